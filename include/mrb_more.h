@@ -1,0 +1,24 @@
+/*
+ * mrb_more.h - entry points of libmrb.so beyond the replacement of the reference's primitives (mrb.h): what this
+ * library's own Python classes need besides. Conventions as in mrb.h; not part of its ABI version.
+ */
+#ifndef MRB_MORE_H_
+#define MRB_MORE_H_
+
+#include <stdint.h>
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* The gradient of mrb_discounted_return: grad_out is the gradient of `out`, grad_reward ([timesteps, batch, inner])
+ * receives the gradient of `reward` and grad_last ([batch, inner], may be NULL) that of `last_value`. With c_t =
+ * (1 - done_t) * gamma it is the same recurrence forwards in time, A_t = grad_out_t + c_{t-1} * A_{t-1} (A_0 = grad_out_0):
+ * grad_reward_t = A_t, grad_last = c_{T-1} * A_{T-1}. One launch; neither waits nor allocates. */
+int mrb_discounted_return_grad(const float *grad_out, const uint8_t *done, float *grad_reward, float *grad_last,
+                               int64_t timesteps, int64_t batch, int64_t inner, float gamma, void *stream);
+
+#ifdef __cplusplus
+}
+#endif
+#endif /* MRB_MORE_H_ */

@@ -68,6 +68,11 @@ SIGNATURES = {
     "mrb_discounted_return": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _f32, _vp],
 }
 
+# the same for include/mrb_more.h
+MORE_SIGNATURES = {
+    "mrb_discounted_return_grad": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _f32, _vp],
+}
+
 _lib = None
 
 
@@ -91,7 +96,7 @@ def lib():
     L = C.CDLL(LIB_PATH)
     L.mrb_last_error.restype = C.c_char_p
     L.mrb_last_error.argtypes = []
-    for name, args in SIGNATURES.items():
+    for name, args in list(SIGNATURES.items()) + list(MORE_SIGNATURES.items()):
         fn = getattr(L, name)
         fn.restype = C.c_int
         fn.argtypes = args

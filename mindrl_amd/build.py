@@ -22,23 +22,45 @@ HIPCC_FLAGS = [
 ]
 
 
+SOURCES = ["mrb.hip", "mrb_returns.hip"]
+
+
 def build(verbose=False):
-    """Compile mindrl_amd/csrc/mrb.hip into mindrl_amd/csrc/libmrb.so. Returns the library path."""
+    """Compile the sources of mindrl_amd/csrc into mindrl_amd/csrc/libmrb.so. Returns the library path."""
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     if not os.path.exists(hipcc):
         hipcc = "hipcc"
     tmp = LIB + ".tmp"
-    cmd = [hipcc] + HIPCC_FLAGS + ["-o", tmp, os.path.join(CSRC, "mrb.hip")]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    flags = [f for f in HIPCC_FLAGS if f != "-shared"]
+    objects = [os.path.join(CSRC, src.replace(".hip", ".o")) for src in SOURCES]
+    commands = [[hipcc] + flags + ["-c", "-o", obj, os.path.join(CSRC, src)] for src, obj in zip(SOURCES, objects)]
+    runs = []
+    for cmd in commands:  # side by side
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        runs.append(subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True))
     noise = "is not a recognized feature for this target"
-    out = "\n".join(l for l in res.stdout.splitlines() if noise not in l)
-    if res.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + out)
-    if verbose and out.strip():
-        print(out)
+
+    def end(run):
+        text = "\n".join(line for line in run.communicate()[0].splitlines() if noise not in line)
+        if run.returncode != 0:
+            raise RuntimeError("hipcc failed:\n" + text)
+        if verbose and text.strip():
+            print(text)
+
+    failures = []
+    for run in runs:
+        try:
+            end(run)
+        except RuntimeError as e:
+            failures.append(str(e))
+    if failures:
+        raise RuntimeError("\n".join(failures))
+    end(subprocess.Popen([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp] + objects, stdout=subprocess.PIPE,
+                         stderr=subprocess.STDOUT, text=True))
     os.replace(tmp, LIB)
+    for obj in objects:
+        os.remove(obj)
     return LIB
 
 

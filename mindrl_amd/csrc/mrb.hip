@@ -16,6 +16,8 @@
 #include <vector>
 
 #include "mrb_kernels.h"
+#include "mrb_returns.h"
+#include "../../include/mrb_more.h"
 
 namespace {
 
@@ -1810,9 +1812,14 @@ int mrb_bench_launch(int kind, void* dst, const void* src, int64_t bytes, void* 
 
 /* ------------------------------------------------------- discounted return */
 
-int mrb_discounted_return(const float* reward, const uint8_t* done, const float* last_value, float* out,
-                          int64_t timesteps, int64_t batch, int64_t inner, float gamma, void* stream) {
-    if (!reward || !done || !last_value || !out) return fail(MRB_EINVAL, "a data pointer is NULL");
+}  // extern "C"
+
+// Both directions of the recurrence (see k_discounted_return): `end_value` is the bootstrap value in or, kBack, its
+// gradient out (may be NULL).
+template <bool kBack>
+static int discounted_return(const float* x, const uint8_t* done, float* end_value, float* out, int64_t timesteps,
+                             int64_t batch, int64_t inner, float gamma, hipStream_t s) {
+    if (!x || !done || (!kBack && !end_value) || !out) return fail(MRB_EINVAL, "a data pointer is NULL");
     if (timesteps <= 0 || batch <= 0 || inner <= 0)
         return fail(MRB_EINVAL, "timesteps %lld, batch %lld, inner %lld must be positive", (long long)timesteps,
                     (long long)batch, (long long)inner);
@@ -1822,19 +1829,30 @@ int mrb_discounted_return(const float* reward, const uint8_t* done, const float*
     if (cols > (1ll << 31) || cols > (1ll << 40) / timesteps)
         return fail(MRB_EINVAL, "%lld columns of %lld steps exceed one call (at most 2^31 columns, 2^40 elements)",
                     (long long)cols, (long long)timesteps);
-    if (cols <= 256 * kDrCols) {
-        // few columns (at most one 64-column tile per compute unit): a thread per column cannot keep
-        // enough loads in flight; stage chunks through LDS
-        hipLaunchKernelGGL(k_discounted_return_tiled, dim3((uint32_t)((cols + kDrCols - 1) / kDrCols)), dim3(kDrWG), 0,
-                           static_cast<hipStream_t>(stream), reward, done, last_value, out, timesteps, batch, inner,
-                           gamma);
-        LAUNCH_CHECK("k_discounted_return_tiled");
+    // A thread per column needs about 65 ns per step however few the columns (a trip to memory per 32 steps) and
+    // streams at up to 6 TB/s when there are many; chunks through LDS need 11 ns per step and stream at 4.8 TB/s.
+    // Measured, us per column / tiled: [1000, 32768] 79 / 61, [1000, 49152] 86 / 94, [250, 32768] 27 / 21, [100, 30001]
+    // 10.7 / 14.3, [100, 16384] 8.5 / 6.8, [20, 16384] 4.1 / 5.1.
+    const bool per_column = cols > 40960 || (cols > 16384 && timesteps <= 128) || (cols > 8192 && timesteps <= 32);
+    if (!per_column) {
+        const hipError_t e = launch_discounted_return_tiled(kBack, x, done, end_value, out, timesteps, batch, inner, gamma, s);
+        if (e != hipSuccess) return fail(MRB_EHIP, "launch k_discounted_return_tiled: %s", hipGetErrorString(e));
         return MRB_OK;
     }
-    hipLaunchKernelGGL(k_discounted_return, dim3(grid_exact((uint64_t)cols)), dim3(kWG), 0,
-                       static_cast<hipStream_t>(stream), reward, done, last_value, out, timesteps, batch, inner, gamma);
+    hipLaunchKernelGGL(k_discounted_return<kBack>, dim3((uint32_t)((cols + kDrWG - 1) / kDrWG)), dim3(kDrWG), 0, s, x, done, end_value, out,
+                       timesteps, batch, inner, gamma);
     LAUNCH_CHECK("k_discounted_return");
     return MRB_OK;
 }
 
+extern "C" {
+
+int mrb_discounted_return(const float* reward, const uint8_t* done, const float* last_value, float* out,
+                          int64_t timesteps, int64_t batch, int64_t inner, float gamma, void* stream) {
+    return discounted_return<false>(reward, done, const_cast<float*>(last_value), out, timesteps, batch, inner, gamma,
+                                    static_cast<hipStream_t>(stream));
+}
+
 }  // extern "C"
+
+#include "mrb_more.inc"

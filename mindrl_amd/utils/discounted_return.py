@@ -18,29 +18,27 @@ def _launch(reward, done, last_value, gamma):
 
 
 class _DiscountedReturnFn(torch.autograd.Function):
-    """Differentiable wrapper. With c_t = (1 - done_t) * gamma the forward recurrence is
-    G_t = R_t + c_t * G_{t+1}; its adjoint runs forwards in time, A_t = dG_t + c_{t-1} * A_{t-1}
-    (A_0 = dG_0), which is the same recurrence on time-reversed inputs, so the same kernel
-    computes it: dR_t = A_t and d(last_state_value) = c_{T-1} * A_{T-1}."""
+    """Differentiable wrapper; the backward pass is one launch (mrb_discounted_return_grad)."""
 
     @staticmethod
     def forward(ctx, reward, done, last_value, gamma):
         ctx.save_for_backward(done)
         ctx.gamma = gamma
+        ctx.last_shape = last_value.shape
         return _launch(reward, done, last_value, gamma)
 
     @staticmethod
     def backward(ctx, grad_out):
         (done,) = ctx.saved_tensors
-        gamma = ctx.gamma
-        g = grad_out.contiguous().flip(0).contiguous()
-        # reversed step s uses c_{T-2-s}; the last reversed step multiplies a zero bootstrap
-        shifted = torch.cat([done[:-1].flip(0), torch.zeros_like(done[:1])], 0).contiguous()
-        zeros = torch.zeros(g.shape[1:], dtype=g.dtype, device=g.device)
-        adj = _launch(g, shifted, zeros, gamma)  # adj[s] = A_{T-1-s}
-        grad_reward = adj.flip(0)
-        keep = (1.0 - done[-1].to(g.dtype)) * gamma
-        grad_last = keep.reshape(keep.shape + (1,) * (adj.dim() - 1 - keep.dim())) * adj[0]
+        g = grad_out.contiguous()
+        timesteps = g.shape[0]
+        batch = done.numel() // timesteps
+        inner = g.numel() // (timesteps * batch)
+        grad_reward = torch.empty_like(g)
+        grad_last = torch.empty(ctx.last_shape, dtype=g.dtype, device=g.device) if ctx.needs_input_grad[2] else None
+        _lib.check(_lib.lib().mrb_discounted_return_grad(
+            g.data_ptr(), done.data_ptr(), grad_reward.data_ptr(), grad_last.data_ptr() if grad_last is not None else None,
+            timesteps, batch, inner, ctx.gamma, stream_ptr()))
         return grad_reward, None, grad_last, None
 
 

@@ -1,0 +1,44 @@
+"""The discounted return and its gradient at the sizes where the tiled kernel's groups and chunks end, and on both sides
+of every line of the dispatch, bit for bit against the oracle's recurrence."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import t2n
+
+pytestmark = pytest.mark.gpu
+
+
+# groups of 16 / 32 / 64 columns and chunks of 64 steps (one short, exact, one over), fewer columns than a quad or a
+# group, several values per environment, the per-column kernel (many columns, or a short time axis)
+SHAPES = [(1, 1, 1), (2, 3, 1), (64, 4, 1), (65, 5, 1), (63, 15, 1), (128, 16, 1), (129, 17, 1), (256, 31, 1), (257, 7, 3),
+          (320, 4096, 1), (70, 4097, 1), (191, 8191, 1), (130, 1400, 3), (128, 8193, 1), (127, 8195, 1), (33, 8200, 1),
+          (32, 8200, 1), (129, 16385, 1), (128, 16385, 1), (3, 40961, 1), (1000, 33, 1)]
+
+
+def oracle_gradient(orc, grad, done, gamma):
+    """A_t = grad_t + c_{t-1} A_{t-1}: the oracle's backward recurrence on time-reversed inputs, flags moved by one."""
+    flags = np.concatenate([done[:-1][::-1], np.zeros_like(done[:1])])
+    a = orc.discounted_return(np.ascontiguousarray(grad[::-1]), np.ascontiguousarray(flags), np.zeros_like(grad[0]), gamma)
+    keep = ((np.float32(1) - done[-1].astype(np.float32)) * np.float32(gamma))[:, None]
+    return a[::-1], keep * a[0]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_return_and_gradient_bit_exact(shape):
+    from mindrl_amd.utils import DiscountedReturn
+    from oracle import orc
+    t, b, inner = shape
+    rng = np.random.default_rng(t * 31 + b)
+    r = rng.normal(size=shape).astype(np.float32)
+    d = rng.random((t, b)) < 0.05
+    v = rng.normal(size=(b, inner)).astype(np.float32)
+    w = rng.normal(size=shape).astype(np.float32)
+    reward = torch.from_numpy(r).cuda().requires_grad_(True)
+    value = torch.from_numpy(v).cuda().requires_grad_(True)
+    out = DiscountedReturn(0.97, need_bprop=True)(reward, torch.from_numpy(d).cuda(), value)
+    assert np.array_equal(t2n(out.detach()), orc.discounted_return(r, d, v, 0.97))
+    grad_reward, grad_value = torch.autograd.grad(out, (reward, value), torch.from_numpy(w).cuda())
+    want_reward, want_value = oracle_gradient(orc, w, d, 0.97)
+    assert np.array_equal(t2n(grad_reward), want_reward)
+    assert np.array_equal(t2n(grad_value), want_value)
