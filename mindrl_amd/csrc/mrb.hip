@@ -580,33 +580,45 @@ int ride_alone_if_large(const UpdateArgs& a, PutArgs& put, hipStream_t s) {
     return MRB_OK;
 }
 
+// A push under at most 16 leaf tiles on a tree with rounds below its top is one launch of one workgroup, a wave per
+// leaf tile (k_push_run; k_tree_fused where an update precedes it in the call): the number of those tiles, 0 where it
+// is not taken. (More than one tile per wave does not pay: the 16 waves of a workgroup share one compute unit's issue
+// slots, and a second tile costs a wave as much as the launch it would save; four cost twice as much.)
+uint32_t run_units(const Per& b, const UpdateArgs& a) {
+    if (a.nrounds == 0 || !b.fused || a.indices) return 0;
+    uint64_t units;
+    if (a.first_slot < 0) {
+        units = push_units(a);  // the slots' start is only known on the device
+    } else {
+        const uint64_t ring_tiles = ((uint64_t)a.capacity + kBlockNodes - 1) / kBlockNodes;
+        const int64_t end = a.first_slot + a.n, first = a.first_slot / kBlockNodes;
+        units = end <= a.capacity ? (uint64_t)((end - 1) / kBlockNodes - first + 1)
+                                  : ring_tiles - first + (uint64_t)((end - a.capacity - 1) / kBlockNodes + 1);
+        if (units > ring_tiles) units = ring_tiles;
+    }
+    return units <= (uint64_t)kRunWaves ? (uint32_t)units : 0u;
+}
+
 // Rebuilds the tree above the leaves that `a` writes: one launch per round, then the top. A push hands
 // its row copy over (`ride`): it is done by extra workgroups of the first launch.
 int tree_rebuild(Per& b, UpdateArgs a, hipStream_t s, const PutArgs* ride = nullptr) {
     PutArgs none{};  // blocks == 0: no copy rides along
-    // One round below the top and at most 16 waves of work (an update: a wave per entry; a push that does
-    // not wrap: a wave per leaf tile under its slots): one launch of one workgroup that goes on to the top.
-    // (More units per wave do not pay: the 16 waves of a workgroup share one compute unit's issue slots, and a
-    // second unit costs a wave as much as the second launch it would save; four cost twice as much.)
-    if (a.nrounds == 1 && b.fused) {
-        uint32_t units = 0, tile_base = 0;
-        if (a.inline_election) {
-            units = (uint32_t)a.n;
-        } else if (!a.indices && a.first_slot < 0) {
-            units = push_units(a);  // the slots' start is only known on the device
-        } else if (!a.indices && a.first_slot + a.n <= a.capacity) {
-            tile_base = (uint32_t)(a.first_slot / kBlockNodes);
-            units = (uint32_t)((a.first_slot + a.n - 1) / kBlockNodes) - tile_base + 1;
-        }
-        if (units > 0 && units <= (uint32_t)(kFusedWG / 64)) {
-            PutArgs put = ride ? *ride : none;
-            if (int rc = ride_alone_if_large(a, put, s)) return rc;
-            put.blocks = (put.blocks + 3) / 4;  // the ride-along copy was sized for workgroups a quarter as large
-            a.readers = 1 + put.blocks;         // (a.advance != 0: this one launch also moves the device's counters on)
-            hipLaunchKernelGGL(k_tree_fused, dim3(1 + put.blocks), dim3(kFusedWG), 0, s, a, tile_base, units, put);
+    if (const uint32_t units = run_units(b, a)) {
+        PutArgs put = ride ? *ride : none;
+        if (int rc = ride_alone_if_large(a, put, s)) return rc;
+        if (a.full_top) {
+            // (the update's launch before this one has carried the row copy)
+            a.readers = 1;
+            hipLaunchKernelGGL(k_tree_fused, dim3(1), dim3(kFusedWG), 0, s, a, (uint32_t)(a.first_slot / kBlockNodes), units);
             LAUNCH_CHECK("k_tree_fused");
             return MRB_OK;
         }
+        const uint32_t threads = units <= kWG / 64 ? (uint32_t)kWG : (uint32_t)kFusedWG;
+        put.blocks = (put.blocks * kWG + threads - 1) / threads;  // the ride-along copy was sized for workgroups of kWG
+        a.readers = 1 + put.blocks;  // (a.advance != 0: this one launch also moves the device's counters on)
+        hipLaunchKernelGGL(k_push_run, dim3(1 + put.blocks), dim3(threads), 0, s, a, units, put);
+        LAUNCH_CHECK("k_push_run");
+        return MRB_OK;
     }
     // A push of at most 1024 rows into a tree of at most 16 levels is one launch: the single workgroup of
     // k_tree_top starts at the leaf level and skips the tiles outside the slot range (such a call is
@@ -1229,16 +1241,19 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
     a.full_top = lead ? 1 : 0;
     // push-then-update: the running max sees every priority of the call, surviving or not, and is
     // raised only after the tree work (a fresh slot with an invalid priority keeps the old running max).
-    // Few rows: the top workgroup scans the priorities itself. More: the leaf-level waves, which compute
-    // every p^alpha anyway, collect their max beside the running max and the top workgroup folds it in.
+    // Few rows on a tree whose leaves the top workgroup rebuilds: it scans the priorities itself. Otherwise the
+    // leaf-level waves, which compute every p^alpha anyway, collect their max beside the running max and the top
+    // workgroup folds it in.
     // Only a call that overwrites rows of its own (more rows than capacity) needs a pass over all priorities.
-    const int fold = !opt_priorities ? 0 : (skip == 0 && nrows <= 1024) ? 1 : (skip == 0 && a.nrounds > 0) ? 2 : 0;
+    a.first_slot = b->device_counters ? -1 : first;
+    a.n = n;
+    const int fold = !opt_priorities ? 0
+                     : (skip == 0 && nrows <= 1024 && !run_units(*b, a)) ? 1
+                     : (skip == 0 && a.nrounds > 0) ? 2 : 0;
     if (opt_priorities) {
         a.priorities = opt_priorities + skip;
         a.fold_max = fold;
     }
-    a.first_slot = b->device_counters ? -1 : first;
-    a.n = n;
     a.advance = b->device_counters ? nrows : 0;  // the call's last launch moves the device's counters on
     const bool stamp_after = opt_priorities && !fold;
     if (!lead && b->fused && nrows == 1 && b->depth <= kPushOneMaxDepth) {
@@ -1373,7 +1388,7 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
     // (2) two launches on a tree with one round of levels below its top: the update's leaf round with the push's
     // row copy riding along, then one workgroup that rebuilds the pushed slots' leaf tiles and the whole top
     if (small_push && b->nrounds == 1 && n <= kElectMax && n > kFusedWG / 64 && b->depth >= 2 &&
-        push_tiles(*b, b->pushes % cap, nrows) <= (uint32_t)(kFusedWG / 64)) {
+        push_tiles(*b, b->pushes % cap, nrows) <= (uint32_t)kRunWaves) {
         int rc = next_epoch(*b, s);
         if (rc) return rc;
         LeadRound lead{update_args(*b)};
@@ -1834,14 +1849,14 @@ static int discounted_return(const float* x, const uint8_t* done, float* end_val
     // Measured, us per column / tiled: [1000, 32768] 79 / 61, [1000, 49152] 86 / 94, [250, 32768] 27 / 21, [100, 30001]
     // 10.7 / 14.3, [100, 16384] 8.5 / 6.8, [20, 16384] 4.1 / 5.1.
     const bool per_column = cols > 40960 || (cols > 16384 && timesteps <= 128) || (cols > 8192 && timesteps <= 32);
-    if (!per_column) {
-        const hipError_t e = launch_discounted_return_tiled(kBack, x, done, end_value, out, timesteps, batch, inner, gamma, s);
-        if (e != hipSuccess) return fail(MRB_EHIP, "launch k_discounted_return_tiled: %s", hipGetErrorString(e));
+    if (per_column) {
+        hipLaunchKernelGGL(k_discounted_return, dim3(grid_exact((uint64_t)cols)), dim3(kWG), 0, s, x, done, end_value, out,
+                           timesteps, batch, inner, gamma, kBack ? 1 : 0);
+        LAUNCH_CHECK("k_discounted_return");
         return MRB_OK;
     }
-    hipLaunchKernelGGL(k_discounted_return<kBack>, dim3((uint32_t)((cols + kDrWG - 1) / kDrWG)), dim3(kDrWG), 0, s, x, done, end_value, out,
-                       timesteps, batch, inner, gamma);
-    LAUNCH_CHECK("k_discounted_return");
+    const hipError_t e = launch_discounted_return_tiled(kBack, x, done, end_value, out, timesteps, batch, inner, gamma, s);
+    if (e != hipSuccess) return fail(MRB_EHIP, "launch k_discounted_return_tiled: %s", hipGetErrorString(e));
     return MRB_OK;
 }
 

@@ -2062,45 +2062,202 @@ __global__ __launch_bounds__(kTopWG) void k_tree_top(UpdateArgs a, PutArgs put) 
 }
 
 // ---------------------------------------------------------------------------
-// A push of few rows, or an update of at most 16 entries, on a tree with one round below the top,
-// in ONE launch: the tile work fits the 16 waves of one workgroup (a wave per leaf tile of a push,
-// or per entry of an update), and the same workgroup goes on to the top after a barrier. Within one
-// workgroup that needs no fence: its waves share a compute unit, and the nodes the top reads were
-// never in that unit's cache before they were written. (Handing the tiles of SEVERAL workgroups to a
-// last one through agent-scope stores, a counter and agent-scope loads was measured too: the three
-// trips through memory cost 2.9 us, more than the second launch they save.)
-//   units      waves with work: entries (update) or leaf tiles from tile_base on (push), at most 16
+// A push under at most 16 leaf tiles on a tree of more than 12 levels, in ONE launch: a run of slots changes one path
+// of tiles - a wave rebuilds each leaf tile, then the tile eight levels up that holds their roots (two where the run
+// crosses its end, one more where it wraps around the ring), then the tile above that, up to the root. Which tiles
+// these are follows from the slots, so all of them are requested when the kernel starts: of their nodes only the
+// lower tiles' roots change, and those reach the wave that holds the tile through LDS. The call is then one trip to
+// memory and two to four rebuilds in a row (within one workgroup, whose waves share a compute unit: no fence), where
+// a launch per eight levels pays a launch, a trip and a rebuild for each. Measured, us per call before and now, plain /
+// with priorities: 64 rows into 2^24 leaves (three launches before) 12.0 / 10.6 and 3.8 / 5.6; 16 rows into 2^20 (one
+// launch that rebuilt the whole top) 4.2 / 6.5 and 3.8 / 5.5; 1024 rows into 2^21 4.8 / 7.4 and 4.3 / 5.9. With 4096
+// priorities the powers of one compute unit are the bound (5.7 / 9.7). The row copy rides along as further workgroups.
+//   units      leaf tiles from the first slot's on, around the ring's end: waves with work
 // ---------------------------------------------------------------------------
 constexpr int kFusedWG = 1024;
+constexpr int kRunWaves = kFusedWG / 64;
+constexpr int kRunLevels = 3;  // tiles above the leaf tiles on a path: trees of at most 8 + 3 * 8 levels
 
-__global__ __launch_bounds__(kFusedWG) void k_tree_fused(UpdateArgs a, uint32_t tile_base, uint32_t units, PutArgs put) {
-    __shared__ unsigned long long s_win[kFusedWG / 64][kBlockNodes];
+__global__ __launch_bounds__(kFusedWG) void k_push_run(UpdateArgs a, uint32_t units, PutArgs put) {
+    __shared__ float s_s[kRunLevels][kRunWaves], s_m[kRunLevels][kRunWaves];
+    __shared__ uint32_t s_new[kRunLevels][kRunWaves];  // whether the wave has a new root for the level above
+    __shared__ float s_largest[kRunWaves];             // the largest leaf of the wave's tile (a push with priorities)
     if (__builtin_expect(blockIdx.x >= 1, 0)) {  // (the tree workgroup's code comes first: it is the one the call waits for)
         rows_put_part(put, blockIdx.x - 1, put.blocks);
         counters_push_done(a.err, a.advance, a.capacity, a.readers);
         rider_ends();
     }
+    const uint32_t lane = threadIdx.x & 63;
+    // (read as a scalar: sixteen waves share the compute unit's issue slots, and what follows from the wave's number
+    // alone - its tiles - then costs them nothing)
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // (a launch that moves the device's counters on: thread 0 takes them now, for the advance at the end)
+    CounterTicket ticket{};
+    if (a.advance > 0 && threadIdx.x == 0) ticket = counters_take(a.err);
+    // (slots and row counts fit 32 bits: the capacity is at most 2^30, the run at most 16 tiles)
+    const uint32_t capacity = (uint32_t)a.capacity, n = (uint32_t)a.n;
+    uint32_t first_slot = (uint32_t)a.first_slot;
+    if (a.first_slot < 0) first_slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)ring_position(counters_behind(a.err), a.capacity));
+    const uint32_t ring_tiles = (capacity + kBlockNodes - 1) / kBlockNodes;  // the ring ends at `capacity`
+    const uint32_t t0 = first_slot / kBlockNodes;
+    auto tile_of = [&](uint32_t unit) -> uint32_t {
+        const uint32_t t = t0 + unit;
+        return t >= ring_tiles ? t - ring_tiles : t;
+    };
+    // of the waves whose leaf tiles lie under one tile l + 1 rounds up the first holds it (the tiles' numbers rise from
+    // wave to wave, and start again from zero where the run wraps)
+    auto holds = [&](uint32_t w, int l) -> bool {
+        const uint32_t up = tile_of(w) >> (8 * (l + 1));
+        return w < units && (w == 0 || (up != tile_of(w - 1) >> (8 * (l + 1)) && up != t0 >> (8 * (l + 1))));
+    };
+    const uint32_t my_tile = tile_of(wave);
+    // The wave's leaf tile, the priorities of its leaves and the running max, all requested before anything is used.
+    const uint32_t leaf = my_tile * kBlockNodes + 4 * lane, leaf_first = (1u << a.depth) + my_tile * kBlockNodes;
+    const bool work = wave < units;  // wave-uniform
+    float4 ls = make_float4(0.f, 0.f, 0.f, 0.f), lm = ls;
+    float old_max = 0.0f, pv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    uint32_t in = 0;  // bit c: the push writes leaf + c
+    if (work) {
+        ls = *reinterpret_cast<const float4*>(a.sum + leaf_first + 4 * lane);
+        lm = *reinterpret_cast<const float4*>(a.mn + leaf_first + 4 * lane);
+        old_max = *a.maxp;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const uint32_t slot = leaf + c, e = slot >= first_slot ? slot - first_slot : slot + capacity - first_slot;
+            if (slot < capacity && e < n) {
+                in |= 1u << c;
+                if (a.priorities) pv[c] = a.priorities[e];
+            }
+        }
+    }
+    // the tiles above
+    float4 vs[kRunLevels], vm[kRunLevels];
+#pragma unroll
+    for (int l = 0; l < kRunLevels; ++l) {
+        const int d = a.depth - kRoundLevels * (l + 1);  // the tile's depth
+        vs[l] = make_float4(0.f, 0.f, 0.f, 0.f);
+        vm[l] = vs[l];
+        if (d <= 0 || !holds(wave, l)) continue;  // wave-uniform
+        if (d == 1) {  // a level of two nodes
+            vs[l].x = a.sum[2], vs[l].y = a.sum[3];
+            vm[l].x = a.mn[2], vm[l].y = a.mn[3];
+        } else if (4 * lane < (1u << d)) {
+            const uint32_t first = (1u << d) + (my_tile >> (8 * (l + 1))) * kBlockNodes + 4 * lane;
+            vs[l] = *reinterpret_cast<const float4*>(a.sum + first);
+            vm[l] = *reinterpret_cast<const float4*>(a.mn + first);
+        }
+    }
+    float rs = 0.0f, rm = 0.0f, largest = 0.0f;
+    const bool changed = work && __any(in != 0);  // (the ring position may be the device's: the last tile may not be met)
+    bool rebuilt = changed;
+    if (changed) {
+        float q[4] = {old_max, old_max, old_max, old_max};
+        if (a.priorities) {
+            const float4 pw = powf_det_x4(make_float4(pv[0], pv[1], pv[2], pv[3]), a.alpha);  // the four together
+            const float p4[4] = {pw.x, pw.y, pw.z, pw.w};
+            bool bad = false;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const bool ok = valid_priority(pv[c]);  // invalid: the fresh slot stays at the running max
+                if (ok) q[c] = p4[c];
+                bad = bad || ((in >> c & 1u) && !ok);
+            }
+            if (bad && a.fold_max) atomicOr(a.err, MRB_DERR_PRIORITY);
+        }
+        if (in & 1u) ls.x = lm.x = q[0];
+        if (in & 2u) ls.y = lm.y = q[1];
+        if (in & 4u) ls.z = lm.z = q[2];
+        if (in & 8u) ls.w = lm.w = q[3];
+        if (in) {
+            *reinterpret_cast<float4*>(a.sum + leaf_first + 4 * lane) = ls;
+            *reinterpret_cast<float4*>(a.mn + leaf_first + 4 * lane) = lm;
+        }
+        // the largest leaf of the tile bounds every p^alpha written here from above, and is itself a p^alpha or a value no
+        // larger than the running max
+        if (a.fold_max) largest = wave_max(fmaxf(fmaxf(ls.x, ls.y), fmaxf(ls.z, ls.w)));
+        tile_parents(a, kRoundLevels, leaf_first, lane, true, ls, lm, &rs, &rm);
+    }
+    if (lane == 0) s_largest[wave] = largest;
+#pragma unroll
+    for (int l = 0; l < kRunLevels; ++l) {
+        const int d = a.depth - kRoundLevels * (l + 1);
+        if (d <= 0) break;  // uniform
+        if (lane == 0) {
+            s_s[l][wave] = rs;
+            s_m[l][wave] = rm;
+            s_new[l][wave] = rebuilt;
+        }
+        lds_barrier();
+        if (l == 0 && a.fold_max && wave == blockDim.x / 64 - 1) {
+            // the running max, by the last wave: every leaf that takes it as it was has been written
+            const float q = wave_max(lane < units ? s_largest[lane] : 0.0f);
+            if (lane == 0 && q > 0.0f) raise_max(a.maxp, q);
+        }
+        rebuilt = false;
+        if (!holds(wave, l)) continue;  // wave-uniform
+        const uint32_t tile0 = (my_tile >> (8 * (l + 1))) * kBlockNodes;  // this tile's first node within its level
+        auto take = [&](uint32_t u, int c) {
+            if (!s_new[l][u]) return;
+            const float ps = s_s[l][u], pm = s_m[l][u];
+            switch (c) {
+                case 0: vs[l].x = ps, vm[l].x = pm; break;
+                case 1: vs[l].y = ps, vm[l].y = pm; break;
+                case 2: vs[l].z = ps, vm[l].z = pm; break;
+                default: vs[l].w = ps, vm[l].w = pm; break;
+            }
+        };
+        if (l == 0) {
+            // the leaf tiles are consecutive: which wave holds a node's follows from the node (all lookups at once)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const uint32_t tile = tile0 + 4 * lane + c;  // the leaf tile under the node
+                const uint32_t u = tile >= t0 ? tile - t0 : tile + ring_tiles - t0;  // (around the ring's end)
+                if (tile < ring_tiles && u < units) take(u, c);
+            }
+        } else {
+            for (uint32_t u = wave; u < units; ++u) {  // scalar: the waves that hold the tiles below (at most three)
+                if (!holds(u, l - 1)) continue;
+                const uint32_t at = (tile_of(u) >> (8 * l)) - tile0;
+                if (at / 4 == lane) take(u, at & 3);
+            }
+        }
+        if (d == 1) {
+            if (lane == 0) {
+                a.sum[1] = vs[l].x + vs[l].y;
+                a.mn[1] = fminf(vm[l].x, vm[l].y);
+            }
+        } else {
+            tile_parents(a, d < kRoundLevels ? d : kRoundLevels, (1u << d) + tile0, lane, 4 * lane < (1u << d), vs[l], vm[l], &rs, &rm);
+            rebuilt = true;
+        }
+    }
+    counters_push_done(a.err, a.advance, a.capacity, a.readers, &ticket);
+}
+
+// ---------------------------------------------------------------------------
+// The second launch of an update and a push as one call (see mrb_per_update_push): the first has written the update's
+// leaf tiles; one workgroup rebuilds the leaf tiles under the pushed slots, a wave each, and the whole top (the update
+// changed nodes anywhere below it).
+//   units      leaf tiles from tile_base on: waves with work, at most 16
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(kFusedWG) void k_tree_fused(UpdateArgs a, uint32_t tile_base, uint32_t units) {
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int top = a.top_depth;
     // (a launch that moves the device's counters on: thread 0 takes them now, for the advance at the end)
     CounterTicket ticket{};
     if (a.advance > 0 && threadIdx.x == 0) ticket = counters_take(a.err);
-    if (!a.inline_election && a.lo[0] == a.depth && a.g[0] == kRoundLevels && top >= kRoundLevels &&
-        (1u << top) / kBlockNodes <= (uint32_t)(kFusedWG / 64)) {
-        // A push: the top's tiles (one per wave) are requested BEFORE the leaf tiles are rebuilt - of all their
-        // nodes only the leaf tiles' roots change, and those reach the waves that hold them through LDS - so the
-        // call has two dependent trips to memory on its path (leaf tiles and top tiles together, then the last
-        // tile) instead of three.
-        __shared__ uint32_t s_root_tile[kFusedWG / 64];
-        __shared__ float s_root_s[kFusedWG / 64], s_root_m[kFusedWG / 64];
-        const uint32_t tiles = (1u << top) / kBlockNodes;
-        uint32_t t_lo = 0, t_hi = tiles - 1;
-        const int64_t first_slot = a.first_slot >= 0 ? a.first_slot : ring_position(counters_behind(a.err), a.capacity);
-        if (!a.full_top && first_slot + a.n <= a.capacity) {
-            t_lo = (uint32_t)(first_slot >> (a.depth - top)) / kBlockNodes;
-            t_hi = (uint32_t)((first_slot + a.n - 1) >> (a.depth - top)) / kBlockNodes;
-        }
-        const bool mine = wave >= t_lo && wave <= t_hi;  // this wave rebuilds the top's tile number `wave`
+    // (device-resident counters: the tiles start at the first slot's tile and wrap around the ring's end)
+    const uint32_t ring_tiles = (uint32_t)((a.capacity + kBlockNodes - 1) / kBlockNodes);
+    const uint32_t tile = a.first_slot >= 0 ? tile_base + wave
+                                            : ((uint32_t)(ring_position(counters_behind(a.err), a.capacity) / kBlockNodes) + wave) % ring_tiles;
+    const uint32_t tiles = (1u << top) / kBlockNodes;
+    if (top >= kRoundLevels && tiles <= (uint32_t)kRunWaves) {
+        // The top's tiles (one per wave) are requested BEFORE the leaf tiles are rebuilt - of all their nodes only the
+        // leaf tiles' roots change, and those reach the waves that hold them through LDS - so the call has two
+        // dependent trips to memory on its path (leaf tiles and top tiles together, then the last tile) instead of three.
+        __shared__ uint32_t s_root_tile[kRunWaves];
+        __shared__ float s_root_s[kRunWaves], s_root_m[kRunWaves];
+        const bool mine = wave < tiles;  // this wave rebuilds the top's tile number `wave`
         const uint32_t top_first = (1u << top) + wave * kBlockNodes;
         float4 tvs = make_float4(0.f, 0.f, 0.f, 0.f), tvm = tvs;
         if (mine) {
@@ -2110,9 +2267,6 @@ __global__ __launch_bounds__(kFusedWG) void k_tree_fused(UpdateArgs a, uint32_t 
         uint32_t leaf_tile = 0xffffffffu;
         float rs = 0.0f, rm = 0.0f;
         if (wave < units) {
-            const uint32_t ring_tiles = (uint32_t)((a.capacity + kBlockNodes - 1) / kBlockNodes);  // the ring ends at `capacity`
-            const uint32_t tile = a.first_slot >= 0 ? tile_base + wave
-                                                    : ((uint32_t)(first_slot / kBlockNodes) + wave) % ring_tiles;
             bool rebuilt = false;
             tile_round(a, a.depth, kRoundLevels, tile, true, nullptr, nullptr, 0, lane, nullptr, &rs, &rm, &rebuilt);
             if (rebuilt) leaf_tile = tile;
@@ -2143,24 +2297,12 @@ __global__ __launch_bounds__(kFusedWG) void k_tree_fused(UpdateArgs a, uint32_t 
             __syncthreads();
             if (wave == 0) tile_round(a, top - kRoundLevels, top - kRoundLevels, 0, false, nullptr, nullptr, 0, lane);
         }
-        if (a.fold_max) fold_push_max(a);
-        counters_push_done(a.err, a.advance, a.capacity, a.readers, &ticket);
-        return;
+    } else {
+        if (wave < units) tile_round(a, a.depth, kRoundLevels, tile, true, nullptr, nullptr, 0, lane);
+        __threadfence_block();  // the tiles' highest nodes, written by other waves of this workgroup, are read below
+        __syncthreads();
+        top_rebuild(a, top, nullptr);
     }
-    if (const uint32_t unit = wave; unit < units) {
-        if (a.inline_election) {
-            entry_tile(a, a.g[0], unit, lane, s_win[wave], nullptr, 0);
-        } else {
-            // (device-resident counters: the tiles start at the first slot's tile and wrap around the level)
-            const uint32_t ring_tiles = (uint32_t)((a.capacity + kBlockNodes - 1) / kBlockNodes);  // the ring ends at `capacity`
-            const uint32_t tile = a.first_slot >= 0 ? tile_base + unit
-                                                    : ((uint32_t)(ring_position(counters_behind(a.err), a.capacity) / kBlockNodes) + unit) % ring_tiles;
-            tile_round(a, a.lo[0], a.g[0], tile, true, nullptr, nullptr, 0, lane);
-        }
-    }
-    __threadfence_block();  // the tiles' highest nodes, written by other waves of this workgroup, are read below
-    __syncthreads();
-    top_rebuild(a, a.top_depth, &s_win[0][0]);
     if (a.fold_max) fold_push_max(a);
     counters_push_done(a.err, a.advance, a.capacity, a.readers, &ticket);
 }
@@ -3399,6 +3541,47 @@ __global__ __launch_bounds__(kWG) void k_tree_paths_push(UpdateArgs a, int64_t s
     __threadfence_block();
     push_one_wave<true>(a.sum, a.mn, a.maxp, slot, a.capacity, a.leaves, a.depth, a.alpha, priority, a.err, threadIdx.x, t,
                         kDev ? a.advance : 0, a.readers);
+}
+
+// The discounted return and its gradient (see mrb_returns.h for the recurrence) of many columns: one thread per (batch,
+// inner) column; neighbouring threads hold neighbouring columns, so every step's loads and stores are coalesced. The
+// loads do not depend on the recurrence, so they are issued UNROLL steps ahead of their use. Step s of the return is
+// time T - 1 - s with that time's flags; of the gradient (`back`) it is time s with the flags of time s - 1 (step 0
+// multiplies a zero: any flag will do). `end_value`: the bootstrap value in, or (back) its gradient out (may be NULL).
+__global__ __launch_bounds__(kWG) void k_discounted_return(const float* __restrict__ x, const uint8_t* __restrict__ done,
+                                                           float* __restrict__ end_value, float* __restrict__ out,
+                                                           int64_t timesteps, int64_t batch, int64_t inner, float gamma,
+                                                           int back) {
+    constexpr int UNROLL = 32;
+    const int64_t cols = batch * inner;
+    const int64_t c = (int64_t)blockIdx.x * kWG + threadIdx.x;
+    if (c >= cols) return;
+    const int64_t b = c / inner;
+    auto time_of = [&](int64_t s) -> int64_t { return back ? s : timesteps - 1 - s; };
+    auto flag_of = [&](int64_t s) -> int64_t { return back ? (s > 0 ? s - 1 : 0) : timesteps - 1 - s; };
+    float last = back ? 0.0f : end_value[c];
+    int64_t s = 0;
+    for (; s + UNROLL <= timesteps; s += UNROLL) {
+        float r[UNROLL];
+        uint32_t d[UNROLL];  // 32-bit: byte-sized register arrays make the compiler pack and unpack them
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            r[u] = __builtin_nontemporal_load(x + time_of(s + u) * cols + c);
+            d[u] = done[flag_of(s + u) * batch + b];
+        }
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            const float scaled = (1.0f - (d[u] ? 1.0f : 0.0f)) * gamma;
+            last = r[u] + scaled * last;
+            __builtin_nontemporal_store(last, out + time_of(s + u) * cols + c);
+        }
+    }
+    for (; s < timesteps; ++s) {
+        const float scaled = (1.0f - (done[flag_of(s) * batch + b] ? 1.0f : 0.0f)) * gamma;
+        last = x[time_of(s) * cols + c] + scaled * last;
+        out[time_of(s) * cols + c] = last;
+    }
+    if (back && end_value) end_value[c] = (1.0f - (done[(timesteps - 1) * batch + b] ? 1.0f : 0.0f)) * gamma * last;
 }
 
 // Device-resident counters (see Counters): after a push, and after a sample that used the generator.

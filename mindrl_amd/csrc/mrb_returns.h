@@ -1,4 +1,5 @@
-// The discounted return's kernels and their gradient's (see mrb_discounted_return, mrb_discounted_return_grad).
+// The discounted return's tiled kernel and its gradient's (see mrb_discounted_return, mrb_discounted_return_grad; the
+// kernel for many columns is k_discounted_return in mrb_kernels.h).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -6,8 +7,6 @@
 #include "mrb_device.h"
 
 namespace mrb {
-
-constexpr int kDrWG = 256;  // threads of the per-column kernel
 
 // ---------------------------------------------------------------------------
 // Discounted return (mindspore_rl/utils/discounted_return.py:84-92) and its gradient. Both are one recurrence over
@@ -23,44 +22,6 @@ template <bool kBack>
 __device__ __forceinline__ int64_t dr_time(int64_t s, int64_t timesteps) { return kBack ? s : timesteps - 1 - s; }
 template <bool kBack>
 __device__ __forceinline__ int64_t dr_flag(int64_t s, int64_t timesteps) { return kBack ? (s > 0 ? s - 1 : 0) : timesteps - 1 - s; }
-
-// Many columns: one thread per column; neighbouring threads hold neighbouring columns, so every step's loads and
-// stores are coalesced. The loads do not depend on the recurrence, so they are issued UNROLL steps ahead of their use.
-// `end_value`: the bootstrap value in, or (kBack) the bootstrap value's gradient out (may be NULL).
-template <bool kBack>
-__global__ __launch_bounds__(kDrWG) void k_discounted_return(const float* __restrict__ x, const uint8_t* __restrict__ done,
-                                                           float* __restrict__ end_value, float* __restrict__ out,
-                                                           int64_t timesteps, int64_t batch, int64_t inner, float gamma) {
-    constexpr int UNROLL = 32;
-    const int64_t cols = batch * inner;
-    const int64_t c = (int64_t)blockIdx.x * kDrWG + threadIdx.x;
-    if (c >= cols) return;
-    const int64_t b = c / inner;
-    float last = kBack ? 0.0f : end_value[c];
-    int64_t s = 0;
-    for (; s + UNROLL <= timesteps; s += UNROLL) {
-        float r[UNROLL];
-        uint32_t d[UNROLL];  // 32-bit: byte-sized register arrays make the compiler pack and unpack them
-#pragma unroll
-        for (int u = 0; u < UNROLL; ++u) {
-            r[u] = __builtin_nontemporal_load(x + dr_time<kBack>(s + u, timesteps) * cols + c);
-            d[u] = done[dr_flag<kBack>(s + u, timesteps) * batch + b];
-        }
-#pragma unroll
-        for (int u = 0; u < UNROLL; ++u) {
-            const float scaled = (1.0f - (d[u] ? 1.0f : 0.0f)) * gamma;
-            last = r[u] + scaled * last;
-            __builtin_nontemporal_store(last, out + dr_time<kBack>(s + u, timesteps) * cols + c);
-        }
-    }
-    for (; s < timesteps; ++s) {
-        const int64_t t = dr_time<kBack>(s, timesteps);
-        const float scaled = (1.0f - (done[dr_flag<kBack>(s, timesteps) * batch + b] ? 1.0f : 0.0f)) * gamma;
-        last = x[t * cols + c] + scaled * last;
-        out[t * cols + c] = last;
-    }
-    if (kBack && end_value) end_value[c] = (1.0f - (done[(timesteps - 1) * batch + b] ? 1.0f : 0.0f)) * gamma * last;
-}
 
 // Fewer columns, where a thread per column leaves the memory system idle: a workgroup takes kCols columns and walks
 // their steps in chunks of kDrChunk through three LDS buffers, as a pipeline whose stages run at the same time on
@@ -292,7 +253,7 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
 }
 
 // Launches k_discounted_return_tiled with the workgroup shape that fits the number of columns (defined in
-// mrb_returns.hip). `x` .. `out` as in k_discounted_return.
+// mrb_returns.hip). `end_value`: the bootstrap value in, or (back) the bootstrap value's gradient out (may be NULL).
 hipError_t launch_discounted_return_tiled(bool back, const float* x, const uint8_t* done, float* end_value, float* out,
                                           int64_t timesteps, int64_t batch, int64_t inner, float gamma, hipStream_t s);
 
