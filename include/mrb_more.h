@@ -18,6 +18,15 @@ extern "C" {
 int mrb_discounted_return_grad(const float *grad_out, const uint8_t *done, float *grad_reward, float *grad_last,
                                int64_t timesteps, int64_t batch, int64_t inner, float gamma, void *stream);
 
+/* Staging memory for rows that lie in host memory: `bytes` (at most 512 KiB) of page-locked memory of buffer `h` (any
+ * kind), which the caller fills and hands to the handle's next push or append on `stream` as if it were device memory:
+ * the kernels read it where it is. Valid for that one call. The memory, 2 MiB per buffer that is pushed host rows, is
+ * allocated by the first call (no device memory) and freed with the buffer; it is handed out in turn, and a call that
+ * comes around to memory given out before waits for the work that read it (calls that change one handle are ordered,
+ * so an event on the stream of the call that moves on covers them all). Refused (MRB_ESTATE) while `stream` is
+ * recorded into a HIP graph. */
+int mrb_stage(int64_t h, int64_t bytes, void **ptr, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -71,9 +71,11 @@ SIGNATURES = {
 # the same for include/mrb_more.h
 MORE_SIGNATURES = {
     "mrb_discounted_return_grad": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _f32, _vp],
+    "mrb_stage": [_i64, _i64, _pvp, _vp],
 }
 
 _lib = None
+_native = None
 
 
 class MrbError(RuntimeError):
@@ -105,6 +107,21 @@ def lib():
                            "`python -m mindrl_amd.build`" % (L.mrb_version(), ABI_VERSION))
     _lib = L
     return L
+
+
+def native():
+    """The extension module mindrl_amd._native (the host side of the buffer classes' calls; csrc/native.cpp), loaded
+    once. Raises if it has not been built."""
+    global _native
+    if _native is None:
+        lib()  # the C ABI it calls
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise RuntimeError("the extension mindrl_amd._native does not load (%s): build it with `python -m "
+                               "mindrl_amd.build`" % e)
+        _native = module
+    return _native
 
 
 def check(rc):

@@ -144,20 +144,23 @@ class FieldLayout:
                 raise ValueError("fields disagree on the number of rows (%d vs %d)" % (n, rows))
         return n
 
-    def rows_if_ready(self, fields, dev):
-        """Number of rows when `fields` already are contiguous device tensors of the declared dtypes holding
-        whole elements (the training path: nothing to convert, one pass), else None."""
-        if len(fields) != len(self.numel):
-            return None
-        n = -1
-        for f, d, numel in zip(fields, self.dtypes, self.numel):
-            if not (isinstance(f, torch.Tensor) and f.dtype == d and f.device == dev and f.is_contiguous()):
-                return None
-            rows, rest = divmod(f.numel(), numel)
-            if rest or (n >= 0 and rows != n):
-                return None
-            n = rows
-        return n
+    def native(self, handle, dev):
+        """The native host side of buffer `handle`'s calls (csrc/native.cpp)."""
+        return _lib.native().Rows(handle, tuple(self.shapes), tuple(self.dtypes), dev.index, _lib.check)
+
+    def put(self, call, fields, dev):
+        """call(fields), a native method that takes rows, for fields it has not taken as they were: converted to the
+        declared dtypes where they lie (host rows pass through the buffer's staging memory), or - where that does not
+        fit the staging memory - as device tensors. Returns the fields that were taken."""
+        self.batch_of(fields)  # raises where the fields are not whole, matching rows
+        fields = [as_tensor(f) for f in fields]
+        fields = [f.to(dtype=d).contiguous() if f.device.type == "cpu" else f.to(device=dev, dtype=d).contiguous()
+                  for f, d in zip(fields, self.dtypes)]
+        if call(fields) is None:
+            fields = self.to_device(fields, dev)
+            if call(fields) is None:
+                raise RuntimeError("rows were refused")
+        return fields
 
     def to_device(self, fields, dev):
         """Contiguous device tensors of the declared dtypes (copies host data if needed)."""

@@ -46,23 +46,50 @@ class PriorityReplayBuffer:
         create_with_layout(packed_rows, lambda: _lib.check(_lib.lib().mrb_per_create(
             self._capacity, self._alpha, len(self._layout), self._layout.c_bytes, seed & (2**64 - 1), C.byref(h))))
         self._h = h.value
+        self._native = self._layout.native(self._h, self._dev)
         self._handle = torch.tensor([self._h], dtype=torch.int64)
         self._keep = None
         self._ring_size = int(output_ring)
         self._ring, self._ring_at = None, 0  # output sets, built by the first sample()
 
     def _next_outputs(self):
-        """The next preallocated (indices, weights, fields, field pointer array) set."""
+        """The next preallocated (indices, weights, fields) set."""
         if self._ring is None:
             n = self._sample_size
-            self._ring = []
-            for _ in range(self._ring_size):
-                fields = self._layout.empty(n, self._dev)
-                self._ring.append((torch.empty(n, dtype=torch.int64, device=self._dev),
-                                   torch.empty(n, dtype=torch.float32, device=self._dev), fields, pointers(fields)))
+            self._ring = [(torch.empty(n, dtype=torch.int64, device=self._dev),
+                           torch.empty(n, dtype=torch.float32, device=self._dev), self._layout.empty(n, self._dev))
+                          for _ in range(self._ring_size)]
         out = self._ring[self._ring_at]
         self._ring_at = (self._ring_at + 1) % self._ring_size
         return out
+
+    def _outputs(self, out):
+        """Where a sample goes that is not to fresh tensors: (indices, weights, [fields]), or None."""
+        if out is not None:
+            idx, w, fields = out
+            return idx, w, self._layout.check_out(fields, self._sample_size, self._dev)
+        return self._next_outputs() if self._ring_size > 0 else None
+
+    def _uniforms(self, uniforms, n, what):
+        u = flat_on_device(uniforms, torch.float32, self._dev)
+        if u.numel() != n:
+            raise ValueError("uniforms must hold %s values" % what)
+        return u
+
+    def _entries(self, indices, priorities):
+        idx = flat_on_device(indices, torch.int64, self._dev)
+        pr = flat_on_device(priorities, torch.float32, self._dev)
+        if idx.numel() != pr.numel():
+            raise ValueError("indices and priorities differ in length")
+        return idx, pr
+
+    def _row_priorities(self, priorities, rows, name):
+        if priorities is None:
+            return None
+        pr = flat_on_device(priorities, torch.float32, self._dev)
+        if pr.numel() != self._layout.batch_of(rows):
+            raise ValueError("%s must hold one value per pushed row" % name)
+        return pr
 
     # -- reference methods ---------------------------------------------------
     def insert(self, *transition, priorities=None):
@@ -73,20 +100,10 @@ class PriorityReplayBuffer:
         tensor int64[1]."""
         if len(transition) == 1 and isinstance(transition[0], (list, tuple)):
             transition = tuple(transition[0])
-        n = self._layout.rows_if_ready(transition, self._dev)
-        if n is not None:
-            src = transition
-        else:
-            n = self._layout.batch_of(transition)
-            src = self._layout.to_device(transition, self._dev)
-        pr = None
-        if priorities is not None:
-            pr = flat_on_device(priorities, torch.float32, self._dev)
-            if pr.numel() != n:
-                raise ValueError("priorities must hold one value per pushed row")
-        _lib.check(_lib.lib().mrb_per_push(self._h, pointers(src), n, pr.data_ptr() if pr is not None else None,
-                                           stream_ptr()))
-        self._keep = (src, pr)
+        if self._native.per_push(transition, priorities) is None:
+            priorities = self._row_priorities(priorities, transition, "priorities")
+            transition = self._layout.put(lambda rows: self._native.per_push(rows, priorities), transition, self._dev)
+        self._keep = (transition, priorities)
         return self._handle
 
     # the reference's own test calls the method by this name (tests/st/test_priority_replay_buffer.py:46)
@@ -103,26 +120,20 @@ class PriorityReplayBuffer:
         `output_ring` > 0: then it comes from that ring of preallocated output sets and stays valid
         until `output_ring` further sample() calls have been made."""
         n = self._sample_size
-        u = None
-        if uniforms is not None:
-            u = flat_on_device(uniforms, torch.float32, self._dev)
-            if u.numel() != n:
-                raise ValueError("uniforms must hold sample_size = %d values" % n)
-        if out is not None:
-            idx, w, fields = out
-            fields = self._layout.check_out(fields, n, self._dev)
-            fptr = pointers(fields)
-        elif self._ring_size > 0:
-            idx, w, fields, fptr = self._next_outputs()
+        given = self._outputs(out)
+        if given is None:
+            res = self._native.per_sample(n, beta, uniforms)
+            if res is None:
+                uniforms = self._uniforms(uniforms, n, "sample_size = %d" % n)
+                res = self._native.per_sample(n, beta, uniforms)
         else:
-            idx = torch.empty(n, dtype=torch.int64, device=self._dev)
-            w = torch.empty(n, dtype=torch.float32, device=self._dev)
-            fields = self._layout.empty(n, self._dev)
-            fptr = pointers(fields)
-        _lib.check(_lib.lib().mrb_per_sample(self._h, n, float(beta), u.data_ptr() if u is not None else None,
-                                             idx.data_ptr(), w.data_ptr(), fptr, stream_ptr()))
-        self._keep = u
-        return (idx, w) + tuple(fields)
+            if uniforms is not None:
+                uniforms = self._uniforms(uniforms, n, "sample_size = %d" % n)
+            if self._native.per_sample_into(n, beta, uniforms, *given) is None:
+                raise ValueError("out must hold contiguous int64 indices, float32 weights and the fields on %s" % self._dev)
+            res = (given[0], given[1]) + tuple(given[2])
+        self._keep = uniforms
+        return res
 
     def sample_with_next(self, beta, slot_field, row_field, uniforms=None):
         """sample(beta) plus, in the same launch, field `row_field` of the row whose slot number each sampled
@@ -134,21 +145,12 @@ class PriorityReplayBuffer:
         slot_field, row_field = int(slot_field), int(row_field)
         if not 0 <= slot_field < len(self._layout) or not 0 <= row_field < len(self._layout):
             raise ValueError("slot_field and row_field must name fields of the transition")
-        u = None
-        if uniforms is not None:
-            u = flat_on_device(uniforms, torch.float32, self._dev)
-            if u.numel() != n:
-                raise ValueError("uniforms must hold sample_size = %d values" % n)
-        idx = torch.empty(n, dtype=torch.int64, device=self._dev)
-        w = torch.empty(n, dtype=torch.float32, device=self._dev)
-        fields = self._layout.empty(n, self._dev)
-        nxt = torch.empty((n,) + tuple(self._layout.shapes[row_field]), dtype=self._layout.dtypes[row_field],
-                          device=self._dev)
-        _lib.check(_lib.lib().mrb_per_sample_next(self._h, n, float(beta), u.data_ptr() if u is not None else None,
-                                                  slot_field, row_field, idx.data_ptr(), w.data_ptr(),
-                                                  pointers(fields), nxt.data_ptr(), stream_ptr()))
-        self._keep = u
-        return (idx, w) + tuple(fields) + (nxt,)
+        res = self._native.per_sample_next(n, beta, uniforms, slot_field, row_field)
+        if res is None:
+            uniforms = self._uniforms(uniforms, n, "sample_size = %d" % n)
+            res = self._native.per_sample_next(n, beta, uniforms, slot_field, row_field)
+        self._keep = uniforms
+        return res
 
     def sample_many(self, nbatch, beta, uniforms=None):
         """`nbatch` batches in one launch: what `nbatch` successive sample(beta) calls would return on an
@@ -156,29 +158,20 @@ class PriorityReplayBuffer:
         [nbatch, B, *shape_i]). For learners that draw several batches between priority updates; one launch
         amortises the launch and the tree descent. `uniforms`: f32[nbatch, B] or None (generator)."""
         nbatch, n = int(nbatch), self._sample_size
-        u = None
-        if uniforms is not None:
-            u = flat_on_device(uniforms, torch.float32, self._dev)
-            if u.numel() != nbatch * n:
-                raise ValueError("uniforms must hold nbatch * sample_size = %d values" % (nbatch * n))
-        idx = torch.empty((nbatch, n), dtype=torch.int64, device=self._dev)
-        w = torch.empty((nbatch, n), dtype=torch.float32, device=self._dev)
-        fields = [torch.empty((nbatch, n) + s, dtype=d, device=self._dev)
-                  for s, d in zip(self._layout.shapes, self._layout.dtypes)]
-        _lib.check(_lib.lib().mrb_per_sample_many(self._h, nbatch, n, float(beta), u.data_ptr() if u is not None else None,
-                                                  idx.data_ptr(), w.data_ptr(), pointers(fields), stream_ptr()))
-        self._keep = u
-        return (idx, w) + tuple(fields)
+        res = self._native.per_sample_many(nbatch, n, beta, uniforms)
+        if res is None:
+            uniforms = self._uniforms(uniforms, nbatch * n, "nbatch * sample_size = %d" % (nbatch * n))
+            res = self._native.per_sample_many(nbatch, n, beta, uniforms)
+        self._keep = uniforms
+        return res
 
     def update_priorities(self, indices, priorities):
         """leaf[indices[j]] = priorities[j] ** alpha in order, last write wins
         (priority_replay_buffer.py:108-120). Returns the handle tensor."""
-        idx = flat_on_device(indices, torch.int64, self._dev)
-        pr = flat_on_device(priorities, torch.float32, self._dev)
-        if idx.numel() != pr.numel():
-            raise ValueError("indices and priorities differ in length")
-        _lib.check(_lib.lib().mrb_per_update(self._h, idx.data_ptr(), pr.data_ptr(), idx.numel(), stream_ptr()))
-        self._keep = (idx, pr)
+        if self._native.per_update(indices, priorities) is None:
+            indices, priorities = self._entries(indices, priorities)
+            self._native.per_update(indices, priorities)
+        self._keep = (indices, priorities)
         return self._handle
 
     def update_priorities_and_insert(self, indices, priorities, *transition, insert_priorities=None):
@@ -186,26 +179,14 @@ class PriorityReplayBuffer:
         as ONE library call (mrb_per_update_push): the result is the two calls', bit for bit, with fewer kernel
         launches - a learner's step is bound by them (the reference's loop issues the two back to back,
         mindspore_rl/algorithm/dqn/dqn_trainer.py:76-87). Returns the handle tensor."""
-        idx = flat_on_device(indices, torch.int64, self._dev)
-        pr = flat_on_device(priorities, torch.float32, self._dev)
-        if idx.numel() != pr.numel():
-            raise ValueError("indices and priorities differ in length")
         if len(transition) == 1 and isinstance(transition[0], (list, tuple)):
             transition = tuple(transition[0])
-        n = self._layout.rows_if_ready(transition, self._dev)
-        if n is not None:
-            src = transition
-        else:
-            n = self._layout.batch_of(transition)
-            src = self._layout.to_device(transition, self._dev)
-        ipr = None
-        if insert_priorities is not None:
-            ipr = flat_on_device(insert_priorities, torch.float32, self._dev)
-            if ipr.numel() != n:
-                raise ValueError("insert_priorities must hold one value per pushed row")
-        _lib.check(_lib.lib().mrb_per_update_push(self._h, idx.data_ptr(), pr.data_ptr(), idx.numel(), pointers(src), n,
-                                                  ipr.data_ptr() if ipr is not None else None, stream_ptr()))
-        self._keep = (idx, pr, src, ipr)
+        if self._native.per_update_push(indices, priorities, transition, insert_priorities) is None:
+            indices, priorities = self._entries(indices, priorities)
+            ipr = insert_priorities = self._row_priorities(insert_priorities, transition, "insert_priorities")
+            transition = self._layout.put(lambda rows: self._native.per_update_push(indices, priorities, rows, ipr),
+                                          transition, self._dev)
+        self._keep = (indices, priorities, transition, insert_priorities)
         return self._handle
 
     def update_priorities_insert_and_sample(self, indices, priorities, *transition, beta, insert_priorities=None,
@@ -216,54 +197,42 @@ class PriorityReplayBuffer:
         are the three calls', bit for bit; on a small buffer (capacity up to 16,384, up to 384 entries, one
         transition, up to 512 sampled rows) they take one kernel launch instead of two or three. Returns what
         sample() returns."""
-        idx = flat_on_device(indices, torch.int64, self._dev)
-        pr = flat_on_device(priorities, torch.float32, self._dev)
-        if idx.numel() != pr.numel():
-            raise ValueError("indices and priorities differ in length")
         if len(transition) == 1 and isinstance(transition[0], (list, tuple)):
             transition = tuple(transition[0])
-        n = self._layout.rows_if_ready(transition, self._dev)
-        if n is not None:
-            src = transition
-        else:
-            n = self._layout.batch_of(transition)
-            src = self._layout.to_device(transition, self._dev)
-        ipr = None
-        if insert_priorities is not None:
-            ipr = flat_on_device(insert_priorities, torch.float32, self._dev)
-            if ipr.numel() != n:
-                raise ValueError("insert_priorities must hold one value per pushed row")
         b = self._sample_size
-        u = None
-        if uniforms is not None:
-            u = flat_on_device(uniforms, torch.float32, self._dev)
-            if u.numel() != b:
-                raise ValueError("uniforms must hold sample_size = %d values" % b)
-        if out is not None:
-            oidx, w, fields = out
-            fields = self._layout.check_out(fields, b, self._dev)
-            fptr = pointers(fields)
-        elif self._ring_size > 0:
-            oidx, w, fields, fptr = self._next_outputs()
-        else:
-            oidx = torch.empty(b, dtype=torch.int64, device=self._dev)
-            w = torch.empty(b, dtype=torch.float32, device=self._dev)
-            fields = self._layout.empty(b, self._dev)
-            fptr = pointers(fields)
-        _lib.check(_lib.lib().mrb_per_update_push_sample(
-            self._h, idx.data_ptr(), pr.data_ptr(), idx.numel(), pointers(src), n,
-            ipr.data_ptr() if ipr is not None else None, b, float(beta), u.data_ptr() if u is not None else None,
-            oidx.data_ptr(), w.data_ptr(), fptr, stream_ptr()))
-        self._keep = (idx, pr, src, ipr, u)
-        return (oidx, w) + tuple(fields)
+        given = self._outputs(out)
+        res = self._native.per_step(indices, priorities, transition, insert_priorities, b, beta, uniforms, given)
+        if res is None:
+            indices, priorities = self._entries(indices, priorities)
+            ipr = insert_priorities = self._row_priorities(insert_priorities, transition, "insert_priorities")
+            if uniforms is not None:
+                uniforms = self._uniforms(uniforms, b, "sample_size = %d" % b)
+            results = []
+
+            def step(rows):
+                r = self._native.per_step(indices, priorities, rows, ipr, b, beta, uniforms, given)
+                results.append(r)
+                return r
+
+            transition = self._layout.put(step, transition, self._dev)
+            res = results[-1]
+        self._keep = (indices, priorities, transition, insert_priorities, uniforms)
+        return res if given is None else (given[0], given[1]) + tuple(given[2])
 
     def gather(self, indices, out=None):
         """Rows at the given slots (int64, each in [0, size)): one [n, *shape_i] tensor per field.
         For transitions that store the slot of their successor instead of a copy of it, e.g.
         `next_rows = buf.gather(sampled_next_idx)`."""
+        if out is None:
+            res = self._native.per_gather(indices)
+            if res is None:
+                indices = flat_on_device(indices, torch.int64, self._dev)
+                res = self._native.per_gather(indices)
+            self._keep = indices
+            return res
         idx = flat_on_device(indices, torch.int64, self._dev)
         n = idx.numel()
-        dst = self._layout.check_out(out, n, self._dev) if out is not None else self._layout.empty(n, self._dev)
+        dst = self._layout.check_out(out, n, self._dev)
         _lib.check(_lib.lib().mrb_per_gather(self._h, idx.data_ptr(), n, pointers(dst), stream_ptr()))
         self._keep = idx
         return tuple(dst)

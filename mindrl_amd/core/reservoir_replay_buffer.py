@@ -6,8 +6,8 @@ import os
 import torch
 
 from .. import _lib
-from ._rows import (FieldLayout, create_with_layout, device, get_counters, load_fields, pointers, save_fields,
-                    set_counters, storage_views, stream_ptr)
+from ._rows import (FieldLayout, create_with_layout, device, get_counters, load_fields, save_fields,
+                    set_counters, storage_views)
 
 
 class ReservoirReplayBuffer:
@@ -35,6 +35,7 @@ class ReservoirReplayBuffer:
         create_with_layout(packed_rows, lambda: _lib.check(_lib.lib().mrb_res_create(
             self._capacity, len(self._layout), self._layout.c_bytes, seed & (2**64 - 1), C.byref(h))))
         self._h = h.value
+        self._native = self._layout.native(self._h, self._dev)
         self._handle = torch.tensor([self._h], dtype=torch.int64)
         self._keep = None
 
@@ -43,22 +44,16 @@ class ReservoirReplayBuffer:
         (reservoir_replay_buffer.py:68-79). Returns the handle tensor int64[1]."""
         if len(transition) == 1 and isinstance(transition[0], (list, tuple)):
             transition = tuple(transition[0])
-        n = self._layout.batch_of(transition)
-        src = self._layout.to_device(transition, self._dev)
-        _lib.check(_lib.lib().mrb_res_push(self._h, pointers(src), n, stream_ptr()))
-        self._keep = src
+        if self._native.res_push(transition) is None:
+            transition = self._layout.put(self._native.res_push, transition, self._dev)
+        self._keep = transition
         return self._handle
 
     insert = push
 
     def sample(self, with_indices=False):
         """`sample_size` rows drawn uniformly with replacement (reservoir_replay_buffer.py:81-89)."""
-        n = self._sample_size
-        dst = self._layout.empty(n, self._dev)
-        idx = torch.empty(n, dtype=torch.int64, device=self._dev) if with_indices else None
-        _lib.check(_lib.lib().mrb_res_sample(self._h, n, idx.data_ptr() if with_indices else None, pointers(dst),
-                                             stream_ptr()))
-        return (idx, tuple(dst)) if with_indices else tuple(dst)
+        return self._native.res_sample(self._sample_size, bool(with_indices))
 
     def destroy(self):
         """Releases the native buffer (reservoir_replay_buffer.py:91-100)."""

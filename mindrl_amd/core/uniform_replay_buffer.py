@@ -6,8 +6,8 @@ import numpy as np
 import torch
 
 from .. import _lib
-from ._rows import (FieldLayout, create_with_layout, device, get_counters, load_fields, pointers, save_fields,
-                    set_counters, storage_views, stream_ptr)
+from ._rows import (FieldLayout, create_with_layout, device, flat_on_device, get_counters, load_fields, pointers,
+                    save_fields, set_counters, storage_views, stream_ptr)
 
 
 class _BufferAppend:
@@ -72,6 +72,7 @@ class UniformReplayBuffer:
         create_with_layout(packed_rows, lambda: _lib.check(_lib.lib().mrb_urb_create(
             self._capacity, len(self._layout), self._layout.c_bytes, C.byref(h))))
         self._h = h.value
+        self._native = self._layout.native(self._h, self._dev)
         _lib.check(_lib.lib().mrb_urb_seed(self._h, int(seed) & (2**64 - 1)))
         self.buffer = storage_views(self._h, self._layout, self._capacity, self, self._dev)
         # Attributes that subclasses and callers of the reference class reach into: the append and sample
@@ -87,10 +88,9 @@ class UniformReplayBuffer:
         """Appends one element (tensors of shape_i) or a batch ([n, *shape_i]); FIFO
         replacement when full. Returns the whole buffer, as the reference does
         (uniform_replay_buffer.py:101-115)."""
-        n = self._layout.batch_of(exp)
-        src = self._layout.to_device(exp, self._dev)
-        _lib.check(_lib.lib().mrb_urb_append(self._h, pointers(src), n, stream_ptr()))
-        self._keep = src  # alive until the next call on this stream-ordered buffer
+        if self._native.urb_append(exp) is None:
+            exp = self._layout.put(self._native.urb_append, exp, self._dev)
+        self._keep = exp  # alive until the next call on this stream-ordered buffer
         return self.buffer
 
     def get_item(self, index):
@@ -106,23 +106,23 @@ class UniformReplayBuffer:
         instead of the buffer's generator (its length sets the batch)."""
         if indices is None:
             n = self._sample_size
-            dst = self._layout.check_out(out, n, self._dev) if out is not None else self._layout.empty(n, self._dev)
+            if out is None:
+                return self._native.urb_sample(n, False)
+            dst = self._layout.check_out(out, n, self._dev)
             _lib.check(_lib.lib().mrb_urb_sample(self._h, n, None, pointers(dst), stream_ptr()))
             return tuple(dst)
-        idx = torch.as_tensor(indices).to(device=self._dev, dtype=torch.int64).contiguous().reshape(-1)
-        n = idx.numel()
-        dst = self._layout.check_out(out, n, self._dev) if out is not None else self._layout.empty(n, self._dev)
-        _lib.check(_lib.lib().mrb_urb_gather(self._h, idx.data_ptr(), n, pointers(dst), stream_ptr()))
+        idx = flat_on_device(indices, torch.int64, self._dev)
         self._keep = idx
+        if out is None:
+            return self._native.urb_gather(idx)
+        n = idx.numel()
+        dst = self._layout.check_out(out, n, self._dev)
+        _lib.check(_lib.lib().mrb_urb_gather(self._h, idx.data_ptr(), n, pointers(dst), stream_ptr()))
         return tuple(dst)
 
     def sample_with_indices(self):
         """As sample(), also returning the drawn slots (int64[sample_size])."""
-        n = self._sample_size
-        dst = self._layout.empty(n, self._dev)
-        idx = torch.empty(n, dtype=torch.int64, device=self._dev)
-        _lib.check(_lib.lib().mrb_urb_sample(self._h, n, idx.data_ptr(), pointers(dst), stream_ptr()))
-        return idx, tuple(dst)
+        return self._native.urb_sample(self._sample_size, True)
 
     def reset(self):
         """count = 0; head is left as it is (uniform_replay_buffer.py:141-150)."""

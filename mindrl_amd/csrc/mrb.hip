@@ -45,6 +45,22 @@ int fail(int code, const char* fmt, ...) {
         if (e_ != hipSuccess) return fail(MRB_EHIP, "launch %s: %s", name, hipGetErrorString(e_)); \
     } while (0)
 
+// Page-locked memory that host rows pass through (mrb_stage): four segments taken in turn.
+constexpr int kStageSegments = 4;
+constexpr int64_t kStageSegment = 512 << 10;
+struct Stage {
+    char* memory = nullptr;
+    int segment = 0;   // the one in use,
+    int64_t at = 0;    // and its first free byte
+    hipEvent_t left[kStageSegments] = {};    // recorded on the stream when a segment was left
+    bool was_left[kStageSegments] = {};
+    ~Stage() {
+        for (auto e : left)
+            if (e) (void)hipEventDestroy(e);
+        if (memory) (void)hipHostFree(memory);
+    }
+};
+
 // Row storage. By default a structure of arrays, field i = [capacity, bytes_i] (reference layout:
 // mindspore_rl/core/uniform_replay_buffer.py:26-47). With the library option "packed_rows" narrow rows are kept
 // packed instead: one [capacity, row_stride] allocation, field i at byte offset_i of every row (each field
@@ -62,6 +78,7 @@ struct RowStore {
     int64_t row_split = 0;  // option "row_split": least number of workgroups per row in the wide-row kernel (0 = auto)
     int64_t row_wave = 0;   // option "row_wave": the wave-per-row sample kernel, 0 = for launches of many rows, 1 = whenever
                             // the rows fit it, 2 = never
+    Stage stage;
 
     ~RowStore() {
         if (packed_base) {
