@@ -64,7 +64,7 @@ struct Stage {
 // Row storage. By default a structure of arrays, field i = [capacity, bytes_i] (reference layout:
 // mindspore_rl/core/uniform_replay_buffer.py:26-47). With the library option "packed_rows" narrow rows are kept
 // packed instead: one [capacity, row_stride] allocation, field i at byte offset_i of every row (each field
-// aligned to its own copy granule), so that a sampled row's fields share cache lines instead of costing one
+// aligned as its size allows), so that a sampled row's fields share cache lines instead of costing one
 // 128-byte line per field. Either way row r of field i starts at data[i] + r * stride[i].
 struct RowStore {
     int64_t capacity = 0;
@@ -73,7 +73,9 @@ struct RowStore {
     int64_t stride[MRB_MAX_FIELDS] = {};
     uint8_t* data[MRB_MAX_FIELDS] = {};
     uint8_t* packed_base = nullptr;  // packed rows: the one allocation (data[i] point into it)
-    uint32_t vec_log2[MRB_MAX_FIELDS] = {};
+    uint32_t align_log2[MRB_MAX_FIELDS] = {};  // log2 of what a row's size is a multiple of, at most 16: the alignment asked
+                                              // of the caller's matrices, and a field's in a packed row
+    uint32_t vec_log2[MRB_MAX_FIELDS] = {};    // copy granule and granules of a row (see granule_offset)
     uint32_t units[MRB_MAX_FIELDS] = {};
     int64_t row_split = 0;  // option "row_split": least number of workgroups per row in the wide-row kernel (0 = auto)
     int64_t row_wave = 0;   // option "row_wave": the wave-per-row sample kernel, 0 = for launches of many rows, 1 = whenever
@@ -107,9 +109,12 @@ int rows_alloc(RowStore& r, int64_t capacity, int nfields, const int64_t* field_
         r.bytes[i] = field_bytes[i];
         uint32_t vl = 4;
         while (vl > 0 && (field_bytes[i] & ((1ll << vl) - 1))) --vl;
-        r.vec_log2[i] = vl;
-        r.units[i] = (uint32_t)(field_bytes[i] >> vl);
-        // where the field would lie in a packed row: at the next multiple of its own copy granule
+        r.align_log2[i] = vl;
+        uint32_t copy = 4;
+        while ((1ll << copy) > field_bytes[i]) --copy;
+        r.vec_log2[i] = copy;
+        r.units[i] = (uint32_t)((field_bytes[i] + (1ll << copy) - 1) >> copy);
+        // where the field would lie in a packed row: at the next multiple of its own alignment
         const int64_t g = 1ll << vl;
         offset[i] = (end + g - 1) / g * g;
         end = offset[i] + field_bytes[i];
@@ -137,15 +142,15 @@ int rows_alloc(RowStore& r, int64_t capacity, int nfields, const int64_t* field_
     return MRB_OK;
 }
 
-// Builds the per-call field table. `io` pointers must honour each field's copy granule.
+// Builds the per-call field table. `io` pointers must be aligned as each field's row size allows.
 int make_table(const RowStore& r, const void* const* io, int64_t n, IoTable& t) {
     if (!io) return fail(MRB_EINVAL, "field pointer array is NULL");
     t.nfields = r.nfields;
     t.prefix[0] = 0;
     for (int i = 0; i < r.nfields; ++i) {
         if (!io[i]) return fail(MRB_EINVAL, "field %d pointer is NULL", i);
-        if (reinterpret_cast<uintptr_t>(io[i]) & ((1u << r.vec_log2[i]) - 1))
-            return fail(MRB_EINVAL, "field %d pointer %p is not %u-byte aligned", i, io[i], 1u << r.vec_log2[i]);
+        if (reinterpret_cast<uintptr_t>(io[i]) & ((1u << r.align_log2[i]) - 1))
+            return fail(MRB_EINVAL, "field %d pointer %p is not %u-byte aligned", i, io[i], 1u << r.align_log2[i]);
         t.store[i] = r.data[i];
         t.io[i] = const_cast<uint8_t*>(static_cast<const uint8_t*>(io[i]));
         t.row_bytes[i] = (uint32_t)r.bytes[i];
@@ -1577,7 +1582,7 @@ int mrb_per_sample_next(int64_t h, int64_t batch, float beta, const float* unifo
     const RowStore& r = b->rows;
     if (slot_field < 0 || slot_field >= r.nfields || r.bytes[slot_field] != 8)
         return fail(MRB_EINVAL, "slot_field %d must name a field of 8 bytes (one int64 slot number per row)", slot_field);
-    if (row_field < 0 || row_field >= r.nfields || r.vec_log2[row_field] != 4)
+    if (row_field < 0 || row_field >= r.nfields || r.align_log2[row_field] != 4)
         return fail(MRB_EINVAL, "row_field %d must name a field whose rows are multiples of 16 bytes", row_field);
     if (!out_next_rows) return fail(MRB_EINVAL, "out_next_rows is NULL");
     if (reinterpret_cast<uintptr_t>(out_next_rows) & 15u) return fail(MRB_EINVAL, "out_next_rows %p is not 16-byte aligned", out_next_rows);
