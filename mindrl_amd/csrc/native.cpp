@@ -6,6 +6,9 @@
 // Python. Here results come straight from torch's caching allocator, the small ones of a call out of one allocation, and a
 // call's host time is the library's and the runtime's launch.
 //
+// A rollout's returns with gradients went through a Python autograd function, whose backward half the engine's thread
+// runs under the interpreter's lock; ReturnBackward needs neither (forward and backward of [1000, 4096] 84 -> 52 us).
+//
 // Every method returns None, having done nothing, when an argument is not what the fast path takes (another dtype or
 // device, not contiguous, rows that do not match): the Python classes then convert it and call again, or raise.
 #define PY_SSIZE_T_CLEAN
@@ -19,7 +22,10 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
 
 #include <cstring>
 #include <new>
@@ -542,6 +548,93 @@ PyObject* put(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {  // put
     END_HANDLE_TH_ERRORS
 }
 
+// ---- discounted return ---------------------------------------------------------------------------------------------
+
+// A fresh contiguous float32 tensor of the given shape.
+at::Tensor new_float(c10::IntArrayRef sizes, int device) {
+    c10::OptionalDeviceGuard guard;
+    if (c10::hip::current_device() != device) guard.reset_device(c10::Device(c10::DeviceType::CUDA, (c10::DeviceIndex)device));
+    at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(new_storage(c10::multiply_integers(sizes) * 4),
+                                                            c10::DispatchKeySet(c10::DispatchKey::CUDA), caffe2::TypeMeta::Make<float>());
+    t.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
+    return t;
+}
+
+// The backward pass of a return that carries gradients: one launch, on the engine's own thread, without the interpreter.
+struct ReturnBackward : torch::autograd::Node {
+    torch::autograd::SavedVariable done;
+    std::vector<int64_t> value_sizes;
+    int64_t timesteps = 0, batch = 0, inner = 0;
+    float gamma = 0.0f;
+    std::string name() const override { return "DiscountedReturnBackward"; }
+    void release_variables() override { done.reset_data(); }
+    torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
+        torch::autograd::variable_list out(2);
+        if (!grads[0].defined()) return out;
+        const at::Tensor flags = done.unpack(), g = grads[0].contiguous();
+        const int device = g.get_device();
+        out[0] = new_float(g.sizes(), device);
+        if (task_should_compute_output(1)) out[1] = new_float(value_sizes, device);
+        const int rc = mrb_discounted_return_grad(g.const_data_ptr<float>(), static_cast<const uint8_t*>(flags.const_data_ptr()),
+                                                  out[0].mutable_data_ptr<float>(),
+                                                  out[1].defined() ? out[1].mutable_data_ptr<float>() : nullptr, timesteps, batch,
+                                                  inner, gamma, stream_of_current_device());
+        TORCH_CHECK(rc == MRB_OK, "libmrb: ", mrb_last_error());
+        if (!task_should_compute_output(0)) out[0] = at::Tensor();
+        return out;
+    }
+};
+
+// discounted_return(reward, done, last_state_value, gamma, differentiable, _lib.check): contiguous tensors on one device,
+// float32 and bool, of matching sizes
+PyObject* discounted_return(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    float gamma;
+    if (nargs != 6) {
+        PyErr_Format(PyExc_TypeError, "expected 6 arguments, got %zd", nargs);
+        return nullptr;
+    }
+    if (!real(args[3], &gamma)) return nullptr;
+    for (int i = 0; i < 3; ++i)
+        if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
+    const at::Tensor &reward = THPVariable_Unpack(args[0]), &done = THPVariable_Unpack(args[1]), &value = THPVariable_Unpack(args[2]);
+    for (const at::Tensor* t : {&reward, &done, &value})
+        if (!t->is_cuda() || t->layout() != c10::kStrided || !t->is_contiguous() || t->get_device() != reward.get_device() ||
+            t->scalar_type() != (t == &done ? at::ScalarType::Bool : at::ScalarType::Float))
+            Py_RETURN_NONE;
+    if (reward.dim() == 0 || done.dim() == 0 || reward.numel() == 0 || done.numel() == 0 || reward.size(0) != done.size(0)) Py_RETURN_NONE;
+    const int64_t timesteps = reward.size(0), batch = done.numel() / timesteps, inner = reward.numel() / done.numel();
+    if (inner * done.numel() != reward.numel() || value.numel() != batch * inner) Py_RETURN_NONE;
+    const int device = reward.get_device();
+    c10::OptionalDeviceGuard guard;
+    if (c10::hip::current_device() != device) guard.reset_device(reward.device());
+    at::Tensor out = new_float(reward.sizes(), device);
+    void* const stream = stream_of_current_device();
+    const float *x = reward.const_data_ptr<float>(), *v = value.const_data_ptr<float>();
+    const uint8_t* d = static_cast<const uint8_t*>(done.const_data_ptr());
+    float* const o = static_cast<float*>(out.mutable_data_ptr());
+    int rc;
+    Py_BEGIN_ALLOW_THREADS rc = mrb_discounted_return(x, d, v, o, timesteps, batch, inner, gamma, stream);
+    Py_END_ALLOW_THREADS if (rc != MRB_OK) {
+        Rows r;
+        r.check = args[5];
+        return failed(&r, rc);
+    }
+    if (args[4] == Py_True && at::GradMode::is_enabled() && (reward.requires_grad() || value.requires_grad())) {
+        std::shared_ptr<ReturnBackward> node(new ReturnBackward(), torch::autograd::deleteNode);
+        node->set_next_edges(torch::autograd::collect_next_edges(reward, value));
+        node->done = torch::autograd::SavedVariable(done, false);
+        node->value_sizes = value.sizes().vec();
+        node->timesteps = timesteps;
+        node->batch = batch;
+        node->inner = inner;
+        node->gamma = gamma;
+        torch::autograd::set_history(out, node);
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
 // ---- the type ----------------------------------------------------------------------------------------------------
 
 // Rows(handle, shapes, dtypes, device index, _lib.check)
@@ -612,7 +705,8 @@ PyMethodDef rows_methods[] = {
 
 PyTypeObject rows_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
-PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "mindrl_amd._native", nullptr, -1, nullptr};
+PyMethodDef module_methods[] = {METHOD("discounted_return", discounted_return), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "mindrl_amd._native", nullptr, -1, module_methods};
 
 }  // namespace
 
