@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "mrb_kernels.h"
+#include "mrb_range.h"
 #include "mrb_returns.h"
 #include "../../include/mrb_more.h"
 
@@ -729,6 +730,24 @@ UpdateArgs update_args(Per& b) {
 // the call's entries); larger calls take the stamp pass (2048 measured: config 4's update 14.0 us against 14.7 with the pass, at twice the waves and four times the comparisons: not taken).
 constexpr int64_t kElectMax = 1024;
 
+// Whether an update goes by runs of leaves (launch_tree_range). Against what it would take otherwise, us per call, before /
+// by runs:
+//   fewest entries  trees of up to 14 levels, 384 / 512 entries: one workgroup along the paths 7.0 / two launches 8.5
+//                   against 6.2 / 6.3; 256 entries 6.6 (14 levels) and 5.0 (12) against 6.1: k_tree_wg keeps those.
+//                   Deeper: 65 entries 7.0 (16 levels), 7.7 (20), 9.9 (22) against 6.2, 6.6, 7.4; up to 64 one wave
+//                   along the paths (k_tree_paths).
+//   most entries    10 levels, 2048 / 4096: 7.7 / 8.4 against 7.7 / 9.3; 12 levels, 8192 / 16,384: 10.0 / 11.4 against
+//                   9.6 / 13.8; 14 levels, 16,384 / 32,768: 11.7 / 12.5 against 11.2 / 16.7; 20 levels 14.4 / 15.4 against
+//                   14.1 / 18.7; 22 levels, 8192 / 16,384: 16.1 / 17.7 against 16.0 / 21.0.
+//   deepest tree    23 and 24 levels leave more than a tile above the runs and bring many runs without an entry: 2048
+//                   entries 14.9 / 15.9 against 14.9 / 23.3.
+bool takes_range(const Per& b, int64_t n) {
+    if (!b.fused || b.depth < 10 || b.depth > 22) return false;
+    const int64_t fewest = b.depth <= kWgMaxDepth ? kWgBestEntries : kPathEntries;
+    const int64_t most = b.depth <= 11 ? 2048 : b.depth == 12 || b.depth == 22 ? 8192 : 16384;
+    return n > fewest && n <= most;
+}
+
 // update_priorities on buffer b with `powered` (device f32[n]) as the scratch that holds the entries'
 // p^alpha between the stamp pass and the leaf writes. Allocates nothing.
 int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t n, float* powered, hipStream_t s) {
@@ -745,6 +764,13 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
             return fail(MRB_ESTATE, "an update of more than %lld entries cannot be recorded into a HIP graph (its "
                                     "election tags are counted on the host); split it into calls of at most %lld",
                         (long long)kElectMax, (long long)kElectMax);
+    }
+    if (takes_range(*b, n)) {
+        hipError_t e = launch_tree_range(indices, priorities, n, b->sum, b->mn, b->maxp, b->err, b->rows.capacity, b->depth, b->alpha, s);
+        if (e != hipSuccess) return fail(MRB_EHIP, "launch k_tree_range: %s", hipGetErrorString(e));
+        e = launch_tree_cap(b->sum, b->mn, b->depth - tree_range_levels(b->depth), s);
+        if (e != hipSuccess) return fail(MRB_EHIP, "launch k_tree_cap: %s", hipGetErrorString(e));
+        return MRB_OK;
     }
     int rc = next_epoch(*b, s);
     if (rc) return rc;

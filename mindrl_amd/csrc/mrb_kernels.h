@@ -7,13 +7,12 @@
 
 #include "../../include/mrb.h"
 #include "mrb_device.h"
+#include "mrb_tree.h"
 
 namespace mrb {
 
 constexpr int kWG = 256;          // threads per workgroup of the row and sample kernels
 constexpr int kLdsWG = kWG + 64;  // the LDS-top sample kernel: kWG strata and a helper wave
-constexpr int kRoundLevels = 8;   // most tree levels rebuilt by one round of k_tree_update
-constexpr int kBlockNodes = 256;  // nodes per wave tile in k_tree_update (float4 per lane)
 constexpr int kTopMaxDepth = 12;  // deepest level k_tree_top normally starts from (4096 nodes)
 
 // Per-call table of the fields of a row, passed to kernels by value.
@@ -1364,15 +1363,6 @@ struct UpdateArgs {
     uint32_t readers;
 };
 
-__device__ __forceinline__ bool valid_priority(float p) { return p >= 0.0f && p <= 3.0e38f; }
-
-// Folds q into the running max priority. Atomics on one address are serialised by the memory
-// system (~11 ns each), so the wave first looks at the current value: the max only grows, hence a
-// q that does not exceed what is already there can never matter, and nearly every wave skips.
-__device__ __forceinline__ void raise_max(float* maxp, float q) {
-    if (q > *reinterpret_cast<volatile float*>(maxp)) atomicMax(reinterpret_cast<unsigned int*>(maxp), __float_as_uint(q));
-}
-
 __global__ __launch_bounds__(kWG) void k_update_stamp(UpdateArgs a) {
     const int64_t j = (int64_t)blockIdx.x * kWG + threadIdx.x;
     float q = 0.0f;
@@ -1442,65 +1432,6 @@ __device__ __forceinline__ bool range_meets(const UpdateArgs& a, int64_t first_s
 //              and the blocks holding a winner are the dirty ones
 // Lanes of clean blocks neither load nor store; the shuffles of a dirty block only mix
 // lanes of that block.
-// The g levels above a tile whose nodes (four per lane, vs / vm) are final: parents by in-lane
-// operations and wave shuffles, stored by the lanes of dirty blocks (`active`). `first`: heap index
-// of the tile's first node.
-// The LDS word a small update's entry bids for its leaf with: the entry's position in the call (plus one, so
-// that zero means no bid) above its priority's bits. An integer max over the bids elects the last entry aimed
-// at the leaf, and the winner's priority comes back with it (no second trip to the call's arrays).
-__device__ __forceinline__ unsigned long long election_key(int64_t j, float p) {
-    return ((unsigned long long)(j + 1) << 32) | (unsigned long long)__float_as_uint(p);
-}
-__device__ __forceinline__ float elected_priority(unsigned long long key) { return __uint_as_float((uint32_t)key); }
-
-// One butterfly step of tile_parents: level 3 + S above the tile, one node per 2^(S+1) lanes.
-template <int S>
-__device__ __forceinline__ void parents_step(const UpdateArgs& a, int g, uint32_t first, uint32_t lane, bool active,
-                                             float& cs, float& cm) {
-    cs = cs + butterfly_peer<S>(cs);
-    cm = fminf(cm, butterfly_peer<S>(cm));
-    if (active && g >= 3 + S && (lane & ((2u << S) - 1)) == 0) {
-        a.sum[(first >> (3 + S)) + (lane >> (S + 1))] = cs;
-        a.mn[(first >> (3 + S)) + (lane >> (S + 1))] = cm;
-    }
-}
-
-// root_s / root_m (optional): the node eight levels above a full tile, as computed here (what is stored when g >= 8).
-__device__ __forceinline__ void tile_parents(const UpdateArgs& a, int g, uint32_t first, uint32_t lane, bool active,
-                                             const float4& vs, const float4& vm, float* root_s = nullptr,
-                                             float* root_m = nullptr) {
-    // one level up: two nodes per lane; two levels up: one node per lane
-    const float s0 = vs.x + vs.y, s1 = vs.z + vs.w;
-    const float m0 = fminf(vm.x, vm.y), m1 = fminf(vm.z, vm.w);
-    float cs = s0 + s1, cm = fminf(m0, m1);
-    if (active && g >= 1) {
-        *reinterpret_cast<float2*>(a.sum + (first >> 1) + 2 * lane) = make_float2(s0, s1);
-        *reinterpret_cast<float2*>(a.mn + (first >> 1) + 2 * lane) = make_float2(m0, m1);
-    }
-    if (active && g >= 2) {
-        a.sum[(first >> 2) + lane] = cs;
-        a.mn[(first >> 2) + lane] = cm;
-    }
-    // three to six levels up: 32, 16, 8, 4 nodes per full tile, a butterfly inside each row of 16 lanes
-    parents_step<0>(a, g, first, lane, active, cs, cm);
-    parents_step<1>(a, g, first, lane, active, cs, cm);
-    parents_step<2>(a, g, first, lane, active, cs, cm);
-    parents_step<3>(a, g, first, lane, active, cs, cm);
-    // seven and eight levels up: the four rows' values, read as scalars (left + right as everywhere)
-    const float s_lo = lane_value(cs, 0) + lane_value(cs, 16), s_hi = lane_value(cs, 32) + lane_value(cs, 48);
-    const float m_lo = fminf(lane_value(cm, 0), lane_value(cm, 16)), m_hi = fminf(lane_value(cm, 32), lane_value(cm, 48));
-    if (active && g >= 7 && (lane & 31) == 0) {
-        a.sum[(first >> 7) + (lane >> 5)] = lane < 32 ? s_lo : s_hi;
-        a.mn[(first >> 7) + (lane >> 5)] = lane < 32 ? m_lo : m_hi;
-    }
-    if (active && g >= 8 && lane == 0) {
-        a.sum[first >> 8] = s_lo + s_hi;
-        a.mn[first >> 8] = fminf(m_lo, m_hi);
-    }
-    if (root_s) *root_s = s_lo + s_hi;
-    if (root_m) *root_m = fminf(m_lo, m_hi);
-}
-
 // root_s / root_m / rebuilt (optional, full tiles with g = 8): the tile's root as stored, and whether the tile
 // was rebuilt at all (its one block was dirty).
 __device__ __forceinline__ void tile_round(const UpdateArgs& a, int lo, int g, uint32_t tile, bool sparse,

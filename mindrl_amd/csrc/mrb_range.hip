@@ -1,0 +1,190 @@
+#include "mrb_range.h"
+
+#include "../../include/mrb.h"
+#include "mrb_tree.h"
+
+namespace mrb {
+
+namespace {
+
+struct Trees {
+    float* sum;
+    float* mn;
+};
+
+// ---------------------------------------------------------------------------
+// update_priorities of a few thousand entries (PriorityReplayBufferUpdate,
+// mindspore_rl/core/priority_replay_buffer.py:71-73,120), divided by LEAVES: a workgroup owns a run of 2^w leaves,
+// looks every entry of the call over for those aimed at its leaves, elects the last one of each leaf in an LDS table
+// with a word per leaf, rebuilds the tiles that changed, a wave each, and goes on with its w levels to the run's root.
+// What is left above is a small tree (k_tree_cap). No stamps in memory, no pass of its own for the election, no wave for
+// a clean tile, no launch between the leaves and the run's root: two launches instead of three or four. What it pays is
+// that every workgroup reads all indices (out of its L2: 16 KB for 2048 entries), which is why larger calls keep the
+// stamp pass (the rule, with both sides measured, is at takes_range).
+// A call is bound by its chain of trips - indices, priorities of a run's own, tiles, then the second launch's tile -, not
+// by bytes. 2048 entries on 2^21 leaves 14.7 -> 9.1 us, 1024 on 2^17 9.4 -> 6.7, 250 on 2^19 7.5 -> 6.8.
+// ---------------------------------------------------------------------------
+constexpr int kRangePer = 8;  // entries of a thread and trip, all requested at once, the next trip's before these are looked at
+
+// kLog2: the table's leaves; w <= kLog2.
+template <int kLog2>
+__global__ __launch_bounds__(1024) void k_tree_range(const int64_t* __restrict__ indices, const float* __restrict__ priorities,
+                                                         float* sum, float* mn, float* maxp, int n, int capacity, int depth_w,
+                                                         float alpha, uint32_t* err) {
+    __shared__ unsigned long long s_win[1 << kLog2];         // per leaf: the latest entry's election_key (with its power)
+    __shared__ uint32_t s_dirty[1 << (kLog2 - 8)];           // per tile
+    __shared__ float s_rs[1 << (kLog2 - 8)], s_rm[1 << (kLog2 - 8)];  // the tiles' roots
+    const int depth = depth_w & 255, w = depth_w >> 8;
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t run = blockIdx.x, leaves = 1u << w, tiles = leaves / kBlockNodes;
+    const Trees trees{sum, mn};
+    const int threads = (int)blockDim.x, trip = kRangePer * threads;
+    auto request = [&](int base, int64_t (&to)[kRangePer]) {
+#pragma unroll
+        for (int q = 0; q < kRangePer; ++q) {
+            const int j = base + q * threads + (int)tid;
+            to[q] = j < n ? indices[j] : -1;
+        }
+    };
+    int64_t idx[kRangePer];
+    request(0, idx);
+    // the roots as they are, for the tiles that stay clean; the table is cleared while the entries are on their way
+    const uint32_t root0 = ((1u << depth) + run * leaves) >> kRoundLevels;
+    if (tid < tiles) {
+        s_rs[tid] = sum[root0 + tid];
+        s_rm[tid] = mn[root0 + tid];
+        s_dirty[tid] = 0;
+    }
+    for (uint32_t i = 2 * tid; i < leaves; i += 2 * threads) *reinterpret_cast<ulonglong2*>(&s_win[i]) = make_ulonglong2(0, 0);
+    lds_barrier();
+    float largest = 0.0f;
+    for (int base = 0; base < n; base += trip) {  // uniform
+        int64_t next[kRangePer];
+        if (base + trip < n) request(base + trip, next);
+        uint32_t mine = 0;
+        float p[kRangePer];
+#pragma unroll
+        for (int q = 0; q < kRangePer; ++q) {
+            const int j = base + q * threads + (int)tid;
+            const bool in = idx[q] >= 0 && idx[q] < capacity;
+            // (entries that name no leaf are the first workgroup's to flag)
+            const bool take = j < n && (in ? (uint32_t)((uint64_t)idx[q] >> w) == run : run == 0);
+            if (take) {
+                mine |= 1u << q;
+                p[q] = priorities[j];
+            }
+        }
+        while (mine) {  // (a thread has one entry of its run, or none, as a rule)
+            const int q = __builtin_ctz(mine);
+            mine &= mine - 1;
+            int64_t i = idx[0];
+            float x = p[0];
+#pragma unroll
+            for (int k = 1; k < kRangePer; ++k) {
+                i = q == k ? idx[k] : i;
+                x = q == k ? p[k] : x;
+            }
+            const bool in = i >= 0 && i < capacity, ok = valid_priority(x);
+            if (!in) atomicOr(err, MRB_DERR_INDEX);
+            if (!ok) atomicOr(err, MRB_DERR_PRIORITY);
+            if (!in || !ok) continue;
+            const float power = powf_det(x, alpha);
+            largest = fmaxf(largest, power);
+            const uint32_t at = (uint32_t)i & (leaves - 1);
+            atomicMax(&s_win[at], election_key(base + q * threads + (int)tid, power));
+            s_dirty[at / kBlockNodes] = 1;
+        }
+        if (base + trip < n) {
+#pragma unroll
+            for (int q = 0; q < kRangePer; ++q) idx[q] = next[q];
+        }
+    }
+    largest = wave_max(largest);
+    if (lane == 0 && largest > 0.0f) raise_max(maxp, largest);
+    lds_barrier();
+    // the tiles that changed, dealt to the waves
+    const unsigned long long dirty = __ballot(lane < tiles && s_dirty[lane < tiles ? lane : 0] != 0);
+    if (dirty == 0) return;  // (the same in every wave)
+    uint32_t nth = 0;
+    for (unsigned long long rest = dirty; rest; rest &= rest - 1, ++nth) {
+        if (nth % (blockDim.x / 64) != wave) continue;
+        const uint32_t t = (uint32_t)__builtin_ctzll(rest);
+        const uint32_t first = (1u << depth) + run * leaves + t * kBlockNodes;
+        float4 vs = *reinterpret_cast<const float4*>(sum + first + 4 * lane);
+        float4 vm = *reinterpret_cast<const float4*>(mn + first + 4 * lane);
+        const ulonglong2 k01 = *reinterpret_cast<const ulonglong2*>(&s_win[t * kBlockNodes + 4 * lane]);
+        const ulonglong2 k23 = *reinterpret_cast<const ulonglong2*>(&s_win[t * kBlockNodes + 4 * lane + 2]);
+        if (k01.x) vs.x = vm.x = elected_priority(k01.x);
+        if (k01.y) vs.y = vm.y = elected_priority(k01.y);
+        if (k23.x) vs.z = vm.z = elected_priority(k23.x);
+        if (k23.y) vs.w = vm.w = elected_priority(k23.y);
+        if (k01.x | k01.y | k23.x | k23.y) {
+            *reinterpret_cast<float4*>(sum + first + 4 * lane) = vs;
+            *reinterpret_cast<float4*>(mn + first + 4 * lane) = vm;
+        }
+        float rs, rm;
+        tile_parents(trees, kRoundLevels, first, lane, true, vs, vm, &rs, &rm);
+        if (lane == 0) {
+            s_rs[t] = rs;
+            s_rm[t] = rm;
+        }
+    }
+    lds_barrier();
+    if (wave != 0 || tiles == 1) return;
+    // from the tiles' roots to the run's (at most six levels)
+    float cs = lane < tiles ? s_rs[lane] : 0.0f, cm = lane < tiles ? s_rm[lane] : 0.0f;
+    for (int l = 1; l <= w - kRoundLevels; ++l) {
+        cs = cs + __shfl_xor(cs, 1 << (l - 1));
+        cm = fminf(cm, __shfl_xor(cm, 1 << (l - 1)));
+        if (lane < tiles && (lane & ((1u << l) - 1)) == 0) {
+            sum[(root0 + lane) >> l] = cs;
+            mn[(root0 + lane) >> l] = cm;
+        }
+    }
+}
+
+// The levels above depth `top` (1 .. 8): one wave, everything it needs in preloaded registers, one trip to memory.
+__global__ __launch_bounds__(64) void k_tree_cap(float* sum, float* mn, int top) {
+    const uint32_t lane = threadIdx.x, nodes = 1u << top;
+    const Trees trees{sum, mn};
+    if (top == 1) {
+        if (lane == 0) {
+            sum[1] = sum[2] + sum[3];
+            mn[1] = fminf(mn[2], mn[3]);
+        }
+        return;
+    }
+    const bool active = 4 * lane < nodes;
+    float4 vs = make_float4(0.f, 0.f, 0.f, 0.f), vm = vs;
+    if (active) {
+        vs = *reinterpret_cast<const float4*>(sum + nodes + 4 * lane);
+        vm = *reinterpret_cast<const float4*>(mn + nodes + 4 * lane);
+    }
+    tile_parents(trees, top, nodes, lane, active, vs, vm);
+}
+
+}  // namespace
+
+// Runs of 256 to 16,384 leaves: 256 of them - and eight levels left above, one tile - where that is possible (16 to 22
+// levels). A table of 16,384 words is 128 KB of a compute unit's LDS.
+int tree_range_levels(int depth) {
+    const int w = depth - kRoundLevels;
+    return w < 8 ? 8 : w > 14 ? 14 : w;
+}
+
+hipError_t launch_tree_range(const int64_t* indices, const float* priorities, int64_t n, float* sum, float* mn, float* maxp,
+                             uint32_t* err, int64_t capacity, int depth, float alpha, hipStream_t s) {
+    const int w = tree_range_levels(depth);
+    const dim3 grid((uint32_t)((capacity + ((int64_t)1 << w) - 1) >> w)), threads(n > 4096 ? 1024 : 512);  // (256: 0.3 to 1.5 us more)
+    auto* const kernel = w <= 10 ? k_tree_range<10> : w <= 12 ? k_tree_range<12> : w == 13 ? k_tree_range<13> : k_tree_range<14>;
+    hipLaunchKernelGGL(kernel, grid, threads, 0, s, indices, priorities, sum, mn, maxp, (int)n, (int)capacity, depth | w << 8, alpha, err);
+    return hipGetLastError();
+}
+
+hipError_t launch_tree_cap(float* sum, float* mn, int top, hipStream_t s) {
+    hipLaunchKernelGGL(k_tree_cap, dim3(1), dim3(64), 0, s, sum, mn, top);
+    return hipGetLastError();
+}
+
+}  // namespace mrb
