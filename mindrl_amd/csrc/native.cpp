@@ -28,6 +28,7 @@
 #include <torch/csrc/autograd/saved_variable.h>
 
 #include <cstring>
+#include <mutex>
 #include <new>
 
 #include "../../include/mrb.h"
@@ -184,10 +185,12 @@ at::ScalarType type_of_format(const char* s, int64_t item) {
     }
 }
 
+PyTypeObject* ndarray_type = nullptr;  // numpy.ndarray
+
 // The rows a call brings: device tensors where they lie; host tensors and arrays copied into the buffer's pinned
 // staging memory (mrb_stage), which the kernels read.
 struct Source {
-    const void* ptr[MRB_MAX_FIELDS];
+    const void* ptr[MRB_MAX_FIELDS] = {};
     int64_t nrows = -1;
     Py_buffer view[MRB_MAX_FIELDS];
     bool viewed[MRB_MAX_FIELDS] = {};
@@ -218,7 +221,7 @@ struct Source {
                 else if (!t.is_cuda() || t.get_device() != r->device) return false;
                 ptr[i] = p;
             } else {
-                if (!PyObject_CheckBuffer(items[i])) return false;
+                if (!PyObject_TypeCheck(items[i], ndarray_type)) return false;
                 if (PyObject_GetBuffer(items[i], &view[i], PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) != 0) {
                     PyErr_Clear();
                     return false;
@@ -567,12 +570,20 @@ struct ReturnBackward : torch::autograd::Node {
     int64_t timesteps = 0, batch = 0, inner = 0;
     float gamma = 0.0f;
     std::string name() const override { return "DiscountedReturnBackward"; }
-    void release_variables() override { done.reset_data(); }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        done.reset_data();
+    }
     torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
         torch::autograd::variable_list out(2);
         if (!grads[0].defined()) return out;
-        const at::Tensor flags = done.unpack(), g = grads[0].contiguous();
+        std::lock_guard<std::mutex> lock(mutex_);
+        const at::Tensor g = grads[0].resolve_neg().contiguous();
         const int device = g.get_device();
+        at::Tensor flags = done.unpack();  // (what saved-tensor hooks made of it)
+        TORCH_CHECK(flags.get_device() == device && flags.scalar_type() == at::ScalarType::Bool && flags.numel() == timesteps * batch,
+                    "the saved flags came back as another tensor");
+        flags = flags.contiguous();
         out[0] = new_float(g.sizes(), device);
         if (task_should_compute_output(1)) out[1] = new_float(value_sizes, device);
         const int rc = mrb_discounted_return_grad(g.const_data_ptr<float>(), static_cast<const uint8_t*>(flags.const_data_ptr()),
@@ -605,13 +616,21 @@ PyObject* discounted_return(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     if (reward.dim() == 0 || done.dim() == 0 || reward.numel() == 0 || done.numel() == 0 || reward.size(0) != done.size(0)) Py_RETURN_NONE;
     const int64_t timesteps = reward.size(0), batch = done.numel() / timesteps, inner = reward.numel() / done.numel();
     if (inner * done.numel() != reward.numel() || value.numel() != batch * inner) Py_RETURN_NONE;
+    const bool differentiable =
+        args[4] == Py_True && at::GradMode::is_enabled() && (reward.requires_grad() || value.requires_grad());
+    if (args[4] == Py_True && (reward.requires_grad() || value.requires_grad()) &&
+        (reward._fw_grad(0).defined() || value._fw_grad(0).defined())) {
+        PyErr_SetString(PyExc_NotImplementedError, "DiscountedReturn has no forward-mode derivative");
+        return nullptr;
+    }
     const int device = reward.get_device();
     c10::OptionalDeviceGuard guard;
     if (c10::hip::current_device() != device) guard.reset_device(reward.device());
     at::Tensor out = new_float(reward.sizes(), device);
     void* const stream = stream_of_current_device();
-    const float *x = reward.const_data_ptr<float>(), *v = value.const_data_ptr<float>();
-    const uint8_t* d = static_cast<const uint8_t*>(done.const_data_ptr());
+    // (data_ptr: raises for tensors without memory)
+    const float *x = static_cast<const float*>(reward.data_ptr()), *v = static_cast<const float*>(value.data_ptr());
+    const uint8_t* d = static_cast<const uint8_t*>(done.data_ptr());
     float* const o = static_cast<float*>(out.mutable_data_ptr());
     int rc;
     Py_BEGIN_ALLOW_THREADS rc = mrb_discounted_return(x, d, v, o, timesteps, batch, inner, gamma, stream);
@@ -620,7 +639,7 @@ PyObject* discounted_return(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
         r.check = args[5];
         return failed(&r, rc);
     }
-    if (args[4] == Py_True && at::GradMode::is_enabled() && (reward.requires_grad() || value.requires_grad())) {
+    if (differentiable) {
         std::shared_ptr<ReturnBackward> node(new ReturnBackward(), torch::autograd::deleteNode);
         node->set_next_edges(torch::autograd::collect_next_edges(reward, value));
         node->done = torch::autograd::SavedVariable(done, false);
@@ -719,6 +738,11 @@ PyMODINIT_FUNC PyInit__native(void) {
     rows_type.tp_dealloc = rows_dealloc;
     rows_type.tp_methods = rows_methods;
     if (PyType_Ready(&rows_type) < 0) return nullptr;
+    PyObject* const numpy = PyImport_ImportModule("numpy");
+    if (!numpy) return nullptr;
+    ndarray_type = reinterpret_cast<PyTypeObject*>(PyObject_GetAttrString(numpy, "ndarray"));
+    Py_DECREF(numpy);
+    if (!ndarray_type) return nullptr;
     PyObject* const m = PyModule_Create(&module_def);
     if (!m) return nullptr;
     Py_INCREF(&rows_type);

@@ -50,7 +50,8 @@ class DiscountedReturn:
                 raise ValueError("last_state_value must be [Batch, ...] matching reward")
             reward, done, last_state_value = r, d, v
             out = self._native(r, d, v, self.gamma, self.need_bprop, _lib.check)
-        self._keep = (reward, done, last_state_value)
+        if not out.requires_grad:  # (a result with a history holds what its gradient needs: no more is kept alive)
+            self._keep = (reward, done, last_state_value)
         return out
 
     __call__ = construct

@@ -42,3 +42,30 @@ def test_return_and_gradient_bit_exact(shape):
     want_reward, want_value = oracle_gradient(orc, w, d, 0.97)
     assert np.array_equal(t2n(grad_reward), want_reward)
     assert np.array_equal(t2n(grad_value), want_value)
+
+
+def test_forward_mode_is_refused():
+    import torch.autograd.forward_ad as fw
+    from mindrl_amd.utils import DiscountedReturn
+    done, value = torch.zeros(5, 3, dtype=torch.bool, device="cuda"), torch.zeros(3, device="cuda")
+    with fw.dual_level():
+        reward = fw.make_dual(torch.ones(5, 3, device="cuda", requires_grad=True), torch.ones(5, 3, device="cuda"))
+        with pytest.raises(NotImplementedError):
+            DiscountedReturn(0.9, need_bprop=True)(reward, done, value)
+
+
+def test_saved_flags_pass_through_hooks():
+    """A hook may hand the flags back in another layout; a gradient may come as an expanded or negated view."""
+    from mindrl_amd.utils import DiscountedReturn
+    reward = torch.randn(70, 9, device="cuda", requires_grad=True)
+    value = torch.randn(9, device="cuda", requires_grad=True)
+    done = torch.rand(70, 9, device="cuda") < 0.1
+    returns = DiscountedReturn(0.9, need_bprop=True)
+    want = torch.autograd.grad(returns(reward, done, value), (reward, value), torch.full((70, 9), 2.0, device="cuda"))
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.cuda().t().contiguous().t()):
+        out = returns(reward, done, value)
+    got = torch.autograd.grad(out, (reward, value), torch.full((), 2.0, device="cuda").expand(70, 9))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    negated = torch._neg_view(torch.full((70, 9), -2.0, device="cuda"))
+    got = torch.autograd.grad(returns(reward, done, value), (reward, value), negated)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
