@@ -489,8 +489,9 @@ struct Per {
     float* mn = nullptr;
     unsigned long long* stamp = nullptr;
     float* maxp = nullptr;
-    // sparse plan for very large trees (see k_tree_sparse): lowest s_g0 levels per entry, then s_rounds tile rounds
-    int s_g0 = 0, s_rounds = 0, s_top = 0;
+    // sparse plan for very large trees (see k_tree_sparse): lowest s_g0 levels per entry, then s_rounds rounds, of which
+    // the last one is k_tree_runs
+    int s_g0 = 0, s_rounds = 0;
     int s_lo[kMaxRounds] = {}, s_g[kMaxRounds] = {};
     uint32_t* s_dirty[kMaxRounds] = {};
     // scratch of update_priorities (p^alpha of the call's entries): sized at create; a call with more
@@ -785,7 +786,6 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
     if (sparse) {
         a.sparse_g0 = b->s_g0;
         a.nrounds = b->s_rounds;
-        a.top_depth = b->s_top;
         for (int r = 0; r < kMaxRounds; ++r) {
             a.dirty[r] = b->s_dirty[r];
             a.lo[r] = b->s_lo[r];
@@ -815,21 +815,26 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
         a.inline_election = 1;
         return tree_rebuild(*b, a, s);
     }
-    hipLaunchKernelGGL(k_update_stamp, dim3(grid_exact((uint64_t)n)), dim3(kWG), 0, s, a);
+    hipLaunchKernelGGL(k_update_stamp, dim3(grid_exact((uint64_t)n)), dim3(kWG), 0, s, a.indices, a.priorities, a.n,
+                       a.capacity, a.alpha, a);
     LAUNCH_CHECK("k_update_stamp");
     if (!sparse) return tree_rebuild(*b, a, s);
-    hipLaunchKernelGGL(k_tree_sparse, dim3(grid_exact((uint64_t)n << (b->s_g0 - 2))), dim3(kWG), 0, s, a);
-    LAUNCH_CHECK("k_tree_sparse");
-    const PutArgs none{};
-    for (int r = 0; r < b->s_rounds; ++r) {
+    const auto checked = [](hipError_t e, const char* name) {
+        return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch %s: %s", name, hipGetErrorString(e));
+    };
+    rc = checked(launch_tree_sparse(a.indices, a.stamp, a.powered, a.sum, a.mn, a.dirty[0], n, a.capacity, a.depth, a.sparse_g0,
+                                    a.g[0], a.epoch, s), "k_tree_sparse");
+    if (rc) return rc;
+    const int last = b->s_rounds - 1;
+    for (int r = 0; r < last; ++r) {
         const uint32_t tiles = (1u << b->s_lo[r]) / kBlockNodes;
         hipLaunchKernelGGL(k_tree_update, dim3((tiles + 3) / 4), dim3(kWG), 0, s, a.indices, a.priorities, a.sum, a.mn, a.n,
-                           a.capacity, r | a.lo[r] << 8 | a.g[r] << 16, a.alpha, a, 0u, none);
+                           a.capacity, r | a.lo[r] << 8 | a.g[r] << 16, a.alpha, a, 0u, PutArgs{});
         LAUNCH_CHECK("k_tree_update");
     }
-    hipLaunchKernelGGL(k_tree_top, dim3(1), dim3(kTopWG), 0, s, a, none);
-    LAUNCH_CHECK("k_tree_top");
-    return MRB_OK;
+    rc = checked(launch_tree_runs(a.sum, a.mn, a.dirty[last], a.lo[last], a.epoch, s), "k_tree_runs");
+    if (rc) return rc;
+    return checked(launch_tree_cap(a.sum, a.mn, kRoundLevels, s), "k_tree_cap");
 }
 
 
@@ -1219,14 +1224,16 @@ int mrb_per_create(int64_t capacity, float alpha, int nfields, const int64_t* fi
     if (b->depth >= 22) {
         // sparse plan: with >= 16384 leaf tiles a call with few entries is better driven by its entries
         b->s_g0 = b->depth - 20 < 4 ? 4 : (b->depth - 20 > 6 ? 6 : b->depth - 20);
-        const int d2 = b->depth - b->s_g0;
-        b->s_top = kTopMaxDepth;
-        const int rest2 = d2 - b->s_top;  // >= 4
-        b->s_rounds = (rest2 + kRoundLevels - 1) / kRoundLevels;
-        for (int r = 0, lo = d2; r < b->s_rounds; ++r) {
-            b->s_lo[r] = lo;
-            b->s_g[r] = rest2 / b->s_rounds + (r < rest2 % b->s_rounds ? 1 : 0);
-            lo -= b->s_g[r];
+        // k_tree_runs takes at most 20 levels; deeper trees go through a round of tiles first (at least two levels, so
+        // that a lane's four nodes share a block)
+        const int d2 = b->depth - b->s_g0, g = d2 <= 20 ? 0 : d2 - 20 < 2 ? 2 : d2 - 20;
+        if (g) {
+            b->s_lo[b->s_rounds] = d2;
+            b->s_g[b->s_rounds++] = g;
+        }
+        b->s_lo[b->s_rounds] = d2 - g;
+        b->s_g[b->s_rounds++] = kRoundLevels;
+        for (int r = 0; r < b->s_rounds; ++r) {
             const size_t nblocks = (size_t)1 << (b->s_lo[r] - b->s_g[r]);
             HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->s_dirty[r]), nblocks * sizeof(uint32_t)));
             HIP_TRY(hipMemset(b->s_dirty[r], 0, nblocks * sizeof(uint32_t)));
@@ -1321,7 +1328,8 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
     if (stamp_after) {
         a.priorities = opt_priorities;
         a.n = nrows;
-        hipLaunchKernelGGL(k_update_stamp, dim3(grid_exact((uint64_t)nrows)), dim3(kWG), 0, s, a);
+        hipLaunchKernelGGL(k_update_stamp, dim3(grid_exact((uint64_t)nrows)), dim3(kWG), 0, s, a.indices, a.priorities, a.n,
+                       a.capacity, a.alpha, a);
         LAUNCH_CHECK("k_update_stamp");
     }
     b->pushes += nrows;

@@ -1363,7 +1363,16 @@ struct UpdateArgs {
     uint32_t readers;
 };
 
-__global__ __launch_bounds__(kWG) void k_update_stamp(UpdateArgs a) {
+// (The leading plain parameters repeat members of `a_in`: preloaded into scalar registers, so the entries are requested
+// when a wave starts.)
+__global__ __launch_bounds__(kWG) void k_update_stamp(const int64_t* __restrict__ lead_indices, const float* __restrict__ lead_priorities,
+                                                      int64_t lead_n, int64_t lead_capacity, float lead_alpha, UpdateArgs a_in) {
+    UpdateArgs a = a_in;
+    a.indices = lead_indices;
+    a.priorities = lead_priorities;
+    a.n = lead_n;
+    a.capacity = lead_capacity;
+    a.alpha = lead_alpha;
     const int64_t j = (int64_t)blockIdx.x * kWG + threadIdx.x;
     float q = 0.0f;
     if (j < a.n) {
@@ -1582,89 +1591,6 @@ __device__ __forceinline__ void tile_round(const UpdateArgs& a, int lo, int g, u
     }
     tile_parents(a, g, first, lane, active, vs, vm, root_s, root_m);
     if (rebuilt) *rebuilt = __any(active);
-}
-
-// ---------------------------------------------------------------------------
-// Sparse lowest round for very large trees (e.g. 2^24 leaves, 65,536 entries): scanning
-// every 256-leaf tile costs more in wave launches than the update itself, so here the
-// ENTRIES drive the work. A group of L = 2^(g0-2) lanes (g0 = 4..6) takes one entry; if
-// that entry owns its block of 2^g0 leaves (it holds the largest of the block's stamps), the
-// group loads the block, replaces the leaves the stamps name, rebuilds the g0 levels
-// above with the same pairwise operations as tile_round and marks the next round's block.
-// ---------------------------------------------------------------------------
-// One butterfly step of k_tree_sparse inside an entry's group of lanes: level 3 + S above its block.
-template <int S>
-__device__ __forceinline__ void sparse_step(const UpdateArgs& a, int g0, uint64_t first, uint32_t sub, bool active,
-                                            float& cs, float& cm) {
-    if (S < g0 - 2) {  // wave-uniform
-        cs = cs + butterfly_peer<S>(cs);
-        cm = fminf(cm, butterfly_peer<S>(cm));
-        if (active && (sub & ((2u << S) - 1)) == 0) {
-            a.sum[(first >> (3 + S)) + (sub >> (S + 1))] = cs;
-            a.mn[(first >> (3 + S)) + (sub >> (S + 1))] = cm;
-        }
-    }
-}
-
-__global__ __launch_bounds__(kWG) void k_tree_sparse(UpdateArgs a) {
-    const int g0 = a.sparse_g0;
-    const uint32_t group = 1u << (g0 - 2);
-    const uint64_t tid = (uint64_t)blockIdx.x * kWG + threadIdx.x;
-    const int64_t j = (int64_t)(tid >> (g0 - 2));
-    const uint32_t sub = (uint32_t)tid & (group - 1);
-    bool active = j < a.n;
-    int64_t idx = 0;
-    if (active) {
-        idx = a.indices[j];
-        active = idx >= 0 && idx < a.capacity && valid_priority(a.priorities[j]);
-    }
-    const uint64_t block = (uint64_t)idx >> g0;
-    const uint64_t first = (uint64_t)a.leaves + (block << g0);  // heap index of the block's first leaf
-    // The block's owner is the entry with the largest stamp of this call among its leaves: every
-    // group aimed at the block reads the same 2^g0 stamps and only the owner's group goes on.
-    unsigned long long top = 0;
-    if (active) {
-        const unsigned long long* st = a.stamp + (block << g0) + 4 * sub;
-        const unsigned long long s0 = st[0], s1 = st[1], s2 = st[2], s3 = st[3];
-        top = s0 > s1 ? s0 : s1;
-        top = top > s2 ? top : s2;
-        top = top > s3 ? top : s3;
-    }
-    for (uint32_t m = 1; m < group; m <<= 1) {
-        const unsigned long long o = __shfl_xor(top, (int)m);
-        top = top > o ? top : o;
-    }
-    active = active && top == (((unsigned long long)a.epoch << 32) | (unsigned long long)j);
-    float4 vs = make_float4(0.f, 0.f, 0.f, 0.f), vm = vs;
-    if (active) {
-        vs = *reinterpret_cast<const float4*>(a.sum + first + 4 * sub);
-        vm = *reinterpret_cast<const float4*>(a.mn + first + 4 * sub);
-        const int64_t leaf0 = (int64_t)((block << g0) + 4 * sub);
-        float q;
-        bool wrote = false;
-        if (leaf_value(a, 0, leaf0 + 0, q)) { vs.x = vm.x = q; wrote = true; }
-        if (leaf_value(a, 0, leaf0 + 1, q)) { vs.y = vm.y = q; wrote = true; }
-        if (leaf_value(a, 0, leaf0 + 2, q)) { vs.z = vm.z = q; wrote = true; }
-        if (leaf_value(a, 0, leaf0 + 3, q)) { vs.w = vm.w = q; wrote = true; }
-        if (wrote) {
-            *reinterpret_cast<float4*>(a.sum + first + 4 * sub) = vs;
-            *reinterpret_cast<float4*>(a.mn + first + 4 * sub) = vm;
-        }
-        if (sub == 0 && a.nrounds) a.dirty[0][block >> a.g[0]] = a.epoch;
-    }
-    const float s0 = vs.x + vs.y, s1 = vs.z + vs.w;
-    const float m0 = fminf(vm.x, vm.y), m1 = fminf(vm.z, vm.w);
-    float cs = s0 + s1, cm = fminf(m0, m1);
-    if (active) {
-        *reinterpret_cast<float2*>(a.sum + (first >> 1) + 2 * sub) = make_float2(s0, s1);
-        *reinterpret_cast<float2*>(a.mn + (first >> 1) + 2 * sub) = make_float2(m0, m1);
-        a.sum[(first >> 2) + sub] = cs;
-        a.mn[(first >> 2) + sub] = cm;
-    }
-    sparse_step<0>(a, g0, first, sub, active, cs, cm);
-    sparse_step<1>(a, g0, first, sub, active, cs, cm);
-    sparse_step<2>(a, g0, first, sub, active, cs, cm);
-    sparse_step<3>(a, g0, first, sub, active, cs, cm);
 }
 
 // Small update on a tree whose leaves the top workgroup itself rebuilds (no stamp pass, no wave per entry):

@@ -144,6 +144,135 @@ __global__ __launch_bounds__(1024) void k_tree_range(const int64_t* __restrict__
     }
 }
 
+// ---------------------------------------------------------------------------
+// Very large trees (22 levels and more) under a call that names few of their leaves (65,536 of 2^24): scanning every
+// 256-leaf tile would cost more in wave launches than the update itself, so the ENTRIES drive the lowest levels. A group
+// of 2^(g0-2) lanes (g0 = 4..6) takes one entry; if that entry owns its block of 2^g0 leaves (it holds the largest of
+// the block's stamps), the group replaces the leaves the stamps name, rebuilds the g0 levels above with tile_parents'
+// operations and marks the tile of the next round.
+// What bounds it: trips to memory that nothing is cached for, and some ten lines per entry written in part. The block's
+// stamps, its nodes and the entry's own power are therefore requested together, as soon as the index is there, whether
+// or not the entry turns out to own the block (nearly every one does), and the arguments are preloaded: two trips where
+// there were five (arguments, index and priority, stamps, nodes, powers). An owner stores all leaves of its block, 64
+// bytes of a line instead of the pieces that changed. 65,536 entries on 2^24 leaves that no cache holds: 19.2 -> 17.7 us,
+// of which the 0.5 million partial lines of the levels between are the rest.
+// ---------------------------------------------------------------------------
+constexpr int kSparseWG = 256;
+
+// Level 3 + S above the block, inside an entry's group of lanes.
+template <int S>
+__device__ __forceinline__ void sparse_step(const Trees& a, int g0, uint32_t first, uint32_t sub, bool active, float& cs, float& cm) {
+    if (S < g0 - 2) {  // uniform
+        cs = cs + butterfly_peer<S>(cs);
+        cm = fminf(cm, butterfly_peer<S>(cm));
+        if (active && (sub & ((2u << S) - 1)) == 0) {
+            a.sum[(first >> (3 + S)) + (sub >> (S + 1))] = cs;
+            a.mn[(first >> (3 + S)) + (sub >> (S + 1))] = cm;
+        }
+    }
+}
+
+// plan: depth | g0 << 8 | g_dirty << 16
+__global__ __launch_bounds__(kSparseWG) void k_tree_sparse(const int64_t* __restrict__ indices,
+                                                           const unsigned long long* __restrict__ stamp,
+                                                           const float* __restrict__ powered, float* sum, float* mn, uint32_t* dirty,
+                                                           int n, uint32_t capacity, uint32_t epoch, int plan) {
+    const int depth = plan & 255, g0 = (plan >> 8) & 255, g_dirty = plan >> 16;
+    const uint32_t group = 1u << (g0 - 2);
+    const uint32_t tid = blockIdx.x * kSparseWG + threadIdx.x;
+    const uint32_t j = tid >> (g0 - 2), sub = tid & (group - 1);
+    const Trees trees{sum, mn};
+    int64_t idx = -1;
+    if (j < (uint32_t)n) idx = indices[j];
+    bool active = idx >= 0 && idx < (int64_t)capacity;
+    const uint32_t block = active ? (uint32_t)idx >> g0 : 0u;
+    const uint32_t first = (1u << depth) + (block << g0);  // heap index of the block's first leaf
+    float4 vs = make_float4(0.f, 0.f, 0.f, 0.f), vm = vs;
+    ulonglong2 s01 = make_ulonglong2(0, 0), s23 = s01;
+    float own = 0.0f;
+    if (active) {
+        const ulonglong2* st = reinterpret_cast<const ulonglong2*>(stamp + ((uint64_t)block << g0) + 4 * sub);
+        s01 = st[0];
+        s23 = st[1];
+        vs = *reinterpret_cast<const float4*>(sum + first + 4 * sub);
+        vm = *reinterpret_cast<const float4*>(mn + first + 4 * sub);
+        own = powered[j];  // (of an invalid priority: whatever lies there; no stamp names it)
+    }
+    // The block's owner is the entry with the largest stamp of this call among its leaves (an entry that is not valid has
+    // raised none).
+    const unsigned long long a01 = s01.x > s01.y ? s01.x : s01.y, a23 = s23.x > s23.y ? s23.x : s23.y;
+    unsigned long long top = a01 > a23 ? a01 : a23;
+    for (uint32_t m = 1; m < group; m <<= 1) {
+        const unsigned long long o = __shfl_xor(top, (int)m);
+        top = top > o ? top : o;
+    }
+    const unsigned long long mine = ((unsigned long long)epoch << 32) | j;
+    active = active && top == mine;
+    if (active) {
+        auto leaf = [&](unsigned long long st, float& ls, float& lm) {
+            if ((uint32_t)(st >> 32) != epoch) return;
+            ls = lm = st == mine ? own : powered[(uint32_t)st];
+        };
+        leaf(s01.x, vs.x, vm.x);
+        leaf(s01.y, vs.y, vm.y);
+        leaf(s23.x, vs.z, vm.z);
+        leaf(s23.y, vs.w, vm.w);
+        *reinterpret_cast<float4*>(sum + first + 4 * sub) = vs;
+        *reinterpret_cast<float4*>(mn + first + 4 * sub) = vm;
+        if (sub == 0) dirty[block >> g_dirty] = epoch;
+    }
+    const float s0 = vs.x + vs.y, s1 = vs.z + vs.w;
+    const float m0 = fminf(vm.x, vm.y), m1 = fminf(vm.z, vm.w);
+    float cs = s0 + s1, cm = fminf(m0, m1);
+    if (active) {
+        *reinterpret_cast<float2*>(sum + (first >> 1) + 2 * sub) = make_float2(s0, s1);
+        *reinterpret_cast<float2*>(mn + (first >> 1) + 2 * sub) = make_float2(m0, m1);
+        sum[(first >> 2) + sub] = cs;
+        mn[(first >> 2) + sub] = cm;
+    }
+    sparse_step<0>(trees, g0, first, sub, active, cs, cm);
+    sparse_step<1>(trees, g0, first, sub, active, cs, cm);
+    sparse_step<2>(trees, g0, first, sub, active, cs, cm);
+    sparse_step<3>(trees, g0, first, sub, active, cs, cm);
+}
+
+// The next levels of such a tree, down to 256 nodes that k_tree_cap takes: a workgroup owns 2^w nodes at depth `top` (w =
+// top - 8, 9 to 12), a wave each tile of 256, and goes on to the run's root. Nodes, dirty word and the root as it is are
+// requested together. With k_tree_cap 6.1 + 1.5 to 3.9 us for 2^20 nodes; a launch for eight levels and one workgroup for
+// the twelve above took 6.1 + 3.9 and their inputs a trip more. (The step on the 24-level tree 55.5 -> 51.5 us.)
+__global__ __launch_bounds__(1024) void k_tree_runs(float* sum, float* mn, const uint32_t* __restrict__ dirty, uint32_t epoch, int top) {
+    __shared__ float s_rs[16], s_rm[16];
+    __shared__ uint32_t s_new[16];
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int up = top - 2 * kRoundLevels;  // levels from the tiles' roots to the run's: 2^up waves
+    const uint32_t tile = (blockIdx.x << up) + wave, first = (1u << top) + tile * kBlockNodes;
+    const Trees trees{sum, mn};
+    const float4 vs = *reinterpret_cast<const float4*>(sum + first + 4 * lane);
+    const float4 vm = *reinterpret_cast<const float4*>(mn + first + 4 * lane);
+    float rs = sum[first >> kRoundLevels], rm = mn[first >> kRoundLevels];
+    const bool changed = dirty[tile] == epoch;
+    if (changed) tile_parents(trees, kRoundLevels, first, lane, true, vs, vm, &rs, &rm);
+    if (lane == 0) {
+        s_rs[wave] = rs;
+        s_rm[wave] = rm;
+        s_new[wave] = changed;
+    }
+    lds_barrier();
+    if (wave != 0) return;
+    const uint32_t tiles = 1u << up;
+    float cs = lane < tiles ? s_rs[lane] : 0.0f, cm = lane < tiles ? s_rm[lane] : 0.0f;
+    if (!__any(lane < tiles && s_new[lane])) return;
+    for (int l = 1; l <= up; ++l) {
+        cs = cs + __shfl_xor(cs, 1 << (l - 1));
+        cm = fminf(cm, __shfl_xor(cm, 1 << (l - 1)));
+        if (lane < tiles && (lane & ((1u << l) - 1)) == 0) {
+            sum[((first >> kRoundLevels) + lane) >> l] = cs;
+            mn[((first >> kRoundLevels) + lane) >> l] = cm;
+        }
+    }
+}
+
 // The levels above depth `top` (1 .. 8): one wave, everything it needs in preloaded registers, one trip to memory.
 __global__ __launch_bounds__(64) void k_tree_cap(float* sum, float* mn, int top) {
     const uint32_t lane = threadIdx.x, nodes = 1u << top;
@@ -179,6 +308,20 @@ hipError_t launch_tree_range(const int64_t* indices, const float* priorities, in
     const dim3 grid((uint32_t)((capacity + ((int64_t)1 << w) - 1) >> w)), threads(n > 4096 ? 1024 : 512);  // (256: 0.3 to 1.5 us more)
     auto* const kernel = w <= 10 ? k_tree_range<10> : w <= 12 ? k_tree_range<12> : w == 13 ? k_tree_range<13> : k_tree_range<14>;
     hipLaunchKernelGGL(kernel, grid, threads, 0, s, indices, priorities, sum, mn, maxp, (int)n, (int)capacity, depth | w << 8, alpha, err);
+    return hipGetLastError();
+}
+
+hipError_t launch_tree_sparse(const int64_t* indices, const unsigned long long* stamp, const float* powered, float* sum, float* mn,
+                              uint32_t* dirty, int64_t n, int64_t capacity, int depth, int g0, int g_dirty, uint32_t epoch,
+                              hipStream_t s) {
+    const dim3 grid((uint32_t)(((n << (g0 - 2)) + kSparseWG - 1) / kSparseWG));
+    hipLaunchKernelGGL(k_tree_sparse, grid, dim3(kSparseWG), 0, s, indices, stamp, powered, sum, mn, dirty, (int)n, (uint32_t)capacity,
+                       epoch, depth | g0 << 8 | g_dirty << 16);
+    return hipGetLastError();
+}
+
+hipError_t launch_tree_runs(float* sum, float* mn, const uint32_t* dirty, int top, uint32_t epoch, hipStream_t s) {
+    hipLaunchKernelGGL(k_tree_runs, dim3(1u << kRoundLevels), dim3(64u << (top - 2 * kRoundLevels)), 0, s, sum, mn, dirty, epoch, top);
     return hipGetLastError();
 }
 
