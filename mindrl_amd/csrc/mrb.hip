@@ -1496,6 +1496,24 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
     return per_push(b.get(), src_fields, nrows, opt_push_priorities, s);
 }
 
+// Whether a sample of `rows` rows (of all its batches) goes to the LDS-top kernel, and the strata of a workgroup there;
+// `rest` is what a row costs it to copy (see k_per_sample_lds). A wave per row carries a row faster, a thread per stratum
+// walks the tree faster, so the line rises with the row's size. Measured, us, wave (workgroup) per row / LDS-top:
+//   8-byte rows, 2^24 slots   2048 rows 6.8 / 6.1, 4096 8.6 / 6.1, 16,384 23 / 6.1
+//   153 bytes, 10^6           2048 rows 6.6 / 7.3, 3000 7.4 / 7.4, 4096 8.9 / 7.3, 16,384 22 / 7.9, 65,536 71 / 13.3
+//   521 bytes, 2^20           4096 rows 8.3 / 8.9, 6000 11.8 / 9.5, 16,384 22 / 11.1
+//   3 KB, 2 * 10^5            8192 rows 17.9 / 21.0, 16,384 29.1 / 26.1; 6 KB: 8192 31.6 / 32.0, 16,384 58 / 39.5
+// and 16 / 32 / 64 / 256 strata to a workgroup: 153 bytes, 16,384 rows 8.5 / 7.9 / 8.7 / 16.1, 65,536 25 / 17 / 13.3 /
+// 16.7, 262,144 84 / 51 / 38 / 31; 521 bytes, 8192 rows 9.6 / 10.7 / 14.0 / 34.5, 32,768 21 / 13.8 / 16.8 / 36; 3 KB,
+// 65,536 rows 99 / 96 / 91 / 201.
+static bool takes_lds(int64_t rows, uint64_t rest) {
+    return rest <= 384 && rows >= (rest <= 16 ? 3072 : rest <= 64 ? 5120 : 12288);
+}
+static int lds_strata(int64_t rows, uint64_t rest) {
+    if (rows <= 20480 && rest > 16) return 16;
+    return rows <= 40960 ? 32 : rows <= 98304 || rest > 64 ? 64 : 256;
+}
+
 // `nbatch` batches of `batch` stratified samples each, as nbatch successive mrb_per_sample calls on
 // an unchanged tree would draw them. Outputs hold nbatch * batch rows, batch after batch.
 static int per_sample_impl(Per* b, int64_t nbatch, int64_t batch, float beta, const float* uniforms,
@@ -1531,10 +1549,11 @@ static int per_sample_impl(Per* b, int64_t nbatch, int64_t batch, float beta, co
         // batch (see generator_calls)
         if (!uniforms) a.calls = 0;
     }
-    const float* const draws = a.uniforms;  // the caller's, or NULL: the generator's, computed by the kernels
-    const int64_t max_bytes = widest_field(b->rows);
+    uint64_t rest = 0;  // granules of a row that the LDS-top kernel's threads do not copy for their own stratum alone
+    for (int f = 0; f < t.nfields; ++f) rest += f < kLdsOwn && t.units[f] == 1 ? 0 : t.units[f];
     int path = (int)b->sample_path;
-    if (path == 0) path = (batch >= 8192 && max_bytes <= 256) ? 2 : 1;
+    if (path == 0) path = takes_lds(nbatch * batch, rest) ? 2 : 1;
+    if (rest > 1u << 23) path = 1;  // (it numbers a workgroup's granules in 32 bits)
     if (next) {
         rc = sample_wide(b->rows, a, t, nbatch, s, next);  // always the wide-row kernel: the gathered field is wide
         if (rc) return rc;
@@ -1542,23 +1561,18 @@ static int per_sample_impl(Per* b, int64_t nbatch, int64_t batch, float beta, co
         rc = sample_wide(b->rows, a, t, nbatch, s);
         if (rc) return rc;
     } else {
-        // the LDS-top kernel takes one batch per launch (its batches are large enough to fill the chip)
         int levels = b->lds_levels > 0 ? (int)b->lds_levels : 9;
         if (levels > b->depth) levels = b->depth;
         const uint32_t ntop = (2u << levels) < 4 ? 4 : (2u << levels);
-        const size_t lds = ntop * sizeof(float) + (kWG + 1) * sizeof(int64_t);
-        for (int64_t i = 0; i < nbatch; ++i) {
-            SampleArgs ai = a;
-            IoTable ti = t;
-            ai.uniforms = draws ? draws + i * batch : nullptr;
-            ai.calls = a.calls + (uint64_t)i;
-            ai.out_idx = out_indices + i * batch;
-            ai.out_w = out_weights + i * batch;
-            for (int f = 0; f < t.nfields; ++f) ti.io[f] = t.io[f] + (uint64_t)i * batch * t.row_bytes[f];
-            hipLaunchKernelGGL(k_per_sample_lds, dim3((uint32_t)((batch + kWG - 1) / kWG)), dim3(kLdsWG), lds, s, ai.sum,
-                               ai.uniforms, ai.mn, ai.depth, levels, (int)batch, beta, ai.seed, ai.calls, ai, ti);
-            LAUNCH_CHECK("k_per_sample_lds");
-        }
+        const int strata = lds_strata(nbatch * batch, rest);
+        const size_t lds = ntop * sizeof(float) + ((size_t)strata + 1) * sizeof(int64_t);
+        auto* const kernel = strata == 16   ? k_per_sample_lds<16>
+                             : strata == 32 ? k_per_sample_lds<32>
+                             : strata == 64 ? k_per_sample_lds<64>
+                                            : k_per_sample_lds<256>;
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)((batch + strata - 1) / strata), (uint32_t)nbatch), dim3(kLdsWG), lds, s, a.sum,
+                           a.uniforms, a.mn, a.depth, levels, (int)batch, beta, a.seed, a.calls, (uint32_t)rest, a, t);
+        LAUNCH_CHECK("k_per_sample_lds");
     }
     if (!uniforms) {
         b->calls += (uint64_t)nbatch;

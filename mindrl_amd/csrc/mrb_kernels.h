@@ -1269,38 +1269,61 @@ __device__ __forceinline__ uint32_t descend_group(const float* __restrict__ sum,
 
 
 // ---------------------------------------------------------------------------
-// PER sample, many narrow rows: one workgroup per 256 strata. The top
+// PER sample, many narrow rows: one workgroup per kStrata strata. The top
 // `lds_levels` levels of the sum tree (nodes [1, 2 << lds_levels)) are staged
 // in LDS once per workgroup, so each thread's descent reads HBM/L2 only for
-// the levels below; then the workgroup gathers its 256 rows with coalesced
+// the levels below; then the workgroup gathers its rows with coalesced
 // writes. Same outputs, bit for bit, as k_per_sample_wide.
+// What bounds it: a chain of trips (the arguments and the top, the descent's two or three, the rows), and, with few
+// workgroups, the compute units that have none: 256 strata to a workgroup used 64 of them for a batch of 16,384. The
+// rows' granules are numbered over all fields and four to a thread are in flight at once; field by field every field was
+// a trip of its own. 16,384 rows of
+// 153 bytes 17.1 -> 7.9 us, 13,764 of 139 bytes 15.8 -> 8.1, 16,384 of 521 bytes 35 -> 11.1.
 // ---------------------------------------------------------------------------
 // sum .. calls repeat members of `a` as plain leading parameters: those are preloaded into scalar
 // registers, so the staging loads go out when the wave starts instead of a round trip to the
 // kernel-argument segment later.
+constexpr int kLdsOwn = 4;  // leading fields whose row is one granule: every thread copies its own stratum's
+
+// rest: granules of a row in the other fields. blockIdx.y: the batch, of several that are drawn at once (each stratified
+// on its own, with the generator's next call counter).
+template <int kStrata>
 __global__ __launch_bounds__(kLdsWG) void k_per_sample_lds(const float* __restrict__ sum, const float* __restrict__ uniforms,
                                                         const float* __restrict__ mn, int depth, int lds_levels,
-                                                        int batch, float beta, uint64_t seed, uint64_t calls,
+                                                        int batch, float beta, uint64_t seed, uint64_t calls, uint32_t rest,
                                                         SampleArgs a, IoTable t) {
-    extern __shared__ float s_top[];  // [2 << lds_levels] floats, then kWG int64 slots
+    extern __shared__ float s_top[];  // [2 << lds_levels] floats, then kStrata + 1 int64: the slots, the number of stored rows
     __shared__ float s_max_w;
+    // the field table (see k_res_push); units: of the fields that make up `rest`
+    __shared__ uint8_t *s_io[MRB_MAX_FIELDS], *s_store[MRB_MAX_FIELDS];
+    __shared__ uint32_t s_bytes[MRB_MAX_FIELDS], s_stride[MRB_MAX_FIELDS], s_units[MRB_MAX_FIELDS], s_vl[MRB_MAX_FIELDS];
     const uint32_t ntop = 2u << lds_levels;
     int64_t* s_slot = reinterpret_cast<int64_t*>(s_top + (ntop < 4 ? 4 : ntop));
-    const int64_t k0 = (int64_t)blockIdx.x * kWG;
-    const int64_t k = k0 + threadIdx.x;
+    const int64_t row0 = (int64_t)blockIdx.y * batch;  // the batch's first row of the call's
+    const int64_t k0 = (int64_t)blockIdx.x * kStrata;
+    const int64_t k = threadIdx.x < kStrata ? k0 + threadIdx.x : batch;
     if (threadIdx.x >= kWG) {
+        const int f = (int)threadIdx.x - kWG;
+        if (f < t.nfields) {
+            s_io[f] = t.io[f];
+            s_store[f] = t.store[f];
+            s_bytes[f] = t.row_bytes[f];
+            s_stride[f] = t.stride[f];
+            s_units[f] = f < kLdsOwn && t.units[f] == 1 ? 0 : t.units[f];
+            s_vl[f] = t.vec_log2[f];
+        }
         // The helper wave: the weights' common denominator (pmin / total * size)^-beta, once per
         // workgroup, off the strata's path (two loads and a power: as long as staging the top).
         // (the number of stored rows: the argument, or read from the device when the counters live there)
-        if (threadIdx.x == kWG) s_slot[kWG] = a.size >= 0 ? a.size : counters_behind(a.err)[kCntSize];
+        if (threadIdx.x == kWG) s_slot[kStrata] = a.size >= 0 ? a.size : counters_behind(a.err)[kCntSize];
         __syncthreads();
-        if (threadIdx.x == kWG) s_max_w = powf_det(mn[1] / sum[1] * (float)s_slot[kWG], -beta);
+        if (threadIdx.x == kWG) s_max_w = powf_det(mn[1] / sum[1] * (float)s_slot[kStrata], -beta);
         __syncthreads();
         return;
     }
     // the stratum's draw is requested together with the top of the tree
     float u = 0.0f;
-    if (k < batch && uniforms) u = uniforms[k];
+    if (k < batch && uniforms) u = uniforms[row0 + k];
     if (ntop >= 4) {
         for (uint32_t i = threadIdx.x * 4; i < ntop; i += kWG * 4)
             *reinterpret_cast<float4*>(s_top + i) = *reinterpret_cast<const float4*>(sum + i);
@@ -1308,12 +1331,11 @@ __global__ __launch_bounds__(kLdsWG) void k_per_sample_lds(const float* __restri
         s_top[threadIdx.x] = sum[threadIdx.x];
     }
     __syncthreads();
-    constexpr int kOwn = 4;  // leading fields whose row is one granule: every thread copies its own stratum's
-    AnyGranule own[kOwn];
+    AnyGranule own[kLdsOwn];
     float weight = 0.0f;
     if (k < batch) {
         const float total = s_top[1];
-        if (!uniforms) u = rng_uniform(seed, generator_calls(uniforms, calls, a.size, a.err), (uint64_t)k);
+        if (!uniforms) u = rng_uniform(seed, generator_calls(uniforms, calls, a.size, a.err) + blockIdx.y, (uint64_t)k);
         float mass = (u + (float)k) * (total / (float)batch);  // each operation rounded once
         uint32_t node = 1;
         int d = 0;
@@ -1351,38 +1373,47 @@ __global__ __launch_bounds__(kLdsWG) void k_per_sample_lds(const float* __restri
         const int64_t slot = idx < a.capacity ? idx : a.capacity - 1;
         // the row's scalar fields are requested now, before the weight's arithmetic and the barrier
 #pragma unroll
-        for (int f = 0; f < kOwn; ++f)
+        for (int f = 0; f < kLdsOwn; ++f)
             if (f < t.nfields && t.units[f] == 1)
                 own[f].load(as_global(t.store[f]) + (uint64_t)slot * t.stride[f], t.vec_log2[f]);
-        a.out_idx[k] = idx;
-        const int64_t size = s_slot[kWG];  // left there by the helper wave before the first barrier
+        a.out_idx[row0 + k] = idx;
+        const int64_t size = s_slot[kStrata];  // left there by the helper wave before the first barrier
         weight = powf_det(picked / total * (float)size, -beta);
         sample_flags(a, total, idx, size);
         s_slot[threadIdx.x] = slot;
     }
     __syncthreads();
-    const uint32_t rows = (uint32_t)((batch - k0) < kWG ? (batch - k0) : kWG);
+    const uint32_t rows = (uint32_t)((batch - k0) < kStrata ? (batch - k0) : kStrata);
     if (k < batch) {
-        a.out_w[k] = weight / s_max_w;
+        a.out_w[row0 + k] = weight / s_max_w;
 #pragma unroll
-        for (int f = 0; f < kOwn; ++f)
+        for (int f = 0; f < kLdsOwn; ++f)
             if (f < t.nfields && t.units[f] == 1)
-                own[f].store(as_global(t.io[f]) + (uint64_t)k * t.row_bytes[f], t.vec_log2[f]);
+                own[f].store(as_global(t.io[f]) + (uint64_t)(row0 + k) * t.row_bytes[f], t.vec_log2[f]);
     }
-    // fields of several granules per row (and fields past the first kOwn): coalesced over the workgroup's rows
-    for (int f = 0; f < t.nfields; ++f) {
-        const uint32_t units = t.units[f];
-        if (f < kOwn && units == 1) continue;
-        const uint32_t vl = t.vec_log2[f];
-        const uint64_t work = (uint64_t)rows * units;
-        for (uint64_t w = threadIdx.x; w < work; w += kWG) {
-            uint64_t r;
-            uint32_t u;
-            split_work(w, units, r, u);
-            const uint32_t off = granule_offset(u, vl, t.row_bytes[f]);
-            copy_granule(as_global(t.io[f]) + (uint64_t)(k0 + (int64_t)r) * t.row_bytes[f] + off,
-                         as_global(t.store[f]) + (uint64_t)s_slot[r] * t.stride[f] + off, vl);
+    // the other granules: field by field and row by row, coalesced over the workgroup's rows
+    const uint32_t work = rows * rest;
+    constexpr int kTrip = 4;
+    for (uint32_t base = threadIdx.x; base < work; base += kTrip * kWG) {
+        gbyte* to[kTrip];
+        uint32_t vl[kTrip];
+        AnyGranule held[kTrip];
+#pragma unroll
+        for (int q = 0; q < kTrip; ++q) {
+            uint32_t w = base + (uint32_t)q * kWG;
+            to[q] = nullptr;
+            if (w >= work) continue;
+            int f = 0;
+            while (w >= rows * s_units[f]) w -= rows * s_units[f++];  // (ends at a field of `rest`: w is below their total)
+            const uint32_t units = s_units[f], r = w / units;
+            vl[q] = s_vl[f];
+            const uint32_t off = granule_offset(w - r * units, vl[q], s_bytes[f]);
+            held[q].load(as_global(s_store[f]) + (uint64_t)s_slot[r] * s_stride[f] + off, vl[q]);
+            to[q] = as_global(s_io[f]) + (uint64_t)(row0 + k0 + r) * s_bytes[f] + off;
         }
+#pragma unroll
+        for (int q = 0; q < kTrip; ++q)
+            if (to[q]) held[q].store(to[q], vl[q]);
     }
 }
 

@@ -1,0 +1,49 @@
+"""Samples of thousands of rows, where the kernel and its workgroups are chosen by the number of rows and their
+size: on both sides of every line of the rules, last workgroups of one stratum, several batches at once (also of fewer rows
+than a workgroup has strata), and the counters on the device. Indices, weights and rows against the oracle, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import assert_sample_equal, random_rows, to_dev, torch_types
+
+pytestmark = pytest.mark.gpu
+
+ROWS = {
+    "tiny": ([(1,), (1,)], [np.int32, np.float32]),
+    "mujoco": ([(17,), (6,), (1,), (17,), (1,)], [np.float32, np.float32, np.float32, np.float32, np.bool_]),
+    "odd": ([(64,), (3,), (1,), (65,), (5,), (1,), (2,)], [np.float32, np.uint8, np.int64, np.float32, np.float16, np.bool_, np.int32]),
+    "wide": ([(1802,), (36,), (364,), (1,)], [np.uint8, np.bool_, np.float16, np.int64]),
+}
+
+
+@pytest.mark.parametrize("rows,cap,batches", [
+    ("tiny", 3000, [(3071, 1), (3072, 1), (3105, 1), (40_960, 1), (40_961, 1), (98_305, 1)]),
+    ("mujoco", 9000, [(3072, 1), (5121, 1), (20_481, 1), (41_025, 1), (98_305, 1), (17, 200), (769, 4), (1, 3072)]),
+    ("odd", 6000, [(5119, 1), (5120, 1), (20_480, 1), (20_481, 1), (40_961, 1), (33, 160)]),
+    ("wide", 2000, [(12_287, 1), (12_288, 1), (20_481, 1), (6145, 2)])])
+@pytest.mark.parametrize("device_counters", [0, 1])
+def test_samples_of_many_rows(rows, cap, batches, device_counters):
+    from mindrl_amd.core import PriorityReplayBuffer
+    from oracle import orc
+    shapes, dtypes = ROWS[rows]
+    rng = np.random.default_rng(cap)
+    g = PriorityReplayBuffer(0.6, cap, 8, shapes, torch_types(dtypes), seed0=2)
+    c = orc.OraclePER(0.6, cap, shapes, dtypes, seed=2)
+    new = random_rows(rng, cap, shapes, dtypes)
+    pr = (np.abs(rng.normal(size=cap)) + 1e-3).astype(np.float32)
+    g.insert(*to_dev(new), priorities=torch.from_numpy(pr).cuda())
+    c.push(new, cap, pr)
+    g.set_option("device_counters", device_counters)
+    for batch, n in batches:
+        what = "%s batch %d x %d" % (rows, batch, n)
+        g._sample_size = batch  # (one buffer for all batch sizes)
+        if n == 1:
+            assert_sample_equal(g.sample(0.4), c.sample(batch, 0.4), what)
+            u = rng.random(batch).astype(np.float32)
+            assert_sample_equal(g.sample(0.4, uniforms=torch.from_numpy(u).cuda()), c.sample(batch, 0.4, u), what)
+        else:
+            out = g.sample_many(n, 0.4)
+            for i in range(n):
+                assert_sample_equal([o[i] for o in out], c.sample(batch, 0.4), "%s number %d" % (what, i))
+    g.destroy()
