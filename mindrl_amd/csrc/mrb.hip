@@ -283,7 +283,7 @@ struct NextRows {
     void* out = nullptr;
 };
 
-constexpr int64_t kRowWaveMinRows = 2048;  // fewest rows of a launch that go to the wave-per-row sample kernel
+constexpr int64_t kRowWaveMinRows = 2048;  // fewest rows of a launch that go to the wave-per-row sample and gather kernels
 
 template <int kInF, bool kTen, bool kOneWide>
 void launch_sample_next(dim3 grid, const SampleArgs& a, const WidePlan& plan, const NextPlan& nx, hipStream_t s) {
@@ -399,7 +399,17 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
         WidePlan plan;
         dim3 grid;
         plan.nbatch = 1;
-        switch (wide_plan(r, t, n, plan, grid)) {
+        const int inflight = wide_plan(r, t, n, plan, grid);
+        // Thousands of rows of up to 4 KB: a wave per row (3 KB, us, workgroup / wave: 1024 rows 6.2 / 6.7, 2048 7.5 / 6.8,
+        // 8192 20.7 / 13.6; 1 KB: 2048 5.2 / 5.5, 4096 7.4 / 5.9).
+        if (r.row_split == 0 && plan.split == 1 && plan.wide_items <= (uint32_t)kRowWaveInF * 64u && plan.narrow_items <= 256u &&
+            inflight != 0 && n >= kRowWaveMinRows) {
+            hipLaunchKernelGGL(k_rows_gather_rows, dim3((uint32_t)((n + kRowWaveWG / 64 - 1) / (kRowWaveWG / 64))), dim3(kRowWaveWG),
+                               0, s, indices, mode, count, fixed_slot, seed, calls, n, out_indices, err, plan);
+            LAUNCH_CHECK("k_rows_gather_rows");
+            return MRB_OK;
+        }
+        switch (inflight) {
             case 0: return MRB_EINVAL;
             case 2: launch_gather_wide<2>(grid, indices, mode, count, fixed_slot, seed, calls, out_indices, err, plan, s); break;
             default: launch_gather_wide<8>(grid, indices, mode, count, fixed_slot, seed, calls, out_indices, err, plan, s); break;

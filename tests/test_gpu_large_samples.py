@@ -1,11 +1,11 @@
-"""Samples of thousands of rows, where the kernel and its workgroups are chosen by the number of rows and their
+"""Samples and gathers of thousands of rows, where the kernel and its workgroups are chosen by the number of rows and their
 size: on both sides of every line of the rules, last workgroups of one stratum, several batches at once (also of fewer rows
 than a workgroup has strata), and the counters on the device. Indices, weights and rows against the oracle, bit for bit."""
 import numpy as np
 import pytest
 import torch
 
-from gpu_util import assert_sample_equal, random_rows, to_dev, torch_types
+from gpu_util import assert_sample_equal, random_rows, t2n, to_dev, torch_types
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +47,28 @@ def test_samples_of_many_rows(rows, cap, batches, device_counters):
             for i in range(n):
                 assert_sample_equal([o[i] for o in out], c.sample(batch, 0.4), "%s number %d" % (what, i))
     g.destroy()
+
+
+@pytest.mark.parametrize("shapes,dtypes", [
+    ([(1024,)], [np.uint8]), ([(376,), (17,), (1,), (376,), (1,)], [np.float32, np.float32, np.float32, np.float32, np.bool_]),
+    ([(4079,), (16,)], [np.uint8, np.uint8]), ([(4097,)], [np.uint8]), ([(2970,)] + [(15,)] * 15, [np.uint8] * 16),
+    ([(1025,)] + [(15,), (13,), (1,)] * 5, [np.uint8] * 16)])
+@pytest.mark.parametrize("packed", [0, 4096])
+def test_gathers_of_many_rows(shapes, dtypes, packed):
+    from mindrl_amd.core import UniformReplayBuffer
+    from oracle import orc
+    if packed and sum(int(np.prod(s)) * np.dtype(d).itemsize for s, d in zip(shapes, dtypes)) > 4000:
+        pytest.skip("rows too large to pack")
+    rng = np.random.default_rng(len(shapes))
+    cap = 4200
+    for batch in (2047, 2048, 4099):
+        g = UniformReplayBuffer(batch, cap, shapes, torch_types(dtypes), seed=4, packed_rows=packed)
+        c = orc.OracleUniform(cap, shapes, dtypes, seed=4)
+        for n in (4100, 500):
+            new = random_rows(rng, n, shapes, dtypes)
+            g.insert(to_dev(new))
+            c.append(new, n)
+        idx, fields = g.sample_with_indices()
+        want_idx, want = c.sample(batch)
+        assert np.array_equal(t2n(idx), want_idx) and all(np.array_equal(t2n(a), b) for a, b in zip(fields, want)), batch
+        g.destroy()
