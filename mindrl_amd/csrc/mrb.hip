@@ -18,6 +18,7 @@
 #include "mrb_kernels.h"
 #include "mrb_range.h"
 #include "mrb_returns.h"
+#include "mrb_samples.h"
 #include "../../include/mrb_more.h"
 
 namespace {
@@ -1573,16 +1574,8 @@ static int per_sample_impl(Per* b, int64_t nbatch, int64_t batch, float beta, co
     } else {
         int levels = b->lds_levels > 0 ? (int)b->lds_levels : 9;
         if (levels > b->depth) levels = b->depth;
-        const uint32_t ntop = (2u << levels) < 4 ? 4 : (2u << levels);
-        const int strata = lds_strata(nbatch * batch, rest);
-        const size_t lds = ntop * sizeof(float) + ((size_t)strata + 1) * sizeof(int64_t);
-        auto* const kernel = strata == 16   ? k_per_sample_lds<16>
-                             : strata == 32 ? k_per_sample_lds<32>
-                             : strata == 64 ? k_per_sample_lds<64>
-                                            : k_per_sample_lds<256>;
-        hipLaunchKernelGGL(kernel, dim3((uint32_t)((batch + strata - 1) / strata), (uint32_t)nbatch), dim3(kLdsWG), lds, s, a.sum,
-                           a.uniforms, a.mn, a.depth, levels, (int)batch, beta, a.seed, a.calls, (uint32_t)rest, a, t);
-        LAUNCH_CHECK("k_per_sample_lds");
+        const hipError_t e = launch_per_sample_lds(a, t, nbatch, lds_strata(nbatch * batch, rest), levels, (uint32_t)rest, s);
+        if (e != hipSuccess) return fail(MRB_EHIP, "launch k_per_sample_lds: %s", hipGetErrorString(e));
     }
     if (!uniforms) {
         b->calls += (uint64_t)nbatch;

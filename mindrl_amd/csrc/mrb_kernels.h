@@ -6,286 +6,12 @@
 #include <stdint.h>
 
 #include "../../include/mrb.h"
-#include "mrb_device.h"
+#include "mrb_rows.h"
 #include "mrb_tree.h"
 
 namespace mrb {
 
-constexpr int kWG = 256;          // threads per workgroup of the row and sample kernels
-constexpr int kLdsWG = kWG + 64;  // the LDS-top sample kernel: kWG strata and a helper wave
 constexpr int kTopMaxDepth = 12;  // deepest level k_tree_top normally starts from (4096 nodes)
-
-// Per-call table of the fields of a row, passed to kernels by value.
-// `store` is the field's place in the buffer - row r of the field at store + r * stride: a [capacity, row_bytes]
-// matrix of its own, or a column of the packed rows -, `io` the caller's contiguous [n, row_bytes] matrix
-// (source of an append, destination of a gather).
-struct IoTable {
-    int nfields;
-    uint8_t* store[MRB_MAX_FIELDS];
-    uint8_t* io[MRB_MAX_FIELDS];
-    uint32_t row_bytes[MRB_MAX_FIELDS];
-    uint32_t stride[MRB_MAX_FIELDS];    // bytes from one row of the field to the next in `store`: row_bytes when every
-                                        // field has an array of its own, the packed row's size when rows are packed
-    uint32_t units[MRB_MAX_FIELDS];     // copy granules of a row: row_bytes / 2^vec_log2, rounded up
-    uint32_t vec_log2[MRB_MAX_FIELDS];  // copy granule: the largest of 16, 8, 4, 2 and 1 bytes that a row holds
-    uint64_t prefix[MRB_MAX_FIELDS + 1];  // running sum of n * units over fields
-};
-
-// Row pointers reach the kernels inside by-value tables, where the compiler cannot
-// see that they point to global memory; the qualified type makes every row access a
-// global_load/global_store rather than a flat one.
-using gbyte = __attribute__((address_space(1))) uint8_t;
-__device__ __forceinline__ gbyte* as_global(uint8_t* p) { return (gbyte*)p; }
-__device__ __forceinline__ const gbyte* as_global(const uint8_t* p) { return (const gbyte*)p; }
-
-// A row of a field is copied in granules of 16 bytes (of 8, 4, 2 or 1 where it has fewer), whatever its size and
-// alignment: granule u starts at byte u * 16, the last one where it ends with the row, over bytes the one before it
-// has too (both bring the same bytes). A granule may lie at any address; the device's loads and stores take that. A row
-// of 147 bytes is then 10 granules rather than 147, one of 111 floats 28 rather than 111. Measured, per call: 250
-// prioritized rows of 925 bytes 8.3 -> 4.4 us, 8192 uniform rows of 268 bytes in odd fields 10.5 -> 5.3 us.
-__device__ __forceinline__ uint32_t granule_offset(uint32_t unit, uint32_t vl, uint32_t row_bytes) {
-    const uint32_t at = unit << vl, last = row_bytes - (1u << vl);
-    return at < last ? at : last;
-}
-
-using granule_t = __attribute__((ext_vector_type(4))) uint32_t;  // one 16-byte copy granule
-// the same, and smaller ones, at any address
-using granule16_u = __attribute__((ext_vector_type(4), aligned(1))) uint32_t;
-using granule8_u = __attribute__((ext_vector_type(2), aligned(1))) uint32_t;
-typedef uint32_t granule4_u __attribute__((aligned(1)));
-typedef uint16_t granule2_u __attribute__((aligned(1)));
-#define MRB_GLOBAL __attribute__((address_space(1)))
-
-// One granule of 1 << vl bytes. Rows are read once and written once, so both
-// sides bypass the caches' retention (non-temporal).
-__device__ __forceinline__ void copy_granule(gbyte* dst, const gbyte* src, uint32_t vl) {
-    switch (vl) {
-        case 4: {
-            const granule16_u t = __builtin_nontemporal_load((const MRB_GLOBAL granule16_u*)src);
-            __builtin_nontemporal_store(t, (MRB_GLOBAL granule16_u*)dst);
-            break;
-        }
-        case 3: {
-            const granule8_u t = __builtin_nontemporal_load((const MRB_GLOBAL granule8_u*)src);
-            __builtin_nontemporal_store(t, (MRB_GLOBAL granule8_u*)dst);
-            break;
-        }
-        case 2: *(MRB_GLOBAL granule4_u*)dst = *(const MRB_GLOBAL granule4_u*)src; break;
-        case 1: *(MRB_GLOBAL granule2_u*)dst = *(const MRB_GLOBAL granule2_u*)src; break;
-        default: *dst = *src; break;
-    }
-}
-
-// One granule of 1 << vl bytes held between its load and its store. vl is wave-uniform; every size
-// has its own member so that no value of one load is merged with another's (a merge would make the
-// compiler wait for the load right away).
-struct AnyGranule {
-    granule_t q;
-    uint64_t d;
-    uint32_t w;
-    uint16_t h;
-    uint8_t b;
-    typedef uint64_t u64_u __attribute__((aligned(1)));
-    __device__ __forceinline__ void load(const gbyte* src, uint32_t vl) {
-        switch (vl) {
-            case 4: q = *(const MRB_GLOBAL granule16_u*)src; break;
-            case 3: d = *(const MRB_GLOBAL u64_u*)src; break;
-            case 2: w = *(const MRB_GLOBAL granule4_u*)src; break;
-            case 1: h = *(const MRB_GLOBAL granule2_u*)src; break;
-            default: b = *src; break;
-        }
-    }
-    __device__ __forceinline__ void store(gbyte* dst, uint32_t vl) const {
-        switch (vl) {
-            case 4: *(MRB_GLOBAL granule16_u*)dst = q; break;
-            case 3: *(MRB_GLOBAL u64_u*)dst = d; break;
-            case 2: *(MRB_GLOBAL granule4_u*)dst = w; break;
-            case 1: *(MRB_GLOBAL granule2_u*)dst = h; break;
-            default: *dst = b; break;
-        }
-    }
-};
-
-__device__ __forceinline__ int field_of(const IoTable& t, uint64_t w) {
-    int f = 0;
-    while (f + 1 < t.nfields && w >= t.prefix[f + 1]) ++f;
-    return f;
-}
-
-__device__ __forceinline__ void split_work(uint64_t local, uint32_t units, uint64_t& row, uint32_t& unit) {
-    if (local <= 0xffffffffull) {
-        const uint32_t l32 = (uint32_t)local;
-        const uint32_t r = l32 / units;
-        row = r;
-        unit = l32 - r * units;
-    } else {
-        row = local / units;
-        unit = (uint32_t)(local - row * units);
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Ring append: rows [0, nrows) of each io matrix go to slots
-// (first_slot + row) mod capacity. Replaces P.BufferAppend
-// (mindspore_rl/core/uniform_replay_buffer.py:82,114) and the row copy of
-// PriorityReplayBufferPush (mindspore_rl/core/priority_replay_buffer.py:67-69).
-// The host guarantees nrows <= capacity, so no two rows share a slot.
-// ---------------------------------------------------------------------------
-// src_capacity > 0: the source is itself a ring of that many rows and row r is read from its
-// slot (src_first + r) mod src_capacity (buffer-to-buffer copy); 0: the source is contiguous.
-struct PutArgs {
-    IoTable t;
-    int64_t capacity, first_slot, src_capacity, src_first;
-    uint32_t blocks;  // workgroups doing this copy when it rides along in another kernel's launch (0: none)
-    // first_slot < 0: the buffer's counters live on the device (see Counters below), the rows go to
-    // (pushes mod capacity) onwards, and src_first - unused then, the source is never a ring - holds the
-    // counters' address
-};
-
-// A prioritized buffer's counters as device memory, for callers that record their loop into a HIP
-// graph: kernels then take the ring position, the number of stored rows and the generator's call
-// counter from here, and a one-thread kernel advances them after each call, so that every replay
-// continues where the one before stopped.
-// Kernels are told through a negative first slot / row count in their arguments and find the counters
-// behind the buffer's error word (one allocation: 16 bytes of flags, then the counters), so that the
-// arguments of the ordinary case are what they were.
-// ([3] counts the reports of a launch that moves the counters on; [4] is the ring position, pushes mod capacity, kept
-// beside the count so that no kernel divides)
-constexpr int kCntPushes = 0, kCntSize = 1, kCntCalls = 2, kCntPos = 4, kCntWords = 5;
-
-__device__ __forceinline__ const int64_t* counters_behind(const uint32_t* err) {
-    return reinterpret_cast<const int64_t*>(err + 4);
-}
-// A prioritized buffer's running max lives in the same allocation, kMaxpBehindErr bytes behind the error word: a
-// kernel that has its address among its preloaded arguments finds the counters without reading another argument.
-constexpr int kMaxpBehindErr = 64;
-__device__ __forceinline__ int64_t* counters_before(float* maxp) {
-    return reinterpret_cast<int64_t*>(reinterpret_cast<char*>(maxp) - kMaxpBehindErr + 16);
-}
-__device__ __forceinline__ int64_t ring_position(const int64_t* counters, int64_t capacity) {
-    return counters[kCntPos];
-}
-// The counters after a push of `pushed` rows (at most `capacity`), stored.
-__device__ __forceinline__ void counters_store_advanced(int64_t* counters, int64_t pushes, int64_t size, int64_t pos,
-                                                        int64_t pushed, int64_t capacity) {
-    counters[kCntPushes] = pushes + pushed;
-    size += pushed;
-    counters[kCntSize] = size < capacity ? size : capacity;
-    pos += pushed;
-    counters[kCntPos] = pos < capacity ? pos : pos - capacity;
-}
-
-// The generator's call counter for a sample kernel: the argument, or - when the counters live on the device (a
-// negative row count tells) and the generator supplies the draws - the device's counter plus the argument (the
-// number of the batch among those the call launches one by one).
-__device__ __forceinline__ uint64_t generator_calls(const float* uniforms, uint64_t calls, int64_t size, const uint32_t* err) {
-    if (uniforms || size >= 0) return calls;
-    return (uint64_t)counters_behind(err)[kCntCalls] + calls;
-}
-
-// The counters as a wave found them, and what its report returned (see counters_report).
-struct CounterTicket {
-    int64_t pushes, size, pos;
-    uint32_t before;  // reports ahead of this wave's
-};
-// (atomic loads: vector loads past the compute unit's caches, which wait for nothing but themselves)
-__device__ __forceinline__ CounterTicket counters_take(const uint32_t* err) {
-    const int64_t* counters = counters_behind(err);
-    CounterTicket t;
-    t.pushes = __hip_atomic_load(counters + kCntPushes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    t.size = __hip_atomic_load(counters + kCntSize, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    t.pos = __hip_atomic_load(counters + kCntPos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    t.before = 0;
-    return t;
-}
-__device__ __forceinline__ int64_t ticket_position(const CounterTicket& t, int64_t capacity) { return t.pos; }
-
-// A push moves the device-resident counters on in its own last launch. Where that launch is also the one whose
-// workgroups read the ring position (`readers` of them: the tree workgroup and the row copy's), every such
-// workgroup reports here when it is done, and the last one to report advances the counters: no workgroup waits
-// for another, and none can read a position already moved on. readers <= 1: the caller is the only reader left.
-// Called by every thread of the workgroup (it contains a barrier); the counters' fourth word counts the reports.
-// `known`: the counters as thread 0 took them when the kernel started (nobody changes them before this advance);
-// without it thread 0 requests them here, ahead of the barrier and the report.
-__device__ __forceinline__ void counters_push_done(uint32_t* err, int64_t pushed, int64_t capacity, uint32_t readers,
-                                                   const CounterTicket* known = nullptr) {
-    if (pushed <= 0) return;  // uniform over the launch
-    CounterTicket t{};
-    if (threadIdx.x == 0) t = known ? *known : counters_take(err);
-    __syncthreads();  // every wave's reads of the position are behind it
-    if (threadIdx.x != 0) return;
-    int64_t* counters = reinterpret_cast<int64_t*>(err + 4);
-    if (readers > 1) {
-        unsigned int* arrived = reinterpret_cast<unsigned int*>(counters + 3);
-        if (atomicAdd(arrived, 1u) != readers - 1) return;
-        atomicExch(arrived, 0u);
-    }
-    counters_store_advanced(counters, t.pushes, t.size, t.pos, pushed, capacity);
-}
-
-// The same for the one-launch pushes whose tree work is a single wave (k_push_one, k_tree_wg_push,
-// k_tree_paths_push), wave by wave and EARLY: what must precede the advance is every wave's READ of the
-// counters, not its work. A wave takes the counters (counters_take: loads only), reports as soon as the values
-// are there (counters_report: one atomic whose operand depends on the loaded values, so that it cannot be issued
-// before they arrive; its result is not awaited here) and goes on with its work; when that is done it looks at
-// what the atomic returned (counters_settle) and, if it was the last of the `readers` waves to report, stores the
-// advanced counters, computed from the values it took - no load, and no round trip to L2 at the kernel's end.
-// All three are called by whole waves; lane 0 acts. readers <= 1: the calling wave is the only reader.
-__device__ __forceinline__ void counters_report(CounterTicket& t, uint32_t* err, uint32_t readers, uint32_t lane) {
-    if (readers <= 1 || lane != 0) return;
-    unsigned int* arrived = reinterpret_cast<unsigned int*>(reinterpret_cast<int64_t*>(err + 4) + 3);
-    // (both counters are non-negative: the operand is 1)
-    t.before = atomicAdd(arrived, 1u + (unsigned int)((uint64_t)(t.pushes | t.size | t.pos) >> 63));
-}
-__device__ __forceinline__ void counters_settle(const CounterTicket& t, uint32_t* err, int64_t pushed, int64_t capacity,
-                                                uint32_t readers, uint32_t lane) {
-    if (lane != 0) return;
-    int64_t* counters = reinterpret_cast<int64_t*>(err + 4);
-    if (readers > 1) {
-        if (t.before != readers - 1) return;
-        atomicExch(reinterpret_cast<unsigned int*>(counters + 3), 0u);
-    }
-    counters_store_advanced(counters, t.pushes, t.size, t.pos, pushed, capacity);
-}
-
-// How a workgroup that carries a row copy in another kernel's launch ends. The compiler lays such a kernel out as
-// if the tree workgroup's code could follow the copy, and without the explicit wait it makes the tree workgroup
-// wait, early on, for loads that only the copy ever issues (its first requests then go out one after the other
-// instead of together: a third of a microsecond on a one-workgroup call).
-__device__ __forceinline__ void rider_ends() {
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_endpgm();
-}
-
-// The copy itself, by workgroup `block` of `nblocks` (grid-stride over the granules). known_first >= 0: the
-// first slot, already read from the device's counters by the caller.
-__device__ __forceinline__ void rows_put_part(const PutArgs& p, uint32_t block, uint32_t nblocks, int64_t known_first = -1) {
-    const IoTable& t = p.t;
-    const uint64_t total = t.prefix[t.nfields];
-    const uint64_t stride = (uint64_t)nblocks * blockDim.x;
-    const int64_t first_slot = known_first >= 0  ? known_first
-                               : p.first_slot >= 0 ? p.first_slot
-                                                   : ring_position(reinterpret_cast<const int64_t*>(p.src_first), p.capacity);
-    for (uint64_t w = (uint64_t)block * blockDim.x + threadIdx.x; w < total; w += stride) {
-        const int f = field_of(t, w);
-        uint64_t row;
-        uint32_t unit;
-        split_work(w - t.prefix[f], t.units[f], row, unit);
-        int64_t slot = first_slot + (int64_t)row;
-        if (slot >= p.capacity) slot -= p.capacity;
-        uint64_t src_row = row;
-        if (p.src_capacity > 0) {
-            int64_t q = p.src_first + (int64_t)row;
-            if (q >= p.src_capacity) q -= p.src_capacity;
-            src_row = (uint64_t)q;
-        }
-        const uint32_t vl = t.vec_log2[f];
-        const uint32_t off = granule_offset(unit, vl, t.row_bytes[f]);
-        // (a source that is itself a ring is another buffer's storage, laid out like this one's)
-        copy_granule(as_global(t.store[f]) + (uint64_t)slot * t.stride[f] + off,
-                     as_global(t.io[f]) + src_row * (p.src_capacity > 0 ? t.stride[f] : t.row_bytes[f]) + off, vl);
-    }
-}
 
 __global__ __launch_bounds__(kWG) void k_rows_put(PutArgs p) { rows_put_part(p, blockIdx.x, gridDim.x); }
 
@@ -457,308 +183,6 @@ __global__ __launch_bounds__(kResWG) void k_res_push(int64_t total, int64_t capa
         if (a.row >= 0 && !s_replaced[a.row]) copy_granule(a.to, a.from, a.vl);
     }
 }
-
-// Arguments of a PER sample (the wide-row kernel takes what its tree walk needs as plain leading
-// parameters instead).
-struct SampleArgs {
-    const float* sum;       // sum tree, heap order
-    const float* uniforms;  // f32[batch] or NULL -> generator
-    int64_t batch;
-    int depth;              // log2(leaves)
-    float beta;
-    uint64_t seed, calls;
-    int64_t leaves;
-    int64_t capacity;
-    int64_t size;           // rows stored; negative: read from the device (see Counters)
-    const float* mn;        // min tree, heap order
-    int64_t* out_idx;
-    float* out_w;
-    uint32_t* err;
-};
-
-// mass of stratum k: (u + k) * (total / batch), each operation rounded once.
-__device__ __forceinline__ float stratum_mass(const SampleArgs& a, float total, int64_t k, float u) {
-    const float seg = total / (float)a.batch;
-    return (u + (float)k) * seg;
-}
-__device__ __forceinline__ float stratum_mass(const SampleArgs& a, float total, int64_t k) {
-    return stratum_mass(a, total, k, a.uniforms ? a.uniforms[k] : rng_uniform(a.seed, a.calls, (uint64_t)k));
-}
-
-// w = (p / total * size)^-beta / (pmin / total * size)^-beta
-__device__ __forceinline__ float is_weight(float p, float total, float pmin, float fsize, float beta) {
-    const float max_w = powf_det(pmin / total * fsize, -beta);
-    return powf_det(p / total * fsize, -beta) / max_w;
-}
-
-__device__ __forceinline__ void sample_flags(const SampleArgs& a, float total, int64_t idx, int64_t size) {
-    if (!(total > 0.0f) || total > 3.0e38f) atomicOr(a.err, MRB_DERR_TOTAL);
-    if (idx >= size) atomicOr(a.err, MRB_DERR_UNFILLED);
-}
-
-// ---------------------------------------------------------------------------
-// Wide rows (at least one field of 1 KB or more): k_per_sample_wide (PER sample)
-// and k_rows_gather_wide (gather at given / drawn / fixed slots).
-//
-// A row's fields are of two kinds: "wide" fields, whose rows have at least
-// 16 bytes and are copied in 16-byte granules, and "narrow" fields (the
-// others: scalars and short vectors), copied byte by byte. The granules
-// (bytes) of each kind are numbered consecutively over the fields. `split` workgroups share a row (one unless a
-// row has more than 2048 wide granules); workgroup `part` copies wide granules
-// [part * share, (part + 1) * share), the row's first workgroup also the
-// narrow ones. A workgroup is one "walker" wave and four copy waves:
-//   walker   finds the row's slot - for a sample by walking the sum tree with
-//            group_request / group_walk (one dependent load per 10 levels; the
-//            first group sits under the root, so it is requested together with
-//            the total and the uniform draw) - using nothing but kernel
-//            arguments preloaded into scalar registers, and publishes it
-//            through LDS. Afterwards it copies the narrow fields, computes the
-//            importance weight (the two powers in two lanes of one instruction
-//            stream) and writes index and weight, off the copy waves' path.
-//   copy     meanwhile every copy thread works out where its up to kInF
-//            granules lie within a row (field, offset, destination) from the
-//            field table, and the first copy wave stages in LDS what the
-//            walker needs afterwards (narrow-field table, output pointers,
-//            the minimum priority). After the barrier one multiply-add per
-//            granule gives the source address; all loads are issued before
-//            the first store: a row costs one memory round trip, not one per
-//            field.
-// Everything read from the kernel-argument segment costs a memory round trip
-// of its own when a kernel starts (nothing is cached across launches), which
-// is why the walker touches none of it before the barrier and the copy waves
-// fetch the table in one round.
-// Sampling reads its rows non-temporally so that they do not push the tree
-// out of the caches; the gathered batch is stored with ordinary stores (it is
-// what the caller reads next).
-// ---------------------------------------------------------------------------
-struct WideField {  // one table entry, 32 bytes
-    const uint8_t* src;  // the field's place in the buffer: row r at src + r * ss
-    uint8_t* dst;        // the caller's [batch, row_bytes] matrix
-    uint32_t rb;         // row_bytes
-    uint32_t first;      // wide field: number of its first granule among the wide ones; narrow: of its first byte
-    uint32_t ss;         // bytes from one row to the next in the buffer (row_bytes, or the packed row's size)
-    uint32_t pad;
-};
-struct WidePlan {
-    int split;              // workgroups per row
-    uint32_t share;         // wide granules per workgroup
-    uint32_t wide_items;    // wide granules per row
-    uint32_t narrow_items;  // bytes of narrow fields per row
-    int nwide, nnarrow;     // fields of each kind
-    uint32_t nbatch;        // host side only: batches in the launch
-    uint32_t pad;
-    WideField f[MRB_MAX_FIELDS];  // the wide fields first, then the narrow ones
-};
-
-// What the walker of a sample needs after the descent.
-struct SampleTail {
-    const float* mn;  // min tree, heap order
-    int64_t* out_idx;
-    float* out_w;
-    uint32_t* err;
-    int64_t size;  // rows stored; negative: read from the device (see Counters)
-    float beta;
-};
-
-constexpr int kCopyWaves = 4;
-constexpr int kCopyThreads = 64 * kCopyWaves;
-constexpr int kWideWG = 64 + kCopyThreads + 64;  // the walker wave, four copy waves and, for rows with narrow
-                                                  // fields, a wave that carries those (launched only then)
-constexpr int kMaxInFlight = 8;             // most granules a copy thread holds between its loads and its stores
-constexpr int kFastWide = 2;                // wide fields whose table entries are fetched unconditionally, in one round
-
-using g16 = MRB_GLOBAL granule16_u;
-
-constexpr int kNarrowInF = 2;  // narrow bytes a thread of the first copy wave holds beside its wide granules
-
-__device__ __forceinline__ uint32_t lane_u32(uint32_t x, int src_lane) {
-    return (uint32_t)__builtin_amdgcn_readlane((int)x, src_lane);
-}
-__device__ __forceinline__ uint64_t lane_u64(uint64_t x, int src_lane) {
-    return ((uint64_t)lane_u32((uint32_t)(x >> 32), src_lane) << 32) | lane_u32((uint32_t)x, src_lane);
-}
-
-// The narrow fields of a row, copied byte by byte by a wave of their own in the row's first
-// workgroup (the sixth; a copy wave that also carried them would hold its wide stores back until
-// the narrow loads have arrived: 0.06 us per launch of 512 Atari-shaped rows): lane l takes bytes l,
-// l + 64, ... of the narrow fields' bytes, numbered consecutively over the fields. Narrow fields are small (scalars such as action, reward, done); byte
-// granularity keeps their copy free of branches on a granule size.
-struct NarrowWork {
-    const gbyte* base[kNarrowInF];
-    gbyte* dst[kNarrowInF];
-    uint32_t rb[kNarrowInF];  // the byte's field: bytes from one row to the next in the buffer
-    uint32_t live;  // bit j: position j holds a byte
-    // the table entry of field `lane` (lanes 0 .. MRB_MAX_FIELDS - 1), kept for bytes past the first ones
-    uint64_t e_src, e_dst;
-    uint32_t e_rb, e_first, e_ss;
-
-    // Each lane finds the fields of its bytes from the table's entries. Up to kNarrowFast narrow fields (the
-    // usual few scalars) are read with wave-uniform indices - scalar loads, issued together, from lines of the
-    // kernel-argument segment that the copy waves' own reads bring into the scalar cache. More fields than that:
-    // lane q fetches entry q with one vector load (a round trip of its own through memory, which holds back the
-    // workgroup's barrier when nothing else, such as a tree descent, takes as long) and the entries are read from
-    // the lanes. Rows with more than 64 * kNarrowInF narrow bytes keep the per-lane copy for store().
-    static constexpr int kNarrowFast = 4;
-    __device__ __forceinline__ void take(const WidePlan& plan, int64_t k, uint32_t lane, uint64_t src_q, uint64_t dst_q,
-                                         uint32_t rb_q, uint32_t first_q, uint32_t ss_q) {
-#pragma unroll
-        for (int j = 0; j < kNarrowInF; ++j) {
-            const uint32_t rel = ((live >> j) & 1u ? lane + 64 * j : 0u) - first_q;  // wraps for bytes of earlier fields
-            if (rel < rb_q) {
-                base[j] = (const gbyte*)(src_q + rel);
-                dst[j] = (gbyte*)(dst_q + rel);
-                rb[j] = ss_q;
-            }
-        }
-    }
-    __device__ __forceinline__ void prepare(const WidePlan& plan, int64_t k, uint32_t lane) {
-        live = 0;
-#pragma unroll
-        for (int j = 0; j < kNarrowInF; ++j) {
-            base[j] = nullptr;
-            dst[j] = nullptr;
-            rb[j] = 0;
-            if (lane + 64 * j < plan.narrow_items) live |= 1u << j;
-        }
-        e_src = e_dst = 0;
-        e_rb = e_first = e_ss = 0;
-        if (plan.nnarrow <= kNarrowFast && plan.narrow_items <= 64u * kNarrowInF) {  // wave-uniform
-            WideField e[kNarrowFast];
-#pragma unroll
-            for (int i = 0; i < kNarrowFast; ++i) e[i] = plan.f[plan.nwide + (i < plan.nnarrow ? i : 0)];
-#pragma unroll
-            for (int i = 0; i < kNarrowFast; ++i)
-                if (i < plan.nnarrow)
-                    take(plan, k, lane, (uint64_t)e[i].src, (uint64_t)e[i].dst + (uint64_t)k * e[i].rb, e[i].rb, e[i].first, e[i].ss);
-            return;
-        }
-        const WideField e = plan.f[lane < MRB_MAX_FIELDS ? lane : 0];
-        e_src = (uint64_t)e.src;
-        e_dst = (uint64_t)e.dst + (uint64_t)k * e.rb;
-        e_rb = e.rb;
-        e_first = e.first;
-        e_ss = e.ss;
-        for (int q = plan.nwide; q < plan.nwide + plan.nnarrow; ++q)
-            take(plan, k, lane, lane_u64(e_src, q), lane_u64(e_dst, q), lane_u32(e_rb, q), lane_u32(e_first, q), lane_u32(e_ss, q));
-    }
-    __device__ __forceinline__ void load(uint32_t slot, uint8_t (&held)[kNarrowInF]) const {
-#pragma unroll
-        for (int j = 0; j < kNarrowInF; ++j) held[j] = *(base[j] + (uint64_t)slot * rb[j]);
-    }
-    __device__ __forceinline__ void store(uint32_t slot, const uint8_t (&held)[kNarrowInF], const WidePlan& plan, uint32_t lane) const {
-#pragma unroll
-        for (int j = 0; j < kNarrowInF; ++j)
-            if (live & (1u << j)) *dst[j] = held[j];
-        if (plan.narrow_items > 64u * kNarrowInF) {  // wave-uniform; rows with many narrow bytes
-            for (int q = plan.nwide; q < plan.nwide + plan.nnarrow; ++q) {
-                const uint64_t src_q = lane_u64(e_src, q) + (uint64_t)slot * lane_u32(e_ss, q), dst_q = lane_u64(e_dst, q);
-                const uint32_t rb_q = lane_u32(e_rb, q), first_q = lane_u32(e_first, q);
-                // bytes of this field numbered 64 * kNarrowInF or more among the narrow bytes
-                uint32_t rel = (first_q >= 64u * kNarrowInF ? 0u : 64u * kNarrowInF - first_q) + lane;
-                for (; rel < rb_q; rel += 64) *((gbyte*)dst_q + rel) = *((const gbyte*)src_q + rel);
-            }
-        }
-    }
-};
-
-// Copy thread `tid` (0 .. kCopyThreads - 1) of workgroup `part` of row k: up to kInF wide granules.
-// A thread without a granule in some position re-reads the workgroup's first granule (a valid
-// address) and skips the store, so that the loads are unconditional and all in flight together.
-// kOneWide: the row has a single wide field (e.g. an image observation beside a few scalars); all
-// addresses are then a wave-uniform row base plus a 32-bit offset, which costs a tenth of the
-// general path's address arithmetic - work that would otherwise compete with the walker for
-// the SIMD's issue slots.
-// kThreads: the threads that share a workgroup's granules (the four copy waves; one wave in k_per_sample_rows).
-template <int kInF, bool kOneWide, int kThreads = kCopyThreads>
-struct CopyWork {
-    const gbyte* base[kOneWide ? 1 : kInF];  // general: field storage + offset of the granule within a row
-    g16* dst[kOneWide ? 1 : kInF];
-    uint32_t rb[kOneWide ? 1 : kInF];        // general: bytes from one row to the next in the buffer
-    uint32_t off[kOneWide ? kInF : 1];       // one wide field: byte offset of the granule within a row
-    const uint8_t* src0;                     // one wide field: storage, destination row, storage row stride (wave-uniform)
-    uint8_t* dst0;
-    uint32_t rb0;
-    uint32_t live;  // bit j: position j holds a granule of this workgroup
-
-    __device__ __forceinline__ void prepare(const WidePlan& plan, int64_t k, uint32_t part, uint32_t tid) {
-        const uint32_t lo = part * plan.share;
-        const uint32_t hi = min(plan.wide_items, lo + plan.share);
-        uint32_t it[kInF];
-        live = 0;
-#pragma unroll
-        for (int j = 0; j < kInF; ++j) {
-            it[j] = lo + j * kThreads + tid;
-            if (it[j] < hi) live |= 1u << j;
-            else it[j] = lo;
-        }
-        if (lo >= hi || tid >= (uint32_t)kThreads) live = 0;  // (a wave past the copy waves carries narrow fields only)
-        if (kOneWide) {
-            const WideField e = plan.f[0];
-            src0 = e.src;
-            rb0 = e.ss;
-            dst0 = e.dst + (uint64_t)k * e.rb;
-#pragma unroll
-            for (int j = 0; j < kInF; ++j) off[j] = granule_offset(it[j], 4, e.rb);
-            return;
-        }
-#pragma unroll
-        for (int j = 0; j < (kOneWide ? 1 : kInF); ++j) {
-            base[j] = nullptr;
-            dst[j] = nullptr;
-            rb[j] = 0;
-        }
-        auto take = [&](int q) {
-            const WideField e = plan.f[q];
-            const uint32_t units = q < plan.nwide ? (e.rb + 15) >> 4 : 0u;
-            const gbyte* s = as_global(e.src);
-            gbyte* d = as_global(e.dst) + (uint64_t)k * e.rb;
-#pragma unroll
-            for (int j = 0; j < (kOneWide ? 1 : kInF); ++j) {
-                const uint32_t rel = it[j] - e.first;  // wraps for granules of earlier fields
-                if (rel < units) {
-                    const uint32_t at = granule_offset(rel, 4, e.rb);
-                    base[j] = s + at;
-                    dst[j] = (g16*)(d + at);
-                    rb[j] = e.ss;
-                }
-            }
-        };
-        // the first entries unconditionally: their (wave-uniform) loads go out together at once
-#pragma unroll
-        for (int q = 0; q < kFastWide; ++q) take(q);
-        for (int q = kFastWide; q < plan.nwide; ++q) take(q);
-    }
-
-    // `narrow`: this thread carries narrow bytes (the wave after the copy waves, in the row's first workgroup)
-    __device__ __forceinline__ void run(uint32_t slot, const WidePlan& plan, bool narrow, const NarrowWork& nw, uint32_t lane) const {
-        uint8_t nheld[kNarrowInF];
-        granule_t held[kInF];
-        if (narrow) nw.load(slot, nheld);
-        if (live) {
-            if (kOneWide) {
-                const gbyte* row = as_global(src0) + (uint64_t)slot * rb0;  // wave-uniform
-#pragma unroll
-                for (int j = 0; j < kInF; ++j) held[j] = __builtin_nontemporal_load((const g16*)(row + off[j]));
-            } else {
-#pragma unroll
-                for (int j = 0; j < kInF; ++j)
-                    held[j] = __builtin_nontemporal_load((const g16*)(base[j < (kOneWide ? 1 : kInF) ? j : 0] + (uint64_t)slot * rb[j < (kOneWide ? 1 : kInF) ? j : 0]));
-            }
-            // every load is issued before the first store (the compiler would otherwise move a load
-            // next to its conditional store, behind the other stores' waits)
-#pragma unroll
-            for (int j = 0; j < kInF; ++j) asm volatile("" : "+v"(held[j]));
-#pragma unroll
-            for (int j = 0; j < kInF; ++j) {
-                if (live & (1u << j)) {
-                    if (kOneWide) *(g16*)(as_global(dst0) + off[j]) = held[j];
-                    else *dst[j < (kOneWide ? 1 : kInF) ? j : 0] = held[j];
-                }
-            }
-        }
-        if (narrow) nw.store(slot, nheld, plan, lane);
-    }
-};
 
 // Replaces PriorityReplayBufferSample (mindspore_rl/core/priority_replay_buffer.py:70,92-106).
 // sum .. calls are the arguments the tree walk needs; they are preloaded into scalar registers.
@@ -1025,6 +449,7 @@ __global__ __launch_bounds__(kWideWG) void k_per_sample_next(const float* __rest
 // a trip to memory of their own when a kernel starts) is read while that group is on its way. Same outputs,
 // bit for bit, as k_per_sample_wide. Rows of at most kRowWaveInF * 64 wide granules (4 KB in 16-byte fields).
 // ---------------------------------------------------------------------------
+
 constexpr int kRowWaveInF = 4;
 constexpr int kRowWaveWG = 256;  // four rows per workgroup
 
@@ -1117,6 +542,7 @@ __global__ __launch_bounds__(kRowWaveWG) void k_per_sample_rows(const float* __r
 // single-row read), given[k] (kFromIndices) or drawn by the counter-based generator uniformly in
 // [0, count) (kFromGenerator). Replaces P.BufferSample / P.BufferGetItem
 // (mindspore_rl/core/uniform_replay_buffer.py:83-89,128,139) for wide rows.
+
 constexpr int kFromIndices = 1, kFromGenerator = 2, kFromFixedSlot = 3;
 
 template <int kInF, bool kOneWide>
@@ -1178,268 +604,6 @@ __global__ __launch_bounds__(kRowWaveWG) void k_rows_gather_rows(const int64_t* 
     }
     if (out_idx && lane == 0) out_idx[k] = slot;
     work.run((uint32_t)slot, plan, narrow, nw, (uint32_t)lane);
-}
-
-// Three levels of the descent from the eight nodes three levels under a node (lo: the first four, hi: the last
-// four): which of them the mass falls into, what is left of the mass inside it, and its value. The sums of the
-// two levels between are the single additions the tree was built with.
-__device__ __forceinline__ uint32_t walk8(const float4 lo, const float4 hi, float& mass, float& picked) {
-    const float a0 = lo.x + lo.y, a1 = lo.z + lo.w, a2 = hi.x + hi.y;
-    const float b0 = a0 + a1;
-    uint32_t p = 0;
-    if (!(mass <= b0)) {
-        mass -= b0;
-        p = 4;
-    }
-    const float left1 = p ? a2 : a0;
-    if (!(mass <= left1)) {
-        mass -= left1;
-        p += 2;
-    }
-    const float n0 = p == 0 ? lo.x : p == 2 ? lo.z : p == 4 ? hi.x : hi.z;
-    const float n1 = p == 0 ? lo.y : p == 2 ? lo.w : p == 4 ? hi.y : hi.w;
-    if (!(mass <= n0)) {
-        mass -= n0;
-        p += 1;
-        picked = n1;
-    } else {
-        picked = n0;
-    }
-    return p;
-}
-
-// Two levels, and one, of the same descent.
-__device__ __forceinline__ uint32_t walk4(const float4 v, float& mass, float& picked) {
-    const float left = v.x + v.y;
-    uint32_t p = 0;
-    if (!(mass <= left)) {
-        mass -= left;
-        p = 2;
-    }
-    const float n0 = p ? v.z : v.x, n1 = p ? v.w : v.y;
-    if (!(mass <= n0)) {
-        mass -= n0;
-        p += 1;
-        picked = n1;
-    } else {
-        picked = n0;
-    }
-    return p;
-}
-__device__ __forceinline__ uint32_t walk2(const float2 pair, float& mass, float& picked) {
-    if (mass <= pair.x) {
-        picked = pair.x;
-        return 0;
-    }
-    mass -= pair.x;
-    picked = pair.y;
-    return 1;
-}
-
-// One dependent load of the thread-per-stratum descent: the 2^g descendants of `node` g levels down (g <= 5: at most
-// one cache line), the levels between rebuilt with the additions the tree was built with. Returns the node the
-// mass falls into, g levels down; `mass` becomes what is left of it inside that node, `picked` the node's value.
-__device__ __forceinline__ uint32_t descend_group(const float* __restrict__ sum, uint32_t node, int g, float& mass, float& picked) {
-    if (g == 5) {
-        const f32x4* src = reinterpret_cast<const f32x4*>(sum + ((uint64_t)node << 5));
-        const f32x4 t0 = src[0], t1 = src[1], t2 = src[2], t3 = src[3], t4 = src[4], t5 = src[5], t6 = src[6], t7 = src[7];
-        const f32x16 lo = __builtin_shufflevector(__builtin_shufflevector(t0, t1, 0, 1, 2, 3, 4, 5, 6, 7),
-                                                  __builtin_shufflevector(t2, t3, 0, 1, 2, 3, 4, 5, 6, 7), 0, 1,
-                                                  2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-        const f32x16 hi = __builtin_shufflevector(__builtin_shufflevector(t4, t5, 0, 1, 2, 3, 4, 5, 6, 7),
-                                                  __builtin_shufflevector(t6, t7, 0, 1, 2, 3, 4, 5, 6, 7), 0, 1,
-                                                  2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-        node = (node << 5) + walk32(lo, hi, mass, picked);
-    } else if (g == 4) {
-        const f32x4* src = reinterpret_cast<const f32x4*>(sum + ((uint64_t)node << 4));
-        const f32x4 t0 = src[0], t1 = src[1], t2 = src[2], t3 = src[3];
-        const f32x16 v = __builtin_shufflevector(__builtin_shufflevector(t0, t1, 0, 1, 2, 3, 4, 5, 6, 7),
-                                                 __builtin_shufflevector(t2, t3, 0, 1, 2, 3, 4, 5, 6, 7), 0, 1,
-                                                 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-        node = (node << 4) + walk16(v, mass, picked);
-    } else if (g == 3) {
-        const float4* src = reinterpret_cast<const float4*>(sum + ((uint64_t)node << 3));
-        const float4 lo = src[0], hi = src[1];
-        node = (node << 3) + walk8(lo, hi, mass, picked);
-    } else if (g == 2) {
-        const float4 v = *reinterpret_cast<const float4*>(sum + ((uint64_t)node << 2));
-        const float left = v.x + v.y;
-        uint32_t p = 0;
-        if (!(mass <= left)) {
-            mass -= left;
-            p = 2;
-        }
-        const float n0 = p ? v.z : v.x, n1 = p ? v.w : v.y;
-        if (!(mass <= n0)) {
-            mass -= n0;
-            p += 1;
-            picked = n1;
-        } else {
-            picked = n0;
-        }
-        node = (node << 2) + p;
-    } else {
-        const float2 pair = *reinterpret_cast<const float2*>(sum + 2 * (uint64_t)node);
-        if (mass <= pair.x) {
-            node = 2 * node;
-            picked = pair.x;
-        } else {
-            mass -= pair.x;
-            node = 2 * node + 1;
-            picked = pair.y;
-        }
-    }
-    return node;
-}
-
-
-// ---------------------------------------------------------------------------
-// PER sample, many narrow rows: one workgroup per kStrata strata. The top
-// `lds_levels` levels of the sum tree (nodes [1, 2 << lds_levels)) are staged
-// in LDS once per workgroup, so each thread's descent reads HBM/L2 only for
-// the levels below; then the workgroup gathers its rows with coalesced
-// writes. Same outputs, bit for bit, as k_per_sample_wide.
-// What bounds it: a chain of trips (the arguments and the top, the descent's two or three, the rows), and, with few
-// workgroups, the compute units that have none: 256 strata to a workgroup used 64 of them for a batch of 16,384. The
-// rows' granules are numbered over all fields and four to a thread are in flight at once; field by field every field was
-// a trip of its own. 16,384 rows of
-// 153 bytes 17.1 -> 7.9 us, 13,764 of 139 bytes 15.8 -> 8.1, 16,384 of 521 bytes 35 -> 11.1.
-// ---------------------------------------------------------------------------
-// sum .. calls repeat members of `a` as plain leading parameters: those are preloaded into scalar
-// registers, so the staging loads go out when the wave starts instead of a round trip to the
-// kernel-argument segment later.
-constexpr int kLdsOwn = 4;  // leading fields whose row is one granule: every thread copies its own stratum's
-
-// rest: granules of a row in the other fields. blockIdx.y: the batch, of several that are drawn at once (each stratified
-// on its own, with the generator's next call counter).
-template <int kStrata>
-__global__ __launch_bounds__(kLdsWG) void k_per_sample_lds(const float* __restrict__ sum, const float* __restrict__ uniforms,
-                                                        const float* __restrict__ mn, int depth, int lds_levels,
-                                                        int batch, float beta, uint64_t seed, uint64_t calls, uint32_t rest,
-                                                        SampleArgs a, IoTable t) {
-    extern __shared__ float s_top[];  // [2 << lds_levels] floats, then kStrata + 1 int64: the slots, the number of stored rows
-    __shared__ float s_max_w;
-    // the field table (see k_res_push); units: of the fields that make up `rest`
-    __shared__ uint8_t *s_io[MRB_MAX_FIELDS], *s_store[MRB_MAX_FIELDS];
-    __shared__ uint32_t s_bytes[MRB_MAX_FIELDS], s_stride[MRB_MAX_FIELDS], s_units[MRB_MAX_FIELDS], s_vl[MRB_MAX_FIELDS];
-    const uint32_t ntop = 2u << lds_levels;
-    int64_t* s_slot = reinterpret_cast<int64_t*>(s_top + (ntop < 4 ? 4 : ntop));
-    const int64_t row0 = (int64_t)blockIdx.y * batch;  // the batch's first row of the call's
-    const int64_t k0 = (int64_t)blockIdx.x * kStrata;
-    const int64_t k = threadIdx.x < kStrata ? k0 + threadIdx.x : batch;
-    if (threadIdx.x >= kWG) {
-        const int f = (int)threadIdx.x - kWG;
-        if (f < t.nfields) {
-            s_io[f] = t.io[f];
-            s_store[f] = t.store[f];
-            s_bytes[f] = t.row_bytes[f];
-            s_stride[f] = t.stride[f];
-            s_units[f] = f < kLdsOwn && t.units[f] == 1 ? 0 : t.units[f];
-            s_vl[f] = t.vec_log2[f];
-        }
-        // The helper wave: the weights' common denominator (pmin / total * size)^-beta, once per
-        // workgroup, off the strata's path (two loads and a power: as long as staging the top).
-        // (the number of stored rows: the argument, or read from the device when the counters live there)
-        if (threadIdx.x == kWG) s_slot[kStrata] = a.size >= 0 ? a.size : counters_behind(a.err)[kCntSize];
-        __syncthreads();
-        if (threadIdx.x == kWG) s_max_w = powf_det(mn[1] / sum[1] * (float)s_slot[kStrata], -beta);
-        __syncthreads();
-        return;
-    }
-    // the stratum's draw is requested together with the top of the tree
-    float u = 0.0f;
-    if (k < batch && uniforms) u = uniforms[row0 + k];
-    if (ntop >= 4) {
-        for (uint32_t i = threadIdx.x * 4; i < ntop; i += kWG * 4)
-            *reinterpret_cast<float4*>(s_top + i) = *reinterpret_cast<const float4*>(sum + i);
-    } else if (threadIdx.x < ntop) {
-        s_top[threadIdx.x] = sum[threadIdx.x];
-    }
-    __syncthreads();
-    AnyGranule own[kLdsOwn];
-    float weight = 0.0f;
-    if (k < batch) {
-        const float total = s_top[1];
-        if (!uniforms) u = rng_uniform(seed, generator_calls(uniforms, calls, a.size, a.err) + blockIdx.y, (uint64_t)k);
-        float mass = (u + (float)k) * (total / (float)batch);  // each operation rounded once
-        uint32_t node = 1;
-        int d = 0;
-        // through the staged levels three at a time: the eight descendants of `node` three levels down are 32
-        // contiguous, aligned bytes of LDS - one read instead of three dependent ones -, the two levels between
-        // are rebuilt with the additions the tree was built with
-        for (; d + 3 <= lds_levels; d += 3) {
-            const float4 lo = *reinterpret_cast<const float4*>(s_top + ((size_t)node << 3));
-            const float4 hi = *reinterpret_cast<const float4*>(s_top + ((size_t)node << 3) + 4);
-            float unused;
-            node = (node << 3) + walk8(lo, hi, mass, unused);
-        }
-        for (; d < lds_levels; ++d) {
-            const float left = s_top[2 * node];
-            if (mass <= left) {
-                node = 2 * node;
-            } else {
-                mass -= left;
-                node = 2 * node + 1;
-            }
-        }
-        // Below the staged levels every dependent load brings up to five levels at once: the 32 (16, 8,
-        // 4, 2) descendants of `node` five (four, ... one) levels down are 128 (64, ... 8) contiguous,
-        // aligned bytes - a whole cache line in the first case; the levels between are rebuilt with
-        // the additions the tree was built with. The remaining levels are taken five at a time, except
-        // that seven are split 4 + 3 (5 + 1 + 1 would be a load more).
-        float picked = depth <= lds_levels ? s_top[node] : 0.0f;
-        while (d < depth) {  // wave-uniform
-            const int rest = depth - d;
-            const int g = rest >= 5 ? (rest == 7 ? 4 : 5) : rest;
-            node = descend_group(sum, node, g, mass, picked);
-            d += g;
-        }
-        const int64_t idx = (int64_t)node - ((int64_t)1 << depth);
-        const int64_t slot = idx < a.capacity ? idx : a.capacity - 1;
-        // the row's scalar fields are requested now, before the weight's arithmetic and the barrier
-#pragma unroll
-        for (int f = 0; f < kLdsOwn; ++f)
-            if (f < t.nfields && t.units[f] == 1)
-                own[f].load(as_global(t.store[f]) + (uint64_t)slot * t.stride[f], t.vec_log2[f]);
-        a.out_idx[row0 + k] = idx;
-        const int64_t size = s_slot[kStrata];  // left there by the helper wave before the first barrier
-        weight = powf_det(picked / total * (float)size, -beta);
-        sample_flags(a, total, idx, size);
-        s_slot[threadIdx.x] = slot;
-    }
-    __syncthreads();
-    const uint32_t rows = (uint32_t)((batch - k0) < kStrata ? (batch - k0) : kStrata);
-    if (k < batch) {
-        a.out_w[row0 + k] = weight / s_max_w;
-#pragma unroll
-        for (int f = 0; f < kLdsOwn; ++f)
-            if (f < t.nfields && t.units[f] == 1)
-                own[f].store(as_global(t.io[f]) + (uint64_t)(row0 + k) * t.row_bytes[f], t.vec_log2[f]);
-    }
-    // the other granules: field by field and row by row, coalesced over the workgroup's rows
-    const uint32_t work = rows * rest;
-    constexpr int kTrip = 4;
-    for (uint32_t base = threadIdx.x; base < work; base += kTrip * kWG) {
-        gbyte* to[kTrip];
-        uint32_t vl[kTrip];
-        AnyGranule held[kTrip];
-#pragma unroll
-        for (int q = 0; q < kTrip; ++q) {
-            uint32_t w = base + (uint32_t)q * kWG;
-            to[q] = nullptr;
-            if (w >= work) continue;
-            int f = 0;
-            while (w >= rows * s_units[f]) w -= rows * s_units[f++];  // (ends at a field of `rest`: w is below their total)
-            const uint32_t units = s_units[f], r = w / units;
-            vl[q] = s_vl[f];
-            const uint32_t off = granule_offset(w - r * units, vl[q], s_bytes[f]);
-            held[q].load(as_global(s_store[f]) + (uint64_t)s_slot[r] * s_stride[f] + off, vl[q]);
-            to[q] = as_global(s_io[f]) + (uint64_t)(row0 + k0 + r) * s_bytes[f] + off;
-        }
-#pragma unroll
-        for (int q = 0; q < kTrip; ++q)
-            if (to[q]) held[q].store(to[q], vl[q]);
-    }
 }
 
 // ---------------------------------------------------------------------------

@@ -1,0 +1,12 @@
+// Samples of thousands of rows (defined in mrb_samples.hip).
+#pragma once
+#include "mrb_rows.h"
+
+namespace mrb {
+
+// nbatch batches of a.batch strata, `strata` (16, 32, 64 or 256) of them to a workgroup, `levels` of the tree in LDS; rest:
+// the granules of a row outside the fields that each thread copies for its own stratum (see kLdsOwn).
+hipError_t launch_per_sample_lds(const SampleArgs& a, const IoTable& t, int64_t nbatch, int strata, int levels, uint32_t rest,
+                                 hipStream_t s);
+
+}  // namespace mrb
