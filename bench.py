@@ -76,9 +76,11 @@ def kernel_sources_sha16():
     """First 16 hex digits of the SHA-256 of the library's kernel sources: names the build a profile was taken of."""
     import hashlib
     h = hashlib.sha256()
-    for name in ("mrb_device.h", "mrb_kernels.h", "mrb.hip"):
-        with open(os.path.join(ROOT, "mindrl_amd", "csrc", name), "rb") as f:
-            h.update(f.read())
+    csrc = os.path.join(ROOT, "mindrl_amd", "csrc")
+    for name in sorted(os.listdir(csrc)):
+        if name.endswith((".h", ".hip", ".inc")):
+            with open(os.path.join(csrc, name), "rb") as f:
+                h.update(f.read())
     return h.hexdigest()[:16]
 
 
