@@ -54,6 +54,7 @@ struct Stage {
     char* memory = nullptr;
     int segment = 0;   // the one in use,
     int64_t at = 0;    // and its first free byte
+    hipStream_t stream = nullptr;  // whose work reads it (a call on another stream goes on to the next segment)
     hipEvent_t left[kStageSegments] = {};    // recorded on the stream when a segment was left
     bool was_left[kStageSegments] = {};
     ~Stage() {

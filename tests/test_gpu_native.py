@@ -108,3 +108,25 @@ def test_calls_follow_the_current_stream():
     s.synchronize()
     assert torch.equal(out, rows[idx])
     b.destroy()
+
+
+def test_host_rows_on_streams_that_run_unordered():
+    """The staging memory's segments come round while the OTHER stream's work that reads them is still queued: the rows of
+    a stream that is far behind are its own all the same."""
+    from mindrl_amd.core import UniformReplayBuffer
+    per_call, calls, floats = 16, 24, 1500  # 96,000 bytes a call: five to a segment
+    b = UniformReplayBuffer(16, per_call * calls, [(floats,)], [torch.float32], seed=2)
+    behind, ahead = torch.cuda.Stream(), torch.cuda.Stream()
+    busy = torch.randn(4096, 4096, device="cuda")
+    torch.cuda.synchronize()
+    for k in range(calls):
+        late = k % 8 == 0
+        with torch.cuda.stream(behind if late else ahead):
+            if late:
+                for _ in range(4):
+                    busy = (busy @ busy).clamp_(-1, 1)
+            b.insert([np.full((per_call, floats), k, np.float32)])
+    torch.cuda.synchronize()
+    want = torch.arange(calls, dtype=torch.float32).repeat_interleave(per_call)
+    assert torch.equal(b.buffer[0].cpu(), want[:, None].expand(-1, floats))
+    b.destroy()
