@@ -192,6 +192,9 @@ PyTypeObject* ndarray_type = nullptr;  // numpy.ndarray
 struct Source {
     const void* ptr[MRB_MAX_FIELDS] = {};
     int64_t nrows = -1;
+    const void* host[MRB_MAX_FIELDS] = {};  // rows in host memory
+    at::Tensor held[MRB_MAX_FIELDS];        // the host tensors among them: they are read without the interpreter's lock
+    int64_t staged = 0;                     // bytes of staging memory they take
     Py_buffer view[MRB_MAX_FIELDS];
     bool viewed[MRB_MAX_FIELDS] = {};
     int nviews = 0;
@@ -200,26 +203,26 @@ struct Source {
             if (viewed[i]) PyBuffer_Release(&view[i]);
     }
     // false: not what the fast path takes (no Python error is left behind)
-    bool take(const Rows* r, PyObject* fields, void* stream) {
+    bool take(const Rows* r, PyObject* fields) {
         PyObject** items;
         if (PyTuple_Check(fields) && PyTuple_GET_SIZE(fields) == r->nfields) items = &PyTuple_GET_ITEM(fields, 0);
         else if (PyList_Check(fields) && PyList_GET_SIZE(fields) == r->nfields) items = &PyList_GET_ITEM(fields, 0);
         else return false;
-        int64_t staged = 0;
-        const void* host[MRB_MAX_FIELDS] = {};
         for (int i = 0; i < r->nfields; ++i) {
             const Field& f = r->f[i];
             int64_t n;
-            void* p;
             nviews = i + 1;
             if (THPVariable_Check(items[i])) {
                 const at::Tensor& t = THPVariable_Unpack(items[i]);
                 if (t.scalar_type() != f.type || !t.is_contiguous() || t.layout() != c10::kStrided) return false;
-                p = t.data_ptr();
+                ptr[i] = t.data_ptr();
                 n = t.numel();
-                if (t.is_cpu()) host[i] = p;
-                else if (!t.is_cuda() || t.get_device() != r->device) return false;
-                ptr[i] = p;
+                if (t.is_cpu()) {
+                    host[i] = ptr[i];
+                    held[i] = t;
+                } else if (!t.is_cuda() || t.get_device() != r->device) {
+                    return false;
+                }
             } else {
                 if (!PyObject_TypeCheck(items[i], ndarray_type)) return false;
                 if (PyObject_GetBuffer(items[i], &view[i], PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) != 0) {
@@ -235,6 +238,11 @@ struct Source {
             nrows = n / f.numel;
             if (host[i]) staged += (nrows * f.bytes + 15) / 16 * 16;
         }
+        return true;
+    }
+    // Copies host rows into the staging memory; false where they do not fit it. Called WITHOUT the interpreter's lock:
+    // mrb_stage may wait for the device, and what the device is waiting for may be another Python thread.
+    bool stage(const Rows* r, void* stream) {
         if (staged == 0 || nrows <= 0) return true;
         void* to = nullptr;
         if (mrb_stage(r->handle, staged, &to, stream) != MRB_OK) return false;
@@ -275,6 +283,14 @@ PyObject* failed(Rows* r, int rc) {
     int rc;                                       \
     Py_BEGIN_ALLOW_THREADS rc = (expr);           \
     Py_END_ALLOW_THREADS if (rc != MRB_OK) return failed(r, rc)
+// the same for a call that brings rows (`src`); None where they do not fit the staging memory
+#define CALL_WITH_ROWS(expr)                              \
+    int rc = MRB_OK;                                      \
+    bool ready;                                           \
+    Py_BEGIN_ALLOW_THREADS ready = src.stage(r, stream);  \
+    if (ready) rc = (expr);                               \
+    Py_END_ALLOW_THREADS if (!ready) Py_RETURN_NONE;      \
+    if (rc != MRB_OK) return failed(r, rc)
 
 #define ARGS(count)                                                                                    \
     Rows* const r = reinterpret_cast<Rows*>(self);                                                     \
@@ -417,8 +433,8 @@ PyObject* per_push(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
     void* pr;
     Source src;
     if (args[1] != Py_None && !THPVariable_Check(args[1])) Py_RETURN_NONE;
-    if (!src.take(r, args[0], stream) || !optional_on_device(r, args[1], at::ScalarType::Float, src.nrows, &pr)) Py_RETURN_NONE;
-    CALL(mrb_per_push(r->handle, src.ptr, src.nrows, static_cast<float*>(pr), stream));
+    if (!src.take(r, args[0]) || !optional_on_device(r, args[1], at::ScalarType::Float, src.nrows, &pr)) Py_RETURN_NONE;
+    CALL_WITH_ROWS(mrb_per_push(r->handle, src.ptr, src.nrows, static_cast<float*>(pr), stream));
     Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
 }
@@ -431,11 +447,11 @@ PyObject* per_update_push(PyObject* self, PyObject* const* args, Py_ssize_t narg
     void *idx, *pr, *ppr;
     int64_t n;
     Source src;
-    if (!entries(r, args[0], args[1], &idx, &pr, &n) || !src.take(r, args[2], stream) ||
+    if (!entries(r, args[0], args[1], &idx, &pr, &n) || !src.take(r, args[2]) ||
         !optional_on_device(r, args[3], at::ScalarType::Float, src.nrows, &ppr))
         Py_RETURN_NONE;
-    CALL(mrb_per_update_push(r->handle, static_cast<int64_t*>(idx), static_cast<float*>(pr), n, src.ptr, src.nrows,
-                             static_cast<float*>(ppr), stream));
+    CALL_WITH_ROWS(mrb_per_update_push(r->handle, static_cast<int64_t*>(idx), static_cast<float*>(pr), n, src.ptr, src.nrows,
+                                       static_cast<float*>(ppr), stream));
     Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
 }
@@ -452,7 +468,7 @@ PyObject* per_step(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
     Source src;
     if (!integer(args[4], &batch) || !real(args[5], &beta)) return nullptr;
     if (!entries(r, args[0], args[1], &idx, &pr, &n) || !optional_on_device(r, args[6], at::ScalarType::Float, batch, &u) ||
-        !src.take(r, args[2], stream) || !optional_on_device(r, args[3], at::ScalarType::Float, src.nrows, &ppr))
+        !src.take(r, args[2]) || !optional_on_device(r, args[3], at::ScalarType::Float, src.nrows, &ppr))
         Py_RETURN_NONE;
     Sampled s;
     void *oidx, *w;
@@ -472,9 +488,9 @@ PyObject* per_step(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
         oidx = s.o[0].ptr;
         w = s.o[1].ptr;
     }
-    CALL(mrb_per_update_push_sample(r->handle, static_cast<int64_t*>(idx), static_cast<float*>(pr), n, src.ptr, src.nrows,
-                                    static_cast<float*>(ppr), batch, beta, static_cast<float*>(u), static_cast<int64_t*>(oidx),
-                                    static_cast<float*>(w), s.fields, stream));
+    CALL_WITH_ROWS(mrb_per_update_push_sample(r->handle, static_cast<int64_t*>(idx), static_cast<float*>(pr), n, src.ptr, src.nrows,
+                                              static_cast<float*>(ppr), batch, beta, static_cast<float*>(u),
+                                              static_cast<int64_t*>(oidx), static_cast<float*>(w), s.fields, stream));
     if (given) Py_RETURN_TRUE;
     return as_tuple(s.o, s.n);
     END_HANDLE_TH_ERRORS
@@ -545,8 +561,8 @@ PyObject* put(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {  // put
     ARGS(1)
     void* const stream = stream_of_current_device();
     Source src;
-    if (!src.take(r, args[0], stream)) Py_RETURN_NONE;
-    CALL(kPut(r->handle, src.ptr, src.nrows, stream));
+    if (!src.take(r, args[0])) Py_RETURN_NONE;
+    CALL_WITH_ROWS(kPut(r->handle, src.ptr, src.nrows, stream));
     Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
 }
