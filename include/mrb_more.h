@@ -27,6 +27,11 @@ int mrb_discounted_return_grad(const float *grad_out, const uint8_t *done, float
  * recorded into a HIP graph. */
 int mrb_stage(int64_t h, int64_t bytes, void **ptr, void *stream);
 
+/* Before the host reads rows at `rows` (n host addresses, NULLs among them are skipped): where one of them is page-locked
+ * memory, waits for the work on `stream`, which may still be writing it (a non-blocking copy from the device). Pageable
+ * memory is not written by queued work, and nothing is waited for (0.1 us an address). */
+int mrb_host_settled(const void *const *rows, int n, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

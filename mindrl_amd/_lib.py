@@ -72,6 +72,7 @@ SIGNATURES = {
 MORE_SIGNATURES = {
     "mrb_discounted_return_grad": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _f32, _vp],
     "mrb_stage": [_i64, _i64, _pvp, _vp],
+    "mrb_host_settled": [_pvp, _int, _vp],
 }
 
 _lib = None

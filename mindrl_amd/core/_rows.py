@@ -154,6 +154,8 @@ class FieldLayout:
         fit the staging memory - as device tensors. Returns the fields that were taken."""
         self.batch_of(fields)  # raises where the fields are not whole, matching rows
         fields = [as_tensor(f) for f in fields]
+        if any(f.device.type == "cpu" and f.is_pinned() for f in fields):
+            torch.cuda.current_stream().synchronize()  # queued work may still be filling them
         fields = [f.to(dtype=d).contiguous() if f.device.type == "cpu" else f.to(device=dev, dtype=d).contiguous()
                   for f, d in zip(fields, self.dtypes)]
         if call(fields) is None:

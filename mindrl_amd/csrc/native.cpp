@@ -240,12 +240,13 @@ struct Source {
         }
         return true;
     }
-    // Copies host rows into the staging memory; false where they do not fit it. Called WITHOUT the interpreter's lock:
-    // mrb_stage may wait for the device, and what the device is waiting for may be another Python thread.
+    // Copies host rows into the staging memory; false where they do not fit it. Page-locked rows may be what work queued
+    // on the stream fills (a non-blocking copy from the device): they are read when that work is done. Called WITHOUT the
+    // interpreter's lock: both may wait for the device, and what the device is waiting for may be another Python thread.
     bool stage(const Rows* r, void* stream) {
         if (staged == 0 || nrows <= 0) return true;
         void* to = nullptr;
-        if (mrb_stage(r->handle, staged, &to, stream) != MRB_OK) return false;
+        if (mrb_stage(r->handle, staged, &to, stream) != MRB_OK || mrb_host_settled(host, r->nfields, stream) != MRB_OK) return false;
         char* at = static_cast<char*>(to);
         for (int i = 0; i < r->nfields; ++i) {
             if (!host[i]) continue;

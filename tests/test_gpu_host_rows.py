@@ -59,3 +59,32 @@ def test_other_threads_run_while_an_insert_waits_for_the_device(form):
     torch.cuda.synchronize()
     assert bool((b.buffer[0] == 1).all())
     b.destroy()
+
+
+@pytest.mark.parametrize("form", ["pinned", "numpy view", "converted", "pageable"])
+@pytest.mark.parametrize("kind", ["uniform", "priority", "reservoir"])
+def test_rows_that_queued_work_is_still_filling(kind, form):
+    """A non-blocking copy from the device into host memory, then the insert, in the order of one stream and with no wait
+    between: the rows are those of the copy, as when the insert itself was a copy on that stream."""
+    from mindrl_amd.core import PriorityReplayBuffer, ReservoirReplayBuffer, UniformReplayBuffer
+    n, shapes, types = 8, [(100,), (1,)], [torch.float32, torch.int64]
+    b = (UniformReplayBuffer(4, n, shapes, types) if kind == "uniform" else
+         PriorityReplayBuffer(0.6, n, 4, shapes, types, seed0=1) if kind == "priority" else
+         ReservoirReplayBuffer(n, 4, shapes, types, seed0=1))
+    ids = torch.arange(n)[:, None]
+    host = torch.zeros((n, 100), dtype=torch.float64 if form == "converted" else torch.float32)
+    if form != "pageable":
+        host = host.pin_memory()
+    rows = [host.numpy() if form == "numpy view" else host, ids]
+    b.insert(rows)  # the staging memory is there: nothing but the rows themselves is waited for below
+    torch.cuda.synchronize()
+    keep_busy(100)
+    host.copy_(torch.ones((n, 100), dtype=host.dtype, device="cuda"), non_blocking=True)
+    b.insert(rows)
+    views = b.buffer if kind == "uniform" else b.storage()
+    stored = views[0].cpu()
+    if kind == "reservoir":  # the second eight rows replace some of the first
+        assert set(stored.sum(1).tolist()) <= {0.0, 100.0} and bool((stored.sum(1) == 100).any())
+    else:
+        assert bool((stored == 1).all())
+    b.destroy()
