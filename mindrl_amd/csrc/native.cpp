@@ -3,8 +3,8 @@
 //
 // A call on a small buffer is 4 to 8 us of kernels, and through ctypes its host side took two to four times as long: a
 // torch.empty for each result (1.1 us each, seven to nine of them), the checks of the arguments and the pointer arrays in
-// Python. Here results come straight from torch's caching allocator, the small ones of a call out of one allocation, and a
-// call's host time is the library's and the runtime's launch.
+// Python. Here results come straight from torch's caching allocator, and a call's host time is theirs, the library's and the
+// runtime's launch.
 //
 // A rollout's returns with gradients went through a Python autograd function, whose backward half the engine's thread
 // runs under the interpreter's lock; ReturnBackward needs neither (forward and backward of [1000, 4096] 84 -> 52 us).
@@ -36,9 +36,6 @@
 
 namespace {
 
-constexpr int64_t kSharedBytes = 64 << 10;  // results of at most this many bytes share one allocation of a call
-constexpr int64_t kAlign = 256;             // where each starts within it
-
 struct Field {
     at::ScalarType type;
     int64_t item, numel, bytes;  // per element, elements and bytes per row
@@ -59,7 +56,7 @@ struct Rows {  // one buffer: its handle and its fields
 
 struct Output {
     at::ScalarType type;
-    int64_t item, bytes;
+    int64_t bytes;
     int ndim;
     int64_t shape[26];
     at::Tensor t;
@@ -73,42 +70,23 @@ c10::Storage new_storage(int64_t bytes) {
                                                               allocator, /*resizable=*/true));
 }
 
-void make(Output& o, c10::Storage storage, int64_t offset) {
-    o.ptr = static_cast<char*>(storage.mutable_data()) + offset;
+void make(Output& o, c10::Storage storage) {
+    o.ptr = storage.mutable_data();
     o.t = at::detail::make_tensor<c10::TensorImpl>(std::move(storage), c10::DispatchKeySet(c10::DispatchKey::CUDA),
                                                    c10::scalarTypeToTypeMeta(o.type));
-    c10::TensorImpl* impl = o.t.unsafeGetTensorImpl();
-    impl->set_sizes_contiguous(c10::IntArrayRef(o.shape, o.ndim));
-    if (offset) impl->set_storage_offset(offset / o.item);
+    o.t.unsafeGetTensorImpl()->set_sizes_contiguous(c10::IntArrayRef(o.shape, o.ndim));
 }
 
+// A storage each: a result can be grown, saved, kept or marked as used on another stream without the call's others.
 void allocate(Output* o, int n, int device) {
     c10::OptionalDeviceGuard guard;
     if (c10::hip::current_device() != device) guard.reset_device(c10::Device(c10::DeviceType::CUDA, (c10::DeviceIndex)device));
-    int64_t shared = 0;
-    int small = 0;
-    for (int i = 0; i < n; ++i)
-        if (o[i].bytes <= kSharedBytes) {
-            shared += (o[i].bytes + kAlign - 1) / kAlign * kAlign;
-            ++small;
-        }
-    c10::Storage slab;
-    if (small > 1) slab = new_storage(shared);
-    int64_t at = 0;
-    for (int i = 0; i < n; ++i) {
-        if (small > 1 && o[i].bytes <= kSharedBytes) {
-            make(o[i], slab, at);
-            at += (o[i].bytes + kAlign - 1) / kAlign * kAlign;
-        } else {
-            make(o[i], new_storage(o[i].bytes), 0);
-        }
-    }
+    for (int i = 0; i < n; ++i) make(o[i], new_storage(o[i].bytes));
 }
 
 // [lead..., *shape_i]; nlead 0..2
 void describe(Output& o, const Field& f, const int64_t* lead, int nlead) {
     o.type = f.type;
-    o.item = f.item;
     o.bytes = f.bytes;
     o.ndim = nlead + f.ndim;
     for (int i = 0; i < nlead; ++i) {
@@ -120,7 +98,6 @@ void describe(Output& o, const Field& f, const int64_t* lead, int nlead) {
 
 void describe(Output& o, at::ScalarType type, int64_t item, const int64_t* lead, int nlead) {
     o.type = type;
-    o.item = item;
     o.bytes = item;
     o.ndim = nlead;
     for (int i = 0; i < nlead; ++i) {

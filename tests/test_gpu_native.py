@@ -1,6 +1,8 @@
 """The native host side of the buffer classes: rows from host memory through the staging memory (numpy arrays, CPU tensors,
 a mix with device tensors, other dtypes, more than the staging memory takes, segments used again while earlier calls are
-still queued), and results that share an allocation without sharing values."""
+still queued), and results that are tensors of their own."""
+import io
+
 import numpy as np
 import pytest
 import torch
@@ -95,6 +97,27 @@ def test_results_are_tensors_of_their_own():
     per.destroy()
     with pytest.raises(ValueError):
         per.sample(0.4)
+
+
+def test_results_have_storages_of_their_own():
+    """A result can be grown in place, given as out= of a larger result, or saved, without the call's other results."""
+    from mindrl_amd.core import PriorityReplayBuffer
+    per = PriorityReplayBuffer(0.6, 400, 16, SHAPES, torch_types(DTYPES), seed0=3)
+    rows = to_dev(random_rows(np.random.default_rng(1), 300, SHAPES, DTYPES))
+    per.insert(*rows)
+    step = lambda: per.update_priorities_insert_and_sample(torch.arange(4, device="cuda"), torch.ones(4, device="cuda"),
+                                                           *[r[:1] for r in rows], beta=0.4)
+    for call in (lambda: per.sample(0.4), lambda: per.sample_many(2, 0.4), lambda: per.gather(torch.arange(16, device="cuda")), step):
+        results = call()
+        kept = [t.clone() for t in results]
+        for i, t in enumerate(results):
+            assert t.untyped_storage().nbytes() == t.numel() * t.element_size() and t.storage_offset() == 0
+            saved = io.BytesIO()
+            torch.save(t, saved)
+            assert torch.equal(torch.load(io.BytesIO(saved.getvalue()), weights_only=True), kept[i])
+            t.resize_(50_000).zero_()
+            assert all(torch.equal(u, kept[j]) for j, u in enumerate(results) if j > i)
+    per.destroy()
 
 
 def test_calls_follow_the_current_stream():
