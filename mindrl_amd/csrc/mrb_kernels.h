@@ -833,6 +833,7 @@ __device__ __forceinline__ void tile_round(const UpdateArgs& a, int lo, int g, u
         }
     }
     float4 vs = make_float4(0.f, 0.f, 0.f, 0.f), vm = vs;
+    float largest = 0.0f;  // p^alpha of those this lane writes (a push with priorities)
     if (active) {
         vs = *reinterpret_cast<const float4*>(a.sum + first + 4 * lane);
         vm = *reinterpret_cast<const float4*>(a.mn + first + 4 * lane);
@@ -871,6 +872,7 @@ __device__ __forceinline__ void tile_round(const UpdateArgs& a, int lo, int g, u
                         if (in[c]) {
                             const bool ok = valid_priority(pv[c]);
                             *vsp[c] = *vmp[c] = ok ? qv[c] : *a.maxp;  // invalid: the fresh slot stays at the running max
+                            if (ok) largest = fmaxf(largest, qv[c]);
                             if (a.fold_max == 2 && !ok) atomicOr(a.err, MRB_DERR_PRIORITY);
                             wrote = true;
                         }
@@ -890,11 +892,7 @@ __device__ __forceinline__ void tile_round(const UpdateArgs& a, int lo, int g, u
         if (dirty_out && ((off & ((1u << g) - 1)) == 0)) dirty_out[(off >> g) >> g_next] = a.epoch;
     }
     if (leaf_level && a.fold_max == 2) {
-        // the largest leaf of the tile bounds every p^alpha written here from above, and is itself a p^alpha or
-        // a value no larger than the running max: folding it in raises the running max to exactly what a pass
-        // over the call's priorities would
-        float q = active ? fmaxf(fmaxf(vs.x, vs.y), fmaxf(vs.z, vs.w)) : 0.0f;
-        q = wave_max(q);
+        const float q = wave_max(largest);
         if (lane == 0 && q > 0.0f) raise_max(a.maxp_next, q);
     }
     tile_parents(a, g, first, lane, active, vs, vm, root_s, root_m);
@@ -1256,7 +1254,7 @@ constexpr int kRunLevels = 3;  // tiles above the leaf tiles on a path: trees of
 __global__ __launch_bounds__(kFusedWG) void k_push_run(UpdateArgs a, uint32_t units, PutArgs put) {
     __shared__ float s_s[kRunLevels][kRunWaves], s_m[kRunLevels][kRunWaves];
     __shared__ uint32_t s_new[kRunLevels][kRunWaves];  // whether the wave has a new root for the level above
-    __shared__ float s_largest[kRunWaves];             // the largest leaf of the wave's tile (a push with priorities)
+    __shared__ float s_largest[kRunWaves];             // the largest p^alpha the wave has written (a push with priorities)
     if (__builtin_expect(blockIdx.x >= 1, 0)) {  // (the tree workgroup's code comes first: it is the one the call waits for)
         rows_put_part(put, blockIdx.x - 1, put.blocks);
         counters_push_done(a.err, a.advance, a.capacity, a.readers);
@@ -1335,7 +1333,10 @@ __global__ __launch_bounds__(kFusedWG) void k_push_run(UpdateArgs a, uint32_t un
             for (int c = 0; c < 4; ++c) {
                 const bool ok = valid_priority(pv[c]);  // invalid: the fresh slot stays at the running max
                 if (ok) q[c] = p4[c];
-                bad = bad || ((in >> c & 1u) && !ok);
+                if (in >> c & 1u) {
+                    if (ok) largest = fmaxf(largest, p4[c]);
+                    bad = bad || !ok;
+                }
             }
             if (bad && a.fold_max) atomicOr(a.err, MRB_DERR_PRIORITY);
         }
@@ -1347,9 +1348,7 @@ __global__ __launch_bounds__(kFusedWG) void k_push_run(UpdateArgs a, uint32_t un
             *reinterpret_cast<float4*>(a.sum + leaf_first + 4 * lane) = ls;
             *reinterpret_cast<float4*>(a.mn + leaf_first + 4 * lane) = lm;
         }
-        // the largest leaf of the tile bounds every p^alpha written here from above, and is itself a p^alpha or a value no
-        // larger than the running max
-        if (a.fold_max) largest = wave_max(fmaxf(fmaxf(ls.x, ls.y), fmaxf(ls.z, ls.w)));
+        if (a.fold_max) largest = wave_max(largest);
         tile_parents(a, kRoundLevels, leaf_first, lane, true, ls, lm, &rs, &rm);
     }
     if (lane == 0) s_largest[wave] = largest;

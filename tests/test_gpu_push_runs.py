@@ -57,3 +57,45 @@ def test_push_runs(cap, starts, device_counters):
         with pytest.raises(ValueError, match="priority"):
             g.check()
         g.destroy()
+
+
+@pytest.mark.parametrize("device_counters", [0, 1])
+@pytest.mark.parametrize("cap", [3000, 20_000, 70_000, 600_000])
+def test_running_max_comes_from_the_pushed_priorities_alone(cap, device_counters):
+    """A loaded state may hold leaves above its running max. A push with priorities raises the running max to the largest of
+    its OWN powers, whatever lies beside its slots: one workgroup's pushes, runs of tiles, more tiles than a run takes, and
+    pushes that follow an update in one call."""
+    from mindrl_amd.core import PriorityReplayBuffer
+    from oracle import orc
+    rng = np.random.default_rng(cap)
+    g = PriorityReplayBuffer(0.6, cap, 8, SHAPES, torch_types(DTYPES), seed0=3)
+    c = orc.OraclePER(0.6, cap, SHAPES, DTYPES, seed=3)
+    rows = random_rows(rng, cap, SHAPES, DTYPES)
+    g.insert(*to_dev(rows), priorities=torch.full((cap,), 20.0, device="cuda"))
+    c.push(rows, cap, np.full(cap, 20.0, np.float32))
+    state = dict(g.state_dict(), max_priority=1e-3)  # far below the leaves, 20 ** 0.6
+    g.load_state_dict(state)
+    c.load_state_dict({**c.state_dict(), "max_priority": 1e-3})
+    g.set_option("device_counters", device_counters)
+    assert np.float32(g.max_priority) == np.float32(c.max_priority)
+    largest = np.float32(1e-3)
+    for step, n in enumerate((1, 3, 255, 900, 1500, 1, 5, 300, 5000)):
+        if n > cap:
+            continue
+        largest *= np.float32(1.5)
+        rows = random_rows(rng, n, SHAPES, DTYPES)
+        pr = (largest * rng.random(n)).astype(np.float32)
+        pr[n // 3] = largest
+        slots = (c.head + np.arange(n)) % cap
+        if step < 5:
+            g.insert(*to_dev(rows), priorities=torch.from_numpy(pr).cuda())
+        else:
+            idx, low = rng.integers(0, cap, 100), np.full(100, 1e-6, np.float32)
+            g.update_priorities_and_insert(torch.from_numpy(idx).cuda(), torch.from_numpy(low).cuda(), *to_dev(rows),
+                                           insert_priorities=torch.from_numpy(pr).cuda())
+            c.update(idx, low)
+        c.push(rows, n)
+        c.update(slots, pr)
+        assert np.float32(g.max_priority) == np.float32(c.max_priority) < np.float32(1.0), (cap, n)
+        assert_tree_equal(g, c, "cap %d n %d" % (cap, n))
+    g.destroy()
