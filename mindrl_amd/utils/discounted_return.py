@@ -44,12 +44,14 @@ class DiscountedReturn:
                 raise ValueError("reward and done must share the leading Timestep axis")
             timesteps = r.shape[0]
             batch = d.numel() // timesteps if timesteps else 0
-            if timesteps == 0 or batch == 0 or d.numel() != timesteps * batch or r.numel() % (timesteps * batch):
+            if batch == 0 or r.numel() == 0 or d.numel() != timesteps * batch or r.numel() % (timesteps * batch):
                 raise ValueError("done must be [Timestep, Batch] and reward [Timestep, Batch, ...]")
             if v.numel() != batch * (r.numel() // (timesteps * batch)):
                 raise ValueError("last_state_value must be [Batch, ...] matching reward")
             reward, done, last_state_value = r, d, v
             out = self._native(r, d, v, self.gamma, self.need_bprop, _lib.check)
+            if out is None:
+                raise ValueError("reward, done and last_state_value must be dense tensors")
         if not out.requires_grad:  # (a result with a history holds what its gradient needs: no more is kept alive)
             self._keep = (reward, done, last_state_value)
         return out

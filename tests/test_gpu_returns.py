@@ -69,3 +69,13 @@ def test_saved_flags_pass_through_hooks():
     negated = torch._neg_view(torch.full((70, 9), -2.0, device="cuda"))
     got = torch.autograd.grad(returns(reward, done, value), (reward, value), negated)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("need_bprop", [False, True])
+def test_empty_inputs_are_refused(need_bprop):
+    from mindrl_amd.utils import DiscountedReturn
+    returns = DiscountedReturn(0.9, need_bprop=need_bprop)
+    for reward, done, value in (((5, 3, 0), (5, 3), (3, 0)), ((5, 0), (5, 0), (0,)), ((0, 3), (0, 3), (3,)), ((0,), (0,), ())):
+        with pytest.raises(ValueError):
+            returns(torch.zeros(reward, device="cuda"), torch.zeros(done, dtype=torch.bool, device="cuda"),
+                    torch.zeros(value, device="cuda"))
