@@ -590,21 +590,22 @@ struct ReturnBackward : torch::autograd::Node {
     }
 };
 
-// discounted_return(reward, done, last_state_value, gamma, differentiable, _lib.check): contiguous tensors on one device,
-// float32 and bool, of matching sizes
+// discounted_return(reward, done, last_state_value, gamma, differentiable, _lib.check, device index): contiguous tensors on
+// that device, float32 and bool, of matching sizes
 PyObject* discounted_return(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     float gamma;
-    if (nargs != 6) {
-        PyErr_Format(PyExc_TypeError, "expected 6 arguments, got %zd", nargs);
+    if (nargs != 7) {
+        PyErr_Format(PyExc_TypeError, "expected 7 arguments, got %zd", nargs);
         return nullptr;
     }
-    if (!real(args[3], &gamma)) return nullptr;
+    int64_t device;
+    if (!real(args[3], &gamma) || !integer(args[6], &device)) return nullptr;
     for (int i = 0; i < 3; ++i)
         if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
     const at::Tensor &reward = THPVariable_Unpack(args[0]), &done = THPVariable_Unpack(args[1]), &value = THPVariable_Unpack(args[2]);
     for (const at::Tensor* t : {&reward, &done, &value})
-        if (!t->is_cuda() || t->layout() != c10::kStrided || !t->is_contiguous() || t->get_device() != reward.get_device() ||
+        if (!t->is_cuda() || t->layout() != c10::kStrided || !t->is_contiguous() || t->get_device() != device ||
             t->scalar_type() != (t == &done ? at::ScalarType::Bool : at::ScalarType::Float))
             Py_RETURN_NONE;
     if (reward.dim() == 0 || done.dim() == 0 || reward.numel() == 0 || done.numel() == 0 || reward.size(0) != done.size(0)) Py_RETURN_NONE;
@@ -617,10 +618,9 @@ PyObject* discounted_return(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
         PyErr_SetString(PyExc_NotImplementedError, "DiscountedReturn has no forward-mode derivative");
         return nullptr;
     }
-    const int device = reward.get_device();
     c10::OptionalDeviceGuard guard;
     if (c10::hip::current_device() != device) guard.reset_device(reward.device());
-    at::Tensor out = new_float(reward.sizes(), device);
+    at::Tensor out = new_float(reward.sizes(), (int)device);
     void* const stream = stream_of_current_device();
     // (data_ptr: raises for tensors without memory)
     const float *x = static_cast<const float*>(reward.data_ptr()), *v = static_cast<const float*>(value.data_ptr());

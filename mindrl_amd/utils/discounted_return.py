@@ -35,7 +35,7 @@ class DiscountedReturn:
         self._native = _lib.native().discounted_return
 
     def construct(self, reward, done, last_state_value):
-        out = self._native(reward, done, last_state_value, self.gamma, self.need_bprop, _lib.check)
+        out = self._native(reward, done, last_state_value, self.gamma, self.need_bprop, _lib.check, self._dev.index)
         if out is None:
             r = torch.as_tensor(reward).to(device=self._dev, dtype=torch.float32).contiguous()
             d = torch.as_tensor(done).to(device=self._dev, dtype=torch.bool).contiguous()
@@ -49,7 +49,7 @@ class DiscountedReturn:
             if v.numel() != batch * (r.numel() // (timesteps * batch)):
                 raise ValueError("last_state_value must be [Batch, ...] matching reward")
             reward, done, last_state_value = r, d, v
-            out = self._native(r, d, v, self.gamma, self.need_bprop, _lib.check)
+            out = self._native(r, d, v, self.gamma, self.need_bprop, _lib.check, self._dev.index)
             if out is None:
                 raise ValueError("reward, done and last_state_value must be dense tensors")
         if not out.requires_grad:  # (a result with a history holds what its gradient needs: no more is kept alive)

@@ -79,3 +79,13 @@ def test_empty_inputs_are_refused(need_bprop):
         with pytest.raises(ValueError):
             returns(torch.zeros(reward, device="cuda"), torch.zeros(done, dtype=torch.bool, device="cuda"),
                     torch.zeros(value, device="cuda"))
+
+
+def test_computes_on_the_device_of_its_own():
+    """Inputs on another device are moved to the one the object was made on: the native call takes none of them as they are."""
+    from mindrl_amd import _lib
+    reward, done = torch.ones(5, 3, device="cuda"), torch.zeros(5, 3, dtype=torch.bool, device="cuda")
+    value = torch.zeros(3, device="cuda")
+    call = _lib.native().discounted_return
+    assert call(reward, done, value, 0.9, False, _lib.check, reward.device.index) is not None
+    assert call(reward, done, value, 0.9, False, _lib.check, reward.device.index + 1) is None
