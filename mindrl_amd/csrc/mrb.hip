@@ -1518,8 +1518,13 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
 // and 16 / 32 / 64 / 256 strata to a workgroup: 153 bytes, 16,384 rows 8.5 / 7.9 / 8.7 / 16.1, 65,536 25 / 17 / 13.3 /
 // 16.7, 262,144 84 / 51 / 38 / 31; 521 bytes, 8192 rows 9.6 / 10.7 / 14.0 / 34.5, 32,768 21 / 13.8 / 16.8 / 36; 3 KB,
 // 65,536 rows 99 / 96 / 91 / 201.
-static bool takes_lds(int64_t rows, uint64_t rest) {
-    return rest <= 384 && rows >= (rest <= 16 ? 3072 : rest <= 64 ? 5120 : 12288);
+// A workgroup has the strata of one batch only, so batches of a few rows leave most of it idle while it stages the top all
+// the same (batches x rows of one): 8-byte rows, 10^6 slots 4096 x 1 6.6 / 20, 4096 x 2 11.0 / 20.6, 2048 x 4 10.9 / 12.1,
+// 2048 x 6 14.6 / 9.9, 1024 x 8 10.8 / 6.4; 521 bytes 2048 x 4 11.0 / 13.8, 4096 x 5 26 / 22; 3 KB 4096 x 3 21 / 30, 4096 x 6
+// 36 / 43, 2048 x 8 26 / 26. (A row above 4 KB takes a whole workgroup there: 6 KB 4096 x 3 46 / 43.)
+static bool takes_lds(int64_t nbatch, int64_t batch, uint64_t rest) {
+    const int64_t rows = nbatch * batch, fewest = rest <= 64 ? 5 : rest <= 256 ? 8 : 1;
+    return rest <= 384 && batch >= fewest && rows >= (rest <= 16 ? 3072 : rest <= 64 ? 5120 : 12288);
 }
 static int lds_strata(int64_t rows, uint64_t rest) {
     if (rows <= 20480 && rest > 16) return 16;
@@ -1564,7 +1569,7 @@ static int per_sample_impl(Per* b, int64_t nbatch, int64_t batch, float beta, co
     uint64_t rest = 0;  // granules of a row that the LDS-top kernel's threads do not copy for their own stratum alone
     for (int f = 0; f < t.nfields; ++f) rest += f < kLdsOwn && t.units[f] == 1 ? 0 : t.units[f];
     int path = (int)b->sample_path;
-    if (path == 0) path = takes_lds(nbatch * batch, rest) ? 2 : 1;
+    if (path == 0) path = takes_lds(nbatch, batch, rest) ? 2 : 1;
     if (rest > 1u << 23) path = 1;  // (it numbers a workgroup's granules in 32 bits)
     if (next) {
         rc = sample_wide(b->rows, a, t, nbatch, s, next);  // always the wide-row kernel: the gathered field is wide
