@@ -70,6 +70,13 @@ class PriorityReplayBuffer:
             return idx, w, self._layout.check_out(fields, self._sample_size, self._dev)
         return self._next_outputs() if self._ring_size > 0 else None
 
+    def _check_given(self, given):
+        """Raises if a sample cannot go to `given` (asked when the native call has taken it for something to convert)."""
+        for t, dtype in zip(given or (), (torch.int64, torch.float32)):
+            if t.dtype != dtype or t.device != self._dev or not t.is_contiguous() or t.numel() < self._sample_size:
+                raise ValueError("out must hold contiguous int64 indices, float32 weights and the fields on %s, of sample_size = "
+                                 "%d rows" % (self._dev, self._sample_size))
+
     def _uniforms(self, uniforms, n, what):
         u = flat_on_device(uniforms, torch.float32, self._dev)
         if u.numel() != n:
@@ -130,7 +137,8 @@ class PriorityReplayBuffer:
             if uniforms is not None:
                 uniforms = self._uniforms(uniforms, n, "sample_size = %d" % n)
             if self._native.per_sample_into(n, beta, uniforms, *given) is None:
-                raise ValueError("out must hold contiguous int64 indices, float32 weights and the fields on %s" % self._dev)
+                self._check_given(given)
+                raise ValueError("out must hold dense tensors")
             res = (given[0], given[1]) + tuple(given[2])
         self._keep = uniforms
         return res
@@ -203,6 +211,7 @@ class PriorityReplayBuffer:
         given = self._outputs(out)
         res = self._native.per_step(indices, priorities, transition, insert_priorities, b, beta, uniforms, given)
         if res is None:
+            self._check_given(given)
             indices, priorities = self._entries(indices, priorities)
             ipr = insert_priorities = self._row_priorities(insert_priorities, transition, "insert_priorities")
             if uniforms is not None:

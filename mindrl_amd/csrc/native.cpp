@@ -325,20 +325,29 @@ PyObject* per_sample(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
-// per_sample_into(batch, beta, uniforms or None, indices, weights, fields): results written to given tensors, which the
-// caller has checked
+// The tensors a sample of `batch` rows goes to: indices and weights that hold them, and the fields, whose shapes the caller
+// has checked.
+bool given_outputs(const Rows* r, PyObject* indices, PyObject* weights, PyObject* fields, int64_t batch, void** idx, void** w,
+                   void** to) {
+    int64_t ni, nw, n;
+    if (!on_device(r, indices, at::ScalarType::Long, idx, &ni) || !on_device(r, weights, at::ScalarType::Float, w, &nw) || ni < batch ||
+        nw < batch || !PyList_Check(fields) || PyList_GET_SIZE(fields) != r->nfields)
+        return false;
+    for (int i = 0; i < r->nfields; ++i)
+        if (!on_device(r, PyList_GET_ITEM(fields, i), r->f[i].type, &to[i], &n)) return false;
+    return true;
+}
+
+// per_sample_into(batch, beta, uniforms or None, indices, weights, fields): results written to given tensors
 PyObject* per_sample_into(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     ARGS(6)
-    int64_t batch, n;
+    int64_t batch;
     float beta;
     void *u, *idx, *w, *fields[MRB_MAX_FIELDS];
     if (!integer(args[0], &batch) || !real(args[1], &beta)) return nullptr;
     if (!optional_on_device(r, args[2], at::ScalarType::Float, batch, &u)) Py_RETURN_NONE;
-    if (!on_device(r, args[3], at::ScalarType::Long, &idx, &n) || !on_device(r, args[4], at::ScalarType::Float, &w, &n)) Py_RETURN_NONE;
-    if (!PyList_Check(args[5]) || PyList_GET_SIZE(args[5]) != r->nfields) Py_RETURN_NONE;
-    for (int i = 0; i < r->nfields; ++i)
-        if (!on_device(r, PyList_GET_ITEM(args[5], i), r->f[i].type, &fields[i], &n)) Py_RETURN_NONE;
+    if (!given_outputs(r, args[3], args[4], args[5], batch, &idx, &w, fields)) Py_RETURN_NONE;
     void* const stream = stream_of_current_device();
     CALL(mrb_per_sample(r->handle, batch, beta, static_cast<float*>(u), static_cast<int64_t*>(idx), static_cast<float*>(w), fields,
                         stream));
@@ -435,13 +444,13 @@ PyObject* per_update_push(PyObject* self, PyObject* const* args, Py_ssize_t narg
 }
 
 // per_step(indices, priorities, fields, push priorities or None, batch, beta, uniforms or None, out or None); `out`:
-// (indices, weights, [fields]) given tensors, which the caller has checked
+// (indices, weights, [fields]) given tensors
 PyObject* per_step(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     ARGS(8)
     void* const stream = stream_of_current_device();
     void *idx, *pr, *ppr, *u;
-    int64_t n, batch, m;
+    int64_t n, batch;
     float beta;
     Source src;
     if (!integer(args[4], &batch) || !real(args[5], &beta)) return nullptr;
@@ -453,13 +462,9 @@ PyObject* per_step(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
     const bool given = args[7] != Py_None;
     if (given) {
         if (!PyTuple_Check(args[7]) || PyTuple_GET_SIZE(args[7]) != 3) Py_RETURN_NONE;
-        PyObject* const fields = PyTuple_GET_ITEM(args[7], 2);
-        if (!on_device(r, PyTuple_GET_ITEM(args[7], 0), at::ScalarType::Long, &oidx, &m) ||
-            !on_device(r, PyTuple_GET_ITEM(args[7], 1), at::ScalarType::Float, &w, &m) || !PyList_Check(fields) ||
-            PyList_GET_SIZE(fields) != r->nfields)
+        if (!given_outputs(r, PyTuple_GET_ITEM(args[7], 0), PyTuple_GET_ITEM(args[7], 1), PyTuple_GET_ITEM(args[7], 2), batch, &oidx, &w,
+                           s.fields))
             Py_RETURN_NONE;
-        for (int i = 0; i < r->nfields; ++i)
-            if (!on_device(r, PyList_GET_ITEM(fields, i), r->f[i].type, &s.fields[i], &m)) Py_RETURN_NONE;
     } else {
         if (!s.prepare(r, &batch, 1)) return refused(r, batch);
         s.finish(r);

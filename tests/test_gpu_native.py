@@ -120,6 +120,27 @@ def test_results_have_storages_of_their_own():
     per.destroy()
 
 
+def test_given_outputs_that_do_not_hold_the_batch_are_refused():
+    """`out` with indices or weights of too few rows, another dtype or device: refused before anything is written or changed."""
+    per, put, _ = buffers()[0]
+    rows = to_dev(random_rows(np.random.default_rng(1), 300, SHAPES, DTYPES))
+    put(rows)
+    good = per.sample(0.4)
+    idx, w, fields = good[0], good[1], list(good[2:])
+    step = lambda out: per.update_priorities_insert_and_sample(torch.arange(4, device="cuda"), torch.ones(4, device="cuda"),
+                                                               *[r[:1] for r in rows], beta=0.4, out=out)
+    for call in (lambda out: per.sample(0.4, out=out), step):
+        size = per.size()
+        for bad in ((idx[:15], w, fields), (idx, w[:15], fields), (idx.int(), w, fields), (idx, w.double(), fields),
+                    (idx.cpu(), w, fields), (idx, torch.empty(32, device="cuda")[::2], fields), (idx, w, fields[:-1])):
+            with pytest.raises(ValueError):
+                call(bad)
+        assert per.size() == size
+        larger = (torch.empty(20, dtype=torch.int64, device="cuda"), torch.empty(20, device="cuda"), fields)
+        assert call(larger)[0] is larger[0]  # more room than needed is fine: the first rows are written
+    per.destroy()
+
+
 def test_calls_follow_the_current_stream():
     from mindrl_amd.core import UniformReplayBuffer
     b = UniformReplayBuffer(64, 64, [(4,)], [torch.float32], seed=2)
