@@ -195,6 +195,7 @@ struct Source {
                 ptr[i] = t.data_ptr();
                 n = t.numel();
                 if (t.is_cpu()) {
+                    if (t.is_neg()) return false;  // (a view that negates: a plain copy of its memory is not its values)
                     host[i] = ptr[i];
                     held[i] = t;
                 } else if (!t.is_cuda() || t.get_device() != r->device) {

@@ -30,13 +30,15 @@ def as_given(rows, form):
         return [torch.from_numpy(r) for r in rows]
     if form == "mixed":
         return [torch.from_numpy(r).cuda() if i % 2 else r for i, r in enumerate(rows)]
+    if form == "negated":  # views whose memory holds the opposite of their values
+        return [torch._neg_view(-torch.from_numpy(r)) if r.dtype in (np.float32, np.int64) else r for r in rows]
     if form == "converted":  # dtypes that need converting, not contiguous
         return [rows[0].astype(np.float64), rows[1].astype(np.int32), rows[2].tolist(), torch.from_numpy(rows[3]).float(),
                 torch.from_numpy(np.repeat(rows[4], 2, axis=1))[:, ::2]]
     return to_dev(rows)
 
 
-@pytest.mark.parametrize("form", ["device", "numpy", "cpu", "mixed", "converted"])
+@pytest.mark.parametrize("form", ["device", "numpy", "cpu", "mixed", "converted", "negated"])
 def test_rows_from_host_memory(form):
     rng = np.random.default_rng(5)
     for buf, put, views in buffers():
