@@ -36,11 +36,13 @@
 
 namespace {
 
+constexpr int kMaxDims = 62;  // of a field: results of two more are what torch's own operations take at most
+
 struct Field {
     at::ScalarType type;
     int64_t item, numel, bytes;  // per element, elements and bytes per row
     int ndim;
-    int64_t shape[24];
+    int64_t shape[kMaxDims];
 };
 
 struct Rows {  // one buffer: its handle and its fields
@@ -58,7 +60,7 @@ struct Output {
     at::ScalarType type;
     int64_t bytes;
     int ndim;
-    int64_t shape[26];
+    int64_t shape[kMaxDims + 2];
     at::Tensor t;
     void* ptr;
 };
@@ -671,8 +673,8 @@ int rows_init(PyObject* self, PyObject* args, PyObject*) {
     for (Py_ssize_t i = 0; i < n; ++i) {
         PyObject* const shape = PyTuple_GET_ITEM(shapes, i);
         PyObject* const type = PyTuple_GET_ITEM(types, i);
-        if (!PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) > 24 || !THPDtype_Check(type)) {
-            PyErr_SetString(PyExc_TypeError, "shapes are tuples of at most 24 numbers, dtypes torch dtypes");
+        if (!PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) > kMaxDims || !THPDtype_Check(type)) {
+            PyErr_SetString(PyExc_TypeError, "shapes are tuples of at most 62 numbers, dtypes torch dtypes");
             return -1;
         }
         Field& f = r->f[i];
