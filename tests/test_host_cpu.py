@@ -165,6 +165,15 @@ def test_only_the_documented_entry_points_wait_or_allocate():
         assert not allocs.search(bodies[name]) and not waits.search(bodies[name]), name
 
 
+def test_failed_staging_leaves_no_error_behind():
+    """A call of mrb_stage that fails in the runtime (no page-locked memory left, say) lets its caller go on without staging
+    memory: it takes the runtime's error with it, or the next launch would report it as its own. Checked on the source, as
+    the runtime cannot be made to fail here; events of a first attempt are kept for the next."""
+    more = open(os.path.join(ROOT, "mindrl_amd", "csrc", "mrb_more.inc")).read()
+    assert re.search(r"rc = stage_take\(.*?if \(rc == MRB_EHIP\) \(void\)hipGetLastError\(\);\s*return rc;", more, re.S)
+    assert re.search(r"if \(!e\) HIP_TRY\(hipEventCreateWithFlags", more)
+
+
 def test_create_replay_buffer_follows_the_reference_config_entry():
     """mindspore_rl/core/msrl.py:270-300: type / number / params-or-(sample_size, capacity) + data_shape / data_type."""
     from mindrl_amd.core import create_replay_buffer
