@@ -24,7 +24,9 @@
  *     enqueued on it in program order. Only *_create, *_destroy, mrb_per_state
  *     (when the running max is asked for), *_check and mrb_per_export_tree wait
  *     for the device (and, around the option "device_counters", what mrb_set_option
- *     says there); only *_create allocates device memory, with one exception:
+ *     says there; of the calls in mrb_more.h, which this library's Python classes add,
+ *     the two that deal with host memory, as they say); only *_create allocates
+ *     device memory, with one exception:
  *     an mrb_per_update of more entries than the buffer has rows and than any
  *     earlier call had enlarges its scratch (hipMalloc; nothing is freed before
  *     *_destroy). Calls that change one handle must be serialised by the caller

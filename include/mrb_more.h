@@ -20,11 +20,12 @@ int mrb_discounted_return_grad(const float *grad_out, const uint8_t *done, float
 
 /* Staging memory for rows that lie in host memory: `bytes` (at most 512 KiB) of page-locked memory of buffer `h` (any
  * kind), which the caller fills and hands to the handle's next push or append on `stream` as if it were device memory:
- * the kernels read it where it is. Valid for that one call. The memory, 2 MiB per buffer that is pushed host rows, is
- * allocated by the first call (no device memory) and freed with the buffer; it is handed out in turn, and a call that
- * comes around to memory given out before waits for the work that read it (calls that change one handle are ordered,
- * so an event on the stream of the call that moves on covers them all). Refused (MRB_ESTATE) while `stream` is
- * recorded into a HIP graph. */
+ * the kernels read it where it is. Valid for that one call. The memory, 2 MiB per buffer that is pushed host rows in four
+ * segments, is allocated by the first call (no device memory) and freed with the buffer. It is handed out in turn. A
+ * segment is read by work on ONE stream: a call on another stream goes on to the next segment. An event on that stream is
+ * recorded when the segment is left, and a call that comes around to it waits for the event (for the whole device, if the
+ * stream is gone by then). Refused (MRB_ESTATE) while `stream` is recorded into a HIP graph. Calls on one handle are
+ * ordered by the caller, as those that change it are. */
 int mrb_stage(int64_t h, int64_t bytes, void **ptr, void *stream);
 
 /* Before the host reads rows at `rows` (n host addresses, NULLs among them are skipped): where one of them is page-locked

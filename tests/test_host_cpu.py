@@ -165,6 +165,81 @@ def test_only_the_documented_entry_points_wait_or_allocate():
         assert not allocs.search(bodies[name]) and not waits.search(bodies[name]), name
 
 
+def more_sources():
+    """What libmrb.so is compiled from beside mrb.hip, and the extension that calls it."""
+    from mindrl_amd import build
+    names = [n for n in build.SOURCES if n != "mrb.hip"] + ["mrb_more.inc", "native.cpp"]
+    return {n: open(os.path.join(build.CSRC, n)).read() for n in names}
+
+
+def test_entry_points_beyond_the_abi_are_declared_bound_and_exported():
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "mrb_more.h")).read(), flags=re.S)
+    names = sorted(set(re.findall(r"\b(mrb_[a-z_0-9]+)\s*\(", text)))
+    assert names == sorted(_lib.MORE_SIGNATURES) == ["mrb_discounted_return_grad", "mrb_host_settled", "mrb_stage"]
+    for n in names:
+        assert hasattr(_lib.lib(), n), "libmrb.so does not export %s" % n
+    # argument checks that need no device
+    L, p = _lib.lib(), C.c_void_p(0)
+    assert L.mrb_stage(42, 64, C.byref(p), None) == _lib.MRB_EHANDLE and L.mrb_stage(42, 0, C.byref(p), None) == _lib.MRB_EINVAL
+    assert L.mrb_stage(42, (512 << 10) + 1, C.byref(p), None) == _lib.MRB_EINVAL and p.value is None
+    assert L.mrb_host_settled(None, 1, None) == _lib.MRB_EINVAL
+    assert L.mrb_host_settled((C.c_void_p * 3)(), 3, None) == _lib.MRB_OK  # no address among them: nothing to wait for
+
+
+def test_only_the_staging_calls_wait_or_allocate_beyond_the_abi():
+    """include/mrb_more.h says which of its calls wait and that one allocates page-locked memory; the launchers in the other
+    source files and the extension do neither (the extension's memory comes from torch's allocator)."""
+    calls = re.compile(r"hip(?:Device|Stream|Event)Synchronize|hipMemcpy\w*\(|hipMalloc|hipFree|hipHost\w+")
+    for name, text in more_sources().items():
+        bodies = {m.group(1): m.group(2) for m in re.finditer(r"^(?:static )?(?:int|hipError_t) (\w+)\([^;{]*\)\s*\{\n(.*?)^\}", text, re.M | re.S)}
+        allowed = {"stage_take": {"hipHostMalloc", "hipDeviceSynchronize", "hipEventSynchronize", "hipHostMallocDefault"},
+                   "mrb_host_settled": {"hipStreamSynchronize"}} if name == "mrb_more.inc" else {}
+        for fn, body in bodies.items():
+            assert set(calls.findall(body)) <= allowed.get(fn, set()), (name, fn)
+        outside = text
+        for body in bodies.values():
+            outside = outside.replace(body, "")
+        assert not calls.findall(outside), name
+    assert "Py_BEGIN_ALLOW_THREADS ready = src.stage(r, stream);" in more_sources()["native.cpp"]
+
+
+@pytest.mark.parametrize("source,count", [("mrb_range.hip", 7), ("mrb_samples.hip", 4), ("mrb_returns.hip", 10)])
+def test_kernels_of_the_other_files_use_no_scratch_memory(source, count, tmp_path):
+    """As test_kernels_use_no_scratch_memory, for the kernels outside mrb.hip."""
+    import subprocess
+    from mindrl_amd import build
+    out = tmp_path / "kernels.s"
+    flags = [f for f in build.HIPCC_FLAGS if f not in ("-shared", "-fPIC")]
+    res = subprocess.run(["/opt/rocm/bin/hipcc"] + flags + ["--cuda-device-only", "-S", "-o", str(out), os.path.join(build.CSRC, source)],
+                         stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert res.returncode == 0, res.stdout
+    kernels = {}
+    for block in out.read_text().split("  - .agpr_count:")[1:]:
+        number = lambda key: int(re.search(r"\.%s:\s+(\d+)" % key, block).group(1))
+        kernels[re.search(r"\.name:\s+(\S+)", block).group(1)] = (
+            number("private_segment_fixed_size"), number("group_segment_fixed_size"), number("vgpr_count"))
+    assert len(kernels) == count, sorted(kernels)
+    for name, (scratch, lds, vgprs) in kernels.items():
+        assert scratch == 0, "%s uses %d bytes of scratch per lane" % (name, scratch)
+        limit = 128
+        if "k_tree_range" in name:
+            # the election words and, per tile, a root of each tree and a mark
+            leaves = 1 << int(re.search(r"k_tree_rangeILi(\d+)E", name).group(1))
+            assert lds == 8 * leaves + 12 * (leaves // 256), (name, lds)
+        elif "k_discounted_return_tiled" in name:
+            cols = int(re.search(r"ELi(\d+)ELi\d+E", name).group(1))
+            assert lds == 2 * 3 * cols * 68 * 4, (name, lds)
+            if cols == 64:
+                # three chunks of sixty-four columns are 104 KB of LDS, one workgroup of nine waves to a compute unit: a
+                # SIMD holds three of them at most, and 168 registers each
+                limit = 168
+        elif "k_per_sample_lds" in name:
+            assert lds <= 1024, (name, lds)  # the field table (what is staged of the tree is sized by the launch)
+        else:
+            assert lds <= 256, (name, lds)
+        assert vgprs <= limit, (name, vgprs)
+
+
 def test_failed_staging_leaves_no_error_behind():
     """A call of mrb_stage that fails in the runtime (no page-locked memory left, say) lets its caller go on without staging
     memory: it takes the runtime's error with it, or the next launch would report it as its own. Checked on the source, as
