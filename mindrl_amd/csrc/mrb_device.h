@@ -413,10 +413,4 @@ __device__ __forceinline__ uint32_t walk32(f32x16 lo, f32x16 hi, float& mass, fl
     return (r ? 16u : 0u) + walk16(r ? hi : lo, mass, picked);
 }
 
-// Number of round trips and the levels taken by each for a tree of `depth` levels.
-__device__ __forceinline__ int group_count(int depth) { return (depth + kGroupMaxLevels - 1) / kGroupMaxLevels; }
-__device__ __forceinline__ int group_levels(int depth, int count, int i) {
-    return depth / count + (i < depth % count ? 1 : 0);
-}
-
 }  // namespace mrb

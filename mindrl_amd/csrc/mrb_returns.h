@@ -15,13 +15,9 @@ namespace mrb {
 // the return backwards in time (x = reward, t' = t, last starts at the bootstrap value), the gradient forwards
 // (kBack; x = the incoming gradient, t' = t - 1, last starts at zero: with c_t = (1 - done_t) * gamma the adjoint of
 // G_t = R_t + c_t G_{t+1} is A_t = dG_t + c_{t-1} A_{t-1}, dR_t = A_t, and the bootstrap value's gradient is
-// c_{T-1} A_{T-1}). Step s of either is time dr_time(s), its factor comes from the flags of time dr_flag(s). (The
-// gradient's step 0 has no factor: it multiplies a zero, so any flag will do.)
+// c_{T-1} A_{T-1}). Step s of the return is time T - 1 - s and its flags', of the gradient time s with the flags of time
+// s - 1. (The gradient's step 0 has no factor: it multiplies a zero, so any flag will do.)
 // ---------------------------------------------------------------------------
-template <bool kBack>
-__device__ __forceinline__ int64_t dr_time(int64_t s, int64_t timesteps) { return kBack ? s : timesteps - 1 - s; }
-template <bool kBack>
-__device__ __forceinline__ int64_t dr_flag(int64_t s, int64_t timesteps) { return kBack ? (s > 0 ? s - 1 : 0) : timesteps - 1 - s; }
 
 // Fewer columns, where a thread per column leaves the memory system idle: a workgroup takes kCols columns and walks
 // their steps in chunks of kDrChunk through three LDS buffers, as a pipeline whose stages run at the same time on

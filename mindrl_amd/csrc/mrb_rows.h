@@ -302,21 +302,6 @@ struct SampleArgs {
     uint32_t* err;
 };
 
-// mass of stratum k: (u + k) * (total / batch), each operation rounded once.
-__device__ __forceinline__ float stratum_mass(const SampleArgs& a, float total, int64_t k, float u) {
-    const float seg = total / (float)a.batch;
-    return (u + (float)k) * seg;
-}
-__device__ __forceinline__ float stratum_mass(const SampleArgs& a, float total, int64_t k) {
-    return stratum_mass(a, total, k, a.uniforms ? a.uniforms[k] : rng_uniform(a.seed, a.calls, (uint64_t)k));
-}
-
-// w = (p / total * size)^-beta / (pmin / total * size)^-beta
-__device__ __forceinline__ float is_weight(float p, float total, float pmin, float fsize, float beta) {
-    const float max_w = powf_det(pmin / total * fsize, -beta);
-    return powf_det(p / total * fsize, -beta) / max_w;
-}
-
 __device__ __forceinline__ void sample_flags(const SampleArgs& a, float total, int64_t idx, int64_t size) {
     if (!(total > 0.0f) || total > 3.0e38f) atomicOr(a.err, MRB_DERR_TOTAL);
     if (idx >= size) atomicOr(a.err, MRB_DERR_UNFILLED);
