@@ -745,8 +745,12 @@ constexpr int64_t kElectMax = 1024;
 
 // Whether an update goes by runs of leaves (launch_tree_range). Against what it would take otherwise, us per call, before /
 // by runs:
-//   fewest entries  trees of up to 14 levels, 384 / 512 entries: one workgroup along the paths 7.0 / two launches 8.5
-//                   against 6.2 / 6.3; 256 entries 6.6 (14 levels) and 5.0 (12) against 6.1: k_tree_wg keeps those.
+//   fewest entries  trees of up to 14 levels: k_tree_wg keeps up to 384 entries, in ONE launch. 65 / 256 / 384 entries, it
+//                   against runs: 10 levels 3.7 / 3.9 / 4.1 against 5.7 / 5.8 / 6.0; 12 levels 4.6 / 4.8 / 5.2 against 6.0 /
+//                   6.1 / 6.4; 13 levels 4.7 / 5.8 / 6.6 against 5.9 / 6.0 / 6.3; 14 levels 4.7 / 6.4 / 7.5 against 5.7 / 5.7 /
+//                   5.8. The last two depths' larger calls are faster by runs only where the host keeps two launches a
+//                   call ahead of the device: in the slower of two processes every call by runs took 7.2 to 8.2 us, and
+//                   k_tree_wg what it takes here. 512 entries without it: two launches with an election 8.5, by runs 6.3.
 //                   Deeper: 65 entries 7.0 (16 levels), 7.7 (20), 9.9 (22) against 6.2, 6.6, 7.4; up to 64 one wave
 //                   along the paths (k_tree_paths).
 //   most entries    10 levels, 2048 / 4096: 7.7 / 8.4 against 7.7 / 9.3; 12 levels, 8192 / 16,384: 10.0 / 11.4 against
@@ -805,7 +809,7 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
         }
     }
     // Up to a few hundred entries on a small tree: one workgroup, a thread per entry, walks the paths in one launch
-    // (k_tree_wg; on deeper trees or with more entries one compute unit's memory traffic costs more than a launch.
+    // (k_tree_wg; on deeper trees or with more entries one compute unit's memory traffic costs more than a launch: takes_range.
     // On these trees it also beats the one-wave kernel below for 64 entries or fewer: 5.45 against 5.87 us at 64.)
     if (!sparse && b->fused && n <= kWgBestEntries && b->depth >= 2 && b->depth <= kWgMaxDepth) {
         // (65 to 128 entries: 1024 threads, eight per entry - the kernel's one-step path below the staged top)

@@ -1071,11 +1071,13 @@ __device__ __forceinline__ void entry_tile(const UpdateArgs& a, int g, uint32_t 
 }
 
 // Calls of more entries than this give each entry two waves (entry_pair): the scan of a short call is too short
-// to be worth a second wave and a barrier (64 entries: no gain on the call, 0.5 us lost in a loop of calls).
+// to be worth a second wave and a barrier. Measured, us per update and push of 4 rows on 10^6 leaves, one wave / two:
+// 32 entries 7.9 / 7.9, 64 8.1 / 8.1, 128 8.4 / 8.3 (no gain worth twice the waves), 192 8.8 / 8.4, 384 9.3 / 8.9, 1024
+// 11.0 / 10.6.
 constexpr int64_t kPairedAbove = 128;
 
-// Two waves per entry (`role` 0 and 1, in one workgroup, `win` shared by the two): the power - some 110
-// dependent double-precision operations - and the election are each a wave's worth of instructions in a row;
+// Two waves per entry (`role` 0 and 1, in one workgroup, `win` shared by the two): the power - 45 double-precision
+// operations, most of them dependent - and the election are each a wave's worth of instructions in a row;
 // side by side they take the time of the longer one. Every wave of the workgroup reaches the one barrier.
 __device__ __forceinline__ void entry_pair(const UpdateArgs& a, int g, uint32_t j, uint32_t role, uint32_t lane,
                                            unsigned long long* win, uint32_t* __restrict__ dirty_out, int g_next) {
@@ -1754,11 +1756,11 @@ __global__ __launch_bounds__(kWG) void k_push_one(float* __restrict__ sum, float
 //     thread picks it up: two barrier steps of 0.7 us become one of 0.6.
 // Why only small trees: every level below the staged top costs an entry six scattered 4-byte accesses to
 // memory (sibling and cousins read, own node written, in both trees), and ONE compute unit moves about one
-// such cache line per nanosecond. Measured per call: 10,000 leaves, 128 / 256 / 384 entries: 6.1 / 6.7 / 7.6 us
-// against 8.1-8.3 us for the two launches; 2^17 leaves (six levels below the top): 8.2 / 9.7 / 11.6 us against
-// 7.7; 2^20 leaves, 512 entries: 22 us against 8.7. On the small trees it also beats the one-wave kernel above
-// for 64 entries or fewer (10,000 leaves: 5.45 against 5.87 us at 64, 5.15 against 5.82 at 16). The kernel itself
-// handles up to 1024 entries and trees of kWgMaxDepth levels.
+// such cache line per nanosecond. The line against the two launches by runs of leaves, with both sides measured, is at
+// takes_range (mrb.hip); against an entry-driven leaf round and the top, 2^17 leaves (six levels below the staged top),
+// 128 / 256 / 384 entries: 8.2 / 9.7 / 11.6 us against 7.7; 2^20 leaves, 512 entries: 22 us against 8.7. On the small
+// trees it also beats the one-wave kernel above for 64 entries or fewer (10,000 leaves: 5.45 against 5.87 us at 64, 5.15
+// against 5.82 at 16). The kernel itself handles up to 1024 entries and trees of kWgMaxDepth levels.
 // ---------------------------------------------------------------------------
 constexpr int kWgMaxEntries = 1024;
 constexpr int kWgMinThreads = 512; // so that kWgPieces 16-byte pieces per thread stage the top of a tree
@@ -1768,7 +1770,7 @@ constexpr int kWgTopNodes = 2 << kWgTopLevels;    // 4096 (node 0 does not exist
 constexpr int kWgSlotsLog2 = 11;
 constexpr int kWgSlots = 1 << kWgSlotsLog2;       // slots per hash table: twice the most entries
 constexpr int kWgMaxDepth = 14;                  // deepest tree the kernel is compiled for
-constexpr int kWgBestEntries = 384;              // most entries for which it beats two launches
+constexpr int kWgBestEntries = 384;              // most entries it is taken for (the line is at takes_range)
 constexpr int kWgHashSteps = (kWgMaxDepth - kWgTopLevels + 1) / 2;  // most two-level steps below the staged top
 constexpr int kWgTopSteps = (kWgTopLevels + 1) / 2;
 

@@ -73,9 +73,9 @@ __device__ __forceinline__ void copy_granule(gbyte* dst, const gbyte* src, uint3
     }
 }
 
-// One granule of 1 << vl bytes held between its load and its store. vl is wave-uniform; every size
-// has its own member so that no value of one load is merged with another's (a merge would make the
-// compiler wait for the load right away).
+// One granule of 1 << vl bytes held between its load and its store. vl may differ from lane to lane (where a wave's
+// lanes copy different fields: k_res_push, k_per_sample_lds); every size has its own member so that no value of one
+// load is merged with another's (a merge would make the compiler wait for the load right away).
 struct AnyGranule {
     granule_t q;
     uint64_t d;
