@@ -102,9 +102,8 @@ int mrb_version(void);
  *                  `capacity` rows, a sample at most 65,536 (its slots are drawn into a device array that
  *                  overlapping sample / get_item calls on one handle would share), mrb_urb_append_from is
  *                  refused, and mrb_urb_state, mrb_urb_reset, mrb_urb_seed and the checkpoint calls wait.
- *   "fused_rebuild" prioritized buffers: 1 (default) = an update of <= 16 entries or a push under <= 16 leaf tiles
- *                  rebuilds the tree in one launch where the tree has one round of levels below its top;
- *                  0 = one launch per round */
+ *   "fused_rebuild" prioritized buffers: 1 (default) = an update of <= 1024 entries on a tree of at most 22 levels
+ *                  or a push under <= 16 leaf tiles rebuilds the tree in one launch; 0 = one launch per round */
 /* Library-wide default, set with handle 0 and taken by buffers created afterwards:
  *   "packed_rows"  N > 0: a buffer whose packed row - every field at the next multiple of its own copy granule
  *                  (the largest power of two <= 16 that divides its size), the row padded to the widest granule -
@@ -210,9 +209,11 @@ int mrb_per_update(int64_t h, const int64_t *indices, const float *priorities, i
  * reference's training loop issues them back to back (mindspore_rl/algorithm/dqn/dqn_trainer.py:76-87). Same
  * result, bit for bit, as the two calls (a pushed row without a priority takes the running max AFTER the
  * update). No counterpart among the reference's primitives: it exists because each of these operations is
- * bound by kernel launches, and together they need fewer - one launch for up to 384 entries and one row on a
- * tree of at most 14 levels (or up to 64 entries on one of at most 25), two launches (instead of three) for up
- * to 1024 entries and a few rows on a tree of 13 to 21 levels; other sizes run as the two calls would. */
+ * bound by kernel launches, and together they need fewer - one launch for up to 1024 entries and 512 rows (whose
+ * own priorities, if they are given, go to slots of one run of leaves) on a tree of 8 to 22 levels, and for one row
+ * and up to 384 entries on a smaller tree or up to 64 on one of at most 25. With device_counters: one launch for up
+ * to 384 entries and one row on a tree of at most 14 levels (64 on one of at most 25), two for up to 1024 entries and a
+ * few rows on a tree of 13 to 21 levels. Other sizes run as the two calls would. */
 int mrb_per_update_push(int64_t h, const int64_t *indices, const float *priorities, int64_t n,
                         const void *const *src_fields, int64_t nrows, const float *opt_push_priorities,
                         void *stream);

@@ -16,7 +16,9 @@
 #include <vector>
 
 #include "mrb_kernels.h"
+#include "mrb_meet.h"
 #include "mrb_range.h"
+#include "mrb_range_one.h"
 #include "mrb_returns.h"
 #include "mrb_samples.h"
 #include "../../include/mrb_more.h"
@@ -743,16 +745,8 @@ UpdateArgs update_args(Per& b) {
 // the call's entries); larger calls take the stamp pass (2048 measured: config 4's update 14.0 us against 14.7 with the pass, at twice the waves and four times the comparisons: not taken).
 constexpr int64_t kElectMax = 1024;
 
-// Whether an update goes by runs of leaves (launch_tree_range). Against what it would take otherwise, us per call, before /
-// by runs:
-//   fewest entries  trees of up to 14 levels: k_tree_wg keeps up to 384 entries, in ONE launch. 65 / 256 / 384 entries, it
-//                   against runs: 10 levels 3.7 / 3.9 / 4.1 against 5.7 / 5.8 / 6.0; 12 levels 4.6 / 4.8 / 5.2 against 6.0 /
-//                   6.1 / 6.4; 13 levels 4.7 / 5.8 / 6.6 against 5.9 / 6.0 / 6.3; 14 levels 4.7 / 6.4 / 7.5 against 5.7 / 5.7 /
-//                   5.8. The last two depths' larger calls are faster by runs only where the host keeps two launches a
-//                   call ahead of the device: in the slower of two processes every call by runs took 7.2 to 8.2 us, and
-//                   k_tree_wg what it takes here. 512 entries without it: two launches with an election 8.5, by runs 6.3.
-//                   Deeper: 65 entries 7.0 (16 levels), 7.7 (20), 9.9 (22) against 6.2, 6.6, 7.4; up to 64 one wave
-//                   along the paths (k_tree_paths).
+// Whether an update of more than 1024 entries goes by runs of leaves (launch_tree_range). Against what it would take
+// otherwise, us per call, before / by runs:
 //   most entries    10 levels, 2048 / 4096: 7.7 / 8.4 against 7.7 / 9.3; 12 levels, 8192 / 16,384: 10.0 / 11.4 against
 //                   9.6 / 13.8; 14 levels, 16,384 / 32,768: 11.7 / 12.5 against 11.2 / 16.7; 20 levels 14.4 / 15.4 against
 //                   14.1 / 18.7; 22 levels, 8192 / 16,384: 16.1 / 17.7 against 16.0 / 21.0.
@@ -760,10 +754,20 @@ constexpr int64_t kElectMax = 1024;
 //                   entries 14.9 / 15.9 against 14.9 / 23.3.
 bool takes_range(const Per& b, int64_t n) {
     if (!b.fused || b.depth < 10 || b.depth > 22) return false;
-    const int64_t fewest = b.depth <= kWgMaxDepth ? kWgBestEntries : kPathEntries;
     const int64_t most = b.depth <= 11 ? 2048 : b.depth == 12 || b.depth == 22 ? 8192 : 16384;
-    return n > fewest && n <= most;
+    return n > kOneMostEntries && n <= most;
 }
+
+// Whether one launch takes an update (and the push that follows it in the call) by runs of leaves: k_range_one. On the
+// device two launches (k_tree_range, k_tree_cap) catch up at 1024 entries on 20 levels and more - 7.7 against 8.1 us, 2048 on
+// 21 levels 9.1 against 10.4 -, where the host's time for the second one (2.7 us) still decides for calls this small. Trees of
+// fewer than 8 levels have no whole tile, those of more than 22 more than 256 runs.
+bool takes_range_one(const Per& b, int64_t n) { return b.fused && n <= kOneMostEntries && b.depth >= 8 && b.depth <= 22; }
+
+// Where one workgroup's update alone (k_tree_wg) is faster than that, us: 13 levels, 1 / 64 / 96 / 128 entries 4.3 / 4.6 / 4.8 /
+// 5.0 against 4.4 / 4.8 / 4.8 / 4.8; 14 levels 4.3 / 4.6 / 4.9 / 5.1 against 4.4 / 4.8 / 4.9 / 4.9. (12 levels, 1 / 64 / 384: 4.4
+// / 4.5 / 5.2 against 4.3 / 4.5 / 5.0.)
+bool takes_wg_rather(const Per& b, int64_t n) { return (b.depth == 13 || b.depth == 14) && n <= 96; }
 
 // update_priorities on buffer b with `powered` (device f32[n]) as the scratch that holds the entries'
 // p^alpha between the stamp pass and the leaf writes. Allocates nothing.
@@ -781,6 +785,10 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
             return fail(MRB_ESTATE, "an update of more than %lld entries cannot be recorded into a HIP graph (its "
                                     "election tags are counted on the host); split it into calls of at most %lld",
                         (long long)kElectMax, (long long)kElectMax);
+    }
+    if (takes_range_one(*b, n) && !takes_wg_rather(*b, n)) {
+        const hipError_t e = launch_range_one(indices, priorities, n, b->sum, b->mn, b->maxp, b->rows.capacity, b->depth, b->alpha, s);
+        return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch k_range_one: %s", hipGetErrorString(e));
     }
     if (takes_range(*b, n)) {
         hipError_t e = launch_tree_range(indices, priorities, n, b->sum, b->mn, b->maxp, b->err, b->rows.capacity, b->depth, b->alpha, s);
@@ -808,9 +816,7 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
             a.g[r] = b->s_g[r];
         }
     }
-    // Up to a few hundred entries on a small tree: one workgroup, a thread per entry, walks the paths in one launch
-    // (k_tree_wg; on deeper trees or with more entries one compute unit's memory traffic costs more than a launch: takes_range.
-    // On these trees it also beats the one-wave kernel below for 64 entries or fewer: 5.45 against 5.87 us at 64.)
+    // Up to a few hundred entries on a small tree: one workgroup, a thread per entry, walks the paths in one launch (k_tree_wg).
     if (!sparse && b->fused && n <= kWgBestEntries && b->depth >= 2 && b->depth <= kWgMaxDepth) {
         // (65 to 128 entries: 1024 threads, eight per entry - the kernel's one-step path below the staged top)
         const uint32_t threads = n > 64 && n <= 128 ? 1024u : n <= kWgMinThreads ? (uint32_t)kWgMinThreads : (uint32_t)((n + 63) / 64 * 64);
@@ -819,7 +825,7 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
         LAUNCH_CHECK("k_tree_wg");
         return MRB_OK;
     }
-    // At most 64 entries on a deeper tree: one wave walks the entries' paths, leaves to root, in one launch (k_tree_paths).
+    // At most 64 entries on a very deep tree: one wave walks the entries' paths, leaves to root, in one launch (k_tree_paths).
     if (!sparse && b->fused && n <= kPathEntries && b->depth <= kPathMaxDepth) {
         hipLaunchKernelGGL(k_tree_paths, dim3(1), dim3(64), 0, s, a);
         LAUNCH_CHECK("k_tree_paths");
@@ -1254,10 +1260,12 @@ int mrb_per_create(int64_t capacity, float alpha, int nfields, const int64_t* fi
     // word), and kMaxpBehindErr bytes in the running max (16 bytes; a kernel that is given its address finds the
     // counters in front of it: counters_before)
     static_assert(16 + kCntWords * sizeof(int64_t) <= kMaxpBehindErr, "the counters end before the running max");
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->err), kMaxpBehindErr + 16));
+    // (and, behind it, what the workgroups of an update meet over: Meet)
+    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->err), kMaxpBehindErr + kMeetBehindMaxp + sizeof(Meet)));
     b->counters = reinterpret_cast<int64_t*>(b->err + 4);
     b->maxp = reinterpret_cast<float*>(reinterpret_cast<char*>(b->err) + kMaxpBehindErr);
     HIP_TRY(hipMemset(b->counters, 0, kCntWords * sizeof(int64_t)));
+    HIP_TRY(hipMemset(reinterpret_cast<char*>(b->maxp) + kMeetBehindMaxp, 0, sizeof(Meet)));
     // update_priorities scratch, sized once: a call rarely names more entries than there are rows
     b->powered_cap = capacity < 4096 ? 4096 : (capacity > (1ll << 20) ? (1ll << 20) : capacity);
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->powered), (size_t)b->powered_cap * sizeof(float)));
@@ -1451,7 +1459,24 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t cap = b->rows.capacity;
     const bool small_push = nrows <= cap && b->fused;
-    // (1) one launch: the one-workgroup or one-wave update, then the walk of the one pushed row by the same workgroup
+    // (1) one launch: the update by runs of leaves, whose workgroups also write the pushed rows' leaves; the ring's position
+    // has to be the host's, and given priorities one run's
+    if (small_push && !b->device_counters && nrows <= kOneMostRows && takes_range_one(*b, n)) {
+        const int64_t first = b->pushes % cap, last = first + nrows - 1;
+        const int w = range_one_levels(b->depth, n);
+        PutArgs put{};
+        int rc = put_args(b->rows, src_fields, 0, nrows, first, put);
+        if (rc) return rc;
+        if (put.blocks <= kOneMostRiders && (!opt_push_priorities || (last < cap && first >> w == last >> w))) {
+            const RangePush push{opt_push_priorities, (uint32_t)first, (uint32_t)nrows};
+            const hipError_t e = launch_range_one_push(indices, priorities, n, b->sum, b->mn, b->maxp, cap, b->depth, b->alpha, push, put, s);
+            if (e != hipSuccess) return fail(MRB_EHIP, "launch k_range_one_push: %s", hipGetErrorString(e));
+            b->pushes += nrows;
+            b->size = b->size + nrows < cap ? b->size + nrows : cap;
+            return MRB_OK;
+        }
+    }
+    // (2) one launch: the one-workgroup or one-wave update, then the walk of the one pushed row by the same workgroup
     const bool wg = n <= kWgBestEntries && b->depth >= 2 && b->depth <= kWgMaxDepth;
     const bool paths = n <= kPathEntries && b->depth <= kPathMaxDepth && b->depth >= 2;
     if (small_push && nrows == 1 && (wg || paths) && b->depth <= kPushOneMaxDepth) {
@@ -1493,7 +1518,7 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
             return MRB_OK;
         }
     }
-    // (2) two launches on a tree with one round of levels below its top: the update's leaf round with the push's
+    // (3) two launches on a tree with one round of levels below its top: the update's leaf round with the push's
     // row copy riding along, then one workgroup that rebuilds the pushed slots' leaf tiles and the whole top
     if (small_push && b->nrounds == 1 && n <= kElectMax && n > kFusedWG / 64 && b->depth >= 2 &&
         push_tiles(*b, b->pushes % cap, nrows) <= (uint32_t)kRunWaves) {
@@ -1506,7 +1531,7 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
         lead.a.inline_election = 1;
         return per_push(b.get(), src_fields, nrows, opt_push_priorities, s, &lead);
     }
-    // (3) otherwise: the two calls, one after the other
+    // (4) otherwise: the two calls, one after the other
     int rc = mrb_per_update(h, indices, priorities, n, stream);
     if (rc) return rc;
     return per_push(b.get(), src_fields, nrows, opt_push_priorities, s);

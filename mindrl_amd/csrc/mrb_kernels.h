@@ -1497,7 +1497,9 @@ __global__ __launch_bounds__(kFusedWG) void k_tree_fused(UpdateArgs a, uint32_t 
 //      active lane (for a left child) or the one before (for a right child). Of two lanes that meet in a
 //      parent the left child's goes on. Every node is the single rounded sum / min of its two final
 //      children, as everywhere.
-// Keys are 32 bits: leaf * 64 + lane, so the tree has at most 2^25 leaves here.
+// Keys are 32 bits: leaf * 64 + lane, so the tree has at most 2^25 leaves here. On trees of up to 22 levels a launch by runs
+// of leaves (k_range_one) is faster at any size: 1 / 64 entries on 2^16 leaves 7.0 / 7.6 us here, 4.6 / 5.0 there, on 2^22 8.5 /
+// 9.7 and 5.6 / 6.0.
 // ---------------------------------------------------------------------------
 constexpr int kPathEntries = 64;
 constexpr int kPathMaxDepth = 25;
@@ -1756,11 +1758,9 @@ __global__ __launch_bounds__(kWG) void k_push_one(float* __restrict__ sum, float
 //     thread picks it up: two barrier steps of 0.7 us become one of 0.6.
 // Why only small trees: every level below the staged top costs an entry six scattered 4-byte accesses to
 // memory (sibling and cousins read, own node written, in both trees), and ONE compute unit moves about one
-// such cache line per nanosecond. The line against the two launches by runs of leaves, with both sides measured, is at
-// takes_range (mrb.hip); against an entry-driven leaf round and the top, 2^17 leaves (six levels below the staged top),
-// 128 / 256 / 384 entries: 8.2 / 9.7 / 11.6 us against 7.7; 2^20 leaves, 512 entries: 22 us against 8.7. On the small
-// trees it also beats the one-wave kernel above for 64 entries or fewer (10,000 leaves: 5.45 against 5.87 us at 64, 5.15
-// against 5.82 at 16). The kernel itself handles up to 1024 entries and trees of kWgMaxDepth levels.
+// such cache line per nanosecond (2^20 leaves, 512 entries: 22 us). Where it is taken, against the launch by runs of leaves:
+// takes_wg_rather (mrb.hip), and trees of fewer than 8 levels. The kernel itself handles up to 1024 entries and trees of
+// kWgMaxDepth levels.
 // ---------------------------------------------------------------------------
 constexpr int kWgMaxEntries = 1024;
 constexpr int kWgMinThreads = 512; // so that kWgPieces 16-byte pieces per thread stage the top of a tree
@@ -1770,7 +1770,7 @@ constexpr int kWgTopNodes = 2 << kWgTopLevels;    // 4096 (node 0 does not exist
 constexpr int kWgSlotsLog2 = 11;
 constexpr int kWgSlots = 1 << kWgSlotsLog2;       // slots per hash table: twice the most entries
 constexpr int kWgMaxDepth = 14;                  // deepest tree the kernel is compiled for
-constexpr int kWgBestEntries = 384;              // most entries it is taken for (the line is at takes_range)
+constexpr int kWgBestEntries = 384;              // most entries it is taken for (one launch by runs of leaves beats it long before: takes_wg_rather)
 constexpr int kWgHashSteps = (kWgMaxDepth - kWgTopLevels + 1) / 2;  // most two-level steps below the staged top
 constexpr int kWgTopSteps = (kWgTopLevels + 1) / 2;
 

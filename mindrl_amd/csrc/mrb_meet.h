@@ -1,0 +1,88 @@
+// How workgroups of one launch hand their subtrees' roots to the last of them.
+//
+// Every workgroup leaves its root, sum and minimum, in a word of its own and raises a counter; the one that finds it was the
+// last takes all the roots and rebuilds what lies above them. A second launch for those levels costs 1.5 us on the device and
+// 2.5 us of the host's time (its arguments go to device memory and are read back once); a fence per workgroup would cost
+// 60 ns each, one after the other, on a part whose dies have caches of their own. So there is no fence: a root's words carry
+// the launch's number beside the value, the last workgroup looks at that, and reads again those (few, if any) whose stores
+// the counter has overtaken. It waits for stores that are on their way, never for a workgroup that has yet to run, so it
+// ends however the workgroups are scheduled; nothing has to be cleared between launches; and a launch replayed from a graph
+// finds its number on the device.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "mrb_rows.h"
+
+namespace mrb {
+
+constexpr int kMeetMost = 256;  // roots: a tile's worth of nodes
+
+// kMeetBehindMaxp bytes behind a buffer's running max (one allocation, see counters_behind).
+constexpr int kMeetBehindMaxp = 64;
+struct Meet {
+    uint32_t arrived;  // of the launch in progress
+    uint32_t turn;     // launches so far
+    uint32_t pad[30];
+    unsigned long long root[kMeetMost][2];  // launch number << 32 | bits: sum, minimum
+};
+
+__device__ __forceinline__ Meet* meet_of(float* maxp) { return reinterpret_cast<Meet*>(reinterpret_cast<char*>(maxp) + kMeetBehindMaxp); }
+__device__ __forceinline__ uint32_t* err_before(float* maxp) {
+    return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(maxp) - kMaxpBehindErr);
+}
+
+// The number of launches before this one (requested when a kernel starts: the last workgroup moves it on).
+__device__ __forceinline__ uint32_t meet_turn(float* maxp) {
+    return __hip_atomic_load(&meet_of(maxp)->turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Called by one whole wave of each of the `count` workgroups that change their root (number `which`). In the last one's it
+// returns true; vs, vm - four roots to a lane, as memory held them when the kernel started - then hold the new ones where
+// `changed` has the root's bit. The roots are requested together with the counter's answer, on the chance that this is the
+// last workgroup and that the others' stores have arrived: then one trip is all it takes.
+__device__ __forceinline__ bool meet(float* maxp, uint32_t turn, uint32_t which, uint32_t count, float root_s, float root_m, uint32_t lane,
+                                     uint32_t changed, float4& vs, float4& vm) {
+    Meet* const m = meet_of(maxp);
+    const uint32_t tag = turn + 1;
+    uint32_t before = 0;
+    if (lane == 0) {
+        const unsigned long long number = (unsigned long long)tag << 32;
+        __hip_atomic_store(&m->root[which][0], number | __float_as_uint(root_s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&m->root[which][1], number | __float_as_uint(root_m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" ::: "memory");  // issued in this order
+        before = __hip_atomic_fetch_add(&m->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    float s[4] = {vs.x, vs.y, vs.z, vs.w}, t[4] = {vm.x, vm.y, vm.z, vm.w};
+    for (;;) {
+        unsigned long long a[4], b[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            a[c] = b[c] = 0;
+            if (changed >> c & 1u) {
+                a[c] = __hip_atomic_load(&m->root[4 * lane + c][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                b[c] = __hip_atomic_load(&m->root[4 * lane + c][1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)before) != count - 1) return false;
+        bool open = false;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (changed >> c & 1u) {
+                open = open || (uint32_t)(a[c] >> 32) != tag || (uint32_t)(b[c] >> 32) != tag;
+                s[c] = __uint_as_float((uint32_t)a[c]);
+                t[c] = __uint_as_float((uint32_t)b[c]);
+            }
+        }
+        if (!__any(open)) break;
+    }
+    vs = make_float4(s[0], s[1], s[2], s[3]);
+    vm = make_float4(t[0], t[1], t[2], t[3]);
+    if (lane == 0) {  // ready for the next launch
+        m->arrived = 0;
+        m->turn = tag;
+    }
+    return true;
+}
+
+}  // namespace mrb

@@ -80,4 +80,37 @@ __device__ __forceinline__ void tile_parents(const Trees& a, int g, uint32_t fir
     if (root_m) *root_m = fminf(m_lo, m_hi);
 }
 
+// The `levels` levels (at most six) above up to 64 consecutive nodes, one to a lane (cs, cm; `first` is the first one's heap
+// index); lane 0 is left with the root.
+template <int S, typename Trees>
+__device__ __forceinline__ void run_step(const Trees& a, int levels, uint32_t first, uint32_t lane, bool active, float& cs, float& cm) {
+    if (S < levels) {  // uniform
+        if constexpr (S < 4) {
+            cs = cs + butterfly_peer<S>(cs);
+            cm = fminf(cm, butterfly_peer<S>(cm));
+        } else if constexpr (S == 4) {
+            const float s0 = lane_value(cs, 0) + lane_value(cs, 16), s1 = lane_value(cs, 32) + lane_value(cs, 48);
+            const float m0 = fminf(lane_value(cm, 0), lane_value(cm, 16)), m1 = fminf(lane_value(cm, 32), lane_value(cm, 48));
+            cs = lane < 32 ? s0 : s1;
+            cm = lane < 32 ? m0 : m1;
+        } else {
+            cs = lane_value(cs, 0) + lane_value(cs, 32);
+            cm = fminf(lane_value(cm, 0), lane_value(cm, 32));
+        }
+        if (active && (lane & ((2u << S) - 1)) == 0) {
+            a.sum[(first + lane) >> (S + 1)] = cs;
+            a.mn[(first + lane) >> (S + 1)] = cm;
+        }
+    }
+}
+template <typename Trees>
+__device__ __forceinline__ void run_parents(const Trees& a, int levels, uint32_t first, uint32_t lane, bool active, float& cs, float& cm) {
+    run_step<0>(a, levels, first, lane, active, cs, cm);
+    run_step<1>(a, levels, first, lane, active, cs, cm);
+    run_step<2>(a, levels, first, lane, active, cs, cm);
+    run_step<3>(a, levels, first, lane, active, cs, cm);
+    run_step<4>(a, levels, first, lane, active, cs, cm);
+    run_step<5>(a, levels, first, lane, active, cs, cm);
+}
+
 }  // namespace mrb

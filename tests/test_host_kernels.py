@@ -1,0 +1,28 @@
+"""The kernels of the source files that tests/test_host_cpu.py does not look at: no scratch memory, no more registers than
+their workgroups' waves have, the LDS their comments state."""
+import os
+import re
+import subprocess
+
+import pytest
+
+
+@pytest.mark.parametrize("source,count", [("mrb_range_one.hip", 8)])
+def test_kernels_use_no_scratch_memory(source, count, tmp_path):
+    from mindrl_amd import build
+    out = tmp_path / "kernels.s"
+    flags = [f for f in build.HIPCC_FLAGS if f not in ("-shared", "-fPIC")]
+    res = subprocess.run(["/opt/rocm/bin/hipcc"] + flags + ["--cuda-device-only", "-S", "-o", str(out), os.path.join(build.CSRC, source)],
+                         stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert res.returncode == 0, res.stdout
+    kernels = {}
+    for block in out.read_text().split("  - .agpr_count:")[1:]:
+        number = lambda key: int(re.search(r"\.%s:\s+(\d+)" % key, block).group(1))
+        kernels[re.search(r"\.name:\s+(\S+)", block).group(1)] = (
+            number("private_segment_fixed_size"), number("group_segment_fixed_size"), number("vgpr_count"))
+    assert len(kernels) == count, sorted(kernels)
+    for name, (scratch, lds, vgprs) in kernels.items():
+        assert scratch == 0 and vgprs <= 128, (name, scratch, vgprs)
+        # the election words, a root of each tree and a mark per tile, the runs' bits and a word per wave
+        leaves = 1 << int(re.search(r"k_range_one(?:_push)?ILi(\d+)E", name).group(1))
+        assert 0 <= lds - (8 * leaves + 12 * (leaves // 256)) <= 64, (name, lds)
