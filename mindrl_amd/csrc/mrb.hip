@@ -192,6 +192,7 @@ int put_args(const RowStore& r, const void* const* src, int64_t skip, int64_t n,
     p.src_capacity = 0;
     p.src_first = 0;
     p.blocks = grid_for(p.t.prefix[p.t.nfields]);
+    p.threads = kWG;
     return MRB_OK;
 }
 
@@ -424,8 +425,9 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
     // a row of workgroups per field, as many as the field with the most granules needs
     uint64_t most = 0;
     for (int f = 0; f < t.nfields; ++f) most = std::max<uint64_t>(most, t.prefix[f + 1] - t.prefix[f]);
-    hipLaunchKernelGGL(k_rows_gather, dim3(grid_for(most), (uint32_t)t.nfields), dim3(kWG), 0, s, t, r.capacity, count,
-                       indices, fixed_slot, seed, calls, out_indices, err);
+    const uint32_t blocks = grid_for(most);
+    hipLaunchKernelGGL(k_rows_gather, dim3(blocks, (uint32_t)t.nfields), dim3(kWG), 0, s, t, r.capacity, count, indices, fixed_slot,
+                       seed, calls, out_indices, err, blocks);
     LAUNCH_CHECK("k_rows_gather");
     return MRB_OK;
 }
@@ -653,6 +655,7 @@ int tree_rebuild(Per& b, UpdateArgs a, hipStream_t s, const PutArgs* ride = null
         }
         const uint32_t threads = units <= kWG / 64 ? (uint32_t)kWG : (uint32_t)kFusedWG;
         put.blocks = (put.blocks * kWG + threads - 1) / threads;  // the ride-along copy was sized for workgroups of kWG
+        put.threads = threads;
         a.readers = 1 + put.blocks;  // (a.advance != 0: this one launch also moves the device's counters on)
         hipLaunchKernelGGL(k_push_run, dim3(1 + put.blocks), dim3(threads), 0, s, a, units, put);
         LAUNCH_CHECK("k_push_run");
@@ -681,12 +684,14 @@ int tree_rebuild(Per& b, UpdateArgs a, hipStream_t s, const PutArgs* ride = null
         }
         const PutArgs& put = (r == 0 && ride) ? *ride : none;
         if (r == 0 && a.inline_election) tiles = (a.n > kPairedAbove ? 2u : 1u) * (uint32_t)a.n;  // one or two waves per entry (see k_tree_update)
-        hipLaunchKernelGGL(k_tree_update, dim3((tiles + 3) / 4 + put.blocks), dim3(kWG), 0, s, a.indices, a.priorities, a.sum, a.mn,
+        a.tile_blocks = (tiles + 3) / 4;
+        hipLaunchKernelGGL(k_tree_update, dim3(a.tile_blocks + put.blocks), dim3(kWG), 0, s, a.indices, a.priorities, a.sum, a.mn,
                            a.n, a.capacity, r | a.lo[r] << 8 | a.g[r] << 16, a.alpha, a, tile_base, put);
         LAUNCH_CHECK("k_tree_update");
     }
     PutArgs put = (a.nrounds == 0 && ride) ? *ride : none;
     if (int rc = ride_alone_if_large(a, put, s)) return rc;
+    put.threads = kTopWG;
     // the top is the call's last launch: it moves the device's counters on (a.advance != 0); only when it is also
     // the first do its workgroups read the ring position
     a.readers = a.nrounds == 0 ? 1 + put.blocks : 0;
@@ -791,7 +796,7 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
         return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch k_range_one: %s", hipGetErrorString(e));
     }
     if (takes_range(*b, n)) {
-        hipError_t e = launch_tree_range(indices, priorities, n, b->sum, b->mn, b->maxp, b->err, b->rows.capacity, b->depth, b->alpha, s);
+        hipError_t e = launch_tree_range(indices, priorities, n, b->sum, b->mn, b->maxp, b->rows.capacity, b->depth, b->alpha, s);
         if (e != hipSuccess) return fail(MRB_EHIP, "launch k_tree_range: %s", hipGetErrorString(e));
         e = launch_tree_cap(b->sum, b->mn, b->depth - tree_range_levels(b->depth), s);
         if (e != hipSuccess) return fail(MRB_EHIP, "launch k_tree_cap: %s", hipGetErrorString(e));
@@ -821,7 +826,7 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
         // (65 to 128 entries: 1024 threads, eight per entry - the kernel's one-step path below the staged top)
         const uint32_t threads = n > 64 && n <= 128 ? 1024u : n <= kWgMinThreads ? (uint32_t)kWgMinThreads : (uint32_t)((n + 63) / 64 * 64);
         hipLaunchKernelGGL(k_tree_wg, dim3(1), dim3(threads), 0, s, a.indices, a.priorities, a.sum, a.mn, a.maxp, (int)a.n,
-                           a.depth, (int)a.capacity, a.alpha, a);
+                           a.depth | (int)threads << 8, (int)a.capacity, a.alpha);
         LAUNCH_CHECK("k_tree_wg");
         return MRB_OK;
     }
@@ -850,7 +855,8 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
     const int last = b->s_rounds - 1;
     for (int r = 0; r < last; ++r) {
         const uint32_t tiles = (1u << b->s_lo[r]) / kBlockNodes;
-        hipLaunchKernelGGL(k_tree_update, dim3((tiles + 3) / 4), dim3(kWG), 0, s, a.indices, a.priorities, a.sum, a.mn, a.n,
+        a.tile_blocks = (tiles + 3) / 4;
+        hipLaunchKernelGGL(k_tree_update, dim3(a.tile_blocks), dim3(kWG), 0, s, a.indices, a.priorities, a.sum, a.mn, a.n,
                            a.capacity, r | a.lo[r] << 8 | a.g[r] << 16, a.alpha, a, 0u, PutArgs{});
         LAUNCH_CHECK("k_tree_update");
     }
@@ -1097,6 +1103,7 @@ int mrb_urb_append_from(int64_t h, int64_t src, int64_t first_logical, int64_t n
     p.src_capacity = from->rows.capacity;
     p.src_first = (src_first + skip) % from->rows.capacity;
     p.blocks = grid_for(p.t.prefix[p.t.nfields]);
+    p.threads = kWG;
     hipLaunchKernelGGL(k_rows_put, dim3(p.blocks), dim3(kWG), 0, static_cast<hipStream_t>(stream), p);
     LAUNCH_CHECK("k_rows_put");
     urb_advance(*b, n);
@@ -1344,8 +1351,9 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
     if (lead) {
         // the update's leaf round (a wave or two per entry), with this push's row copy as further workgroups
         const uint32_t waves = (lead->a.n > kPairedAbove ? 2u : 1u) * (uint32_t)lead->a.n;
-        const UpdateArgs& la = lead->a;
-        hipLaunchKernelGGL(k_tree_update, dim3((waves + 3) / 4 + put.blocks), dim3(kWG), 0, s, la.indices, la.priorities, la.sum,
+        UpdateArgs la = lead->a;
+        la.tile_blocks = (waves + 3) / 4;
+        hipLaunchKernelGGL(k_tree_update, dim3(la.tile_blocks + put.blocks), dim3(kWG), 0, s, la.indices, la.priorities, la.sum,
                            la.mn, la.n, la.capacity, 0 | la.lo[0] << 8 | la.g[0] << 16, la.alpha, la, 0u, put);
         LAUNCH_CHECK("k_tree_update");
         put.blocks = 0;
@@ -1503,8 +1511,10 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
                 // (65 to 128 entries: 1024 threads, eight per entry - the kernel's one-step path below the staged top)
         const uint32_t threads = n > 64 && n <= 128 ? 1024u : n <= kWgMinThreads ? (uint32_t)kWgMinThreads : (uint32_t)((n + 63) / 64 * 64);
                 a.readers = 1 + put.blocks * (threads / 64);
+                put.threads = threads;
                 hipLaunchKernelGGL(b->device_counters ? k_tree_wg_push<true> : k_tree_wg_push<false>, dim3(1 + put.blocks),
-                                   dim3(threads), 0, s, a.indices, a.priorities, a.sum, a.mn, a.maxp, (int)a.n, a.depth,
+                                   dim3(threads), 0, s, a.indices, a.priorities, a.sum, a.mn, a.maxp, (int)a.n,
+                                   a.depth | (int)threads << 8,
                                    (int)a.capacity, a.alpha, a, slot, opt_push_priorities, put);
                 LAUNCH_CHECK("k_tree_wg_push");
             } else {

@@ -12,8 +12,9 @@
 namespace mrb {
 
 constexpr int kTopMaxDepth = 12;  // deepest level k_tree_top normally starts from (4096 nodes)
+constexpr int kTopWG = 1024;
 
-__global__ __launch_bounds__(kWG) void k_rows_put(PutArgs p) { rows_put_part(p, blockIdx.x, gridDim.x); }
+__global__ __launch_bounds__(kWG) void k_rows_put(PutArgs p) { rows_put_part(p, blockIdx.x, p.blocks); }
 
 // ---------------------------------------------------------------------------
 // Gather: io_f[k] = store_f[slot_k]. slot_k is `fixed_slot` when that is >= 0
@@ -25,7 +26,7 @@ __global__ __launch_bounds__(kWG) void k_rows_gather(IoTable t, int64_t capacity
                                                      const int64_t* __restrict__ indices, int64_t fixed_slot,
                                                      uint64_t seed, uint64_t calls,
                                                      int64_t* __restrict__ out_indices,
-                                                     uint32_t* __restrict__ err) {
+                                                     uint32_t* __restrict__ err, uint32_t blocks) {
     // blockIdx.y is the field: the table's entries for it are the same for every thread of the launch's row of
     // workgroups and come through scalar registers, requested with the other arguments. (Indexed by a field number
     // each thread works out for itself they were two more dependent trips to memory in a kernel that is a chain of
@@ -35,7 +36,7 @@ __global__ __launch_bounds__(kWG) void k_rows_gather(IoTable t, int64_t capacity
     const gbyte* const store = as_global(t.store[f]);
     gbyte* const io = as_global(t.io[f]);
     const uint64_t total = t.prefix[f + 1] - t.prefix[f];  // rows * units
-    const uint64_t step = (uint64_t)gridDim.x * kWG;
+    const uint64_t step = (uint64_t)blocks * kWG;
     for (uint64_t w = (uint64_t)blockIdx.x * kWG + threadIdx.x; w < total; w += step) {
         uint64_t row;
         uint32_t unit;
@@ -669,6 +670,7 @@ struct UpdateArgs {
     // the workgroups of this launch that read the ring position (see counters_push_done)
     int64_t advance;
     uint32_t readers;
+    uint32_t tile_blocks;  // workgroups of k_tree_update that work on tiles (those behind them carry a push's row copy)
 };
 
 // (The leading plain parameters repeat members of `a_in`: preloaded into scalar registers, so the entries are requested
@@ -935,7 +937,7 @@ __device__ __forceinline__ void fold_push_max(const UpdateArgs& a) {
         return;
     }
     float q = 0.0f;
-    for (int64_t j = threadIdx.x; j < a.n; j += blockDim.x) {
+    for (int64_t j = threadIdx.x; j < a.n; j += kTopWG) {
         const float p = a.priorities[j];
         if (valid_priority(p)) {
             q = fmaxf(q, powf_det_call(p, a.alpha));
@@ -1116,7 +1118,7 @@ __device__ __forceinline__ void entry_pair(const UpdateArgs& a, int g, uint32_t 
 // is the leaf level, clean tiles are skipped like in a round. `win`: 256 eight-byte words of LDS per wave
 // (see tile_round).
 __device__ __forceinline__ void top_rebuild(const UpdateArgs& a, int top, unsigned long long* win) {
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = kTopWG >> 6;
     const int g1 = top < kRoundLevels ? top : kRoundLevels;
     const uint32_t tiles = (1u << top) <= (uint32_t)kBlockNodes ? 1u : (1u << top) / kBlockNodes;
     if (a.inline_election && top == a.depth) entry_duty(a, wave, nwaves, lane);
@@ -1163,7 +1165,7 @@ __global__ __launch_bounds__(kWG) void k_tree_update(const int64_t* __restrict__
                                                      int64_t lead_n, int64_t lead_capacity, int plan, float lead_alpha,
                                                      UpdateArgs a_in, uint32_t tile_base, PutArgs put) {
     __shared__ unsigned long long s_win[kWG / 64][kBlockNodes];
-    const uint32_t tile_blocks = gridDim.x - put.blocks;
+    const uint32_t tile_blocks = a_in.tile_blocks;
     if (blockIdx.x >= tile_blocks) {
         rows_put_part(put, blockIdx.x - tile_blocks, put.blocks);
         rider_ends();
@@ -1220,7 +1222,6 @@ __global__ __launch_bounds__(kWG) void k_tree_update(const int64_t* __restrict__
 // A separate launch rather than a continuation of the last round by its last workgroup: publishing
 // the rounds' stores to that workgroup needs an agent-scope fence per workgroup, which on this
 // multi-die part costs far more than a launch.
-constexpr int kTopWG = 1024;
 __global__ __launch_bounds__(kTopWG) void k_tree_top(UpdateArgs a, PutArgs put) {
     __shared__ unsigned long long s_win[kTopWG / 64][kBlockNodes];
     if (__builtin_expect(blockIdx.x >= 1, 0)) {  // (the tree workgroup's code comes first: it is the one the call waits for)
@@ -1364,7 +1365,7 @@ __global__ __launch_bounds__(kFusedWG) void k_push_run(UpdateArgs a, uint32_t un
             s_new[l][wave] = rebuilt;
         }
         lds_barrier();
-        if (l == 0 && a.fold_max && wave == blockDim.x / 64 - 1) {
+        if (l == 0 && a.fold_max && wave == put.threads / 64 - 1) {
             // the running max, by the last wave: every leaf that takes it as it was has been written
             const float q = wave_max(lane < units ? s_largest[lane] : 0.0f);
             if (lane == 0 && q > 0.0f) raise_max(a.maxp, q);
@@ -1872,17 +1873,17 @@ __device__ __forceinline__ void top_write_back_by(const UpdateArgs& a, const flo
 // caller before the workgroup's first barrier) receives what StepShared describes, watch_leaf being the heap
 // number of the leaf the caller writes next - with kStep == 2 taken from `step` (left there before the first
 // barrier: the caller had to read it from the device).
-template <bool kTake, int kStep = 0, int kThreads = 0>
-__device__ __forceinline__ void tree_wg_body(const UpdateArgs& a, CounterTicket& ticket, float*& staged_s, float*& staged_m,
-                                             StepShared* step = nullptr, uint32_t watch_leaf = 0) {
+template <bool kTake, int kStep = 0>
+__device__ __forceinline__ void tree_wg_body(const UpdateArgs& a, const uint32_t nthreads, CounterTicket& ticket, float*& staged_s,
+                                             float*& staged_m, StepShared* step = nullptr, uint32_t watch_leaf = 0) {
     __shared__ __align__(16) float top_s[kWgTopNodes];
     __shared__ __align__(16) float top_m[kWgTopNodes];
     staged_s = top_s;
     staged_m = top_m;
     __shared__ __align__(16) uint32_t keys[3][kWgSlots];
     __shared__ __align__(16) unsigned long long vals[3][kWgSlots];
-    // (kThreads: the caller's fixed number of threads - the launch's own is a read of the kernel-argument segment)
-    const uint32_t tid = threadIdx.x, nthreads = kThreads ? (uint32_t)kThreads : blockDim.x, lane = tid & 63u;
+    // (nthreads: the workgroup's, from the caller - asking the launch for it is a read of the kernel-argument segment)
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const int D = a.depth;                                // 2 .. kWgMaxDepth
     const int T = D < kWgTopLevels ? D : kWgTopLevels;    // the staged top ends at level T
     const int H = D - T;                                  // levels below it
@@ -2182,12 +2183,12 @@ struct WgLead {
     const int64_t* indices;
     const float* priorities;
     float *sum, *mn, *maxp;
-    int n, depth, capacity;
+    int n, depth_threads, capacity;  // depth | threads of the workgroup << 8
     float alpha;
 };
 #define MRB_WG_LEAD_PARAMS                                                                                      \
     const int64_t *__restrict__ lead_indices, const float *__restrict__ lead_priorities, float *lead_sum, float *lead_mn, \
-        float *lead_maxp, int lead_n, int lead_depth, int lead_capacity, float lead_alpha
+        float *lead_maxp, int lead_n, int lead_plan, int lead_capacity, float lead_alpha
 __device__ __forceinline__ UpdateArgs with_lead(const UpdateArgs& from, const WgLead& lead) {
     UpdateArgs a = from;
     a.indices = lead.indices;
@@ -2196,19 +2197,20 @@ __device__ __forceinline__ UpdateArgs with_lead(const UpdateArgs& from, const Wg
     a.mn = lead.mn;
     a.maxp = lead.maxp;
     a.n = lead.n;
-    a.depth = lead.depth;
-    a.leaves = (int64_t)1 << lead.depth;
+    a.depth = lead.depth_threads & 255;
+    a.leaves = (int64_t)1 << a.depth;
     a.capacity = lead.capacity;
     a.alpha = lead.alpha;
     return a;
 }
-#define MRB_WG_LEAD WgLead{lead_indices, lead_priorities, lead_sum, lead_mn, lead_maxp, lead_n, lead_depth, lead_capacity, lead_alpha}
+#define MRB_WG_LEAD WgLead{lead_indices, lead_priorities, lead_sum, lead_mn, lead_maxp, lead_n, lead_plan, lead_capacity, lead_alpha}
 
-__global__ __launch_bounds__(kWgMaxEntries) void k_tree_wg(MRB_WG_LEAD_PARAMS, UpdateArgs a_in) {
-    const UpdateArgs a = with_lead(a_in, MRB_WG_LEAD);
+__global__ __launch_bounds__(kWgMaxEntries) void k_tree_wg(MRB_WG_LEAD_PARAMS) {
+    UpdateArgs a = with_lead(UpdateArgs{}, MRB_WG_LEAD);
+    a.err = err_before(lead_maxp);
     CounterTicket none{};
     float *top_s, *top_m;
-    tree_wg_body<false>(a, none, top_s, top_m);
+    tree_wg_body<false>(a, (uint32_t)lead_plan >> 8, none, top_s, top_m);
 }
 
 // ---------------------------------------------------------------------------
@@ -2234,10 +2236,11 @@ __global__ __launch_bounds__(kWgMaxEntries) void k_tree_wg_push(MRB_WG_LEAD_PARA
     // The device's counters are the last wave's business: it requests them among the update's first requests, hands
     // the position to the walking wave through LDS and moves the counters on while that wave walks.
     __shared__ int64_t s_position;
-    const bool keeper = kDev && threadIdx.x >= blockDim.x - 64;
+    const uint32_t nthreads = (uint32_t)lead_plan >> 8;
+    const bool keeper = kDev && threadIdx.x >= nthreads - 64;
     CounterTicket t{};
     float *top_s, *top_m;
-    tree_wg_body<kDev>(a, t, top_s, top_m);
+    tree_wg_body<kDev>(a, nthreads, t, top_s, top_m);
     if (keeper && (threadIdx.x & 63u) == 0) s_position = ticket_position(t, a.capacity);
     __threadfence_block();
     __syncthreads();
@@ -2562,7 +2565,7 @@ __global__ __launch_bounds__(kThreads) void k_tree_wg_push_sample(const int64_t*
     }
     CounterTicket none{};
     float *top_s, *top_m;
-    tree_wg_body<false, kDev ? 2 : 1, kThreads>(a, none, top_s, top_m, &s_step, leaf_node);  // (ends behind a barrier)
+    tree_wg_body<false, kDev ? 2 : 1>(a, (uint32_t)kThreads, none, top_s, top_m, &s_step, leaf_node);  // (ends behind a barrier)
     if (kDev) {
         if (walker) {  // the counters moved on (this launch has no other reader of them)
             int64_t* const cnt = counters_before(maxp);

@@ -28,9 +28,6 @@ struct Meet {
 };
 
 __device__ __forceinline__ Meet* meet_of(float* maxp) { return reinterpret_cast<Meet*>(reinterpret_cast<char*>(maxp) + kMeetBehindMaxp); }
-__device__ __forceinline__ uint32_t* err_before(float* maxp) {
-    return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(maxp) - kMaxpBehindErr);
-}
 
 // The number of launches before this one (requested when a kernel starts: the last workgroup moves it on).
 __device__ __forceinline__ uint32_t meet_turn(float* maxp) {

@@ -10,7 +10,7 @@ namespace mrb {
 int tree_range_levels(int depth);
 // indices and priorities of n entries -> leaves and the tree_range_levels(depth) levels above them.
 hipError_t launch_tree_range(const int64_t* indices, const float* priorities, int64_t n, float* sum, float* mn, float* maxp,
-                             uint32_t* err, int64_t capacity, int depth, float alpha, hipStream_t s);
+                             int64_t capacity, int depth, float alpha, hipStream_t s);
 // An update driven by its entries on a very large tree, after k_update_stamp: the lowest g0 levels (4 to 6), and `dirty`
 // gets the epoch for each run of 2^g_dirty of the nodes at depth - g0 that has a changed one.
 hipError_t launch_tree_sparse(const int64_t* indices, const unsigned long long* stamp, const float* powered, float* sum, float* mn,

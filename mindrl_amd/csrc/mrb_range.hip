@@ -1,6 +1,7 @@
 #include "mrb_range.h"
 
 #include "../../include/mrb.h"
+#include "mrb_rows.h"
 #include "mrb_tree.h"
 
 namespace mrb {
@@ -24,13 +25,15 @@ struct Trees {
 // A call is bound by its chain of trips - indices, priorities of a run's own, tiles, then the second launch's tile -, not
 // by bytes. 2048 entries on 2^21 leaves 14.7 -> 9.1 us, 1024 on 2^17 9.4 -> 6.7, 250 on 2^19 7.5 -> 6.8.
 // ---------------------------------------------------------------------------
+// (no argument for what the kernel can tell: see PutArgs::threads)
+__host__ __device__ constexpr int range_threads(int64_t n) { return n > 4096 ? 1024 : 512; }  // (256: 0.3 to 1.5 us more)
 constexpr int kRangePer = 8;  // entries of a thread and trip, all requested at once, the next trip's before these are looked at
 
 // kLog2: the table's leaves; w <= kLog2.
 template <int kLog2>
 __global__ __launch_bounds__(1024) void k_tree_range(const int64_t* __restrict__ indices, const float* __restrict__ priorities,
                                                          float* sum, float* mn, float* maxp, int n, int capacity, int depth_w,
-                                                         float alpha, uint32_t* err) {
+                                                         float alpha) {
     __shared__ unsigned long long s_win[1 << kLog2];         // per leaf: the latest entry's election_key (with its power)
     __shared__ uint32_t s_dirty[1 << (kLog2 - 8)];           // per tile
     __shared__ float s_rs[1 << (kLog2 - 8)], s_rm[1 << (kLog2 - 8)];  // the tiles' roots
@@ -39,7 +42,8 @@ __global__ __launch_bounds__(1024) void k_tree_range(const int64_t* __restrict__
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t run = blockIdx.x, leaves = 1u << w, tiles = leaves / kBlockNodes;
     const Trees trees{sum, mn};
-    const int threads = (int)blockDim.x, trip = kRangePer * threads;
+    const int threads = range_threads(n), trip = kRangePer * threads;
+    uint32_t* const err = err_before(maxp);
     auto request = [&](int base, int64_t (&to)[kRangePer]) {
 #pragma unroll
         for (int q = 0; q < kRangePer; ++q) {
@@ -108,7 +112,7 @@ __global__ __launch_bounds__(1024) void k_tree_range(const int64_t* __restrict__
     if (dirty == 0) return;  // (the same in every wave)
     uint32_t nth = 0;
     for (unsigned long long rest = dirty; rest; rest &= rest - 1, ++nth) {
-        if (nth % (blockDim.x / 64) != wave) continue;
+        if (nth % ((uint32_t)threads / 64) != wave) continue;
         const uint32_t t = (uint32_t)__builtin_ctzll(rest);
         const uint32_t first = (1u << depth) + run * leaves + t * kBlockNodes;
         float4 vs = *reinterpret_cast<const float4*>(sum + first + 4 * lane);
@@ -303,11 +307,11 @@ int tree_range_levels(int depth) {
 }
 
 hipError_t launch_tree_range(const int64_t* indices, const float* priorities, int64_t n, float* sum, float* mn, float* maxp,
-                             uint32_t* err, int64_t capacity, int depth, float alpha, hipStream_t s) {
+                             int64_t capacity, int depth, float alpha, hipStream_t s) {
     const int w = tree_range_levels(depth);
-    const dim3 grid((uint32_t)((capacity + ((int64_t)1 << w) - 1) >> w)), threads(n > 4096 ? 1024 : 512);  // (256: 0.3 to 1.5 us more)
+    const dim3 grid((uint32_t)((capacity + ((int64_t)1 << w) - 1) >> w)), threads(range_threads(n));
     auto* const kernel = w <= 10 ? k_tree_range<10> : w <= 12 ? k_tree_range<12> : w == 13 ? k_tree_range<13> : k_tree_range<14>;
-    hipLaunchKernelGGL(kernel, grid, threads, 0, s, indices, priorities, sum, mn, maxp, (int)n, (int)capacity, depth | w << 8, alpha, err);
+    hipLaunchKernelGGL(kernel, grid, threads, 0, s, indices, priorities, sum, mn, maxp, (int)n, (int)capacity, depth | w << 8, alpha);
     return hipGetLastError();
 }
 

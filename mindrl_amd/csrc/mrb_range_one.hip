@@ -274,6 +274,7 @@ hipError_t launch_range_one_push(const int64_t* indices, const float* priorities
     const uint32_t runs = runs_of(capacity, w);
     PutArgs ride = put;  // (its workgroups were counted for kWG threads)
     ride.blocks = (put.blocks * kWG + kOneWG - 1) / kOneWG;
+    ride.threads = kOneWG;
     auto* const kernel = w <= 10 ? k_range_one_push<10> : w <= 12 ? k_range_one_push<12> : w == 13 ? k_range_one_push<13> : k_range_one_push<14>;
     hipLaunchKernelGGL(kernel, dim3(runs + ride.blocks), dim3(kOneWG), 0, s, indices, priorities, sum, mn, maxp, (int)n, (int)capacity,
                        depth | w << 8, alpha, runs, push, ride);

@@ -64,7 +64,7 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
     const int64_t cols = batch * inner;
     // Workgroups are dealt to the chip's eight dies in turn, and each die has its own L2. Neighbouring column groups
     // share cache lines (a group's flags of a step are kCols bytes), so they go to the SAME die.
-    const uint32_t per = gridDim.x >> 3, more = gridDim.x & 7u, die = blockIdx.x & 7u;
+    const uint32_t groups = (uint32_t)((cols + kCols - 1) / kCols), per = groups >> 3, more = groups & 7u, die = blockIdx.x & 7u;
     const uint32_t group = die * per + (die < more ? die : more) + (blockIdx.x >> 3);
     // every group is full when there are kCols columns at all: the last one is moved back
     const int64_t c_last = cols > kCols ? cols - kCols : 0;

@@ -134,6 +134,8 @@ struct PutArgs {
     IoTable t;
     int64_t capacity, first_slot, src_capacity, src_first;
     uint32_t blocks;  // workgroups doing this copy when it rides along in another kernel's launch (0: none)
+    uint32_t threads; // of each. (From the host: a kernel that asks for its launch's size gets 256 bytes more of arguments,
+                      // and a launch of more than 1 KB of them costs the host half a microsecond more than one of less.)
     // first_slot < 0: the buffer's counters live on the device (see Counters below), the rows go to
     // (pushes mod capacity) onwards, and src_first - unused then, the source is never a ring - holds the
     // counters' address
@@ -158,6 +160,9 @@ __device__ __forceinline__ const int64_t* counters_behind(const uint32_t* err) {
 constexpr int kMaxpBehindErr = 64;
 __device__ __forceinline__ int64_t* counters_before(float* maxp) {
     return reinterpret_cast<int64_t*>(reinterpret_cast<char*>(maxp) - kMaxpBehindErr + 16);
+}
+__device__ __forceinline__ uint32_t* err_before(float* maxp) {
+    return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(maxp) - kMaxpBehindErr);
 }
 __device__ __forceinline__ int64_t ring_position(const int64_t* counters, int64_t capacity) {
     return counters[kCntPos];
@@ -259,11 +264,11 @@ __device__ __forceinline__ void rider_ends() {
 __device__ __forceinline__ void rows_put_part(const PutArgs& p, uint32_t block, uint32_t nblocks, int64_t known_first = -1) {
     const IoTable& t = p.t;
     const uint64_t total = t.prefix[t.nfields];
-    const uint64_t stride = (uint64_t)nblocks * blockDim.x;
+    const uint64_t stride = (uint64_t)nblocks * p.threads;
     const int64_t first_slot = known_first >= 0  ? known_first
                                : p.first_slot >= 0 ? p.first_slot
                                                    : ring_position(reinterpret_cast<const int64_t*>(p.src_first), p.capacity);
-    for (uint64_t w = (uint64_t)block * blockDim.x + threadIdx.x; w < total; w += stride) {
+    for (uint64_t w = (uint64_t)block * p.threads + threadIdx.x; w < total; w += stride) {
         const int f = field_of(t, w);
         uint64_t row;
         uint32_t unit;
