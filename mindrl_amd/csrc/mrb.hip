@@ -21,6 +21,7 @@
 #include "mrb_range_one.h"
 #include "mrb_returns.h"
 #include "mrb_samples.h"
+#include "mrb_short.h"
 #include "../../include/mrb_more.h"
 
 namespace {
@@ -86,8 +87,10 @@ struct RowStore {
     int64_t row_wave = 0;   // option "row_wave": the wave-per-row sample kernel, 0 = for launches of many rows, 1 = whenever
                             // the rows fit it, 2 = never
     Stage stage;
+    RowTable* table = nullptr;  // on the device: what launches with short arguments find there
 
     ~RowStore() {
+        if (table) (void)hipFree(table);
         if (packed_base) {
             (void)hipFree(packed_base);
             return;
@@ -100,6 +103,47 @@ struct RowStore {
 // Library-wide default of the option "packed_rows" (mrb_set_option with handle 0): buffers created afterwards
 // keep their rows packed when a packed row takes at most this many bytes; 0 = every field an array of its own.
 std::atomic<int64_t> g_packed_rows{0};
+
+// What a buffer's launches with short arguments find on the device (but for the flags, which its create function adds).
+RowTable row_table(const RowStore& r) {
+    RowTable t{};
+    t.t.nfields = r.nfields;
+    for (int i = 0; i < r.nfields; ++i) {
+        t.t.store[i] = r.data[i];
+        t.t.row_bytes[i] = (uint32_t)r.bytes[i];
+        t.t.stride[i] = (uint32_t)r.stride[i];
+        t.t.units[i] = r.units[i];
+        t.t.vec_log2[i] = r.vec_log2[i];
+        t.t.prefix[i + 1] = t.t.prefix[i] + r.units[i];
+    }
+    t.capacity = r.capacity;
+    return t;
+}
+
+// A call's matrices as kernels with short arguments take them; false where these cannot say where they are.
+bool short_io(const void* const* at, int n, ShortIo& io) {
+    if (n > kShortPointers) return false;
+    io.base = reinterpret_cast<uint64_t>(at[0]);
+    uint64_t any = 1ull << 12;
+    for (int i = 1; i < n; ++i) any |= reinterpret_cast<uint64_t>(at[i]) - io.base;
+    io.shift = (uint32_t)__builtin_ctzll(any);
+    for (int i = 1; i < n; ++i) {
+        const int64_t away = static_cast<int64_t>(reinterpret_cast<uint64_t>(at[i]) - io.base) >> io.shift;
+        if (away != (int32_t)away) return false;
+        io.away[i - 1] = (int32_t)away;
+    }
+    return true;
+}
+bool short_io(const IoTable& t, ShortIo& io) { return short_io(reinterpret_cast<const void* const*>(t.io), t.nfields, io); }
+// The same with one or two matrices in front.
+bool short_io(const void* first, const void* second, const IoTable& t, ShortIo& io) {
+    const void* at[MRB_MAX_FIELDS + 2];
+    int n = 0;
+    at[n++] = first;
+    if (second) at[n++] = second;
+    for (int i = 0; i < t.nfields; ++i) at[n++] = t.io[i];
+    return short_io(at, n, io);
+}
 
 int rows_alloc(RowStore& r, int64_t capacity, int nfields, const int64_t* field_bytes) {
     if (capacity <= 0 || capacity > (1ll << 30)) return fail(MRB_EINVAL, "capacity %lld outside [1, 2^30]", (long long)capacity);
@@ -135,15 +179,18 @@ int rows_alloc(RowStore& r, int64_t capacity, int nfields, const int64_t* field_
             r.stride[i] = packed_row;
         }
         r.nfields = nfields;
-        return MRB_OK;
+    } else {
+        for (int i = 0; i < nfields; ++i) {
+            const size_t total = (size_t)capacity * (size_t)field_bytes[i];
+            HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r.data[i]), total));
+            r.nfields = i + 1;  // so the destructor frees what exists
+            r.stride[i] = field_bytes[i];
+            HIP_TRY(hipMemset(r.data[i], 0, total));
+        }
     }
-    for (int i = 0; i < nfields; ++i) {
-        const size_t total = (size_t)capacity * (size_t)field_bytes[i];
-        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r.data[i]), total));
-        r.nfields = i + 1;  // so the destructor frees what exists
-        r.stride[i] = field_bytes[i];
-        HIP_TRY(hipMemset(r.data[i], 0, total));
-    }
+    const RowTable table = row_table(r);
+    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r.table), sizeof(table)));
+    HIP_TRY(hipMemcpy(r.table, &table, sizeof(table), hipMemcpyHostToDevice));
     return MRB_OK;
 }
 
@@ -196,10 +243,21 @@ int put_args(const RowStore& r, const void* const* src, int64_t skip, int64_t n,
     return MRB_OK;
 }
 
+// Granules of the field that has the most.
+uint64_t most_granules(const IoTable& t) {
+    uint64_t most = 0;
+    for (int f = 0; f < t.nfields; ++f) most = std::max<uint64_t>(most, t.prefix[f + 1] - t.prefix[f]);
+    return most;
+}
+
 int rows_put(const RowStore& r, const void* const* src, int64_t skip, int64_t n, int64_t first_slot, hipStream_t s) {
     PutArgs p{};
     int rc = put_args(r, src, skip, n, first_slot, p);
     if (rc) return rc;
+    if (ShortIo io{}; short_io(p.t, io)) {
+        const hipError_t e = launch_short_put(r.table, io, r.nfields, first_slot, n, most_granules(p.t), s);
+        return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch k_short_put: %s", hipGetErrorString(e));
+    }
     hipLaunchKernelGGL(k_rows_put, dim3(p.blocks), dim3(kWG), 0, s, p);
     LAUNCH_CHECK("k_rows_put");
     return MRB_OK;
@@ -423,9 +481,11 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
         return MRB_OK;
     }
     // a row of workgroups per field, as many as the field with the most granules needs
-    uint64_t most = 0;
-    for (int f = 0; f < t.nfields; ++f) most = std::max<uint64_t>(most, t.prefix[f + 1] - t.prefix[f]);
-    const uint32_t blocks = grid_for(most);
+    const uint32_t blocks = grid_for(most_granules(t));
+    if (ShortIo io{}; fixed_slot < 0 && n <= 0xffffffffll && (out_indices ? short_io(out_indices, nullptr, t, io) : short_io(t, io))) {
+        const hipError_t e = launch_short_gather(r.table, io, t.nfields, indices, count, seed, calls, n, blocks, out_indices != nullptr, s);
+        return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch k_short_gather: %s", hipGetErrorString(e));
+    }
     hipLaunchKernelGGL(k_rows_gather, dim3(blocks, (uint32_t)t.nfields), dim3(kWG), 0, s, t, r.capacity, count, indices, fixed_slot,
                        seed, calls, out_indices, err, blocks);
     LAUNCH_CHECK("k_rows_gather");
@@ -656,6 +716,10 @@ int tree_rebuild(Per& b, UpdateArgs a, hipStream_t s, const PutArgs* ride = null
         const uint32_t threads = units <= kWG / 64 ? (uint32_t)kWG : (uint32_t)kFusedWG;
         put.blocks = (put.blocks * kWG + threads - 1) / threads;  // the ride-along copy was sized for workgroups of kWG
         put.threads = threads;
+        if (ShortIo io{}; put.blocks && a.first_slot >= 0 && a.advance == 0 && a.fold_max != 1 && short_io(put.t, io)) {
+            const hipError_t e = launch_short_push_run(b.rows.table, io, put.t.nfields, a, units, most_granules(put.t), threads, s);
+            return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch k_short_push_run: %s", hipGetErrorString(e));
+        }
         a.readers = 1 + put.blocks;  // (a.advance != 0: this one launch also moves the device's counters on)
         hipLaunchKernelGGL(k_push_run, dim3(1 + put.blocks), dim3(threads), 0, s, a, units, put);
         LAUNCH_CHECK("k_push_run");
@@ -1029,6 +1093,7 @@ int mrb_urb_create(int64_t capacity, int nfields, const int64_t* field_bytes, in
     if (rc) return rc;
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->err), 16 + kCntWords * sizeof(int64_t)));
     HIP_TRY(hipMemset(b->err, 0, 16 + kCntWords * sizeof(int64_t)));
+    HIP_TRY(hipMemcpy(&b->rows.table->err, &b->err, sizeof(b->err), hipMemcpyHostToDevice));
     b->counters = reinterpret_cast<int64_t*>(b->err + 4);
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->slots), kUrbDrawMax * sizeof(int64_t)));
     HIP_TRY(hipDeviceSynchronize());  // the zero-fills ran on the null stream; the caller's stream may not wait for it
@@ -1273,6 +1338,7 @@ int mrb_per_create(int64_t capacity, float alpha, int nfields, const int64_t* fi
     b->maxp = reinterpret_cast<float*>(reinterpret_cast<char*>(b->err) + kMaxpBehindErr);
     HIP_TRY(hipMemset(b->counters, 0, kCntWords * sizeof(int64_t)));
     HIP_TRY(hipMemset(reinterpret_cast<char*>(b->maxp) + kMeetBehindMaxp, 0, sizeof(Meet)));
+    HIP_TRY(hipMemcpy(&b->rows.table->err, &b->err, sizeof(b->err), hipMemcpyHostToDevice));
     // update_priorities scratch, sized once: a call rarely names more entries than there are rows
     b->powered_cap = capacity < 4096 ? 4096 : (capacity > (1ll << 20) ? (1ll << 20) : capacity);
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->powered), (size_t)b->powered_cap * sizeof(float)));
@@ -1383,10 +1449,16 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
         // one row: one wave walks from its leaf to the root (k_push_one)
         rc = ride_alone_if_large(a, put, s);
         if (rc) return rc;
-        hipLaunchKernelGGL(b->device_counters ? k_push_one<true> : k_push_one<false>, dim3(1 + put.blocks), dim3(kWG), 0, s,
-                           a.sum, a.mn, a.maxp, a.first_slot, a.capacity, a.leaves, a.depth, a.alpha, opt_priorities, a.err, put,
-                           a.advance, 1 + put.blocks * (kWG / 64));
-        LAUNCH_CHECK("k_push_one");
+        if (ShortIo io{}; put.blocks && !b->device_counters && short_io(put.t, io)) {
+            const hipError_t e = launch_short_push_one(b->rows.table, io, put.t.nfields, a.sum, a.mn, a.maxp, a.first_slot, a.depth,
+                                                       a.alpha, opt_priorities, most_granules(put.t), s);
+            if (e != hipSuccess) return fail(MRB_EHIP, "launch k_short_push_one: %s", hipGetErrorString(e));
+        } else {
+            hipLaunchKernelGGL(b->device_counters ? k_push_one<true> : k_push_one<false>, dim3(1 + put.blocks), dim3(kWG), 0, s,
+                               a.sum, a.mn, a.maxp, a.first_slot, a.capacity, a.leaves, a.depth, a.alpha, opt_priorities, a.err, put,
+                               a.advance, 1 + put.blocks * (kWG / 64));
+            LAUNCH_CHECK("k_push_one");
+        }
         b->pushes += nrows;
         b->size = b->size + nrows < cap ? b->size + nrows : cap;
         return MRB_OK;
@@ -1796,6 +1868,7 @@ int mrb_res_create(int64_t capacity, int nfields, const int64_t* field_bytes, ui
     HIP_TRY(hipMemset(b->stamp, 0, (size_t)capacity * sizeof(unsigned long long)));
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->err), 16));
     HIP_TRY(hipMemset(b->err, 0, 16));
+    HIP_TRY(hipMemcpy(&b->rows.table->err, &b->err, sizeof(b->err), hipMemcpyHostToDevice));
     HIP_TRY(hipDeviceSynchronize());  // as in mrb_urb_create
     std::lock_guard<std::mutex> lk(g_mu);
     *out_handle = g_next++;

@@ -103,6 +103,18 @@ struct AnyGranule {
     }
 };
 
+// A call's fields as the gather looks at them: of a by-value table, or (ShortRows, mrb_short.h) of one in device memory.
+struct FullRows {
+    const IoTable& t;
+    __device__ __forceinline__ uint32_t units(int f) const { return t.units[f]; }
+    __device__ __forceinline__ uint32_t vl(int f) const { return t.vec_log2[f]; }
+    __device__ __forceinline__ uint32_t row_bytes(int f) const { return t.row_bytes[f]; }
+    __device__ __forceinline__ uint32_t stride(int f) const { return t.stride[f]; }
+    __device__ __forceinline__ uint8_t* store(int f) const { return t.store[f]; }
+    __device__ __forceinline__ uint8_t* io(int f) const { return t.io[f]; }
+    __device__ __forceinline__ uint64_t granules(int f) const { return t.prefix[f + 1] - t.prefix[f]; }
+};
+
 __device__ __forceinline__ int field_of(const IoTable& t, uint64_t w) {
     int f = 0;
     while (f + 1 < t.nfields && w >= t.prefix[f + 1]) ++f;

@@ -1,0 +1,71 @@
+// Kernels whose arguments are short (defined in mrb_short.hip): the same bodies as the kernels of mrb_kernels.h with the
+// buffer's constant tables read from device memory and the caller's matrices given as distances from the first.
+//
+// A launch's arguments are written across the bus and the last of them is read back before the launch: up to 112 bytes cost a
+// process whose memory is far from the device 2.7 us of host time, 120 to 960 bytes 3.1 to 3.9, more than a kilobyte 4.1 to 4.5.
+// By-value field tables are 550 to 1000 bytes, and nearly all of them is the same in every call. On the device a kernel's first
+// trip reads what it needs of the table into scalar registers, and the copies have a row of workgroups per field instead of a
+// search for each granule's field. Device time per call, us, by value / short: an append of 1 row 2.85 / 2.04, of 1000 rows of
+// 133 bytes 3.08 / 2.39, of 57.5 MB (read and written) 15.5 / 12.2; a gather of 256 rows of 162 bytes 3.17 / 2.66, of 8192 rows
+// of 133 bytes 4.87 / 4.25; a push of 1 row 2.86 / 2.28, of 64 3.09 / 2.84, of 1000 3.56 / 3.13, of 4096 with priorities
+// 8.7 / 8.8. Host time of one uniform insert and sample 10.0 / 9.2.
+//
+// By value stay: more than kShortPointers matrices, matrices too far apart at an odd address, device-resident counters, single-row
+// reads, copies from another buffer's ring; the sampling kernels and the reservoir's push (3.35 / 3.40 and 2.8 / 2.9 when they
+// were tried: their row copies come last, so the table's trip is not hidden); and the gather of wide rows, which takes a plan
+// that a wave divides its lanes by (within 4 % of each other either way, 24,831-byte rows slower short).
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "mrb_push.h"
+#include "mrb_rows.h"
+
+namespace mrb {
+
+constexpr int kShortPointers = 8;
+
+// The matrices of a call: up to kShortPointers addresses, as distances from the first in units of 1 << shift bytes (what
+// torch's allocator gives lies 512 bytes from each other or a multiple of that, and anywhere in the device's address space).
+struct ShortIo {
+    uint64_t base;
+    uint32_t shift;
+    int32_t away[kShortPointers - 1];
+    __device__ __forceinline__ uint8_t* at(int i) const {
+        return reinterpret_cast<uint8_t*>(base + (i ? (uint64_t)((int64_t)away[i - 1] << shift) : 0));
+    }
+};
+
+// What stays the same of a buffer's arguments from call to call, in device memory.
+struct RowTable {
+    IoTable t;  // (store, row_bytes, stride, units and vec_log2 of it)
+    int64_t capacity;
+    uint32_t* err;  // the buffer's flags
+};
+
+// The fields of n rows (see FullRows); `first`: the number of the first field's matrix in io.
+struct ShortRows {
+    const RowTable* r;
+    const ShortIo& s;
+    uint64_t n;
+    int first;
+    __device__ __forceinline__ uint32_t units(int f) const { return r->t.units[f]; }
+    __device__ __forceinline__ uint32_t vl(int f) const { return r->t.vec_log2[f]; }
+    __device__ __forceinline__ uint32_t row_bytes(int f) const { return r->t.row_bytes[f]; }
+    __device__ __forceinline__ uint32_t stride(int f) const { return r->t.stride[f]; }
+    __device__ __forceinline__ uint8_t* store(int f) const { return r->t.store[f]; }
+    __device__ __forceinline__ uint8_t* io(int f) const { return s.at(first + f); }
+    __device__ __forceinline__ uint64_t granules(int f) const { return n * r->t.units[f]; }
+};
+
+hipError_t launch_short_gather(const RowTable* table, const ShortIo& io, int nfields, const int64_t* indices, int64_t count, uint64_t seed,
+                               uint64_t calls, int64_t n, uint32_t blocks, bool with_indices, hipStream_t s);
+// (granules: the field's with the most)
+hipError_t launch_short_put(const RowTable* table, const ShortIo& io, int nfields, int64_t first_slot, int64_t n, uint64_t granules,
+                            hipStream_t s);
+hipError_t launch_short_push_one(const RowTable* table, const ShortIo& io, int nfields, float* sum, float* mn, float* maxp, int64_t first_slot,
+                                 int depth, float alpha, const float* priority, uint64_t granules, hipStream_t s);
+hipError_t launch_short_push_run(const RowTable* table, const ShortIo& io, int nfields, const UpdateArgs& a, uint32_t units, uint64_t granules,
+                                 uint32_t threads, hipStream_t s);
+
+}  // namespace mrb

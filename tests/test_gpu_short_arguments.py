@@ -1,0 +1,134 @@
+"""Calls whose launches take their tables from device memory and the caller's matrices as distances, against the same calls over
+matrices that cannot be given so (more than 2^31 bytes apart at an odd address): rows, trees, running max, outputs and flags,
+bit for bit. Rows from 1 byte to several granules, aligned and not, packed, from host memory and from views that begin anywhere;
+pushes of one row to many, around the ring's end, with valid and invalid priorities; gathers by generator and by index."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import bits, random_rows, t2n
+
+pytestmark = pytest.mark.gpu
+
+SETS = {  # (the field of single bytes is the one that is placed far away)
+    "small": ([(3,), (1,), (2,)], [np.float32, np.uint8, np.int64]),
+    "odd": ([(61,), (37,), (5, 3), (1,)], [np.int32, np.uint8, np.float32, np.bool_]),
+    "wide": ([(1024,), (4097,), (1,)], [np.float32, np.uint8, np.int32]),
+    "two": ([(4,), (17,)], [np.float32, np.uint8]),
+    "nine": ([(2,)] * 8 + [(7,)], [np.float32] * 8 + [np.uint8]),
+}
+
+
+@pytest.fixture(scope="module")
+def big():
+    return torch.empty((1 << 31) + (1 << 25), dtype=torch.uint8, device="cuda")
+
+
+def dev(rows, shift):
+    """On the device, the fields of single bytes as views that begin `shift` bytes into an allocation."""
+    out = []
+    for r in rows:
+        if r.dtype == np.uint8:
+            whole = torch.zeros(r.size + shift, dtype=torch.uint8, device="cuda")
+            whole[shift:].copy_(torch.from_numpy(r.reshape(-1)))
+            out.append(whole[shift:].view(r.shape))
+        else:
+            out.append(torch.from_numpy(r).cuda())
+    return out
+
+
+def far(big, rows):
+    """The same with the first field at the start of `big` and the one of single bytes beyond 2^31 bytes, at an odd address."""
+    out = []
+    for k, r in enumerate(rows):
+        if k == 0:
+            t = big[: r.nbytes].view(torch.from_numpy(r).dtype).view(r.shape)
+        elif r.dtype == np.uint8:
+            t = big[(1 << 31) + 4099 : (1 << 31) + 4099 + r.nbytes].view(r.shape)
+        else:
+            t = torch.empty(r.shape, dtype=torch.from_numpy(r).dtype, device="cuda")
+        t.copy_(torch.from_numpy(r))
+        out.append(t)
+    return out
+
+
+def same_rows(a, b, what):
+    for k, (x, y) in enumerate(zip(a, b)):
+        assert np.ascontiguousarray(t2n(x)).tobytes() == np.ascontiguousarray(t2n(y)).tobytes(), (what, k)
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("name", sorted(SETS))
+def test_uniform(name, packed, big):
+    from mindrl_amd.core import UniformReplayBuffer
+    shapes, types = SETS[name]
+    tt = [torch.from_numpy(np.zeros(1, t)).dtype for t in types]
+    cap, batch = 1009, 515
+    a, b = (UniformReplayBuffer(batch, cap, shapes, tt, seed=5, packed_rows=packed) for _ in range(2))
+    rng = np.random.default_rng(1)
+    for step, n in enumerate((515, 1, 2, 255, 256, 257, 1009, 3, 700, 64)):
+        rows = random_rows(rng, n, shapes, types)
+        a.insert(dev(rows, step % 4 * 3) if step % 3 else [torch.from_numpy(r) for r in rows])
+        b.insert(far(big, rows))
+        same_rows(a.buffer, b.buffer, (name, n))
+        same_rows(a.sample(), b.sample(out=far(big, random_rows(rng, batch, shapes, types))), (name, n, "generator"))
+        idx = torch.from_numpy(rng.integers(0, a.size(), 77)).cuda()
+        same_rows(a.sample(indices=idx), b.sample(indices=idx, out=far(big, random_rows(rng, 77, shapes, types))), (name, n, "indices"))
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("cap", [200, 1009, 70_001])
+@pytest.mark.parametrize("name", ["small", "odd", "nine"])
+def test_pushes(name, cap, packed, big):
+    from mindrl_amd.core import PriorityReplayBuffer
+    shapes, types = SETS[name]
+    tt = [torch.from_numpy(np.zeros(1, t)).dtype for t in types]
+    a, b = (PriorityReplayBuffer(0.7, cap, 8, shapes, tt, seed0=5, packed_rows=packed) for _ in range(2))
+    rng = np.random.default_rng(2)
+    for step, n in enumerate((cap // 2 + 1, 1, 3, 63, 256, cap, 1, 200, 257, 1, 1024, 4000, 4096, cap - 1, 5)):
+        n = min(n, cap)
+        rows = random_rows(rng, n, shapes, types)
+        for how in range(3):
+            pr = None
+            if how:
+                pr = (rng.pareto(1.5, n) + 1e-6).astype(np.float32)
+                if how == 2:
+                    pr[rng.integers(0, n, 1 + n // 50)] = [-1.0, np.inf, np.nan][step % 3]
+                pr = torch.from_numpy(pr).cuda()
+            a.insert(*(dev(rows, step % 5) if step % 4 else [torch.from_numpy(r) for r in rows]), priorities=pr)
+            b.insert(*far(big, rows), priorities=pr)
+            what = (name, cap, packed, n, how)
+            for x, y in zip(a.export_tree(), b.export_tree()):
+                assert np.array_equal(bits(x[1:]), bits(y[1:])), what
+            assert bits([a.max_priority]).tolist() == bits([b.max_priority]).tolist(), what
+            same_rows(a.storage(), b.storage(), what)
+            bad = []
+            for buf in (a, b):
+                try:
+                    buf.check()
+                    bad.append(None)
+                except Exception as e:
+                    bad.append(str(e))
+            assert bad[0] == bad[1], what
+
+
+def test_replays():
+    """A recorded gather and a recorded insert, on other contents than they were recorded with."""
+    from mindrl_amd.core import UniformReplayBuffer
+    u = UniformReplayBuffer(64, 128, [(3,)], [torch.float32], seed=1)
+    rows = torch.arange(384, dtype=torch.float32, device="cuda").view(128, 3)
+    u.insert([rows])
+    idx = torch.arange(64, device="cuda")
+    out = [torch.empty(64, 3, device="cuda")]
+    u.sample(indices=idx, out=out)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        u.sample(indices=idx, out=out)
+    for k in range(4):
+        idx.copy_((torch.arange(64, device="cuda") * 5 + k) % 128)
+        u.insert([rows[k : k + 2] * 0 - k])
+        g.replay()
+        torch.cuda.synchronize()
+        eager = u.sample(indices=idx)
+        assert torch.equal(out[0], eager[0] if isinstance(eager, (list, tuple)) else eager), k
