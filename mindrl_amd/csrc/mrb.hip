@@ -17,6 +17,7 @@
 
 #include "mrb_kernels.h"
 #include "mrb_meet.h"
+#include "mrb_push_many.h"
 #include "mrb_range.h"
 #include "mrb_range_one.h"
 #include "mrb_returns.h"
@@ -770,6 +771,16 @@ void fill_zero(void* p, size_t bytes, hipStream_t s) {
     hipLaunchKernelGGL(k_fill_f32, dim3(grid_for(n)), dim3(kWG), 0, s, static_cast<float*>(p), 0.0f, n);
 }
 
+// A push whose leaf tiles are rebuilt by several workgroups, or whose powers one shares out over its threads (k_push_many): with
+// priorities always; without, one tile (us, k_push_run / this: 3.6 / 3.3) or eight and more (1024 rows 4.2 / 4.7, 1500 4.5 / 4.8,
+// 2048 4.9 / 4.8, 3000 5.4 / 4.8: up to seven the roots' meeting costs more than sharing the tiles out saves).
+constexpr int64_t kManyLeastTiles = 8;
+bool takes_push_many(const Per& b, int64_t first, int64_t n, bool with_priorities) {
+    if (b.device_counters || !b.fused || b.nrounds == 0 || first + n > b.rows.capacity) return false;
+    const int64_t tiles = (first + n - 1) / kBlockNodes - first / kBlockNodes + 1;
+    return (with_priorities || tiles == 1 || tiles >= kManyLeastTiles) && tiles <= kManyMostTiles;
+}
+
 // Starts a new tree-update epoch. Epochs tag stamps and dirty words so that
 // neither needs clearing between calls; when the 32-bit tag would wrap, both
 // are cleared once.
@@ -1407,6 +1418,14 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
     if (b->device_counters) {  // the kernels take the first slot from the device
         put.first_slot = -1;
         put.src_first = reinterpret_cast<int64_t>(b->counters);
+    }
+    if (ShortIo io{}; !lead && skip == 0 && n > 1 && takes_push_many(*b, first, n, opt_priorities != nullptr) && short_io(put.t, io)) {
+        const hipError_t e = launch_push_many(b->rows.table, io, put.t.nfields, b->sum, b->mn, b->maxp, opt_priorities, first, n, b->depth,
+                                              b->alpha, most_granules(put.t), s);
+        if (e != hipSuccess) return fail(MRB_EHIP, "launch k_push_many: %s", hipGetErrorString(e));
+        b->pushes += nrows;
+        b->size = b->size + nrows < cap ? b->size + nrows : cap;
+        return MRB_OK;
     }
     // A large copy gets its own launch; a small one rides along in the first tree launch.
     if (put.blocks > 2048u) {

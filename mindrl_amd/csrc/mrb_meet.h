@@ -24,7 +24,8 @@ struct Meet {
     uint32_t arrived;  // of the launch in progress
     uint32_t turn;     // launches so far
     uint32_t pad[30];
-    unsigned long long root[kMeetMost][2];  // launch number << 32 | bits: sum, minimum
+    unsigned long long root[kMeetMost][2];   // launch number << 32 | bits: sum, minimum
+    unsigned long long largest[kMeetMost];  // and, of a push, the largest power
 };
 
 __device__ __forceinline__ Meet* meet_of(float* maxp) { return reinterpret_cast<Meet*>(reinterpret_cast<char*>(maxp) + kMeetBehindMaxp); }

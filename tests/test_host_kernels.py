@@ -7,7 +7,7 @@ import subprocess
 import pytest
 
 
-@pytest.mark.parametrize("source,count", [("mrb_range_one.hip", 8), ("mrb_short.hip", 4)])
+@pytest.mark.parametrize("source,count", [("mrb_range_one.hip", 8), ("mrb_short.hip", 4), ("mrb_push_many.hip", 3)])
 def test_kernels_use_no_scratch_memory(source, count, tmp_path):
     from mindrl_amd import build
     out = tmp_path / "kernels.s"
@@ -24,8 +24,8 @@ def test_kernels_use_no_scratch_memory(source, count, tmp_path):
     for name, (scratch, lds, vgprs) in kernels.items():
         assert scratch == 0 and vgprs <= 128, (name, scratch, vgprs)
         runs = re.search(r"k_range_one(?:_push)?ILi(\d+)E", name)
-        if not runs:  # three levels of a pair of roots and a mark per wave, at most
-            assert lds <= 1024, (name, lds)
+        if not runs:  # a tile's leaves, or three levels of a pair of roots and a mark per wave
+            assert lds <= 1088, (name, lds)
             continue
         # the election words, a root of each tree and a mark per tile, the runs' bits and a word per wave
         leaves = 1 << int(runs.group(1))
