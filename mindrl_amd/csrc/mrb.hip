@@ -825,7 +825,15 @@ UpdateArgs update_args(Per& b) {
 // the call's entries); larger calls take the stamp pass (2048 measured: config 4's update 14.0 us against 14.7 with the pass, at twice the waves and four times the comparisons: not taken).
 constexpr int64_t kElectMax = 1024;
 
-// Whether an update of more than 1024 entries goes by runs of leaves (launch_tree_range). Against what it would take
+// Whether one launch takes an update by runs of leaves: k_range_one. More than 1024 entries on 21 levels and more are faster on
+// the device by two (k_tree_range, k_tree_cap): 2048 8.7 against 9.1 us, 4096 10.2 against 10.7; on 20 levels 8.4 / 8.5 and
+// 9.3 / 9.4, and the host is spared a launch (2.7 us). Trees of fewer than 8 levels have no whole tile, those of more than 22 more
+// than 256 runs.
+bool takes_range_one(const Per& b, int64_t n) {
+    return b.fused && n <= (b.depth <= 20 ? kOneMostEntries : kElectMax) && b.depth >= 8 && b.depth <= 22;
+}
+
+// Whether an update goes by runs of leaves in two launches (launch_tree_range). Against what it would take
 // otherwise, us per call, before / by runs:
 //   most entries    10 levels, 2048 / 4096: 7.7 / 8.4 against 7.7 / 9.3; 12 levels, 8192 / 16,384: 10.0 / 11.4 against
 //                   9.6 / 13.8; 14 levels, 16,384 / 32,768: 11.7 / 12.5 against 11.2 / 16.7; 20 levels 14.4 / 15.4 against
@@ -835,14 +843,8 @@ constexpr int64_t kElectMax = 1024;
 bool takes_range(const Per& b, int64_t n) {
     if (!b.fused || b.depth < 10 || b.depth > 22) return false;
     const int64_t most = b.depth <= 11 ? 2048 : b.depth == 12 || b.depth == 22 ? 8192 : 16384;
-    return n > kOneMostEntries && n <= most;
+    return !takes_range_one(b, n) && n <= most;
 }
-
-// Whether one launch takes an update (and the push that follows it in the call) by runs of leaves: k_range_one. On the
-// device two launches (k_tree_range, k_tree_cap) catch up at 1024 entries on 20 levels and more - 7.7 against 8.1 us, 2048 on
-// 21 levels 9.1 against 10.4 -, where the host's time for the second one (2.7 us) still decides for calls this small. Trees of
-// fewer than 8 levels have no whole tile, those of more than 22 more than 256 runs.
-bool takes_range_one(const Per& b, int64_t n) { return b.fused && n <= kOneMostEntries && b.depth >= 8 && b.depth <= 22; }
 
 // Where one workgroup's update alone (k_tree_wg) is faster than that, us: 13 levels, 1 / 64 / 96 / 128 entries 4.3 / 4.6 / 4.8 /
 // 5.0 against 4.4 / 4.8 / 4.8 / 4.8; 14 levels 4.3 / 4.6 / 4.9 / 5.1 against 4.4 / 4.8 / 4.9 / 4.9. (12 levels, 1 / 64 / 384: 4.4
@@ -1560,7 +1562,7 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
     const bool small_push = nrows <= cap && b->fused;
     // (1) one launch: the update by runs of leaves, whose workgroups also write the pushed rows' leaves; the ring's position
     // has to be the host's, and given priorities one run's
-    if (small_push && !b->device_counters && nrows <= kOneMostRows && takes_range_one(*b, n)) {
+    if (small_push && !b->device_counters && nrows <= kOneMostRows && n <= kElectMax && takes_range_one(*b, n)) {
         const int64_t first = b->pushes % cap, last = first + nrows - 1;
         const int w = range_one_levels(b->depth, n);
         PutArgs put{};

@@ -17,6 +17,10 @@
 namespace mrb {
 
 constexpr int kMeetMost = 256;  // roots: a tile's worth of nodes
+// Atomics on one word are served one after the other, 11 ns each. More than kMeetDirect workgroups count themselves in groups of
+// 16 roots, of which the last to come counts for its group: one trip more (0.6 us), 32 in a row at most instead of 256.
+constexpr int kMeetGroup = 16;
+constexpr uint32_t kMeetDirect = 96;
 
 // kMeetBehindMaxp bytes behind a buffer's running max (one allocation, see counters_behind).
 constexpr int kMeetBehindMaxp = 64;
@@ -24,6 +28,7 @@ struct Meet {
     uint32_t arrived;  // of the launch in progress
     uint32_t turn;     // launches so far
     uint32_t pad[30];
+    uint32_t group[kMeetMost / kMeetGroup][32];  // as `arrived`, of the workgroups of a group; a line each
     unsigned long long root[kMeetMost][2];   // launch number << 32 | bits: sum, minimum
     unsigned long long largest[kMeetMost];  // and, of a push, the largest power
 };
@@ -35,12 +40,39 @@ __device__ __forceinline__ uint32_t meet_turn(float* maxp) {
     return __hip_atomic_load(&meet_of(maxp)->turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Called by one whole wave of each of the `count` workgroups that change their root (number `which`). In the last one's it
-// returns true; vs, vm - four roots to a lane, as memory held them when the kernel started - then hold the new ones where
-// `changed` has the root's bit. The roots are requested together with the counter's answer, on the chance that this is the
+// Who meets: a bit for each of a lane's four roots that changes - the same in every workgroup -, and, worked out from them by
+// one whole wave (early, while it waits for memory), how many count themselves.
+struct MeetPlan {
+    uint32_t changed;
+    uint32_t count;     // on `arrived`
+    uint32_t of_group;  // on the group's counter; 0: there are none
+};
+__device__ __forceinline__ MeetPlan meet_plan(uint32_t changed, uint32_t which, uint32_t lane) {
+    MeetPlan p{changed, 0, 0};
+    uint32_t of = 0;
+    unsigned long long any = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const unsigned long long bits = __ballot(changed >> c & 1u);
+        p.count += (uint32_t)__popcll(bits);
+        of += (uint32_t)__popcll(bits >> (which / kMeetGroup * (kMeetGroup / 4)) & 15u);
+        any |= bits;
+    }
+    if (p.count <= kMeetDirect) return p;  // uniform
+    any |= any >> 1;
+    any |= any >> 2;
+    p.count = (uint32_t)__popcll(any & 0x1111111111111111ull);
+    p.of_group = of;
+    return p;
+}
+
+// Called by one whole wave of each of the workgroups that change their root (number `which`). In the last one's it returns true;
+// vs, vm - four roots to a lane, as memory held them when the kernel started - then hold the new ones where
+// the plan has the root's bit. The roots are requested together with the counter's answer, on the chance that this is the
 // last workgroup and that the others' stores have arrived: then one trip is all it takes.
-__device__ __forceinline__ bool meet(float* maxp, uint32_t turn, uint32_t which, uint32_t count, float root_s, float root_m, uint32_t lane,
-                                     uint32_t changed, float4& vs, float4& vm) {
+__device__ __forceinline__ bool meet(float* maxp, uint32_t turn, uint32_t which, float root_s, float root_m, uint32_t lane,
+                                     const MeetPlan& p, float4& vs, float4& vm) {
+    const uint32_t changed = p.changed;
     Meet* const m = meet_of(maxp);
     const uint32_t tag = turn + 1;
     uint32_t before = 0;
@@ -49,6 +81,14 @@ __device__ __forceinline__ bool meet(float* maxp, uint32_t turn, uint32_t which,
         __hip_atomic_store(&m->root[which][0], number | __float_as_uint(root_s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(&m->root[which][1], number | __float_as_uint(root_m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("" ::: "memory");  // issued in this order
+    }
+    if (p.of_group) {  // uniform
+        uint32_t* const counter = m->group[which / kMeetGroup];
+        if (lane == 0) before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)before) != p.of_group - 1) return false;
+        if (lane == 0) *counter = 0;  // ready for the next launch
+    }
+    if (lane == 0) {
         before = __hip_atomic_fetch_add(&m->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     float s[4] = {vs.x, vs.y, vs.z, vs.w}, t[4] = {vm.x, vm.y, vm.z, vm.w};
@@ -62,7 +102,7 @@ __device__ __forceinline__ bool meet(float* maxp, uint32_t turn, uint32_t which,
                 b[c] = __hip_atomic_load(&m->root[4 * lane + c][1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
-        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)before) != count - 1) return false;
+        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)before) != p.count - 1) return false;
         bool open = false;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {

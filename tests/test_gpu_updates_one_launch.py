@@ -1,4 +1,4 @@
-"""Updates of up to 1024 entries, and the push that follows one in the same call, in one launch: on both sides of the lines of
+"""Updates of up to 4096 entries, and the push that follows one of up to 1024 in the same call, in one launch: on both sides of the lines of
 their rules (tree levels, entries, how many runs of leaves the tree is divided into), against the oracle bit for bit. Forms:
 duplicates, entries that name no leaf and invalid priorities, everything in one tile, consecutive slots; pushes of one row to
 more than a launch takes, across a run's end and around the ring's, over slots the entries name, with a new running max in the
@@ -59,7 +59,7 @@ def same(g, c, what):
 def test_updates(cap):
     g, c, rng = pair(cap, cap if cap < 200_000 else 150_000)
     flags(g)
-    for n in (1, 2, 64, 96, 97, 255, 256, 257, 512, 513, 1024):
+    for n in (1, 2, 64, 96, 97, 192, 193, 255, 256, 257, 512, 513, 1024, 1025, 2049, 4096, 4097):
         for form in range(5):
             idx, pr, ok = entries(rng, cap, n, form)
             g.update_priorities(*to_dev([idx, pr]))
