@@ -105,7 +105,7 @@ struct RowStore {
 // keep their rows packed when a packed row takes at most this many bytes; 0 = every field an array of its own.
 std::atomic<int64_t> g_packed_rows{0};
 
-// What a buffer's launches with short arguments find on the device (but for the flags, which its create function adds).
+// What a buffer's launches with short arguments find on the device.
 RowTable row_table(const RowStore& r) {
     RowTable t{};
     t.t.nfields = r.nfields;
@@ -146,7 +146,8 @@ bool short_io(const void* first, const void* second, const IoTable& t, ShortIo& 
     return short_io(at, n, io);
 }
 
-int rows_alloc(RowStore& r, int64_t capacity, int nfields, const int64_t* field_bytes) {
+// `flags`: `behind` zeroed bytes behind the table, in one allocation with it and filled by the copy that fills it.
+int rows_alloc(RowStore& r, int64_t capacity, int nfields, const int64_t* field_bytes, size_t behind, uint32_t** flags) {
     if (capacity <= 0 || capacity > (1ll << 30)) return fail(MRB_EINVAL, "capacity %lld outside [1, 2^30]", (long long)capacity);
     if (nfields <= 0 || nfields > MRB_MAX_FIELDS) return fail(MRB_EINVAL, "nfields %d outside [1, %d]", nfields, MRB_MAX_FIELDS);
     if (!field_bytes) return fail(MRB_EINVAL, "field_bytes is NULL");
@@ -189,9 +190,14 @@ int rows_alloc(RowStore& r, int64_t capacity, int nfields, const int64_t* field_
             HIP_TRY(hipMemset(r.data[i], 0, total));
         }
     }
-    const RowTable table = row_table(r);
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r.table), sizeof(table)));
-    HIP_TRY(hipMemcpy(r.table, &table, sizeof(table), hipMemcpyHostToDevice));
+    constexpr size_t kTableBytes = (sizeof(RowTable) + 255) / 256 * 256;
+    std::vector<char> fill(kTableBytes + behind, 0);
+    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r.table), fill.size()));
+    *flags = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(r.table) + kTableBytes);
+    RowTable table = row_table(r);
+    table.err = *flags;
+    memcpy(fill.data(), &table, sizeof(table));
+    HIP_TRY(hipMemcpy(r.table, fill.data(), fill.size(), hipMemcpyHostToDevice));
     return MRB_OK;
 }
 
@@ -528,12 +534,11 @@ struct Urb {
     RowStore rows;
     int64_t count = 0, head = 0;
     uint64_t seed = 0, calls = 0;
-    uint32_t* err = nullptr;       // 16 bytes of flags, then the device copy of the counters (kUrb* in mrb_kernels.h)
+    uint32_t* err = nullptr;       // (behind rows.table) 16 bytes of flags, then the device copy of the counters (kUrb* in mrb_kernels.h)
     int64_t* counters = nullptr;   // = err + 16 bytes
     int64_t* slots = nullptr;      // device array of kUrbDrawMax slots: drawn there when the counters live on the device
     int64_t device_counters = 0;   // option "device_counters"
     ~Urb() {
-        if (err) (void)hipFree(err);
         if (slots) (void)hipFree(slots);
     }
 };
@@ -598,7 +603,6 @@ struct Per {
         for (auto* d : retired) (void)hipFree(d);
         for (auto* d : s_dirty)
             if (d) (void)hipFree(d);
-        if (err) (void)hipFree(err);
         for (auto* d : dirty)
             if (d) (void)hipFree(d);
     }
@@ -612,7 +616,6 @@ struct Res {
     uint32_t* err = nullptr;
     ~Res() {
         if (stamp) (void)hipFree(stamp);
-        if (err) (void)hipFree(err);
     }
 };
 
@@ -1102,11 +1105,8 @@ int mrb_urb_create(int64_t capacity, int nfields, const int64_t* field_bytes, in
     if (!out_handle) return fail(MRB_EINVAL, "out_handle is NULL");
     if (capacity > 0x7fffffffll) return fail(MRB_EINVAL, "capacity %lld does not fit the int32 count", (long long)capacity);
     auto b = std::make_shared<Urb>();
-    int rc = rows_alloc(b->rows, capacity, nfields, field_bytes);
+    int rc = rows_alloc(b->rows, capacity, nfields, field_bytes, 16 + kCntWords * sizeof(int64_t), &b->err);
     if (rc) return rc;
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->err), 16 + kCntWords * sizeof(int64_t)));
-    HIP_TRY(hipMemset(b->err, 0, 16 + kCntWords * sizeof(int64_t)));
-    HIP_TRY(hipMemcpy(&b->rows.table->err, &b->err, sizeof(b->err), hipMemcpyHostToDevice));
     b->counters = reinterpret_cast<int64_t*>(b->err + 4);
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->slots), kUrbDrawMax * sizeof(int64_t)));
     HIP_TRY(hipDeviceSynchronize());  // the zero-fills ran on the null stream; the caller's stream may not wait for it
@@ -1314,7 +1314,7 @@ int mrb_per_create(int64_t capacity, float alpha, int nfields, const int64_t* fi
     if (!out_handle) return fail(MRB_EINVAL, "out_handle is NULL");
     if (!(alpha >= 0.0f) || alpha > 16.0f) return fail(MRB_EINVAL, "alpha %g outside [0, 16]", (double)alpha);
     auto b = std::make_shared<Per>();
-    int rc = rows_alloc(b->rows, capacity, nfields, field_bytes);
+    int rc = rows_alloc(b->rows, capacity, nfields, field_bytes, kMaxpBehindErr + kMeetBehindMaxp + sizeof(Meet), &b->err);
     if (rc) return rc;
     while (b->leaves < capacity) {
         b->leaves <<= 1;
@@ -1341,17 +1341,13 @@ int mrb_per_create(int64_t capacity, float alpha, int nfields, const int64_t* fi
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->sum), nodes * sizeof(float)));
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->mn), nodes * sizeof(float)));
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->stamp), (size_t)b->leaves * sizeof(unsigned long long)));
-    // one allocation: the error word (16 bytes), the device copy of the counters (kernels find them behind the error
+    // one allocation, behind the row table: the error word (16 bytes), the device copy of the counters (kernels find them behind the error
     // word), and kMaxpBehindErr bytes in the running max (16 bytes; a kernel that is given its address finds the
     // counters in front of it: counters_before)
     static_assert(16 + kCntWords * sizeof(int64_t) <= kMaxpBehindErr, "the counters end before the running max");
     // (and, behind it, what the workgroups of an update meet over: Meet)
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->err), kMaxpBehindErr + kMeetBehindMaxp + sizeof(Meet)));
     b->counters = reinterpret_cast<int64_t*>(b->err + 4);
     b->maxp = reinterpret_cast<float*>(reinterpret_cast<char*>(b->err) + kMaxpBehindErr);
-    HIP_TRY(hipMemset(b->counters, 0, kCntWords * sizeof(int64_t)));
-    HIP_TRY(hipMemset(reinterpret_cast<char*>(b->maxp) + kMeetBehindMaxp, 0, sizeof(Meet)));
-    HIP_TRY(hipMemcpy(&b->rows.table->err, &b->err, sizeof(b->err), hipMemcpyHostToDevice));
     // update_priorities scratch, sized once: a call rarely names more entries than there are rows
     b->powered_cap = capacity < 4096 ? 4096 : (capacity > (1ll << 20) ? (1ll << 20) : capacity);
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->powered), (size_t)b->powered_cap * sizeof(float)));
@@ -1361,7 +1357,6 @@ int mrb_per_create(int64_t capacity, float alpha, int nfields, const int64_t* fi
     if (rc) return rc;
     HIP_TRY(hipMemset(b->sum, 0, nodes * sizeof(float)));
     HIP_TRY(hipMemset(b->stamp, 0, (size_t)b->leaves * sizeof(unsigned long long)));
-    HIP_TRY(hipMemset(b->err, 0, 16));
     for (int r = 0; r < b->nrounds; ++r) {
         const size_t nblocks = (size_t)1 << (b->lo[r] - b->g[r]);
         HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->dirty[r]), nblocks * sizeof(uint32_t)));
@@ -1882,14 +1877,11 @@ int mrb_per_destroy(int64_t h) {
 int mrb_res_create(int64_t capacity, int nfields, const int64_t* field_bytes, uint64_t seed, int64_t* out_handle) {
     if (!out_handle) return fail(MRB_EINVAL, "out_handle is NULL");
     auto b = std::make_shared<Res>();
-    int rc = rows_alloc(b->rows, capacity, nfields, field_bytes);
+    int rc = rows_alloc(b->rows, capacity, nfields, field_bytes, 16, &b->err);
     if (rc) return rc;
     b->seed = seed;
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->stamp), (size_t)capacity * sizeof(unsigned long long)));
     HIP_TRY(hipMemset(b->stamp, 0, (size_t)capacity * sizeof(unsigned long long)));
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->err), 16));
-    HIP_TRY(hipMemset(b->err, 0, 16));
-    HIP_TRY(hipMemcpy(&b->rows.table->err, &b->err, sizeof(b->err), hipMemcpyHostToDevice));
     HIP_TRY(hipDeviceSynchronize());  // as in mrb_urb_create
     std::lock_guard<std::mutex> lk(g_mu);
     *out_handle = g_next++;
