@@ -776,12 +776,14 @@ void fill_zero(void* p, size_t bytes, hipStream_t s) {
 
 // A push whose leaf tiles are rebuilt by several workgroups, or whose powers one shares out over its threads (k_push_many): with
 // priorities always; without, one tile (us, k_push_run / this: 3.6 / 3.3) or eight and more (1024 rows 4.2 / 4.7, 1500 4.5 / 4.8,
-// 2048 4.9 / 4.8, 3000 5.4 / 4.8: up to seven the roots' meeting costs more than sharing the tiles out saves).
+// 2048 4.9 / 4.8, 3000 5.4 / 4.8: up to seven the roots' meeting costs more than sharing the tiles out saves), or a copy of more than
+// kManyCopy workgroups, which waits for k_push_run's large ones (300 rows of 28 KB 9.3 / 4.9, 1000 18.2 / 10.9).
 constexpr int64_t kManyLeastTiles = 8;
-bool takes_push_many(const Per& b, int64_t first, int64_t n, bool with_priorities) {
+constexpr uint32_t kManyCopy = 1024;
+bool takes_push_many(const Per& b, int64_t first, int64_t n, bool with_priorities, uint32_t copy_blocks) {
     if (b.device_counters || !b.fused || b.nrounds == 0 || first + n > b.rows.capacity) return false;
     const int64_t tiles = (first + n - 1) / kBlockNodes - first / kBlockNodes + 1;
-    return (with_priorities || tiles == 1 || tiles >= kManyLeastTiles) && tiles <= kManyMostTiles;
+    return (with_priorities || tiles == 1 || tiles >= kManyLeastTiles || copy_blocks > kManyCopy) && tiles <= kManyMostTiles;
 }
 
 // Starts a new tree-update epoch. Epochs tag stamps and dirty words so that
@@ -1416,7 +1418,7 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
         put.first_slot = -1;
         put.src_first = reinterpret_cast<int64_t>(b->counters);
     }
-    if (ShortIo io{}; !lead && skip == 0 && n > 1 && takes_push_many(*b, first, n, opt_priorities != nullptr) && short_io(put.t, io)) {
+    if (ShortIo io{}; !lead && skip == 0 && n > 1 && takes_push_many(*b, first, n, opt_priorities != nullptr, put.blocks) && short_io(put.t, io)) {
         const hipError_t e = launch_push_many(b->rows.table, io, put.t.nfields, b->sum, b->mn, b->maxp, opt_priorities, first, n, b->depth,
                                               b->alpha, most_granules(put.t), s);
         if (e != hipSuccess) return fail(MRB_EHIP, "launch k_push_many: %s", hipGetErrorString(e));
@@ -1426,8 +1428,13 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
     }
     // A large copy gets its own launch; a small one rides along in the first tree launch.
     if (put.blocks > 2048u) {
-        hipLaunchKernelGGL(k_rows_put, dim3(put.blocks), dim3(kWG), 0, s, put);
-        LAUNCH_CHECK("k_rows_put");
+        if (ShortIo io{}; !b->device_counters && short_io(put.t, io)) {
+            const hipError_t e = launch_short_put(b->rows.table, io, put.t.nfields, first, n, most_granules(put.t), s);
+            if (e != hipSuccess) return fail(MRB_EHIP, "launch k_short_put: %s", hipGetErrorString(e));
+        } else {
+            hipLaunchKernelGGL(k_rows_put, dim3(put.blocks), dim3(kWG), 0, s, put);
+            LAUNCH_CHECK("k_rows_put");
+        }
         put.blocks = 0;
     }
     if (lead) {

@@ -6,9 +6,9 @@
 // By-value field tables are 550 to 1000 bytes, and nearly all of them is the same in every call. On the device a kernel's first
 // trip reads what it needs of the table into scalar registers, and the copies have a row of workgroups per field instead of a
 // search for each granule's field. Device time per call, us, by value / short: an append of 1 row 2.85 / 2.04, of 1000 rows of
-// 133 bytes 3.08 / 2.39, of 57.5 MB (read and written) 15.5 / 12.2; a gather of 256 rows of 162 bytes 3.17 / 2.66, of 8192 rows
-// of 133 bytes 4.87 / 4.25; a push of 1 row 2.86 / 2.28, of 64 3.09 / 2.84, of 1000 3.56 / 3.13, of 4096 with priorities
-// 8.7 / 8.8. Host time of one uniform insert and sample 10.0 / 9.2.
+// 133 bytes 3.08 / 2.39, of 57.5 MB (read and written) 15.5 / 11.4; a gather of 256 rows of 162 bytes 3.17 / 2.66, of 8192 rows
+// of 133 bytes 4.87 / 4.25; a push of 1 row 2.86 / 2.28, of 64 3.09 / 2.84, of 1000 3.56 / 3.13. Host
+// time of one uniform insert and sample 10.0 / 9.2.
 //
 // By value stay: more than kShortPointers matrices, matrices too far apart at an odd address, device-resident counters, single-row
 // reads, copies from another buffer's ring; the sampling kernels and the reservoir's push (3.35 / 3.40 and 2.8 / 2.9 when they
@@ -62,6 +62,7 @@ struct ShortRows {
 // workgroups per field: what the table says of it is the same for all its threads and comes in one trip through scalar
 // registers.) A thread has up to four granules on their way before it stores the first.
 constexpr int kPutTrip = 4;
+constexpr uint32_t kPutFew = 512;  // workgroups up to which a thread has one
 
 __device__ __forceinline__ void put_field(const RowTable* __restrict__ table, const ShortIo& io, int f, uint32_t first_slot, uint32_t n,
                                           uint32_t block, uint32_t blocks, uint32_t threads) {
@@ -69,7 +70,10 @@ __device__ __forceinline__ void put_field(const RowTable* __restrict__ table, co
     const uint32_t units = rows.units(f), vl = rows.vl(f), row_bytes = rows.row_bytes(f), stride = rows.stride(f);
     gbyte* const store = as_global(rows.store(f));
     const gbyte* const from = as_global((const uint8_t*)rows.io(f));
-    const uint64_t ring = (uint64_t)table->capacity, total = (uint64_t)n * units, step = (uint64_t)blocks * threads;
+    const uint64_t ring = (uint64_t)table->capacity, total = (uint64_t)n * units;
+    // granules of a thread and trip: side by side those of a workgroup, which keeps what is in flight within few pages
+    const uint32_t per = total > (uint64_t)kPutFew * threads ? kPutTrip : 1;
+    const uint64_t step = (uint64_t)blocks * threads * per;
     auto place = [&](uint64_t w, const gbyte*& src) -> gbyte* {
         uint64_t row;
         uint32_t unit;
@@ -80,26 +84,25 @@ __device__ __forceinline__ void put_field(const RowTable* __restrict__ table, co
         src = from + row * row_bytes + off;
         return store + slot * stride + off;
     };
-    uint64_t w = (uint64_t)block * threads + threadIdx.x;
-    if (vl == 4) {  // (uniform)
-        for (; w < total; w += kPutTrip * step) {
+    if (vl == 4 && per > 1) {  // (uniform)
+        for (uint64_t w = (uint64_t)block * threads * kPutTrip + threadIdx.x; w < total; w += step) {
             granule_t held[kPutTrip];
             gbyte* to[kPutTrip];
 #pragma unroll
             for (int q = 0; q < kPutTrip; ++q) {
                 const gbyte* src;
-                to[q] = place(w + q * step < total ? w + q * step : w, src);  // (past the end: the thread's first again)
+                to[q] = place(w + q * threads < total ? w + q * threads : w, src);  // (past the end: the thread's first again)
                 held[q] = __builtin_nontemporal_load((const g16*)src);
             }
 #pragma unroll
             for (int q = 0; q < kPutTrip; ++q) asm volatile("" : "+v"(held[q]));
 #pragma unroll
             for (int q = 0; q < kPutTrip; ++q)
-                if (w + q * step < total) __builtin_nontemporal_store(held[q], (g16*)to[q]);
+                if (w + q * threads < total) __builtin_nontemporal_store(held[q], (g16*)to[q]);
         }
         return;
     }
-    for (; w < total; w += step) {
+    for (uint64_t w = (uint64_t)block * threads + threadIdx.x; w < total; w += (uint64_t)blocks * threads) {
         const gbyte* src;
         gbyte* const to = place(w, src);
         copy_granule(to, src, vl);
@@ -107,10 +110,12 @@ __device__ __forceinline__ void put_field(const RowTable* __restrict__ table, co
 }
 
 // Workgroups per field: one granule to a thread where that is all there is to do, four where the launch would be tens of
-// thousands of waves (a call of 32 MB: 9.1 us with one, 6.5 with four).
+// thousands of waves (16 MB
+// 4.8 us with one, 3.4 with four; 57 MB of odd rows 15.0 / 11.4; 200 MB 44.9 / 35.2; 500 MB 110 / 85, and 92 with a thread's four
+// a launch's width apart).
 inline uint32_t put_blocks(uint64_t granules, uint32_t threads) {
     uint64_t blocks = (granules + threads - 1) / threads;
-    if (blocks > 512) blocks = (blocks + kPutTrip - 1) / kPutTrip;
+    if (blocks > kPutFew) blocks = (blocks + kPutTrip - 1) / kPutTrip;
     return (uint32_t)(blocks < 16384 ? blocks : 16384);
 }
 

@@ -73,6 +73,26 @@ def test_push(cap, first, n, big):
         assert flags(a) == flags(b), how
 
 
+@pytest.mark.parametrize("n", [3, 290, 700, 9000])
+def test_large_copies(n):
+    """Copies of several granules to a thread, with the tiles' work and ahead of it: the rows lie where they belong."""
+    from mindrl_amd.core import PriorityReplayBuffer, UniformReplayBuffer
+    cap = 10_000
+    shapes, types = [(4099,), (1031,), (1,)], [torch.int32, torch.uint8, torch.int64]
+    a, u = PriorityReplayBuffer(0.7, cap, 8, shapes, types), UniformReplayBuffer(8, cap, shapes, types)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    for first in (0, n):
+        rows = [torch.randint(0, 200, (n,) + s, device="cuda", generator=g).to(t) for s, t in zip(shapes, types)]
+        a.insert(*rows)
+        u.insert(rows)
+        for stored in (a.storage(), u.buffer):
+            for x, y in zip(stored, rows):
+                kept = min(n, cap - first)
+                assert torch.equal(x[first : first + kept], y[:kept]) and torch.equal(x[: n - kept], y[kept:]), first
+    s, m = a.export_tree()
+    assert s[1] == min(2 * n, cap) and m[1] == 1.0
+
+
 def test_replays():
     """A recorded call is replayed between the program's own."""
     from mindrl_amd.core import PriorityReplayBuffer
