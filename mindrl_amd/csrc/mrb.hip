@@ -262,7 +262,7 @@ int rows_put(const RowStore& r, const void* const* src, int64_t skip, int64_t n,
     int rc = put_args(r, src, skip, n, first_slot, p);
     if (rc) return rc;
     if (ShortIo io{}; short_io(p.t, io)) {
-        const hipError_t e = launch_short_put(r.table, io, r.nfields, first_slot, n, most_granules(p.t), s);
+        const hipError_t e = launch_short_put(r.table, io, p.t, first_slot, n, s);
         return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch k_short_put: %s", hipGetErrorString(e));
     }
     hipLaunchKernelGGL(k_rows_put, dim3(p.blocks), dim3(kWG), 0, s, p);
@@ -1419,8 +1419,8 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
         put.src_first = reinterpret_cast<int64_t>(b->counters);
     }
     if (ShortIo io{}; !lead && skip == 0 && n > 1 && takes_push_many(*b, first, n, opt_priorities != nullptr, put.blocks) && short_io(put.t, io)) {
-        const hipError_t e = launch_push_many(b->rows.table, io, put.t.nfields, b->sum, b->mn, b->maxp, opt_priorities, first, n, b->depth,
-                                              b->alpha, most_granules(put.t), s);
+        const hipError_t e = launch_push_many(b->rows.table, io, put.t, b->sum, b->mn, b->maxp, opt_priorities, first, n, b->depth,
+                                              b->alpha, s);
         if (e != hipSuccess) return fail(MRB_EHIP, "launch k_push_many: %s", hipGetErrorString(e));
         b->pushes += nrows;
         b->size = b->size + nrows < cap ? b->size + nrows : cap;
@@ -1429,7 +1429,7 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
     // A large copy gets its own launch; a small one rides along in the first tree launch.
     if (put.blocks > 2048u) {
         if (ShortIo io{}; !b->device_counters && short_io(put.t, io)) {
-            const hipError_t e = launch_short_put(b->rows.table, io, put.t.nfields, first, n, most_granules(put.t), s);
+            const hipError_t e = launch_short_put(b->rows.table, io, put.t, first, n, s);
             if (e != hipSuccess) return fail(MRB_EHIP, "launch k_short_put: %s", hipGetErrorString(e));
         } else {
             hipLaunchKernelGGL(k_rows_put, dim3(put.blocks), dim3(kWG), 0, s, put);

@@ -10,8 +10,8 @@ namespace mrb {
 constexpr uint32_t kManyMostTiles = 256;  // (their roots lie under two tiles at most)
 
 // A push of n rows to consecutive slots from first_slot on (not around the ring's end), on a tree of more than 8 levels, with
-// its row copy (granules: of the field that has the most). With priorities, running max included.
-hipError_t launch_push_many(const RowTable* table, const ShortIo& io, int nfields, float* sum, float* mn, float* maxp, const float* priorities,
-                            int64_t first_slot, int64_t n, int depth, float alpha, uint64_t granules, hipStream_t s);
+// its row copy (t: the call's table). With priorities, running max included.
+hipError_t launch_push_many(const RowTable* table, const ShortIo& io, const IoTable& t, float* sum, float* mn, float* maxp, const float* priorities,
+                            int64_t first_slot, int64_t n, int depth, float alpha, hipStream_t s);
 
 }  // namespace mrb

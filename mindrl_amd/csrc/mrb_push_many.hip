@@ -41,7 +41,7 @@ __global__ __launch_bounds__(kWG) void k_push_many(float* sum, float* mn, float*
     __shared__ uint32_t s_new[2], s_before;
     const uint32_t groups = plan >> 8;
     if (__builtin_expect(blockIdx.x >= groups || blockIdx.y != 0, 0)) {
-        if (blockIdx.x >= groups) put_field(table, io, blockIdx.y, first_slot, n, blockIdx.x - groups, blocks, kWG);
+        if (blockIdx.x >= groups) put_fields(table, io, first_slot, n, blockIdx.x - groups, blocks);
         rider_ends();
     }
     const int depth = (int)(plan & 255u);
@@ -266,14 +266,16 @@ __global__ __launch_bounds__(kWG) void k_push_many(float* sum, float* mn, float*
 
 }  // namespace
 
-hipError_t launch_push_many(const RowTable* table, const ShortIo& io, int nfields, float* sum, float* mn, float* maxp, const float* priorities,
-                            int64_t first_slot, int64_t n, int depth, float alpha, uint64_t granules, hipStream_t s) {
+hipError_t launch_push_many(const RowTable* table, const ShortIo& io, const IoTable& t, float* sum, float* mn, float* maxp, const float* priorities,
+                            int64_t first_slot, int64_t n, int depth, float alpha, hipStream_t s) {
     const uint32_t tiles = (uint32_t)((first_slot + n - 1) / kBlockNodes - first_slot / kBlockNodes + 1);
-    const uint32_t per = tiles == 1 || (priorities && tiles <= kManyApart) ? 1 : 4, groups = (tiles + per - 1) / per, blocks = put_blocks(granules, kWG);
+    const uint32_t per = tiles == 1 || (priorities && tiles <= kManyApart) ? 1 : 4, groups = (tiles + per - 1) / per;
+    uint32_t blocks;
+    const dim3 grid = put_grid(t, groups, blocks);
     auto* kernel = k_push_many<4, false>;
     if (per == 1) kernel = k_push_many<1, false>;
     if (tiles == 1) kernel = k_push_many<1, true>;
-    hipLaunchKernelGGL(kernel, dim3(groups + blocks, (uint32_t)nfields), dim3(kWG), 0, s, sum, mn, maxp,
+    hipLaunchKernelGGL(kernel, grid, dim3(kWG), 0, s, sum, mn, maxp,
                        priorities, table, (uint32_t)first_slot, (uint32_t)n, (uint32_t)depth | groups << 8, alpha, blocks, io);
     return hipGetLastError();
 }

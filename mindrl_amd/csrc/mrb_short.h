@@ -58,11 +58,22 @@ struct ShortRows {
     __device__ __forceinline__ uint64_t granules(int f) const { return n * r->t.units[f]; }
 };
 
+constexpr int kPutTrip = 4;
+constexpr uint32_t kPutFew = 512;  // workgroups up to which a thread has one
+
+// Workgroups per field: one granule to a thread where that is all there is to do, four where the launch would be tens of
+// thousands of waves (16 MB
+// 4.8 us with one, 3.4 with four; 57 MB of odd rows 15.0 / 11.4; 200 MB 44.9 / 35.2; 500 MB 110 / 85, and 92 with a thread's four
+// a launch's width apart).
+__host__ __device__ inline uint32_t put_blocks(uint64_t granules, uint32_t threads) {
+    uint64_t blocks = (granules + threads - 1) / threads;
+    if (blocks > kPutFew) blocks = (blocks + kPutTrip - 1) / kPutTrip;
+    return (uint32_t)(blocks < 16384 ? blocks : 16384);
+}
+
 // The copy of a ring append, one field's n rows by workgroup `block` of `blocks` with `threads` threads each. (A row of
 // workgroups per field: what the table says of it is the same for all its threads and comes in one trip through scalar
 // registers.) A thread has up to four granules on their way before it stores the first.
-constexpr int kPutTrip = 4;
-constexpr uint32_t kPutFew = 512;  // workgroups up to which a thread has one
 
 __device__ __forceinline__ void put_field(const RowTable* __restrict__ table, const ShortIo& io, int f, uint32_t first_slot, uint32_t n,
                                           uint32_t block, uint32_t blocks, uint32_t threads) {
@@ -109,21 +120,40 @@ __device__ __forceinline__ void put_field(const RowTable* __restrict__ table, co
     }
 }
 
-// Workgroups per field: one granule to a thread where that is all there is to do, four where the launch would be tens of
-// thousands of waves (16 MB
-// 4.8 us with one, 3.4 with four; 57 MB of odd rows 15.0 / 11.4; 200 MB 44.9 / 35.2; 500 MB 110 / 85, and 92 with a thread's four
-// a launch's width apart).
-inline uint32_t put_blocks(uint64_t granules, uint32_t threads) {
-    uint64_t blocks = (granules + threads - 1) / threads;
-    if (blocks > kPutFew) blocks = (blocks + kPutTrip - 1) / kPutTrip;
-    return (uint32_t)(blocks < 16384 ? blocks : 16384);
+// A launch of few workgroups has as many for every field (blockIdx.y). Of one of many those of the small fields would do nothing, and
+// 65,536 workgroups that leave at once take 15 us: it has each field's own number of them, one field's behind the other's.
+__device__ __forceinline__ void put_fields(const RowTable* __restrict__ table, const ShortIo& io, uint32_t first_slot, uint32_t n,
+                                           uint32_t block, uint32_t blocks) {
+    if (blocks) {  // uniform
+        put_field(table, io, blockIdx.y, first_slot, n, block, blocks, kWG);
+        return;
+    }
+    int f = 0;
+    for (;;) {
+        blocks = put_blocks((uint64_t)n * table->t.units[f], kWG);
+        if (block < blocks || f + 1 == table->t.nfields) break;
+        block -= blocks;
+        ++f;
+    }
+    put_field(table, io, f, first_slot, n, block, blocks, kWG);
+}
+
+// `blocks` of such a launch, and its grid behind (in x) `in_front` other workgroups. (t: the call's table.)
+inline dim3 put_grid(const IoTable& t, uint32_t in_front, uint32_t& blocks) {
+    uint32_t most = 0, all = 0;
+    for (int f = 0; f < t.nfields; ++f) {
+        const uint32_t b = put_blocks(t.prefix[f + 1] - t.prefix[f], kWG);
+        most = b > most ? b : most;
+        all += b;
+    }
+    blocks = most <= kPutFew ? most : 0;
+    return blocks ? dim3(in_front + blocks, (uint32_t)t.nfields) : dim3(in_front + all);
 }
 
 hipError_t launch_short_gather(const RowTable* table, const ShortIo& io, int nfields, const int64_t* indices, int64_t count, uint64_t seed,
                                uint64_t calls, int64_t n, uint32_t blocks, bool with_indices, hipStream_t s);
+hipError_t launch_short_put(const RowTable* table, const ShortIo& io, const IoTable& t, int64_t first_slot, int64_t n, hipStream_t s);
 // (granules: the field's with the most)
-hipError_t launch_short_put(const RowTable* table, const ShortIo& io, int nfields, int64_t first_slot, int64_t n, uint64_t granules,
-                            hipStream_t s);
 hipError_t launch_short_push_one(const RowTable* table, const ShortIo& io, int nfields, float* sum, float* mn, float* maxp, int64_t first_slot,
                                  int depth, float alpha, const float* priority, uint64_t granules, hipStream_t s);
 hipError_t launch_short_push_run(const RowTable* table, const ShortIo& io, int nfields, const UpdateArgs& a, uint32_t units, uint64_t granules,

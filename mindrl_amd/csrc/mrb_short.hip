@@ -15,7 +15,7 @@ __global__ __launch_bounds__(kWG) void k_short_gather(const RowTable* __restrict
 
 __global__ __launch_bounds__(kWG) void k_short_put(const RowTable* __restrict__ table, uint32_t first_slot, uint32_t n, uint32_t blocks,
                                                    ShortIo io) {
-    put_field(table, io, blockIdx.y, first_slot, n, blockIdx.x, blocks, kWG);
+    put_fields(table, io, first_slot, n, blockIdx.x, blocks);
 }
 
 // Pushes: workgroup (0, 0) does the tree's work, those with a column of at least 1 copy rows of field blockIdx.y.
@@ -66,10 +66,10 @@ hipError_t launch_short_gather(const RowTable* table, const ShortIo& io, int nfi
     return hipGetLastError();
 }
 
-hipError_t launch_short_put(const RowTable* table, const ShortIo& io, int nfields, int64_t first_slot, int64_t n, uint64_t granules,
-                            hipStream_t s) {
-    const uint32_t blocks = put_blocks(granules, kWG);
-    hipLaunchKernelGGL(k_short_put, dim3(blocks, (uint32_t)nfields), dim3(kWG), 0, s, table, (uint32_t)first_slot, (uint32_t)n, blocks, io);
+hipError_t launch_short_put(const RowTable* table, const ShortIo& io, const IoTable& t, int64_t first_slot, int64_t n, hipStream_t s) {
+    uint32_t blocks;
+    const dim3 grid = put_grid(t, 0, blocks);
+    hipLaunchKernelGGL(k_short_put, grid, dim3(kWG), 0, s, table, (uint32_t)first_slot, (uint32_t)n, blocks, io);
     return hipGetLastError();
 }
 
