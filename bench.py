@@ -774,7 +774,7 @@ def bench_uniform(a):
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "u8", "data": "synthetic",
         "config": {"workload": "config 2: SAC-shaped UniformReplayBuffer, capacity %d, 165 B rows, batch 256, "
                                "host-drawn indices" % capacity, "row_bytes": row_bytes},
-        "roofline": roofline("k_rows_gather", algo, kern_s, wall / K, "c2", "batch * (2 * row_bytes + 8)"),
+        "roofline": roofline("k_short_gather", algo, kern_s, wall / K, "c2", "batch * (2 * row_bytes + 8)"),
         "extras": {"inserts_per_s": capacity / ins_s, "insert_chunk": chunk},
         "cpu_baseline": None,
     }
@@ -851,7 +851,7 @@ def bench_reservoir(a):
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "u8", "data": "synthetic",
         "config": {"workload": "ReservoirReplayBuffer, capacity %d, 92 B rows, push 4096 per call past capacity, "
                                "sample 256 per call" % capacity, "row_bytes": row_bytes},
-        "roofline": roofline("k_rows_gather", algo, kern_s, wall / K, "res", "batch * 2 * row_bytes"),
+        "roofline": roofline("k_short_gather", algo, kern_s, wall / K, "res", "batch * 2 * row_bytes"),
         "extras": {"pushes_per_s": n_push * chunk / push_s, "push_chunk": chunk},
         "cpu_baseline": None,
     }

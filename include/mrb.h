@@ -102,8 +102,8 @@ int mrb_version(void);
  *                  `capacity` rows, a sample at most 65,536 (its slots are drawn into a device array that
  *                  overlapping sample / get_item calls on one handle would share), mrb_urb_append_from is
  *                  refused, and mrb_urb_state, mrb_urb_reset, mrb_urb_seed and the checkpoint calls wait.
- *   "fused_rebuild" prioritized buffers: 1 (default) = an update of <= 1024 entries on a tree of at most 22 levels
- *                  or a push under <= 16 leaf tiles rebuilds the tree in one launch; 0 = one launch per round */
+ *   "fused_rebuild" prioritized buffers: 1 (default) = an update of <= 1024 entries on a tree of at most 22 levels (<= 4096
+ *                  on one of at most 20) or a push under <= 256 leaf tiles (16 around the ring's end) rebuilds the tree in one launch; 0 = one launch per round */
 /* Library-wide default, set with handle 0 and taken by buffers created afterwards:
  *   "packed_rows"  N > 0: a buffer whose packed row - every field at the next multiple of its own copy granule
  *                  (the largest power of two <= 16 that divides its size), the row padded to the widest granule -
