@@ -68,6 +68,7 @@ extern "C" {
 #define MRB_DERR_PRIORITY 2u  /* update_priorities/push: negative or non-finite priority — entry skipped */
 #define MRB_DERR_TOTAL 4u     /* sample: tree total not finite or <= 0 */
 #define MRB_DERR_UNFILLED 8u  /* sample: descent ended on a slot >= size */
+#define MRB_DERR_OVERLAP 16u  /* update/push: calls that change the handle ran side by side — levels at the tree's top not rebuilt */
 
 /* ---- library ---------------------------------------------------------- */
 

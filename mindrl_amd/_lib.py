@@ -10,7 +10,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libmrb.so")
 
 MRB_OK, MRB_EINVAL, MRB_EHANDLE, MRB_EHIP, MRB_ESTATE, MRB_EDEVICE = 0, 1, 2, 3, 4, 5
-DERR_INDEX, DERR_PRIORITY, DERR_TOTAL, DERR_UNFILLED = 1, 2, 4, 8
+DERR_INDEX, DERR_PRIORITY, DERR_TOTAL, DERR_UNFILLED, DERR_OVERLAP = 1, 2, 4, 8, 16
 MAX_FIELDS = 16
 ABI_VERSION = 4  # MRB_ABI_VERSION of include/mrb.h this binding was written against
 

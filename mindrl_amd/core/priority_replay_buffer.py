@@ -340,6 +340,8 @@ class PriorityReplayBuffer:
             raise ValueError("update_priorities: negative or non-finite priority")
         if f & _lib.DERR_TOTAL:
             raise ValueError("sample: total priority is not positive and finite")
+        if f & _lib.DERR_OVERLAP:
+            raise RuntimeError("calls that change the buffer ran side by side (on several streams, not ordered)")
         return f
 
     def set_option(self, name, value):

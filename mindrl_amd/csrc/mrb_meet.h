@@ -8,11 +8,18 @@
 // the counter has overtaken. It waits for stores that are on their way, never for a workgroup that has yet to run, so it
 // ends however the workgroups are scheduled; nothing has to be cleared between launches; and a launch replayed from a graph
 // finds its number on the device.
+//
+// Calls that change one buffer must not run side by side (mrb.h). Where two did all the same, they share the counters and the
+// number, so what the counters hold afterwards is anybody's guess and a root may never come. Two things keep that from outliving
+// those calls. Whoever counts itself at or behind the last place, not only at it, takes the roots, after all of them have
+// this launch's number: from whatever count a launch starts, at least one workgroup does, with every root, and several write
+// the same values. And the wait ends after kMeetLooks looks, which leaves the roots that did not come as they were and says so
+// in the buffer's flags.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "mrb_rows.h"
+#include "../../include/mrb.h"
 
 namespace mrb {
 
@@ -21,6 +28,8 @@ constexpr int kMeetMost = 256;  // roots: a tile's worth of nodes
 // 16 roots, of which the last to come counts for its group: one trip more (0.6 us), 32 in a row at most instead of 256.
 constexpr int kMeetGroup = 16;
 constexpr uint32_t kMeetDirect = 96;
+// Looks at the roots at most. One is a trip to memory, half a microsecond or more, and stores on their way take a few: 30 ms and more.
+constexpr uint32_t kMeetLooks = 1u << 16;
 
 // kMeetBehindMaxp bytes behind a buffer's running max (one allocation, see counters_behind).
 constexpr int kMeetBehindMaxp = 64;
@@ -38,6 +47,15 @@ __device__ __forceinline__ Meet* meet_of(float* maxp) { return reinterpret_cast<
 // The number of launches before this one (requested when a kernel starts: the last workgroup moves it on).
 __device__ __forceinline__ uint32_t meet_turn(float* maxp) {
     return __hip_atomic_load(&meet_of(maxp)->turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Whether a workgroup that `before` others came ahead of, of `count` that come, is to take the roots.
+__device__ __forceinline__ bool meet_last(uint32_t before, uint32_t count) { return before + 1 >= count; }
+__device__ __forceinline__ bool meet_here(unsigned long long word, uint32_t tag) { return (uint32_t)(word >> 32) == tag; }
+// By one thread, when every root has been looked at for the last time: ready for the next launch.
+__device__ __forceinline__ void meet_over(Meet* m, uint32_t tag) {
+    m->arrived = 0;
+    m->turn = tag;
 }
 
 // Who meets: a bit for each of a lane's four roots that changes - the same in every workgroup -, and, worked out from them by
@@ -68,9 +86,9 @@ __device__ __forceinline__ MeetPlan meet_plan(uint32_t changed, uint32_t which, 
 
 // Called by one whole wave of each of the workgroups that change their root (number `which`). In the last one's it returns true;
 // vs, vm - four roots to a lane, as memory held them when the kernel started - then hold the new ones where
-// the plan has the root's bit. The roots are requested together with the counter's answer, on the chance that this is the
-// last workgroup and that the others' stores have arrived: then one trip is all it takes.
-__device__ __forceinline__ bool meet(float* maxp, uint32_t turn, uint32_t which, float root_s, float root_m, uint32_t lane,
+// the plan has the root's bit. (Two trips to memory: the counter's answer, which the compiler waits for where one lane asks, and
+// the roots, more where stores are still on their way.)
+__device__ __forceinline__ bool meet(float* maxp, uint32_t* err, uint32_t turn, uint32_t which, float root_s, float root_m, uint32_t lane,
                                      const MeetPlan& p, float4& vs, float4& vm) {
     const uint32_t changed = p.changed;
     Meet* const m = meet_of(maxp);
@@ -85,14 +103,14 @@ __device__ __forceinline__ bool meet(float* maxp, uint32_t turn, uint32_t which,
     if (p.of_group) {  // uniform
         uint32_t* const counter = m->group[which / kMeetGroup];
         if (lane == 0) before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)before) != p.of_group - 1) return false;
+        if (!meet_last((uint32_t)__builtin_amdgcn_readfirstlane((int)before), p.of_group)) return false;
         if (lane == 0) *counter = 0;  // ready for the next launch
     }
     if (lane == 0) {
         before = __hip_atomic_fetch_add(&m->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     float s[4] = {vs.x, vs.y, vs.z, vs.w}, t[4] = {vm.x, vm.y, vm.z, vm.w};
-    for (;;) {
+    for (uint32_t looks = 1;; ++looks) {
         unsigned long long a[4], b[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
@@ -102,24 +120,29 @@ __device__ __forceinline__ bool meet(float* maxp, uint32_t turn, uint32_t which,
                 b[c] = __hip_atomic_load(&m->root[4 * lane + c][1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
-        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)before) != p.count - 1) return false;
+        if (!meet_last((uint32_t)__builtin_amdgcn_readfirstlane((int)before), p.count)) return false;
         bool open = false;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             if (changed >> c & 1u) {
-                open = open || (uint32_t)(a[c] >> 32) != tag || (uint32_t)(b[c] >> 32) != tag;
+                open = open || !meet_here(a[c], tag) || !meet_here(b[c], tag);
                 s[c] = __uint_as_float((uint32_t)a[c]);
                 t[c] = __uint_as_float((uint32_t)b[c]);
             }
         }
         if (!__any(open)) break;
+        if (looks == kMeetLooks) {
+            const float was_s[4] = {vs.x, vs.y, vs.z, vs.w}, was_m[4] = {vm.x, vm.y, vm.z, vm.w};
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (!meet_here(a[c], tag) || !meet_here(b[c], tag)) s[c] = was_s[c], t[c] = was_m[c];
+            if (lane == 0) atomicOr(err, MRB_DERR_OVERLAP);
+            break;
+        }
     }
     vs = make_float4(s[0], s[1], s[2], s[3]);
     vm = make_float4(t[0], t[1], t[2], t[3]);
-    if (lane == 0) {  // ready for the next launch
-        m->arrived = 0;
-        m->turn = tag;
-    }
+    if (lane == 0) meet_over(m, tag);
     return true;
 }
 

@@ -177,25 +177,30 @@ __global__ __launch_bounds__(kWG) void k_push_many(float* sum, float* mn, float*
     if (!kAlone) {
         if (threadIdx.x == 0) s_before = before;
         lds_barrier();
-        if (s_before != groups - 1) return;  // uniform
+        if (!meet_last(s_before, groups)) return;  // uniform
     }
     if (takes && !kAlone) {
-        for (;;) {
+        for (uint32_t looks = 1;; ++looks) {
             bool open = false;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) open = open || (uint32_t)(a[c] >> 32) != tag || (uint32_t)(b[c] >> 32) != tag;
+            for (int c = 0; c < 4; ++c) open = open || !meet_here(a[c], tag) || !meet_here(b[c], tag);
             if (!__any(open)) break;
+            if (looks == kMeetLooks) {
+                if (lane == 0) atomicOr(err_before(maxp), MRB_DERR_OVERLAP);
+                break;
+            }
             request();
         }
     }
-    if (threadIdx.x == 0 && !kAlone) {  // ready for the next launch
-        m->arrived = 0;
-        m->turn = tag;
+    if (!kAlone) {
+        lds_barrier();  // every wave has the roots that it waited for
+        if (threadIdx.x == kWG - 1) meet_over(m, tag);  // (of the wave that waits for none)
     }
     if (powers) {
         float largest = 0.0f;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) largest = fmaxf(largest, __uint_as_float((uint32_t)a[c]));
+        for (int c = 0; c < 4; ++c)
+            if (meet_here(a[c], tag)) largest = fmaxf(largest, __uint_as_float((uint32_t)a[c]));
         largest = wave_max(largest);
         // (every leaf that takes the running max as it was has been written)
         if (lane == 0 && largest > 0.0f) raise_max(maxp, largest);
@@ -205,7 +210,7 @@ __global__ __launch_bounds__(kWG) void k_push_many(float* sum, float* mn, float*
         float* const m4[4] = {&vm[0].x, &vm[0].y, &vm[0].z, &vm[0].w};
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            if (up * kBlockNodes + 4 * lane + c - t0 < tiles) {
+            if (up * kBlockNodes + 4 * lane + c - t0 < tiles && meet_here(a[c], tag) && meet_here(b[c], tag)) {
                 *s4[c] = __uint_as_float((uint32_t)a[c]);
                 *m4[c] = __uint_as_float((uint32_t)b[c]);
             }

@@ -245,7 +245,7 @@ __device__ __forceinline__ void range_one(const int64_t* __restrict__ indices, c
     run_parents(trees, w - kRoundLevels, root0, lane, lane < tiles, cs, cm);
     if (top == 0) return;
     // and from the runs' to the tree's
-    if (!meet(maxp, turn, run, cs, cm, lane, plan, vs, vm)) return;
+    if (!meet(maxp, err, turn, run, cs, cm, lane, plan, vs, vm)) return;
     tile_parents(trees, top, 1u << top, lane, 4 * lane < (1u << top), vs, vm);
 }
 
