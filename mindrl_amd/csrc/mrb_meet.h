@@ -35,7 +35,7 @@ constexpr uint32_t kMeetLooks = 1u << 16;
 constexpr int kMeetBehindMaxp = 64;
 struct Meet {
     uint32_t arrived;  // of the launch in progress
-    uint32_t turn;     // launches so far
+    uint32_t turn;     // launches so far, of a lap of 2^32 - 1
     uint32_t pad[30];
     uint32_t group[kMeetMost / kMeetGroup][32];  // as `arrived`, of the workgroups of a group; a line each
     unsigned long long root[kMeetMost][2];   // launch number << 32 | bits: sum, minimum
@@ -44,7 +44,8 @@ struct Meet {
 
 __device__ __forceinline__ Meet* meet_of(float* maxp) { return reinterpret_cast<Meet*>(reinterpret_cast<char*>(maxp) + kMeetBehindMaxp); }
 
-// The number of launches before this one (requested when a kernel starts: the last workgroup moves it on).
+// The number of launches before this one; its own is one more, never 0, which is what a word that no launch of the lap has
+// written holds (requested when a kernel starts: the last workgroup moves it on).
 __device__ __forceinline__ uint32_t meet_turn(float* maxp) {
     return __hip_atomic_load(&meet_of(maxp)->turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -56,6 +57,11 @@ __device__ __forceinline__ bool meet_here(unsigned long long word, uint32_t tag)
 __device__ __forceinline__ void meet_over(Meet* m, uint32_t tag) {
     m->arrived = 0;
     m->turn = tag;
+    if (__builtin_expect(tag == 0xffffffffu, 0)) {  // the lap's last: its numbers come again
+        m->turn = 0;
+#pragma clang loop unroll(disable)
+        for (int r = 0; r < kMeetMost; ++r) m->root[r][0] = m->root[r][1] = m->largest[r] = 0;
+    }
 }
 
 // Who meets: a bit for each of a lane's four roots that changes - the same in every workgroup -, and, worked out from them by

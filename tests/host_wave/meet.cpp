@@ -112,11 +112,24 @@ void missing_root() {
     }
 }
 
+// Launches around the last of the 2^32 numbers, on words that the lap before left: none holds a later launch's number.
+void last_number() {
+    for (int lap = 0; lap < 40; ++lap) {
+        Buffer b;
+        b.words.meet.turn = 0xfffffffdu;
+        if (lap % 2)
+            for (uint32_t r = 0; r < 256; ++r) b.words.meet.root[r][0] = b.words.meet.root[r][1] = b.words.meet.largest[r] = (uint64_t)(1 + r % 4) << 32;
+        for (int k = 1; k < 8; ++k) CHECK(launch(b, some(k < 6 ? 2 + (uint32_t)lap : 120), k) == 1, "launch %d", k);
+        CHECK(at_rest(b.words.meet) && b.words.err[0] == 0, "lap %d", lap);
+    }
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "launches") launches();
     else if (what == "any_count") any_count();
     else if (what == "missing_root") missing_root();
+    else if (what == "last_number") last_number();
     else return 2;
     printf("%d wrong\n", wrong);
     return wrong != 0;
