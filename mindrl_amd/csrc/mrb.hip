@@ -851,10 +851,11 @@ bool takes_range(const Per& b, int64_t n) {
     return !takes_range_one(b, n) && n <= most;
 }
 
-// Where one workgroup's update alone (k_tree_wg) is faster than that, us: 13 levels, 1 / 64 / 96 / 128 entries 4.3 / 4.6 / 4.8 /
-// 5.0 against 4.4 / 4.8 / 4.8 / 4.8; 14 levels 4.3 / 4.6 / 4.9 / 5.1 against 4.4 / 4.8 / 4.9 / 4.9. (12 levels, 1 / 64 / 384: 4.4
-// / 4.5 / 5.2 against 4.3 / 4.5 / 5.0.)
-bool takes_wg_rather(const Per& b, int64_t n) { return (b.depth == 13 || b.depth == 14) && n <= 96; }
+// Where one workgroup's update alone (k_tree_wg) is faster than that. 1 / 16 / 64 / 96 / 128 entries, us, it against runs: 10 levels
+// 3.5 / 3.5 / 3.5 / 3.6 / 3.6 against 3.2 / 3.4 / 3.4 / 3.4 / 3.4; 11 levels 3.8 / 3.8 / 3.8 / 3.9 / 3.9 against 3.2 / 3.9 / 4.0 / 4.0 / 4.0; 12 levels
+// 4.1 / 4.2 / 4.3 / 4.6 / 4.7 against 4.4 / 4.7 / 4.7 / 4.7 / 4.7. 1 / 64 / 96 / 128: 13 levels 4.1 / 4.4 / 4.6 / 4.8 against 4.6 / 4.7 / 4.7 / 4.7; 14
+// levels 4.1 / 4.4 / 4.7 / 4.9 against 4.5 / 4.7 / 4.7 / 4.8.
+bool takes_wg_rather(const Per& b, int64_t n) { return b.depth >= 12 && b.depth <= kWgMaxDepth && n <= 96; }
 
 // update_priorities on buffer b with `powered` (device f32[n]) as the scratch that holds the entries'
 // p^alpha between the stamp pass and the leaf writes. Allocates nothing.
