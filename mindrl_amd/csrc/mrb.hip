@@ -775,15 +775,21 @@ void fill_zero(void* p, size_t bytes, hipStream_t s) {
 }
 
 // A push whose leaf tiles are rebuilt by several workgroups, or whose powers one shares out over its threads (k_push_many): with
-// priorities always; without, one tile (us, k_push_run / this: 3.6 / 3.3) or eight and more (1024 rows 4.2 / 4.7, 1500 4.5 / 4.8,
-// 2048 4.9 / 4.8, 3000 5.4 / 4.8: up to seven the roots' meeting costs more than sharing the tiles out saves), or a copy of more than
-// kManyCopy workgroups, which waits for k_push_run's large ones (300 rows of 28 KB 9.3 / 4.9, 1000 18.2 / 10.9).
-constexpr int64_t kManyLeastTiles = 8;
+// priorities always; without, one tile (us, k_push_run / this: 3.6 / 3.3), more than k_push_run takes, or on more than 16 levels
+// twelve and more: up to there, and on trees with one tile above the leaf tiles, the roots' meeting costs more than sharing the
+// tiles out saves (1024 / 2048 / 2560 / 3072 / 3584 rows of 37 bytes, 14 levels 3.1 / 3.4 / 3.4 / 3.6 / 3.6 against 3.8 / 3.8 / 3.8 / 3.8 / 3.9, 16
+// levels 3.2 / 3.4 / 3.5 / 3.6 / 3.7 against 4.0 each, 17 levels 3.9 / 4.4 / 4.5 / 4.9 / 5.0 against 4.5 / 4.6 / 4.6 / 4.6 / 4.6, 20 levels
+// 4.1 / 4.6 / 4.8 / 5.1 / 5.2 against 4.8 / 4.9 / 4.9 / 4.9 / 4.9). Or a copy of more than kManyCopy workgroups, which waits for
+// k_push_run's large ones (300 rows of 28 KB 9.3 / 4.9, 1000 18.2 / 10.9).
+constexpr int64_t kManyLeastTiles = 12;
+constexpr int kManyLeastDepth = 17;
 constexpr uint32_t kManyCopy = 1024;
 bool takes_push_many(const Per& b, int64_t first, int64_t n, bool with_priorities, uint32_t copy_blocks) {
     if (b.device_counters || !b.fused || b.nrounds == 0 || first + n > b.rows.capacity) return false;
     const int64_t tiles = (first + n - 1) / kBlockNodes - first / kBlockNodes + 1;
-    return (with_priorities || tiles == 1 || tiles >= kManyLeastTiles || copy_blocks > kManyCopy) && tiles <= kManyMostTiles;
+    if (tiles > kManyMostTiles) return false;
+    return with_priorities || tiles == 1 || tiles > kRunWaves || (tiles >= kManyLeastTiles && b.depth >= kManyLeastDepth) ||
+           copy_blocks > kManyCopy;
 }
 
 // Starts a new tree-update epoch. Epochs tag stamps and dirty words so that

@@ -33,6 +33,7 @@ T = 256
 CASES = [  # capacity, first slot, rows
     (5000, 0, 2), (5000, 100, 156), (5000, 100, 157), (5000, 255, 2), (5000, 4999, 1), (5000, 4000, 1000), (5000, 4001, 1000),
     (5000, 0, 5000), (4097, 1, 4096), (100_000, 7 * T, 7 * T), (100_000, 7 * T, 8 * T), (100_000, 7 * T + 1, 8 * T),
+    (100_000, 7 * T, 11 * T), (100_000, 7 * T, 12 * T), (60_000, 5, 12 * T), (60_000, T, 16 * T), (60_000, T + 1, 16 * T),
     (100_000, 65_536 - T, 2 * T), (100_000, 65_535, 2), (100_000, 60_000, 40_000), (100_000, 3, 160 * T), (100_000, 3, 159 * T),
     (200_000, 5, 256 * T), (200_000, 0, 256 * T), (200_000, 5, 255 * T), (200_000, 65_536 + 9, 97 * T),
     ((1 << 24) + 70_000, (1 << 24) - 300, 2), ((1 << 24) + 70_000, (1 << 24) - 300, 600), ((1 << 24) + 70_000, (1 << 24) - 2000, 65_000),
