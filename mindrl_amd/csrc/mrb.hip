@@ -493,8 +493,8 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
         const hipError_t e = launch_short_gather(r.table, io, t.nfields, indices, count, seed, calls, n, blocks, out_indices != nullptr, s);
         return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch k_short_gather: %s", hipGetErrorString(e));
     }
-    hipLaunchKernelGGL(k_rows_gather, dim3(blocks, (uint32_t)t.nfields), dim3(kWG), 0, s, t, r.capacity, count, indices, fixed_slot,
-                       seed, calls, out_indices, err, blocks);
+    hipLaunchKernelGGL(k_rows_gather, dim3(blocks, (uint32_t)t.nfields), dim3(kWG), 0, s, indices, fixed_slot, seed, calls,
+                       count, out_indices, err, r.capacity, blocks, t);
     LAUNCH_CHECK("k_rows_gather");
     return MRB_OK;
 }

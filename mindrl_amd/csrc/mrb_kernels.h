@@ -18,9 +18,10 @@ constexpr int kTopWG = 1024;
 
 __global__ __launch_bounds__(kWG) void k_rows_put(PutArgs p) { rows_put_part(p, blockIdx.x, p.blocks); }
 
-__global__ __launch_bounds__(kWG) void k_rows_gather(IoTable t, int64_t capacity, int64_t count, const int64_t* __restrict__ indices,
-                                                     int64_t fixed_slot, uint64_t seed, uint64_t calls, int64_t* __restrict__ out_indices,
-                                                     uint32_t* __restrict__ err, uint32_t blocks) {
+// (The leading plain parameters are preloaded into scalar registers.)
+__global__ __launch_bounds__(kWG) void k_rows_gather(const int64_t* __restrict__ indices, int64_t fixed_slot, uint64_t seed, uint64_t calls,
+                                                     int64_t count, int64_t* __restrict__ out_indices, uint32_t* __restrict__ err,
+                                                     int64_t capacity, uint32_t blocks, IoTable t) {
     gather_body(FullRows{t}, capacity, count, indices, fixed_slot, seed, calls, out_indices, err, blocks);
 }
 
