@@ -179,18 +179,26 @@ __global__ __launch_bounds__(kWG) void k_push_many(float* sum, float* mn, float*
         lds_barrier();
         if (!meet_last(s_before, groups)) return;  // uniform
     }
+    bool late = false;
     if (takes && !kAlone) {
-        for (uint32_t looks = 1;; ++looks) {
+        for (uint32_t looks = 0; looks < kMeetLooks; ++looks) {
             bool open = false;
 #pragma unroll
             for (int c = 0; c < 4; ++c) open = open || !meet_here(a[c], tag) || !meet_here(b[c], tag);
-            if (!__any(open)) break;
-            if (looks == kMeetLooks) {
-                if (lane == 0) atomicOr(err_before(maxp), MRB_DERR_OVERLAP);
-                break;
-            }
+            late = __any(open);
+            if (!late) break;
             request();
         }
+    }
+    if (__builtin_expect(late, 0)) {  // what did not come stays as it was (see mrb_meet.h); a look at each root below would cost every push 0.1 us
+        const float was_s[4] = {vs[0].x, vs[0].y, vs[0].z, vs[0].w}, was_m[4] = {vm[0].x, vm[0].y, vm[0].z, vm[0].w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (meet_here(a[c], tag) && meet_here(b[c], tag)) continue;
+            a[c] = powers ? 0 : __float_as_uint(was_s[c]);
+            b[c] = __float_as_uint(was_m[c]);
+        }
+        if (lane == 0) atomicOr(err_before(maxp), MRB_DERR_OVERLAP);
     }
     if (!kAlone) {
         lds_barrier();  // every wave has the roots that it waited for
@@ -199,8 +207,7 @@ __global__ __launch_bounds__(kWG) void k_push_many(float* sum, float* mn, float*
     if (powers) {
         float largest = 0.0f;
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (meet_here(a[c], tag)) largest = fmaxf(largest, __uint_as_float((uint32_t)a[c]));
+        for (int c = 0; c < 4; ++c) largest = fmaxf(largest, __uint_as_float((uint32_t)a[c]));
         largest = wave_max(largest);
         // (every leaf that takes the running max as it was has been written)
         if (lane == 0 && largest > 0.0f) raise_max(maxp, largest);
@@ -210,7 +217,7 @@ __global__ __launch_bounds__(kWG) void k_push_many(float* sum, float* mn, float*
         float* const m4[4] = {&vm[0].x, &vm[0].y, &vm[0].z, &vm[0].w};
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            if (up * kBlockNodes + 4 * lane + c - t0 < tiles && meet_here(a[c], tag) && meet_here(b[c], tag)) {
+            if (up * kBlockNodes + 4 * lane + c - t0 < tiles) {
                 *s4[c] = __uint_as_float((uint32_t)a[c]);
                 *m4[c] = __uint_as_float((uint32_t)b[c]);
             }
