@@ -846,15 +846,13 @@ bool takes_range_one(const Per& b, int64_t n) {
 
 // Whether an update goes by runs of leaves in two launches (launch_tree_range). Against what it would take
 // otherwise, us per call, before / by runs:
-//   most entries    10 levels, 2048 / 4096: 7.7 / 8.4 against 7.7 / 9.3; 12 levels, 8192 / 16,384: 10.0 / 11.4 against
-//                   9.6 / 13.8; 14 levels, 16,384 / 32,768: 11.7 / 12.5 against 11.2 / 16.7; 20 levels 14.4 / 15.4 against
+//   most entries    12 levels, 8192 / 16,384: 10.0 / 11.4 against 9.6 / 13.8; 14 levels, 16,384 / 32,768: 11.7 / 12.5 against 11.2 / 16.7; 20 levels 14.4 / 15.4 against
 //                   14.1 / 18.7; 22 levels, 8192 / 16,384: 16.1 / 17.7 against 16.0 / 21.0.
 //   deepest tree    23 and 24 levels leave more than a tile above the runs and bring many runs without an entry: 2048
 //                   entries 14.9 / 15.9 against 14.9 / 23.3.
 bool takes_range(const Per& b, int64_t n) {
-    if (!b.fused || b.depth < 10 || b.depth > 22) return false;
-    const int64_t most = b.depth <= 11 ? 2048 : b.depth == 12 || b.depth == 22 ? 8192 : 16384;
-    return !takes_range_one(b, n) && n <= most;
+    if (!b.fused || b.depth < 12 || b.depth > 22) return false;
+    return !takes_range_one(b, n) && n <= (b.depth == 12 || b.depth == 22 ? 8192 : 16384);
 }
 
 // Where one workgroup's update alone (k_tree_wg) is faster than that. 1 / 16 / 64 / 96 / 128 entries, us, it against runs: 10 levels

@@ -20,7 +20,7 @@ struct RangePush {
 
 // Levels of the runs that a launch for n entries divides a tree of `depth` (8 to 22) levels into.
 int range_one_levels(int depth, int64_t n);
-// indices and priorities of n entries (1 .. kOneMostEntries) -> the trees and the running max.
+// indices and priorities of n entries (1 .. kOneMostEntries; more than 1024 on trees of at most 20 levels) -> the trees and the running max.
 hipError_t launch_range_one(const int64_t* indices, const float* priorities, int64_t n, float* sum, float* mn, float* maxp,
                             int64_t capacity, int depth, float alpha, hipStream_t s);
 // The same (of up to 1024 entries) and then a push whose row copy is `put`, in one launch. With priorities the slots must lie in one run.

@@ -286,8 +286,10 @@ hipError_t launch_range_one(const int64_t* indices, const float* priorities, int
                             int64_t capacity, int depth, float alpha, hipStream_t s) {
     const int w = range_one_levels(depth, n);
     auto* kernel = w <= 10 ? k_range_one<10, kOneFew> : w <= 12 ? k_range_one<12, kOneFew> : w == 13 ? k_range_one<13, kOneFew> : k_range_one<14, kOneFew>;
-    if (n > kOneFew * kOneWG)
-        kernel = w <= 10 ? k_range_one<10, kOneMany> : w <= 12 ? k_range_one<12, kOneMany> : w == 13 ? k_range_one<13, kOneMany> : k_range_one<14, kOneMany>;
+    if (n > kOneFew * kOneWG) {
+        if (w > 12) return hipErrorInvalidValue;  // (more than 20 levels: not taken, see takes_range_one)
+        kernel = w <= 10 ? k_range_one<10, kOneMany> : k_range_one<12, kOneMany>;
+    }
     hipLaunchKernelGGL(kernel, dim3(runs_of(capacity, w)), dim3(kOneWG), 0, s, indices, priorities, sum, mn, maxp, (int)n, (int)capacity,
                        depth | w << 8, alpha);
     return hipGetLastError();
