@@ -1,12 +1,13 @@
-"""Pushes whose tiles several workgroups rebuild, against the kernels that take the same call where its matrices lie too far apart
-to be given as distances (more than 2^31 bytes at an odd address): trees, running max, rows and flags, bit for bit. Runs of 1 to 257
+"""Pushes whose tiles several workgroups rebuild, against the oracle (buffers of up to 200,000 slots) and against the kernels that take
+the same call where its matrices lie too far apart to be given as distances (more than 2^31 bytes at an odd address): trees, running
+max, rows and flags, bit for bit. Runs of 1 to 257
 tiles, aligned and not, up to the ring's end and around it, across the boundaries of the tiles 8 and 16 levels up; some priorities
 invalid."""
 import numpy as np
 import pytest
 import torch
 
-from gpu_util import bits, t2n
+from gpu_util import assert_tree_equal, bits, t2n
 
 pytestmark = pytest.mark.gpu
 
@@ -44,7 +45,9 @@ CASES = [  # capacity, first slot, rows
 @pytest.mark.parametrize("cap,first,n", CASES)
 def test_push(cap, first, n, big):
     from mindrl_amd.core import PriorityReplayBuffer
+    from oracle import orc
     a, b = (PriorityReplayBuffer(0.7, cap, 8, [(1,), (3,)], [torch.int32, torch.uint8], seed0=5) for _ in range(2))
+    c = orc.OraclePER(0.7, cap, [(1,), (3,)], [np.int32, np.uint8]) if cap <= 200_000 else None
     rng = np.random.default_rng(first + n)
     for how in range(3):
         # up to the slot `first`: the ring's head is a multiple of the capacity away after each round
@@ -54,6 +57,9 @@ def test_push(cap, first, n, big):
                 x = torch.arange(lead, device="cuda")
                 buf.insert((x % 1000)[:, None].int(), (x[:, None] % torch.tensor([3, 5, 7], device="cuda")).to(torch.uint8),
                            priorities=(x % 97).float() + 0.5)
+        if c is not None and lead:
+            x = np.arange(lead)
+            c.push([(x % 1000)[:, None].astype(np.int32), (x[:, None] % np.array([3, 5, 7])).astype(np.uint8)], lead, (x % 97 + 0.5).astype(np.float32))
         wide = torch.from_numpy(rng.integers(0, 1 << 30, (n, 1), dtype=np.int32)).cuda()
         small = torch.from_numpy(rng.integers(0, 256, (n, 3), dtype=np.uint8)).cuda()
         far0, far1 = big[: 4 * n].view(torch.int32).view(n, 1), big[(1 << 31) + 4099 : (1 << 31) + 4099 + 3 * n].view(n, 3)
@@ -72,6 +78,16 @@ def test_push(cap, first, n, big):
         for x, y in zip(a.storage(), b.storage()):
             assert np.array_equal(t2n(x), t2n(y)), how
         assert flags(a) == flags(b), how
+        if c is not None:
+            head, values = c.head, None if pr is None else t2n(pr)
+            c.push([t2n(wide), t2n(small)], n)
+            if pr is not None:  # (a row whose priority is invalid takes the running max)
+                ok = (values >= 0) & (values <= 3e38)
+                c.update(((head + np.arange(n)) % cap)[ok], values[ok])
+            assert_tree_equal(a, c, how)
+            assert np.float32(a.max_priority) == np.float32(c.max_priority), how
+            for k, x in enumerate(a.storage()):
+                assert np.array_equal(t2n(x), c.field(k).reshape(x.shape)), how
 
 
 @pytest.mark.parametrize("n", [3, 290, 700, 9000])

@@ -1,12 +1,12 @@
 """Calls whose launches take their tables from device memory and the caller's matrices as distances, against the same calls over
 matrices that cannot be given so (more than 2^31 bytes apart at an odd address): rows, trees, running max, outputs and flags,
-bit for bit. Rows from 1 byte to several granules, aligned and not, packed, from host memory and from views that begin anywhere;
+bit for bit; the rows and trees of the pushes against the oracle, too. Rows from 1 byte to several granules, aligned and not, packed, from host memory and from views that begin anywhere;
 pushes of one row to many, around the ring's end, with valid and invalid priorities; gathers by generator and by index."""
 import numpy as np
 import pytest
 import torch
 
-from gpu_util import bits, random_rows, t2n
+from gpu_util import assert_tree_equal, bits, random_rows, t2n
 
 pytestmark = pytest.mark.gpu
 
@@ -83,7 +83,9 @@ def test_pushes(name, cap, packed, big):
     from mindrl_amd.core import PriorityReplayBuffer
     shapes, types = SETS[name]
     tt = [torch.from_numpy(np.zeros(1, t)).dtype for t in types]
+    from oracle import orc
     a, b = (PriorityReplayBuffer(0.7, cap, 8, shapes, tt, seed0=5, packed_rows=packed) for _ in range(2))
+    c = orc.OraclePER(0.7, cap, shapes, types)
     rng = np.random.default_rng(2)
     for step, n in enumerate((cap // 2 + 1, 1, 3, 63, 256, cap, 1, 200, 257, 1, 1024, 4000, 4096, cap - 1, 5)):
         n = min(n, cap)
@@ -110,25 +112,52 @@ def test_pushes(name, cap, packed, big):
                 except Exception as e:
                     bad.append(str(e))
             assert bad[0] == bad[1], what
+            head = c.head
+            c.push(rows, n)
+            if pr is not None:  # (a row whose priority is invalid takes the running max)
+                values = t2n(pr)
+                ok = (values >= 0) & (values <= 3e38)
+                c.update(((head + np.arange(n)) % cap)[ok], values[ok])
+            assert_tree_equal(a, c, what)
+            assert np.float32(a.max_priority) == np.float32(c.max_priority), what
+            same_rows(a.storage(), [torch.from_numpy(c.field(k)) for k in range(len(shapes))], what)
 
 
 def test_replays():
-    """A recorded gather and a recorded insert, on other contents than they were recorded with."""
+    """A recorded gather and a recorded insert, on other contents than they were recorded with. (A replayed insert writes the slots
+    that it was recorded for.)"""
     from mindrl_amd.core import UniformReplayBuffer
-    u = UniformReplayBuffer(64, 128, [(3,)], [torch.float32], seed=1)
-    rows = torch.arange(384, dtype=torch.float32, device="cuda").view(128, 3)
-    u.insert([rows])
+    u = UniformReplayBuffer(64, 128, [(3,), (5,)], [torch.float32, torch.uint8], seed=1)
+    rows = [torch.arange(384, dtype=torch.float32, device="cuda").view(128, 3), torch.arange(640, device="cuda").to(torch.uint8).view(128, 5)]
+    u.insert(rows)
     idx = torch.arange(64, device="cuda")
-    out = [torch.empty(64, 3, device="cuda")]
+    out = [torch.empty(64, 3, device="cuda"), torch.empty(64, 5, dtype=torch.uint8, device="cuda")]
+    new = [torch.zeros(7, 3, device="cuda"), torch.zeros(7, 5, dtype=torch.uint8, device="cuda")]
     u.sample(indices=idx, out=out)
+    u.insert([r[:124] for r in rows])  # (so that the recorded one goes around the ring's end)
     torch.cuda.synchronize()
-    g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
+    slots = (124 + torch.arange(7, device="cuda")) % 128
+    gather, insert = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(gather):
         u.sample(indices=idx, out=out)
+    with torch.cuda.graph(insert):
+        u.insert(new)
+    want = [x.clone() for x in u.buffer]  # (recording writes nothing)
+    head = 131 % 128
     for k in range(4):
         idx.copy_((torch.arange(64, device="cuda") * 5 + k) % 128)
-        u.insert([rows[k : k + 2] * 0 - k])
-        g.replay()
+        for r, t in zip(new, want):
+            r.copy_(torch.arange(r.numel(), device="cuda").view(r.shape) % 50 + 10 * k)
+            t[slots] = r
+        insert.replay()
+        eager = [rows[0][k : k + 2] * 0 - k, rows[1][k : k + 2] // 2]
+        u.insert(eager)
+        for r, t in zip(eager, want):
+            t[torch.arange(head, head + 2, device="cuda")] = r
+        head += 2
+        gather.replay()
         torch.cuda.synchronize()
-        eager = u.sample(indices=idx)
-        assert torch.equal(out[0], eager[0] if isinstance(eager, (list, tuple)) else eager), k
+        for k2, (x, t, o) in enumerate(zip(u.buffer, want, out)):
+            assert torch.equal(x, t) and torch.equal(o, t[idx]), (k, k2)
+        for x, o in zip(u.sample(indices=idx), out):
+            assert torch.equal(x, o), k
