@@ -103,8 +103,12 @@ int mrb_version(void);
  *                  `capacity` rows, a sample at most 65,536 (its slots are drawn into a device array that
  *                  overlapping sample / get_item calls on one handle would share), mrb_urb_append_from is
  *                  refused, and mrb_urb_state, mrb_urb_reset, mrb_urb_seed and the checkpoint calls wait.
- *   "fused_rebuild" prioritized buffers: 1 (default) = an update of <= 1024 entries on a tree of at most 22 levels (<= 4096
- *                  on one of at most 20) or a push under <= 256 leaf tiles (16 around the ring's end) rebuilds the tree in one launch; 0 = one launch per round */
+ *   "fused_rebuild" prioritized buffers: 1 (default) = the tree is rebuilt in one launch by an update of <= 1024 entries on a tree
+ *                  of 8 to 22 levels (<= 4096 on one of at most 20; <= 384 on a smaller tree, <= 64 on one of 23 to 25), by a push
+ *                  of one row, under <= 16 leaf tiles (of 256 slots each) or on a tree of at most 12 levels; and under <= 256 leaf
+ *                  tiles where it does not go around the ring's end, the counters are on the host and the matrices are at
+ *                  most 8, each less than 2^31 units from the first (a unit: the largest power of two, up to 4096, that
+ *                  divides all the distances); 0 = one launch per round */
 /* Library-wide default, set with handle 0 and taken by buffers created afterwards:
  *   "packed_rows"  N > 0: a buffer whose packed row - every field at the next multiple of its own copy granule
  *                  (the largest power of two <= 16 that divides its size), the row padded to the widest granule -

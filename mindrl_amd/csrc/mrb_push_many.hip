@@ -22,11 +22,11 @@ struct Trees {
 // workgroup per tile a thread takes one, 0.35 us, so with priorities kTiles is 1 - until so many workgroups raise the one counter
 // that it costs more (11 ns each: 65 tiles 5.9 against 7.0 us with four tiles to a workgroup, 129 6.7 / 7.2, 254 8.4 / 7.7). A single
 // tile (kAlone) meets nobody. In front of this one workgroup did it all up to 16 tiles (k_push_run), beyond that launches per eight
-// levels (k_tree_update, k_tree_top). Device time per call, us, before / now, plain and with priorities (i4;f4 rows, 2^24 leaves):
-//   2 rows      4.0 / 3.3   5.3 / 3.6      4096 rows   9.0 / 4.9   10.8 / 5.5
-//   200 rows    4.0 / 3.9   5.4 / 4.7      32768 rows  9.5 / 5.3   12.0 / 6.7
-//   1000 rows   4.5 / 4.3   6.4 / 5.2      65000 rows  9.8 / 5.9   13.8 / 7.8
-// (524-byte rows, 2^21 leaves: 4096 rows 7.0 / 5.0 and 8.8 / 5.6, 16384 rows 12.6 / 5.9 and 15.3 / 7.0.)
+// levels (k_tree_update, k_tree_top). Device time per call, us, before / now (i4;f4 rows, 2^24 leaves):
+//   with priorities  2 rows 5.4 / 3.5, 200 5.5 / 4.7, 1000 6.5 / 5.2, 4096 10.9 / 5.6, 32768 12.3 / 6.9, 65000 14.1 / 7.8
+//   plain            2 rows 3.9 / 3.2 (where they lie under one tile), 4096 9.1 / 4.8, 32768 9.6 / 5.3, 65000 10.1 / 5.9
+// (524-byte rows, 2^21 leaves: 4096 rows plain 5.6 / 4.7 and with priorities 8.8 / 5.5, 16384 rows 12.8 / 5.7 and 15.1 / 6.8.) Plain pushes
+// in between are k_short_push_run's: the rule, with both sides measured, is at takes_push_many (mrb.hip).
 //   plan: depth | columns of workgroups that rebuild tiles << 8; those behind them, (x, y), copy rows of field y
 // ---------------------------------------------------------------------------
 constexpr uint32_t kManyApart = 160;

@@ -23,7 +23,8 @@ struct Trees {
 // that every workgroup reads all indices (out of its L2: 16 KB for 2048 entries), which is why larger calls keep the
 // stamp pass (the rule, with both sides measured, is at takes_range).
 // A call is bound by its chain of trips - indices, priorities of a run's own, tiles, then the second launch's tile -, not
-// by bytes. 2048 entries on 2^21 leaves 14.7 -> 9.1 us, 1024 on 2^17 9.4 -> 6.7, 250 on 2^19 7.5 -> 6.8.
+// by bytes. 2048 entries on 2^21 leaves 14.7 -> 8.6 us. (Up to 1024 entries, up to 4096 on at most 20 levels, one launch does the same:
+// k_range_one.)
 // ---------------------------------------------------------------------------
 // (no argument for what the kernel can tell: see PutArgs::threads)
 __host__ __device__ constexpr int range_threads(int64_t n) { return n > 4096 ? 1024 : 512; }  // (256: 0.3 to 1.5 us more)

@@ -27,15 +27,15 @@ constexpr int kOneHeld = 2;                        // changed tiles of a wave th
 // on their way while the powers are taken and the leaves elected), the roots' meeting (0.9 us; with one run there is none), and
 // with more than a thousand entries the looking them over. us per call queued behind a busy device, the kernels before (two
 // launches; one wave along the paths; one workgroup) / this:
-//   64 entries   2^10 leaves 3.7 / 3.3, 2^12 4.5 / 4.7, 2^16 7.6 / 5.0, 2^20 8.9 / 5.4, 2^22 9.7 / 6.0
-//   256 entries  2^10 3.9 / 3.4, 2^14 6.5 / 5.0, 2^16 6.1 / 5.2, 2^19 6.7 / 5.5, 2^21 7.0 / 5.9
-//   512 entries  2^14 6.3 / 5.1, 2^17 6.7 / 5.5, 2^20 7.2 / 6.1; 1024  2^14 6.6 / 5.3, 2^17 6.8 / 5.8, 2^20 7.7 / 7.0
-//   2048 entries 2^10 7.8 / 5.9, 2^12 7.2 / 6.4, 2^14 6.7 / 6.3, 2^18 7.4 / 7.2, 2^20 8.3 / 8.5; 4096  2^14 7.1 / 6.9, 2^18 7.9 / 7.6
+//   64 entries   2^10 leaves 3.7 / 3.4, 2^16 7.7 / 5.0, 2^20 9.0 / 5.4, 2^22 9.7 / 6.0
+//   256 entries  2^10 3.9 / 3.4, 2^14 6.5 / 4.9, 2^16 6.2 / 5.3, 2^19 6.8 / 5.6, 2^21 7.0 / 5.8
+//   512 entries  2^14 6.0 / 5.1, 2^17 6.7 / 5.6, 2^20 7.4 / 6.1; 1024  2^14 6.3 / 5.3, 2^17 6.8 / 5.9, 2^20 7.8 / 7.0
+//   2048 entries 2^10 7.7 / 6.6, 2^12 6.9 / 6.4, 2^14 6.6 / 6.3, 2^18 7.5 / 7.2, 2^20 8.6 / 8.5; 4096  2^14 7.0 / 6.8, 2^18 8.0 / 7.5
 // and the host issues one launch instead of two (6.8 -> 4.1 us), which is what bounds a training program's step.
 // kPush: the rows a push of the same call writes come after the entries - slots first_slot .. + nrows - 1 take the running
 // max as the update leaves it, or their own priorities -, in the runs that hold those slots; further workgroups carry the
 // row copy. (Only one workgroup may raise the running max for pushed rows, while others read it: one run with priorities.)
-// 512 entries and 4 rows: 2^14 leaves 9.5 / 5.7, 2^17 8.8 / 6.3, 2^20 9.2 / 7.6; 64 and 1: 2^14 5.8 / 5.1, 2^20 10.3 / 5.9.
+// 512 entries and 4 rows: 2^14 leaves 9.5 / 5.4, 2^17 8.7 / 5.9, 2^20 9.2 / 6.5; 64 and 1: 2^14 5.8 / 5.3, 2^20 10.4 / 5.6.
 // ---------------------------------------------------------------------------
 template <int kLog2, bool kPush, int kPer>  // (kPush: kPer == kOneFew)
 __device__ __forceinline__ void range_one(const int64_t* __restrict__ indices, const float* __restrict__ priorities, float* sum,
