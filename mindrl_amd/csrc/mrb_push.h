@@ -60,7 +60,8 @@ struct UpdateArgs {
 // a launch per eight levels pays a launch, a trip and a rebuild for each. Measured, us per call before and now, plain /
 // with priorities: 64 rows into 2^24 leaves (three launches before) 12.0 / 10.6 and 3.8 / 5.6; 16 rows into 2^20 (one
 // launch that rebuilt the whole top) 4.2 / 6.5 and 3.8 / 5.3; 1024 rows into 2^21 4.8 / 7.4 and 4.3 / 5.6. With 4096
-// priorities the powers of one compute unit are the bound (5.6 / 8.7). The row copy rides along as further workgroups of the
+// priorities the powers of one compute unit are the bound (5.6 / 8.7): k_push_many, which shares them out, takes pushes with
+// priorities where it can (takes_push_many). The row copy rides along as further workgroups of the
 // kernels that call this (k_push_run, k_short_push_run).
 //   threads    of the workgroup
 //   units      leaf tiles from the first slot's on, around the ring's end: waves with work
