@@ -2091,11 +2091,13 @@ static int discounted_return(const float* x, const uint8_t* done, float* end_val
     if (cols > (1ll << 31) || cols > (1ll << 40) / timesteps)
         return fail(MRB_EINVAL, "%lld columns of %lld steps exceed one call (at most 2^31 columns, 2^40 elements)",
                     (long long)cols, (long long)timesteps);
-    // A thread per column needs about 65 ns per step however few the columns (a trip to memory per 32 steps) and
-    // streams at up to 6 TB/s when there are many; chunks through LDS need 11 ns per step and stream at 4.8 TB/s.
-    // Measured, us per column / tiled: [1000, 32768] 79 / 61, [1000, 49152] 86 / 94, [250, 32768] 27 / 21, [100, 30001]
-    // 10.7 / 14.3, [100, 16384] 8.5 / 6.8, [20, 16384] 4.1 / 5.1.
-    const bool per_column = cols > 40960 || (cols > 16384 && timesteps <= 128) || (cols > 8192 && timesteps <= 32);
+    // A thread per column needs about 65 to 100 ns per step however few the columns (a trip to memory per 32 steps) and
+    // streams at up to 6 TB/s when there are many; chunks through LDS need 8 to 11 ns per step and stream at 4.8 TB/s.
+    // Measured, us per column / tiled: [20, 9000] 5.0 / 4.7, [32, 30001] 5.3 / 7.8; [64, 30000] 8.8 / 8.0, [64, 40000] 8.7 / 9.7, [48, 30001] 10.8 /
+    // 8.2; [100, 38000] 14.2 / 10.9, [200, 45000] 26.7 / 22.0, [128, 65536] 16.8 / 21.4, [200, 65536] 27.4 / 29.4; [256, 65536] 31.9 / 32.5, [300, 65536] 41.3 /
+    // 35.0, [1000, 65536] 123 / 113, [256, 80000] 38.0 / 40.5, [1000, 131072] 195 / 247.
+    const int64_t most = timesteps <= 32 ? 8192 : timesteps <= 64 ? 32768 : timesteps < 256 ? 40960 : 65536;
+    const bool per_column = cols > most;
     if (per_column) {
         hipLaunchKernelGGL(k_discounted_return, dim3(grid_exact((uint64_t)cols)), dim3(kWG), 0, s, x, done, end_value, out,
                            timesteps, batch, inner, gamma, kBack ? 1 : 0);

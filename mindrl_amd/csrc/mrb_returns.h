@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "mrb_device.h"
 
 namespace mrb {
@@ -20,37 +22,46 @@ namespace mrb {
 // ---------------------------------------------------------------------------
 
 // Fewer columns, where a thread per column leaves the memory system idle: a workgroup takes kCols columns and walks
-// their steps in chunks of kDrChunk through three LDS buffers, as a pipeline whose stages run at the same time on
-// consecutive chunks:
-//   deposit  the movers (four waves, or eight) put chunk s, requested kDrAhead stages ago, into its LDS buffer ...
-//   request  ... request chunk s + kDrAhead into the registers just emptied (independent, coalesced loads) ...
-//   drain    ... and write chunk s - 2's results from LDS to memory, while ...
-//   recur    ... wave 0 runs the recurrence over chunk s - 1 out of LDS (lane = column).
-// One LDS barrier per stage (lds_barrier: requests and results stay in flight across it).
+// their steps in chunks of kDrChunk through three LDS buffers, as a pipeline. Wave 0 runs the recurrence out of LDS (lane =
+// column) and meets the movers - four waves, or eight - at a barrier in the MIDDLE of every chunk, so that the next chunk's
+// first steps are there, and are read, before it comes to them. Between the barriers in chunks c - 1 and c the movers
+//   take     chunk c - 2's results out of its LDS buffer,
+//   deposit  chunk c + 1, requested kDrAhead stages ago, into that buffer, each mover over what it has itself read there,
+//   request  chunk c + 1 + kDrAhead into the registers just emptied (independent, coalesced loads),
+//   store    and write chunk c - 2's results to memory.
+// (lds_barrier: requests and results stay in flight across it.)
 //
 // What bounds it: for few columns the recurrence, a chain of two dependent operations per step in ONE wave; for many
-// the memory. The chain is kept as short as it can be: a column's steps lie one after the other in LDS, so that one
-// 16-byte read brings four steps' values (one more their factors, one 16-byte write takes the results), and a batch
-// of steps is read while the one before runs (read 15 at a time just before their use, and two LDS accesses a step,
-// a step took 54 cycles: [1000, 4096] 22.9 us, now 14.5; [1000, 32] 24 us, now 11.9, of which the chain alone, with the
-// movers idle, takes 11.2). kCols is small so that a few thousand columns spread over all
+// the memory. A chain in registers alone takes 10 cycles a step; an LDS access of that wave costs it 9 to 20 more, wherever it is
+// put (between the two operations of a step it costs most), so there are few: a column's steps lie one after the other, one 16-byte
+// read brings four steps' values and one more their factors, sixteen steps ahead; and up to sixteen columns to a workgroup it leaves
+// only every fourth result (4 bytes, where four results are 16: 16 cycles a step against 21), from which the movers, who have time, work
+// out the three before. More columns are bound by the movers and the memory: there it leaves all results (at 32 columns with every
+// fourth [2000, 8000] took 32.5 us, with all 30.3). Loads are cached: neighbouring groups on one die share 128-byte lines, and read as
+// streams their second halves came from memory again (13.4 -> 12.5 us at [1000, 4096]). us before / now, forward and backward:
+//   [1000, 4096] 14.3 14.2 / 11.8 11.8, [1000, 32] 12.4 12.9 / 11.2 11.4, [2000, 3001] 27.6 27.7 / 20.9 21.1, [65, 4825] 5.3 5.4 / 4.4 4.5,
+//   [1000, 8192] 17.8 17.5 / 15.8 16.5, [2000, 8000] 28.5 29.1 / 28.4 29.2, [2000, 7501] 40.0 40.5 / 33.4 33.7, [1000, 16384] 30.2 30.8 / 28.7 28.5,
+//   [1011, 204, 3] 14.6 14.6 / 12.2 12.0, [1000, 3000, 3] 25.8 26.1 / 19.4 18.9; [4000, 8192], 300 MB that no cache holds, 57.0 56.0 / 54.4 57.6.
+// kCols is small so that a few thousand columns spread over all
 // compute units, several workgroups to each when there are more. The pad of four floats puts the sixteen columns'
 // 16-byte reads into different banks, and the movers' scalar writes likewise.
 //
-// Every mover issues the SAME number of loads and stores in every stage, without a branch around any of them: a step
-// past the end of the time axis is replaced by the last one (loaded again, stored again with the same value), a
+// Every mover issues the SAME number of loads and stores in every stage but the last, without a branch around any of them: a step
+// past the end of the time axis is replaced by the last one (loaded again, not stored), a
 // column past the last one by a column before it. Only so can the compiler count what is in flight: with a branch per
-// element it would wait for EVERYTHING before each deposit.
+// element, or a way out of the loop in the middle of its three stages, it would wait for EVERYTHING before a deposit.
 //   kQuad   a mover carries four neighbouring columns of one step, one 16-byte load and store (4-byte aligned when
 //           the number of columns is not a multiple of four) and the four flags as one 4-byte load; needs inner == 1
 //           and at least four columns. The last quad is moved back so that it ends with the last column.
 //   else    a mover carries four steps of one column.
 constexpr int kDrChunk = 64;  // steps
-constexpr int kDrAhead = 4;   // chunks on their way from memory at any time
+constexpr int kDrAhead = 3;   // chunks on their way from memory at any time
+constexpr int kDrBuffers = 3;
 constexpr int kDrPitch = kDrChunk + 4;
 
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));      // four floats at any float's address
 typedef uint32_t u32_u __attribute__((aligned(1)));                         // four flags at any address
+#define MRB_GLOBAL __attribute__((address_space(1)))
 
 template <bool kBack, bool kQuad, int kCols, int kMovers>
 __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
@@ -58,9 +69,13 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
     int64_t timesteps, int64_t batch, int64_t inner, float gamma) {
     constexpr int kPer = kDrChunk * kCols / 4 / kMovers;  // groups of four elements of a chunk that a mover carries
     constexpr int kSteps = kDrChunk / kPer;                 // steps the movers cover at once
+    constexpr bool kAll = kCols > 16;                       // the recurrence leaves every result, else every fourth
+    constexpr int kSpan = 256 / kCols;                      // consecutive steps that a wave of movers carries
+    static_assert(kAll || kDrChunk / kSpan <= 2 * (kDrPitch - kDrChunk), "a pad for each");
+
     static_assert(kPer >= 1 && kSteps * kPer == kDrChunk && kSteps % 4 == 0, "the movers share a chunk evenly");
-    __shared__ float s_x[3][kCols][kDrPitch];  // a step's value in, its result out
-    __shared__ float s_f[3][kCols][kDrPitch];  // its factor (1 - done) * gamma
+    __shared__ float s_x[kDrBuffers][kCols][kDrPitch];  // a step's value in, its result out
+    __shared__ float s_f[kDrBuffers][kCols][kDrPitch];  // its factor (1 - done) * gamma
     const int64_t cols = batch * inner;
     // Workgroups are dealt to the chip's eight dies in turn, and each die has its own L2. Neighbouring column groups
     // share cache lines (a group's flags of a step are kCols bytes), so they go to the SAME die.
@@ -82,54 +97,65 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
         return q < ncols ? q : ncols - 1;
     };
 
+    // The result in front of the first step that a wave of movers carries, kept in the pads: the step before belongs to another wave,
+    // which may have put the next chunk there.
+    auto in_front = [&](int buf, int q, int at) -> float& {
+        const int nth = at / kSpan;
+        return nth < 4 ? s_x[buf][q][kDrChunk + nth] : s_f[buf][q][kDrChunk + nth - 4];
+    };
+
     if (threadIdx.x < 64) {
         // ---- wave 0: the recurrence
         const int q = lane < kCols ? lane : 0;
         const int64_t col = c0 + column_of(q);
         float last = kBack ? 0.0f : end_value[col];
+        f32x4 xa[4], fa[4], xb[4], fb[4];
+        auto fetch = [&](int buf, int at, f32x4 (&xs)[4], f32x4 (&fs)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                xs[i] = *reinterpret_cast<const f32x4*>(&s_x[buf][q][at + 4 * i]);
+                fs[i] = *reinterpret_cast<const f32x4*>(&s_f[buf][q][at + 4 * i]);
+            }
+        };
+        auto sixteen = [&](int buf, int at, f32x4 (&xs)[4], const f32x4 (&fs)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    last = xs[i][j] + fs[i][j] * last;
+                    if (kAll) xs[i][j] = last;
+                }
+                if (kAll)
+                    *reinterpret_cast<f32x4*>(&s_x[buf][q][at + 4 * i]) = xs[i];
+                else
+                    s_x[buf][q][at + 4 * i + 3] = last;
+                if (!kAll && (at + 4 * i + 4) % kSpan == 0 && at + 4 * i + 4 < kDrChunk) in_front(buf, q, at + 4 * i + 4) = last;
+            }
+        };
         lds_barrier();
+        if (lane < kCols) fetch(0, 0, xa, fa);
         int buf = 0;
         for (int64_t c = 0; c < nchunks; ++c) {
+            const int next = buf == kDrBuffers - 1 ? 0 : buf + 1;
             if (lane < kCols) {
-                float* const vx = s_x[buf][q];
-                const float* const vf = s_f[buf][q];
-                // sixteen steps at a time, the next sixteen requested before these run (a short last chunk runs its
-                // doubled steps too: nobody looks at what they leave)
-                f32x4 xa[4], fa[4], xb[4], fb[4];
-                auto fetch = [&](int at, f32x4 (&xs)[4], f32x4 (&fs)[4]) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        xs[i] = *reinterpret_cast<const f32x4*>(vx + at + 4 * i);
-                        fs[i] = *reinterpret_cast<const f32x4*>(vf + at + 4 * i);
-                    }
-                };
-                auto steps16 = [&](int at, f32x4 (&xs)[4], f32x4 (&fs)[4]) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            last = xs[i][j] + fs[i][j] * last;
-                            xs[i][j] = last;
-                        }
-                        *reinterpret_cast<f32x4*>(vx + at + 4 * i) = xs[i];
-                    }
-                };
-                fetch(0, xa, fa);
-#pragma unroll
-                for (int at = 0; at < kDrChunk; at += 32) {
-                    fetch(at + 16, xb, fb);
-                    steps16(at, xa, fa);
-                    if (at + 32 < kDrChunk) fetch(at + 32, xa, fa);
-                    steps16(at + 16, xb, fb);
-                }
-                if (kBack && c == nchunks - 1) last = vx[timesteps - 1 - c * kDrChunk];  // step T - 1, not a doubled one
+                if (!kAll) in_front(buf, q, 0) = last;
+                fetch(buf, 16, xb, fb);
+                sixteen(buf, 0, xa, fa);
+                fetch(buf, 32, xa, fa);
+                sixteen(buf, 16, xb, fb);
             }
-            buf = buf == 2 ? 0 : buf + 1;
             lds_barrier();
+            // (a short last chunk runs doubled steps to the end of its half: nobody looks at what they leave)
+            if (lane < kCols && timesteps - c * kDrChunk > kDrChunk / 2) {
+                fetch(buf, 48, xb, fb);
+                sixteen(buf, 32, xa, fa);
+                fetch(next, 0, xa, fa);  // (behind the last chunk: what nobody uses)
+                sixteen(buf, 48, xb, fb);
+            }
+            buf = next;
         }
+        if (nchunks == 1) lds_barrier();
         lds_barrier();
-        if (kBack && end_value && lane < kCols)
-            end_value[col] = (1.0f - (done[(timesteps - 1) * batch + col / inner] ? 1.0f : 0.0f)) * gamma * last;
         return;
     }
     // ---- the movers
@@ -160,24 +186,29 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
     auto base_of = [&](int64_t c) -> int64_t {  // the earliest time of chunk c
         return kBack ? first_of(c) : timesteps - 1 - first_of(c) - last_of(c);
     };
+    // (Read through addresses that the compiler knows nothing of: what it knows to be constant it would request behind the barriers
+    // in front of its use, a trip to memory later.)
+    const MRB_GLOBAL char* from_x = (const MRB_GLOBAL char*)x;
+    const MRB_GLOBAL char* from_f = (const MRB_GLOBAL char*)done;
+    asm volatile("" : "+s"(from_x), "+s"(from_f));
     auto request = [&](int64_t c, f32x4 (&xr)[kPer], uint32_t (&dr)[kPer][kFlags]) {
         const int last = last_of(c);
         const int64_t t0 = base_of(c);
-        const char* const bx = reinterpret_cast<const char*>(x + t0 * cols);
-        const uint8_t* const bf = done + (kBack && t0 > 0 ? t0 - 1 : t0) * batch;
+        const MRB_GLOBAL char* const bx = from_x + t0 * cols * 4;
+        const MRB_GLOBAL char* const bf = from_f + (kBack && t0 > 0 ? t0 - 1 : t0) * batch;
         const uint32_t back = kBack && t0 == 0 ? 1u : 0u;  // the first chunk's flags start a row late: step 0 takes any
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             if (kQuad) {
                 const uint32_t row = row_of(i * kSteps + step, last);
-                xr[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_u*>(bx + (row * row_x + off_x)));
-                dr[i][0] = *reinterpret_cast<const u32_u*>(bf + ((row > back ? row - back : 0u) * row_f + off_f));
+                xr[i] = *(const MRB_GLOBAL f32x4_u*)(bx + (row * row_x + off_x));
+                dr[i][0] = *(const MRB_GLOBAL u32_u*)(bf + ((row > back ? row - back : 0u) * row_f + off_f));
             } else {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const uint32_t row = row_of(i * kSteps + step + j, last);
-                    xr[i][j] = __builtin_nontemporal_load(reinterpret_cast<const float*>(bx + (row * row_x + off_x)));
-                    dr[i][kQuad ? 0 : j] = bf[(row > back ? row - back : 0u) * row_f + off_f];
+                    xr[i][j] = *(const MRB_GLOBAL float*)(bx + (row * row_x + off_x));
+                    dr[i][kQuad ? 0 : j] = (uint8_t)bf[(row > back ? row - back : 0u) * row_f + off_f];
                 }
             }
         }
@@ -201,49 +232,111 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
             }
         }
     };
-    auto drain = [&](int64_t c, int buf) {
-        const int last = last_of(c);
+    // A chunk's results, from LDS to registers: of each four steps the recurrence has left the last one's. A mover works the three
+    // before it out again, from the result in front of them, for four steps of one column; one that carries a step of four
+    // columns hands them to the others that carry these four steps, all in its own wave, through LDS.
+    auto take = [&](int buf, f32x4 (&v)[kPer]) {
+        if (kAll) {
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) {
+                if (!kQuad) v[i] = *reinterpret_cast<const f32x4*>(&s_x[buf][own][i * kSteps + step]);
+#pragma unroll
+                for (int j = 0; kQuad && j < 4; ++j) v[i][j] = s_x[buf][4 * quad + j][i * kSteps + step];
+            }
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int of = kQuad ? 4 * quad + (step & 3) : own, at = i * kSteps + (step & ~3);
+            const f32x4 f = *reinterpret_cast<const f32x4*>(&s_f[buf][of][at]);
+            float last = at % kSpan ? s_x[buf][of][at ? at - 1 : 0] : in_front(buf, of, at);
+            v[i] = *reinterpret_cast<const f32x4*>(&s_x[buf][of][at]);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) v[i][j] = last = v[i][j] + f[j] * last;
+            if (kQuad) *reinterpret_cast<f32x4*>(&s_x[buf][of][at]) = v[i];
+        }
+        if (kQuad) {
+#pragma unroll
+            for (int i = 0; i < kPer; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[i][j] = s_x[buf][4 * quad + j][i * kSteps + step];
+        }
+    };
+    auto store = [&](int64_t c, const f32x4 (&v)[kPer], auto whole, int last) {
         char* const bo = reinterpret_cast<char*>(out + base_of(c) * cols);
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
+            const int k = i * kSteps + step;
             if (kQuad) {
-                const int k = i * kSteps + step < last ? i * kSteps + step : last;
-                f32x4 v;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = s_x[buf][4 * quad + j][k];
-                __builtin_nontemporal_store(v, reinterpret_cast<f32x4_u*>(bo + (row_of(k, last) * row_x + off_x)));
+                if (decltype(whole)::value || k <= last) __builtin_nontemporal_store(v[i], reinterpret_cast<f32x4_u*>(bo + (row_of(k, last) * row_x + off_x)));
             } else {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int k = i * kSteps + step + j < last ? i * kSteps + step + j : last;
-                    __builtin_nontemporal_store(s_x[buf][own][k], reinterpret_cast<float*>(bo + (row_of(k, last) * row_x + off_x)));
-                }
+                for (int j = 0; j < 4; ++j)
+                    if (decltype(whole)::value || k + j <= last)
+                        __builtin_nontemporal_store(v[i][j], reinterpret_cast<float*>(bo + (row_of(k + j, last) * row_x + off_x)));
             }
         }
     };
+    const int end = last_of(nchunks - 1);  // the last chunk's last step
 #pragma unroll
     for (int j = 0; j < kDrAhead; ++j) request(j, xs[j], ds[j]);
-    static_assert(kDrAhead >= 3, "the two stages without a drain use the first two register sets");
+    uint32_t end_flags[kFlags];  // the last step's, for the bootstrap value's gradient
+    if (kBack) {
+        if (kQuad)
+            end_flags[0] = *reinterpret_cast<const u32_u*>(done + (timesteps - 1) * batch + off_f);
+        else
+            end_flags[0] = done[(timesteps - 1) * batch + off_f];
+    }
+    __builtin_amdgcn_sched_barrier(0);  // all of them now: none behind the wait for the first
+    // Chunk k lies in buffer k % 3 and comes through register set k % kDrAhead. Between the recurrence's barriers in the middle
+    // of chunks c - 1 and c: take chunk c - 2's results out of its buffer and put chunk c + 1 (past the end: a chunk nobody
+    // reads) there, each mover its own places.
+    static_assert(kDrAhead == 3 && kDrBuffers == 3, "the sets and buffers below");
+    f32x4 v[kPer];
     deposit(0, xs[0], ds[0]);
     request(kDrAhead, xs[0], ds[0]);
     lds_barrier();
     deposit(1, xs[1], ds[1]);
     request(kDrAhead + 1, xs[1], ds[1]);
     lds_barrier();
-    // stage s, s = 2 .. nchunks + 1: deposit chunk s (past the end: a chunk nobody reads, into a buffer nobody uses),
-    // drain chunk s - 2. Buffers: chunk c lies in buffer c % 3.
-    int put = 2, take = 0;
-    for (int64_t s = 2; s < nchunks + 2; s += kDrAhead) {
+    deposit(2, xs[2], ds[2]);
+    request(kDrAhead + 2, xs[2], ds[2]);
+    lds_barrier();
+    auto stage = [&](int64_t c, auto nth) {
+        constexpr int j = decltype(nth)::value;
+        take(j, v);
+        deposit(j, xs[j], ds[j]);
+        request(c + 1 + kDrAhead, xs[j], ds[j]);
+        store(c - 2, v, std::true_type{}, kDrChunk - 1);
+        lds_barrier();
+        __builtin_amdgcn_sched_barrier(0);  // (the next chunk's flags are not looked at, that is waited for, before its time)
+    };
+    int64_t c = 2;
+    for (; c + 2 < nchunks; c += 3) {  // (no way out in the middle: what is in flight is counted exactly)
+        stage(c, std::integral_constant<int, 0>{});
+        stage(c + 1, std::integral_constant<int, 1>{});
+        stage(c + 2, std::integral_constant<int, 2>{});
+    }
+    int buf = 0;
+    if (c < nchunks) stage(c, std::integral_constant<int, 0>{}), buf = 1;
+    if (c + 1 < nchunks) stage(c + 1, std::integral_constant<int, 1>{}), buf = 2;
+    if (nchunks > 1) {
+        take(buf, v);
+        store(nchunks - 2, v, std::true_type{}, kDrChunk - 1);
+        buf = buf == kDrBuffers - 1 ? 0 : buf + 1;
+    }
+    lds_barrier();
+    take(buf, v);
+    store(nchunks - 1, v, std::false_type{}, end);
+    if (kBack && end_value) {
 #pragma unroll
-        for (int j = 0; j < kDrAhead; ++j) {
-            if (s + j >= nchunks + 2) break;  // (uniform; nothing is requested or stored after the loop)
-            const int set = (2 + j) % kDrAhead;  // = (s + j) % kDrAhead, known when the loop is unrolled
-            deposit(put, xs[set], ds[set]);
-            request(s + j + kDrAhead, xs[set], ds[set]);
-            drain(s + j - 2, take);
-            put = put == 2 ? 0 : put + 1;
-            take = take == 2 ? 0 : take + 1;
-            lds_barrier();
+        for (int i = 0; i < kPer; ++i) {
+            const int k = i * kSteps + step;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const bool flag = kQuad ? (end_flags[0] >> (8 * j)) & 255u : end_flags[0] != 0;
+                if (k + (kQuad ? 0 : j) == end) end_value[col + (kQuad ? j : 0)] = (1.0f - (flag ? 1.0f : 0.0f)) * gamma * v[i][j];
+            }
         }
     }
 }

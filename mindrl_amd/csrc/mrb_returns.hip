@@ -19,23 +19,23 @@ void launch(bool back, const float* x, const uint8_t* done, float* end_value, fl
 
 }  // namespace
 
-// Columns per workgroup: sixteen while that fills at most one workgroup per compute unit (4096 columns), thirty-two up
-// to 8192, sixty-four beyond. Narrow groups spread the recurrence's waves and the memory traffic over more compute
-// units; wide ones read longer pieces of a row, which the memory serves better (3.1, 4.4 and 4.8 TB/s for 16, 32 and
-// 64 columns when every compute unit has work). Measured, us for 16 / 32 / 64 columns per group: [1000, 32] 11.9 /
-// 13.7 / 17.9, [1000, 4096] 14.5 / 15.8 / 21.8, [1000, 8192] 26.2 / 17.7 / 24.1, [1000, 16384] 48 / 34.5 / 30.6. A short
-// time axis keeps thirty-two ([100, 16384]: 7.9 / 6.8 / 7.6). Sixty-four columns take the movers that carry four steps of
-// one column: the other kind's scalar LDS writes meet in the same banks there (29 us at [1000, 32]).
+// Columns per workgroup. Narrow groups spread the recurrence's waves and the memory traffic over more compute units; wide ones read
+// longer pieces of a row, which the memory serves better, and which counts when the call is more than the caches hold. Measured, us for
+// 16 / 32 / 64 columns per group: [1000, 4096] 11.8 / 15.4 / 16.1, [1000, 8192] 15.3 / 15.8 / 16.6, [2000, 8192] 43 / 29.5 / 40, [1000, 12000] 31.6 / 26.1 /
+// 22.7, [1000, 16384] 43 / 33 / 28.7, [500, 20000] 28.6 / 21.3 / 22.8, [1000, 40000] 67 / 60 / 57. A short time axis moves less, and sixteen stay
+// the best or within 0.2 us of it: [100, 8192] 4.6 / 4.5 / 5.2, [100, 16384] 5.8 / 6.0 / 5.8, [64, 20000] 5.8 / 6.6 / 8.4, [100, 30001] 10.5 / 13.1 /
+// 10.7. Sixty-four columns take the movers that carry four steps of one column: the other kind's scalar LDS writes meet in the
+// same banks there.
 hipError_t launch_discounted_return_tiled(bool back, const float* x, const uint8_t* done, float* end_value, float* out,
                                           int64_t timesteps, int64_t batch, int64_t inner, float gamma, hipStream_t s) {
     const int64_t cols = batch * inner;
     const bool quad = inner == 1 && cols >= 4;
-    if (cols > 8192 && timesteps >= 128)
-        launch<false, 64, 512>(back, x, done, end_value, out, timesteps, batch, inner, gamma, s);
-    else if (cols > 4096)
+    if (cols <= 4096 || timesteps < 128)
+        (quad ? launch<true, 16, 256> : launch<false, 16, 256>)(back, x, done, end_value, out, timesteps, batch, inner, gamma, s);
+    else if (cols <= 8192)
         (quad ? launch<true, 32, 256> : launch<false, 32, 512>)(back, x, done, end_value, out, timesteps, batch, inner, gamma, s);
     else
-        (quad ? launch<true, 16, 256> : launch<false, 16, 256>)(back, x, done, end_value, out, timesteps, batch, inner, gamma, s);
+        launch<false, 64, 512>(back, x, done, end_value, out, timesteps, batch, inner, gamma, s);
     return hipGetLastError();
 }
 

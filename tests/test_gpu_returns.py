@@ -44,6 +44,34 @@ def test_return_and_gradient_bit_exact(shape):
     assert np.array_equal(t2n(grad_value), want_value)
 
 
+# the pipeline's first, second and third chunk and the stages behind its loop of three, each with a last chunk of one step, of
+# half and whole, at either side of sixteen and eight steps; the lines between the kernels and the groups' widths
+EDGES = [(t, b, inner) for b, inner in ((5, 1), (3, 2), (4101, 1)) for t in (1, 16, 17, 32, 33, 48, 64, 96, 97, 128, 129, 192, 193, 256, 257, 320, 321, 385)]
+EDGES += [(33, 32768, 1), (33, 32769, 1), (64, 32769, 1), (65, 32769, 1), (65, 40961, 1), (127, 8193, 1), (128, 4097, 1), (127, 4097, 1),
+          (255, 40961, 1), (256, 40961, 1), (257, 65537, 1), (130, 2731, 3), (100, 5461, 3)]
+
+
+@pytest.mark.parametrize("shape", EDGES)
+def test_every_stage_of_the_pipeline(shape):
+    """Results and both gradients bit for bit, with infinities and numbers that are none among the inputs: they reach every earlier
+    (of the gradient: later) step of their column up to the next end, and no other column."""
+    from mindrl_amd.utils import DiscountedReturn
+    from oracle import orc
+    t, b, inner = shape
+    rng = np.random.default_rng(t * 7 + b + inner)
+    r, w = rng.normal(size=shape).astype(np.float32), rng.normal(size=shape).astype(np.float32)
+    for x in (r, w):
+        x[rng.integers(0, t), rng.integers(0, b)] = np.inf
+        x[rng.integers(0, t), rng.integers(0, b)] = np.nan
+    d = rng.random((t, b)) < 0.03
+    v = rng.normal(size=(b, inner)).astype(np.float32)
+    reward, value = torch.from_numpy(r).cuda().requires_grad_(True), torch.from_numpy(v).cuda().requires_grad_(True)
+    out = DiscountedReturn(0.99, need_bprop=True)(reward, torch.from_numpy(d).cuda(), value)
+    got = (out.detach(),) + torch.autograd.grad(out, (reward, value), torch.from_numpy(w).cuda())
+    for g, want in zip(got, (orc.discounted_return(r, d, v, 0.99),) + oracle_gradient(orc, w, d, 0.99)):
+        assert np.array_equal(t2n(g), want, equal_nan=True)
+
+
 def test_forward_mode_is_refused():
     import torch.autograd.forward_ad as fw
     from mindrl_amd.utils import DiscountedReturn
