@@ -1661,9 +1661,26 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
 // the same (batches x rows of one): 8-byte rows, 10^6 slots 4096 x 1 6.6 / 20, 4096 x 2 11.0 / 20.6, 2048 x 4 10.9 / 12.1,
 // 2048 x 6 14.6 / 9.9, 1024 x 8 10.8 / 6.4; 521 bytes 2048 x 4 11.0 / 13.8, 4096 x 5 26 / 22; 3 KB 4096 x 3 21 / 30, 4096 x 6
 // 36 / 43, 2048 x 8 26 / 26. (A row above 4 KB takes a whole workgroup there: 6 KB 4096 x 3 46 / 43.)
-static bool takes_lds(int64_t nbatch, int64_t batch, uint64_t rest) {
+// `lanes`: whether sixteen lanes to a stratum could take it (takes_lanes), which is the better one up to (lanes / LDS-top, us) 8-byte rows 8192
+// 4.5 / 5.1, 16,384 6.0 / 5.3; 41 bytes 12,288 5.7 / 6.2, 16,384 6.8 / 6.2; 153 bytes 16,384 7.4 / 7.5, 32,768 13.0 / 9.0; 521 bytes 16,384 7.9 / 9.0,
+// 32,768 14.0 / 11.6; 899 bytes in odd fields 12,288 9.5 / 9.8, 16,384 14.2 / 10.8; 1 KB 12,000 10.9 against a wave's 18.9, 16,384 14.2 / 12.4; 2.4 KB
+// 16,384 22.9 / 21.5.
+static bool takes_lds(int64_t nbatch, int64_t batch, uint64_t rest, bool lanes) {
     const int64_t rows = nbatch * batch, fewest = rest <= 64 ? 5 : rest <= 256 ? 8 : 1;
-    return rest <= 384 && batch >= fewest && rows >= (rest <= 16 ? 3072 : rest <= 64 ? 5120 : 12288);
+    const int64_t least = lanes ? (rest <= 16 ? 14336 : rest <= 40 ? 20480 : 12288) : (rest <= 16 ? 3072 : rest <= 64 ? 5120 : 12288);
+    return rest <= 384 && batch >= fewest && rows >= least;
+}
+// Whether sixteen lanes to a stratum (k_per_sample_lanes) can take a sample, and from how many rows on they are the better ones. Workgroup per row
+// (k_per_sample_light) / lanes, us: 41 bytes 1024 rows 3.8 / 4.1, 1280 4.1 / 4.0; 153 bytes, 5 * 10^4 slots 1024 3.8 / 3.5, 10^5 3.85 / 3.9, 10^6 3.8 / 4.3;
+// 899 bytes in odd fields 1280 4.4 / 5.0, 1536 5.0 / 5.1; 1 KB 1536 4.75 / 5.0, 2048 6.4 / 5.1; 2.4 KB 1500 5.2 / 5.5, 2048 7.2 / 5.8; 13 KB 1024
+// 8.2 / 9.3, 2048 15.7 / 14.4; 20 KB 1024 13.8 / 13.8, 2048 23.2 / 20.8; 28 KB 2048 23.8 / 24.7, 4096 40.9 / 44.7. On 21 levels and more, whose walk takes
+// the workgroup longer: 153 bytes 1024 5.6 / 4.8, 521 bytes 5.4 / 4.7.
+static bool takes_lanes(const Per& b, const WidePlan& plan) {
+    return b.rows.row_split == 0 && b.rows.row_wave == 0 && b.depth >= kLanesFewestLevels && plan.narrow_items <= kLanesMostNarrow &&
+           plan.wide_items <= 1280;
+}
+static int64_t lanes_fewest_rows(int depth, uint32_t wide_items) {
+    return wide_items > 64 ? 2048 : depth >= 21 ? 1024 : wide_items <= 32 ? 1280 : 1536;
 }
 static int lds_strata(int64_t rows, uint64_t rest) {
     if (rows <= 20480 && rest > 16) return 16;
@@ -1708,7 +1725,17 @@ static int per_sample_impl(Per* b, int64_t nbatch, int64_t batch, float beta, co
     uint64_t rest = 0;  // granules of a row that the LDS-top kernel's threads do not copy for their own stratum alone
     for (int f = 0; f < t.nfields; ++f) rest += f < kLdsOwn && t.units[f] == 1 ? 0 : t.units[f];
     int path = (int)b->sample_path;
-    if (path == 0) path = takes_lds(nbatch, batch, rest) ? 2 : 1;
+    if (path == 0) {
+        WidePlan plan;
+        dim3 grid;
+        plan.nbatch = (uint32_t)nbatch;
+        const bool lanes = !next && nbatch * batch >= 1024 && wide_plan(b->rows, t, nbatch * batch, plan, grid) && takes_lanes(*b, plan);
+        path = takes_lds(nbatch, batch, rest, lanes) ? 2 : lanes && nbatch * batch >= lanes_fewest_rows(b->depth, plan.wide_items) ? 3 : 1;
+        if (path == 3) {
+            const hipError_t e = launch_per_sample_lanes(a, plan, nbatch, s);
+            if (e != hipSuccess) return fail(MRB_EHIP, "launch k_per_sample_lanes: %s", hipGetErrorString(e));
+        }
+    }
     if (rest > 1u << 23) path = 1;  // (it numbers a workgroup's granules in 32 bits)
     if (next) {
         rc = sample_wide(b->rows, a, t, nbatch, s, next);  // always the wide-row kernel: the gathered field is wide
@@ -1716,7 +1743,7 @@ static int per_sample_impl(Per* b, int64_t nbatch, int64_t batch, float beta, co
     } else if (path == 1) {
         rc = sample_wide(b->rows, a, t, nbatch, s);
         if (rc) return rc;
-    } else {
+    } else if (path == 2) {
         int levels = b->lds_levels > 0 ? (int)b->lds_levels : 9;
         if (levels > b->depth) levels = b->depth;
         const hipError_t e = launch_per_sample_lds(a, t, nbatch, lds_strata(nbatch * batch, rest), levels, (uint32_t)rest, s);

@@ -1,4 +1,4 @@
-// Samples of thousands of rows (defined in mrb_samples.hip).
+// Samples of thousands of rows (defined in mrb_samples.hip and mrb_sample_lanes.hip).
 #pragma once
 #include "mrb_rows.h"
 
@@ -8,5 +8,11 @@ namespace mrb {
 // the granules of a row outside the fields that each thread copies for its own stratum (see kLdsOwn).
 hipError_t launch_per_sample_lds(const SampleArgs& a, const IoTable& t, int64_t nbatch, int strata, int levels, uint32_t rest,
                                  hipStream_t s);
+
+// The same by sixteen lanes for each stratum: trees of at least kLanesFewestLevels levels, rows of at most kLanesMostNarrow bytes in
+// narrow fields.
+constexpr int kLanesFewestLevels = 7;
+constexpr uint32_t kLanesMostNarrow = 48;
+hipError_t launch_per_sample_lanes(const SampleArgs& a, const WidePlan& plan, int64_t nbatch, hipStream_t s);
 
 }  // namespace mrb
