@@ -847,12 +847,25 @@ bool takes_range_one(const Per& b, int64_t n) {
 // Whether an update goes by runs of leaves in two launches (launch_tree_range). Against what it would take
 // otherwise, us per call, before / by runs:
 //   most entries    12 levels, 8192 / 16,384: 10.0 / 11.4 against 9.6 / 13.8; 14 levels, 16,384 / 32,768: 11.7 / 12.5 against 11.2 / 16.7; 20 levels 14.4 / 15.4 against
-//                   14.1 / 18.7; 22 levels, 8192 / 16,384: 16.1 / 17.7 against 16.0 / 21.0.
+//                   14.1 / 18.7. On 21 levels and more what its entries drive is the other way: see takes_sparse.
 //   deepest tree    23 and 24 levels leave more than a tile above the runs and bring many runs without an entry: 2048
 //                   entries 14.9 / 15.9 against 14.9 / 23.3.
 bool takes_range(const Per& b, int64_t n) {
     if (!b.fused || b.depth < 12 || b.depth > 22) return false;
-    return !takes_range_one(b, n) && n <= (b.depth == 12 || b.depth == 22 ? 8192 : 16384);
+    return !takes_range_one(b, n) && n <= (b.depth == 22 ? 4096 : b.depth == 12 || b.depth == 21 ? 8192 : 16384);
+}
+
+// Whether the entries drive the lowest levels of an update (launch_tree_sparse), with more than the 1024 that elect among themselves. The other ways
+// look at every tile of the tree, or at every entry in every workgroup. us per call, by tiles (runs of leaves up to 8192 entries) / by entries, slots at random and,
+// behind the comma, one after the other:
+//   21 levels  8193 12.1 / 11.4, 16,384 14.9 / 12.4, 32,768 20.7 / 14.7, 10.9 / 10.4; 65,536 23.4 / 19.7, 11.0 / 11.6; 131,072 27.9 / 29.0
+//   22 levels  4096 10.8 / 11.1, 5000 12.0 / 11.2, 8192 13.2 / 11.6, 32,768 29.6 / 15.0, 131,072 38.7 / 32.0, 14.6 / 13.2; 200,000 43.3 / 43.0, 15.2 / 16.2
+//   23 levels  131,072 56 / 34, 262,144 66 / 56, 19.7 / 18.2; 524,288 83 / 95
+//   24 levels  131,072 93 / 36, 262,144 116 / 63, 27 / 18; 524,288 138 / 156; 25 levels  262,144 189 / 110, 524,288 235 / 173
+//   26 levels  524,288 368 / 338, 75 / 50; 1,048,576 458 / 599; deeper trees were not measured
+bool takes_sparse(const Per& b, int64_t n) {
+    const int share = b.depth == 22 || b.depth == 23 ? 5 : b.depth <= 25 ? 6 : b.depth == 26 ? 7 : 8;
+    return b.s_g0 > 0 && n > kElectMax && n <= b.leaves >> share;
 }
 
 // Where one workgroup's update alone (k_tree_wg) is faster than that. 1 / 16 / 64 / 96 / 128 entries, us, it against runs: 10 levels
@@ -896,9 +909,7 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
     a.indices = indices;
     a.priorities = priorities;
     a.n = n;
-    // Few entries (but more than the 1024 that elect among themselves, below) on a very large tree: rebuild
-    // the lowest levels per entry, not per tile.
-    const bool sparse = b->s_g0 > 0 && n > kElectMax && n <= (b->leaves >> 8);
+    const bool sparse = takes_sparse(*b, n);
     if (sparse) {
         a.sparse_g0 = b->s_g0;
         a.nrounds = b->s_rounds;
@@ -1369,8 +1380,8 @@ int mrb_per_create(int64_t capacity, float alpha, int nfields, const int64_t* fi
         HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->dirty[r]), nblocks * sizeof(uint32_t)));
         HIP_TRY(hipMemset(b->dirty[r], 0, nblocks * sizeof(uint32_t)));
     }
-    if (b->depth >= 22) {
-        // sparse plan: with >= 16384 leaf tiles a call with few entries is better driven by its entries
+    if (b->depth >= 21) {
+        // sparse plan: with thousands of leaf tiles a call with few entries is better driven by its entries (takes_sparse)
         b->s_g0 = b->depth - 20 < 4 ? 4 : (b->depth - 20 > 6 ? 6 : b->depth - 20);
         // k_tree_runs takes at most 20 levels; deeper trees go through a round of tiles first (at least two levels, so
         // that a lane's four nodes share a block)
