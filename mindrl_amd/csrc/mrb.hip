@@ -958,9 +958,7 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
                            a.capacity, r | a.lo[r] << 8 | a.g[r] << 16, a.alpha, a, 0u, PutArgs{});
         LAUNCH_CHECK("k_tree_update");
     }
-    rc = checked(launch_tree_runs(a.sum, a.mn, a.dirty[last], a.lo[last], a.epoch, s), "k_tree_runs");
-    if (rc) return rc;
-    return checked(launch_tree_cap(a.sum, a.mn, kRoundLevels, s), "k_tree_cap");
+    return checked(launch_tree_runs(a.sum, a.mn, a.dirty[last], a.maxp, a.lo[last], a.epoch, s), "k_tree_runs");
 }
 
 

@@ -16,8 +16,8 @@ hipError_t launch_tree_range(const int64_t* indices, const float* priorities, in
 hipError_t launch_tree_sparse(const int64_t* indices, const unsigned long long* stamp, const float* powered, float* sum, float* mn,
                               uint32_t* dirty, int64_t n, int64_t capacity, int depth, int g0, int g_dirty, uint32_t epoch,
                               hipStream_t s);
-// From depth `top` (17 to 20) to depth 8: the tiles of 256 nodes whose word in `dirty` carries the epoch.
-hipError_t launch_tree_runs(float* sum, float* mn, const uint32_t* dirty, int top, uint32_t epoch, hipStream_t s);
+// From depth `top` (17 to 20) to the root: the tiles of 256 nodes whose word in `dirty` carries the epoch.
+hipError_t launch_tree_runs(float* sum, float* mn, const uint32_t* dirty, float* maxp, int top, uint32_t epoch, hipStream_t s);
 // The levels above depth `top`, at most 8.
 hipError_t launch_tree_cap(float* sum, float* mn, int top, hipStream_t s);
 

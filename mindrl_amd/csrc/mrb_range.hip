@@ -1,6 +1,7 @@
 #include "mrb_range.h"
 
 #include "../../include/mrb.h"
+#include "mrb_meet.h"
 #include "mrb_rows.h"
 #include "mrb_tree.h"
 
@@ -241,11 +242,12 @@ __global__ __launch_bounds__(kSparseWG) void k_tree_sparse(const int64_t* __rest
     sparse_step<3>(trees, g0, first, sub, active, cs, cm);
 }
 
-// The next levels of such a tree, down to 256 nodes that k_tree_cap takes: a workgroup owns 2^w nodes at depth `top` (w =
-// top - 8, 9 to 12), a wave each tile of 256, and goes on to the run's root. Nodes, dirty word and the root as it is are
-// requested together. With k_tree_cap 6.1 + 1.5 to 3.9 us for 2^20 nodes; a launch for eight levels and one workgroup for
-// the twelve above took 6.1 + 3.9 and their inputs a trip more. (The step on the 24-level tree 55.5 -> 51.5 us.)
-__global__ __launch_bounds__(1024) void k_tree_runs(float* sum, float* mn, const uint32_t* __restrict__ dirty, uint32_t epoch, int top) {
+// The levels above: a workgroup owns 2^w nodes at depth `top` (w = top - 8, 9 to 12), a wave each tile of 256, and goes on to
+// the run's root; the last of the 256 workgroups to get there rebuilds the eight levels above the runs (mrb_meet.h; all of them meet: which runs
+// changed, nobody knows but they). Nodes, dirty word and the root as it is are requested together. With a launch of its own
+// for the eight levels 16,384 entries on 2^22 leaves took 12.6 us, now 12.0, 65,536 on 2^24 23.9, now 22.9. (A launch for eight levels and one workgroup
+// for the twelve above took 3 us more.)
+__global__ __launch_bounds__(1024) void k_tree_runs(float* sum, float* mn, const uint32_t* __restrict__ dirty, float* maxp, uint32_t epoch, int top) {
     __shared__ float s_rs[16], s_rm[16];
     __shared__ uint32_t s_new[16];
     const uint32_t lane = threadIdx.x & 63;
@@ -257,6 +259,13 @@ __global__ __launch_bounds__(1024) void k_tree_runs(float* sum, float* mn, const
     const float4 vm = *reinterpret_cast<const float4*>(mn + first + 4 * lane);
     float rs = sum[first >> kRoundLevels], rm = mn[first >> kRoundLevels];
     const bool changed = dirty[tile] == epoch;
+    uint32_t turn = 0;
+    float4 roots_s = vs, roots_m = vm;
+    if (wave == 0) {
+        turn = meet_turn(maxp);
+        roots_s = *reinterpret_cast<const float4*>(sum + kBlockNodes + 4 * lane);
+        roots_m = *reinterpret_cast<const float4*>(mn + kBlockNodes + 4 * lane);
+    }
     if (changed) tile_parents(trees, kRoundLevels, first, lane, true, vs, vm, &rs, &rm);
     if (lane == 0) {
         s_rs[wave] = rs;
@@ -265,17 +274,13 @@ __global__ __launch_bounds__(1024) void k_tree_runs(float* sum, float* mn, const
     }
     lds_barrier();
     if (wave != 0) return;
+    const MeetPlan plan = meet_plan(15u, blockIdx.x, lane);
     const uint32_t tiles = 1u << up;
+    const bool any = __any(lane < tiles && s_new[lane < tiles ? lane : 0]);
     float cs = lane < tiles ? s_rs[lane] : 0.0f, cm = lane < tiles ? s_rm[lane] : 0.0f;
-    if (!__any(lane < tiles && s_new[lane])) return;
-    for (int l = 1; l <= up; ++l) {
-        cs = cs + __shfl_xor(cs, 1 << (l - 1));
-        cm = fminf(cm, __shfl_xor(cm, 1 << (l - 1)));
-        if (lane < tiles && (lane & ((1u << l) - 1)) == 0) {
-            sum[((first >> kRoundLevels) + lane) >> l] = cs;
-            mn[((first >> kRoundLevels) + lane) >> l] = cm;
-        }
-    }
+    run_parents(trees, up, first >> kRoundLevels, lane, any && lane < tiles, cs, cm);  // (of a clean run: its root as it is)
+    if (!meet(maxp, err_before(maxp), turn, blockIdx.x, cs, cm, lane, plan, roots_s, roots_m)) return;
+    tile_parents(trees, kRoundLevels, kBlockNodes, lane, true, roots_s, roots_m);
 }
 
 // The levels above depth `top` (1 .. 8): one wave, everything it needs in preloaded registers, one trip to memory.
@@ -325,8 +330,8 @@ hipError_t launch_tree_sparse(const int64_t* indices, const unsigned long long* 
     return hipGetLastError();
 }
 
-hipError_t launch_tree_runs(float* sum, float* mn, const uint32_t* dirty, int top, uint32_t epoch, hipStream_t s) {
-    hipLaunchKernelGGL(k_tree_runs, dim3(1u << kRoundLevels), dim3(64u << (top - 2 * kRoundLevels)), 0, s, sum, mn, dirty, epoch, top);
+hipError_t launch_tree_runs(float* sum, float* mn, const uint32_t* dirty, float* maxp, int top, uint32_t epoch, hipStream_t s) {
+    hipLaunchKernelGGL(k_tree_runs, dim3(1u << kRoundLevels), dim3(64u << (top - 2 * kRoundLevels)), 0, s, sum, mn, dirty, maxp, epoch, top);
     return hipGetLastError();
 }
 
