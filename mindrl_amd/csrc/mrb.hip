@@ -940,8 +940,8 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
         a.inline_election = 1;
         return tree_rebuild(*b, a, s);
     }
-    hipLaunchKernelGGL(k_update_stamp, dim3(grid_exact((uint64_t)n)), dim3(kWG), 0, s, a.indices, a.priorities, a.n,
-                       a.capacity, a.alpha, a);
+    hipLaunchKernelGGL(k_update_stamp, dim3(grid_exact((uint64_t)n)), dim3(kWG), 0, s, a.indices, a.priorities, a.stamp, a.powered, a.maxp,
+                       (uint32_t)a.n, (uint32_t)a.capacity, a.epoch, a.alpha, !sparse && a.nrounds ? a.dirty[0] : nullptr, a.g[0]);
     LAUNCH_CHECK("k_update_stamp");
     if (!sparse) return tree_rebuild(*b, a, s);
     const auto checked = [](hipError_t e, const char* name) {
@@ -1505,8 +1505,9 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
     if (stamp_after) {
         a.priorities = opt_priorities;
         a.n = nrows;
-        hipLaunchKernelGGL(k_update_stamp, dim3(grid_exact((uint64_t)nrows)), dim3(kWG), 0, s, a.indices, a.priorities, a.n,
-                       a.capacity, a.alpha, a);
+        // (no indices: nothing to elect, the priorities are looked at and folded into the running max)
+        hipLaunchKernelGGL(k_update_stamp, dim3(grid_exact((uint64_t)nrows)), dim3(kWG), 0, s, a.indices, a.priorities, a.stamp, a.powered, a.maxp,
+                           (uint32_t)a.n, (uint32_t)a.capacity, a.epoch, a.alpha, static_cast<uint32_t*>(nullptr), 0);
         LAUNCH_CHECK("k_update_stamp");
     }
     b->pushes += nrows;

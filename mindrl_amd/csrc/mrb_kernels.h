@@ -602,36 +602,32 @@ __global__ __launch_bounds__(kRowWaveWG) void k_rows_gather_rows(const int64_t* 
 // behind; recomputing a clean node reproduces its bits. No float is ever
 // accumulated atomically.
 // ---------------------------------------------------------------------------
-// (The leading plain parameters repeat members of `a_in`: preloaded into scalar registers, so the entries are requested
-// when a wave starts.)
-__global__ __launch_bounds__(kWG) void k_update_stamp(const int64_t* __restrict__ lead_indices, const float* __restrict__ lead_priorities,
-                                                      int64_t lead_n, int64_t lead_capacity, float lead_alpha, UpdateArgs a_in) {
-    UpdateArgs a = a_in;
-    a.indices = lead_indices;
-    a.priorities = lead_priorities;
-    a.n = lead_n;
-    a.capacity = lead_capacity;
-    a.alpha = lead_alpha;
-    const int64_t j = (int64_t)blockIdx.x * kWG + threadIdx.x;
+// (Everything but the dirty words comes in preloaded arguments, and an entry bids for its leaf before its power is taken: what bounds this kernel is a
+// chain of two trips, the entry and the bid, and the power need not stand between them. An update of 16,384 entries on 2^22 leaves 12.0 -> 11.5 us, of 65,536
+// on 2^24 22.9 -> 22.1, on 2^20 16.5 -> 16.0.)
+__global__ __launch_bounds__(kWG) void k_update_stamp(const int64_t* __restrict__ indices, const float* __restrict__ priorities,
+                                                      unsigned long long* __restrict__ stamp, float* __restrict__ powered, float* maxp, uint32_t n,
+                                                      uint32_t capacity, uint32_t epoch, float alpha, uint32_t* __restrict__ dirty, int g) {
+    const uint64_t j = (uint64_t)blockIdx.x * kWG + threadIdx.x;
     float q = 0.0f;
-    if (j < a.n) {
-        const float p = a.priorities[j];
-        int64_t idx = a.indices ? a.indices[j] : 0;
-        const bool idx_ok = !a.indices || (idx >= 0 && idx < a.capacity);
-        if (!idx_ok) atomicOr(a.err, MRB_DERR_INDEX);
-        if (!valid_priority(p)) atomicOr(a.err, MRB_DERR_PRIORITY);
-        if (idx_ok && valid_priority(p)) {
-            q = powf_det_call(p, a.alpha);
-            if (a.indices) {
-                a.powered[j] = q;
-                atomicMax(&a.stamp[idx], ((unsigned long long)a.epoch << 32) | (unsigned long long)j);
-                if (!a.sparse_g0 && a.nrounds) a.dirty[0][idx >> a.g[0]] = a.epoch;
+    if (j < n) {
+        const float p = priorities[j];
+        const int64_t idx = indices ? indices[j] : 0;
+        const bool idx_ok = idx >= 0 && idx < (int64_t)capacity, ok = valid_priority(p);
+        if (!idx_ok) atomicOr(err_before(maxp), MRB_DERR_INDEX);
+        if (!ok) atomicOr(err_before(maxp), MRB_DERR_PRIORITY);
+        if (idx_ok && ok) {
+            if (indices) {
+                atomicMax(&stamp[idx], ((unsigned long long)epoch << 32) | j);
+                if (dirty) dirty[idx >> g] = epoch;
             }
+            q = powf_det(p, alpha);
+            if (indices) powered[j] = q;
         }
     }
     // wave max, then one integer atomic per wave
     q = wave_max(q);
-    if ((threadIdx.x & 63) == 0 && q > 0.0f) raise_max(a.maxp, q);
+    if ((threadIdx.x & 63) == 0 && q > 0.0f) raise_max(maxp, q);
 }
 
 // New value of leaf `leaf`, if this call writes it.
