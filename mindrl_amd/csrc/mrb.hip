@@ -836,15 +836,15 @@ UpdateArgs update_args(Per& b) {
 // the call's entries); larger calls take the stamp pass (2048 measured: config 4's update 14.0 us against 14.7 with the pass, at twice the waves and four times the comparisons: not taken).
 constexpr int64_t kElectMax = 1024;
 
-// Whether one launch takes an update by runs of leaves: k_range_one. More than 1024 entries on 21 levels and more are faster on
-// the device by two (k_tree_range, k_tree_cap): 2048 8.7 against 9.1 us, 4096 10.2 against 10.7; on 20 levels 8.4 / 8.5 and
-// 9.3 / 9.4, and the host is spared a launch (2.7 us). Trees of fewer than 8 levels have no whole tile, those of more than 22 more
-// than 256 runs.
+// Whether an update of few entries goes by runs of leaves in k_range_one, whose workgroups read the priorities with the indices and leave where
+// they have no entry, rather than in k_tree_range. us, 20 levels: 1024 entries 6.9 / 7.3, 1500 8.0 / 7.7, 4096 9.3 / 8.9, one after the other 1500 7.4 / 7.5, 3000
+// 9.4 / 9.7, 4096 10.8 / 11.3; 21 levels 512 6.4 / 7.1, 1024 7.5 / 7.5; 22 levels 1024 7.8 / 8.0. Trees of fewer than 8 levels have no whole tile, those of
+// more than 22 more than 256 runs.
 bool takes_range_one(const Per& b, int64_t n) {
     return b.fused && n <= (b.depth <= 20 ? kOneMostEntries : kElectMax) && b.depth >= 8 && b.depth <= 22;
 }
 
-// Whether an update goes by runs of leaves in two launches (launch_tree_range). Against what it would take
+// Whether an update of more entries goes by runs of leaves (launch_tree_range). Against what it would take
 // otherwise, us per call, before / by runs:
 //   most entries    12 levels, 8192 / 16,384: 10.0 / 11.4 against 9.6 / 13.8; 14 levels, 16,384 / 32,768: 11.7 / 12.5 against 11.2 / 16.7; 20 levels 14.4 / 15.4 against
 //                   14.1 / 18.7. On 21 levels and more what its entries drive is the other way: see takes_sparse.
@@ -852,14 +852,15 @@ bool takes_range_one(const Per& b, int64_t n) {
 //                   entries 14.9 / 15.9 against 14.9 / 23.3.
 bool takes_range(const Per& b, int64_t n) {
     if (!b.fused || b.depth < 12 || b.depth > 22) return false;
-    return !takes_range_one(b, n) && n <= (b.depth == 22 ? 4096 : b.depth == 12 || b.depth == 21 ? 8192 : 16384);
+    return !takes_range_one(b, n) && n <= (b.depth >= 21 ? 3072 : b.depth == 12 ? 8192 : 16384);
 }
 
 // Whether the entries drive the lowest levels of an update (launch_tree_sparse), with more than the 1024 that elect among themselves. The other ways
-// look at every tile of the tree, or at every entry in every workgroup. us per call, by tiles (runs of leaves up to 8192 entries) / by entries, slots at random and,
+// look at every tile of the tree, or at every entry in every workgroup. us per call, by tiles (up to 8193 entries by runs of leaves) / by entries, slots at random and,
 // behind the comma, one after the other:
-//   21 levels  8193 12.1 / 11.4, 16,384 14.9 / 12.4, 32,768 20.7 / 14.7, 10.9 / 10.4; 65,536 23.4 / 19.7, 11.0 / 11.6; 131,072 27.9 / 29.0
-//   22 levels  4096 10.8 / 11.1, 5000 12.0 / 11.2, 8192 13.2 / 11.6, 32,768 29.6 / 15.0, 131,072 38.7 / 32.0, 14.6 / 13.2; 200,000 43.3 / 43.0, 15.2 / 16.2
+//   21 levels  3000 9.0 / 9.5, 10.1 / 8.6; 4096 9.6 / 9.5, 11.7 / 8.8; 8193 11.1 / 10.1, 16,384 14.9 / 11.4, 32,768 20.7 / 13.5, 10.9 / 9.5; 65,536 23.4 / 19.7,
+//              11.0 / 11.6; 131,072 27.9 / 29.0
+//   22 levels  2048 9.5 / 9.3, 3000 9.7 / 9.6, 10.7 / 8.8; 4096 10.7 / 9.7, 8192 13.2 / 10.2, 32,768 29.6 / 13.9, 131,072 38.7 / 32.0, 14.6 / 13.2; 200,000 43.3 / 43.0, 15.2 / 16.2
 //   23 levels  131,072 56 / 34, 262,144 66 / 56, 19.7 / 18.2; 524,288 83 / 95
 //   24 levels  131,072 93 / 36, 262,144 116 / 63, 27 / 18; 524,288 138 / 156; 25 levels  262,144 189 / 110, 524,288 235 / 173
 //   26 levels  524,288 368 / 338, 75 / 50; 1,048,576 458 / 599; deeper trees were not measured
@@ -896,10 +897,8 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
         return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch k_range_one: %s", hipGetErrorString(e));
     }
     if (takes_range(*b, n)) {
-        hipError_t e = launch_tree_range(indices, priorities, n, b->sum, b->mn, b->maxp, b->rows.capacity, b->depth, b->alpha, s);
+        const hipError_t e = launch_tree_range(indices, priorities, n, b->sum, b->mn, b->maxp, b->rows.capacity, b->depth, b->alpha, s);
         if (e != hipSuccess) return fail(MRB_EHIP, "launch k_tree_range: %s", hipGetErrorString(e));
-        e = launch_tree_cap(b->sum, b->mn, b->depth - tree_range_levels(b->depth), s);
-        if (e != hipSuccess) return fail(MRB_EHIP, "launch k_tree_cap: %s", hipGetErrorString(e));
         return MRB_OK;
     }
     int rc = next_epoch(*b, s);

@@ -1,4 +1,4 @@
-// update_priorities of a few thousand entries as two launches, and the rebuild of very large trees (defined in
+// update_priorities of a few thousand entries by runs of leaves, and the rebuild of very large trees (defined in
 // mrb_range.hip).
 #pragma once
 #include <hip/hip_runtime.h>
@@ -18,7 +18,5 @@ hipError_t launch_tree_sparse(const int64_t* indices, const unsigned long long* 
                               hipStream_t s);
 // From depth `top` (17 to 20) to the root: the tiles of 256 nodes whose word in `dirty` carries the epoch.
 hipError_t launch_tree_runs(float* sum, float* mn, const uint32_t* dirty, float* maxp, int top, uint32_t epoch, hipStream_t s);
-// The levels above depth `top`, at most 8.
-hipError_t launch_tree_cap(float* sum, float* mn, int top, hipStream_t s);
 
 }  // namespace mrb

@@ -19,13 +19,14 @@ struct Trees {
 // mindspore_rl/core/priority_replay_buffer.py:71-73,120), divided by LEAVES: a workgroup owns a run of 2^w leaves,
 // looks every entry of the call over for those aimed at its leaves, elects the last one of each leaf in an LDS table
 // with a word per leaf, rebuilds the tiles that changed, a wave each, and goes on with its w levels to the run's root.
-// What is left above is a small tree (k_tree_cap). No stamps in memory, no pass of its own for the election, no wave for
-// a clean tile, no launch between the leaves and the run's root: two launches instead of three or four. What it pays is
-// that every workgroup reads all indices (out of its L2: 16 KB for 2048 entries), which is why larger calls keep the
+// The last workgroup to get there rebuilds the levels above the runs (mrb_meet.h; all of them meet, also those without an entry, whose
+// root is as it was). No stamps in memory, no pass of its own for the election, no wave for a clean tile, one launch instead of three or
+// four. What it pays is that every workgroup reads all indices (out of its L2: 16 KB for 2048 entries), which is why larger calls keep the
 // stamp pass (the rule, with both sides measured, is at takes_range).
-// A call is bound by its chain of trips - indices, priorities of a run's own, tiles, then the second launch's tile -, not
-// by bytes. 2048 entries on 2^21 leaves 14.7 -> 8.6 us. (Up to 1024 entries, up to 4096 on at most 20 levels, one launch does the same:
-// k_range_one.)
+// A call is bound by its chain of trips - indices, priorities of a run's own, tiles, the roots' meeting -, not
+// by bytes. 2048 entries on 2^21 leaves 14.7 -> 8.6 us, and 8.4 with the meeting in the place of a
+// second launch (5000 on 2^20 9.5 -> 9.0, 5000 one after the other on 2^14 6.7 -> 6.5), which a host that is behind takes 2.7 us longer to issue. (Up to 1024 entries, up to
+// 4096 on at most 20 levels, k_range_one, whose workgroups read the priorities with the indices, is faster.)
 // ---------------------------------------------------------------------------
 // (no argument for what the kernel can tell: see PutArgs::threads)
 __host__ __device__ constexpr int range_threads(int64_t n) { return n > 4096 ? 1024 : 512; }  // (256: 0.3 to 1.5 us more)
@@ -46,6 +47,8 @@ __global__ __launch_bounds__(1024) void k_tree_range(const int64_t* __restrict__
     const Trees trees{sum, mn};
     const int threads = range_threads(n), trip = kRangePer * threads;
     uint32_t* const err = err_before(maxp);
+    const int top = depth - w;  // levels above the runs, at least two
+    const uint32_t runs = ((uint32_t)capacity + leaves - 1) >> w;
     auto request = [&](int base, int64_t (&to)[kRangePer]) {
 #pragma unroll
         for (int q = 0; q < kRangePer; ++q) {
@@ -55,6 +58,19 @@ __global__ __launch_bounds__(1024) void k_tree_range(const int64_t* __restrict__
     };
     int64_t idx[kRangePer];
     request(0, idx);
+    // the launch's number and the runs' roots as they are, this one's among them
+    uint32_t turn = 0;
+    float4 vs = make_float4(0.f, 0.f, 0.f, 0.f), vm = vs;
+    float cs = 0.0f, cm = 0.0f;
+    if (wave == 0) {
+        turn = meet_turn(maxp);
+        cs = sum[(1u << top) + run];
+        cm = mn[(1u << top) + run];
+        if (4 * lane < (1u << top)) {
+            vs = *reinterpret_cast<const float4*>(sum + (1u << top) + 4 * lane);
+            vm = *reinterpret_cast<const float4*>(mn + (1u << top) + 4 * lane);
+        }
+    }
     // the roots as they are, for the tiles that stay clean; the table is cleared while the entries are on their way
     const uint32_t root0 = ((1u << depth) + run * leaves) >> kRoundLevels;
     if (tid < tiles) {
@@ -111,43 +127,44 @@ __global__ __launch_bounds__(1024) void k_tree_range(const int64_t* __restrict__
     lds_barrier();
     // the tiles that changed, dealt to the waves
     const unsigned long long dirty = __ballot(lane < tiles && s_dirty[lane < tiles ? lane : 0] != 0);
-    if (dirty == 0) return;  // (the same in every wave)
+    if (dirty == 0 && wave != 0) return;
     uint32_t nth = 0;
     for (unsigned long long rest = dirty; rest; rest &= rest - 1, ++nth) {
         if (nth % ((uint32_t)threads / 64) != wave) continue;
         const uint32_t t = (uint32_t)__builtin_ctzll(rest);
         const uint32_t first = (1u << depth) + run * leaves + t * kBlockNodes;
-        float4 vs = *reinterpret_cast<const float4*>(sum + first + 4 * lane);
-        float4 vm = *reinterpret_cast<const float4*>(mn + first + 4 * lane);
+        float4 ls = *reinterpret_cast<const float4*>(sum + first + 4 * lane);
+        float4 lm = *reinterpret_cast<const float4*>(mn + first + 4 * lane);
         const ulonglong2 k01 = *reinterpret_cast<const ulonglong2*>(&s_win[t * kBlockNodes + 4 * lane]);
         const ulonglong2 k23 = *reinterpret_cast<const ulonglong2*>(&s_win[t * kBlockNodes + 4 * lane + 2]);
-        if (k01.x) vs.x = vm.x = elected_priority(k01.x);
-        if (k01.y) vs.y = vm.y = elected_priority(k01.y);
-        if (k23.x) vs.z = vm.z = elected_priority(k23.x);
-        if (k23.y) vs.w = vm.w = elected_priority(k23.y);
+        if (k01.x) ls.x = lm.x = elected_priority(k01.x);
+        if (k01.y) ls.y = lm.y = elected_priority(k01.y);
+        if (k23.x) ls.z = lm.z = elected_priority(k23.x);
+        if (k23.y) ls.w = lm.w = elected_priority(k23.y);
         if (k01.x | k01.y | k23.x | k23.y) {
-            *reinterpret_cast<float4*>(sum + first + 4 * lane) = vs;
-            *reinterpret_cast<float4*>(mn + first + 4 * lane) = vm;
+            *reinterpret_cast<float4*>(sum + first + 4 * lane) = ls;
+            *reinterpret_cast<float4*>(mn + first + 4 * lane) = lm;
         }
         float rs, rm;
-        tile_parents(trees, kRoundLevels, first, lane, true, vs, vm, &rs, &rm);
+        tile_parents(trees, kRoundLevels, first, lane, true, ls, lm, &rs, &rm);
         if (lane == 0) {
             s_rs[t] = rs;
             s_rm[t] = rm;
         }
     }
-    lds_barrier();
-    if (wave != 0 || tiles == 1) return;
-    // from the tiles' roots to the run's (at most six levels)
-    float cs = lane < tiles ? s_rs[lane] : 0.0f, cm = lane < tiles ? s_rm[lane] : 0.0f;
-    for (int l = 1; l <= w - kRoundLevels; ++l) {
-        cs = cs + __shfl_xor(cs, 1 << (l - 1));
-        cm = fminf(cm, __shfl_xor(cm, 1 << (l - 1)));
-        if (lane < tiles && (lane & ((1u << l) - 1)) == 0) {
-            sum[(root0 + lane) >> l] = cs;
-            mn[(root0 + lane) >> l] = cm;
-        }
+    if (dirty != 0) {  // (the same in every wave)
+        lds_barrier();
+        if (wave != 0) return;
+        // from the tiles' roots to the run's (at most six levels)
+        cs = lane < tiles ? s_rs[lane] : 0.0f;
+        cm = lane < tiles ? s_rm[lane] : 0.0f;
+        run_parents(trees, w - kRoundLevels, root0, lane, lane < tiles, cs, cm);
     }
+    // and from the runs' to the tree's
+    const uint32_t mine = 4 * lane < runs ? (runs - 4 * lane >= 4 ? 15u : (1u << (runs - 4 * lane)) - 1) : 0u;
+    const MeetPlan plan = meet_plan(mine, run, lane);
+    if (!meet(maxp, err, turn, run, cs, cm, lane, plan, vs, vm)) return;
+    tile_parents(trees, top, 1u << top, lane, 4 * lane < (1u << top), vs, vm);
 }
 
 // ---------------------------------------------------------------------------
@@ -178,12 +195,13 @@ __device__ __forceinline__ void sparse_step(const Trees& a, int g0, uint32_t fir
     }
 }
 
-// plan: depth | g0 << 8 | g_dirty << 16
+// plan: depth | g0 << 8 | g_dirty << 16. kG0: g0 where the compiler is to know it (four: trees of up to 24 levels), or 0.
+template <int kG0>
 __global__ __launch_bounds__(kSparseWG) void k_tree_sparse(const int64_t* __restrict__ indices,
                                                            const unsigned long long* __restrict__ stamp,
                                                            const float* __restrict__ powered, float* sum, float* mn, uint32_t* dirty,
                                                            int n, uint32_t capacity, uint32_t epoch, int plan) {
-    const int depth = plan & 255, g0 = (plan >> 8) & 255, g_dirty = plan >> 16;
+    const int depth = plan & 255, g0 = kG0 ? kG0 : (plan >> 8) & 255, g_dirty = plan >> 16;
     const uint32_t group = 1u << (g0 - 2);
     const uint32_t tid = blockIdx.x * kSparseWG + threadIdx.x;
     const uint32_t j = tid >> (g0 - 2), sub = tid & (group - 1);
@@ -283,26 +301,6 @@ __global__ __launch_bounds__(1024) void k_tree_runs(float* sum, float* mn, const
     tile_parents(trees, kRoundLevels, kBlockNodes, lane, true, roots_s, roots_m);
 }
 
-// The levels above depth `top` (1 .. 8): one wave, everything it needs in preloaded registers, one trip to memory.
-__global__ __launch_bounds__(64) void k_tree_cap(float* sum, float* mn, int top) {
-    const uint32_t lane = threadIdx.x, nodes = 1u << top;
-    const Trees trees{sum, mn};
-    if (top == 1) {
-        if (lane == 0) {
-            sum[1] = sum[2] + sum[3];
-            mn[1] = fminf(mn[2], mn[3]);
-        }
-        return;
-    }
-    const bool active = 4 * lane < nodes;
-    float4 vs = make_float4(0.f, 0.f, 0.f, 0.f), vm = vs;
-    if (active) {
-        vs = *reinterpret_cast<const float4*>(sum + nodes + 4 * lane);
-        vm = *reinterpret_cast<const float4*>(mn + nodes + 4 * lane);
-    }
-    tile_parents(trees, top, nodes, lane, active, vs, vm);
-}
-
 }  // namespace
 
 // Runs of 256 to 16,384 leaves: 256 of them - and eight levels left above, one tile - where that is possible (16 to 22
@@ -325,18 +323,13 @@ hipError_t launch_tree_sparse(const int64_t* indices, const unsigned long long* 
                               uint32_t* dirty, int64_t n, int64_t capacity, int depth, int g0, int g_dirty, uint32_t epoch,
                               hipStream_t s) {
     const dim3 grid((uint32_t)(((n << (g0 - 2)) + kSparseWG - 1) / kSparseWG));
-    hipLaunchKernelGGL(k_tree_sparse, grid, dim3(kSparseWG), 0, s, indices, stamp, powered, sum, mn, dirty, (int)n, (uint32_t)capacity,
+    hipLaunchKernelGGL(g0 == 4 ? k_tree_sparse<4> : k_tree_sparse<0>, grid, dim3(kSparseWG), 0, s, indices, stamp, powered, sum, mn, dirty, (int)n, (uint32_t)capacity,
                        epoch, depth | g0 << 8 | g_dirty << 16);
     return hipGetLastError();
 }
 
 hipError_t launch_tree_runs(float* sum, float* mn, const uint32_t* dirty, float* maxp, int top, uint32_t epoch, hipStream_t s) {
     hipLaunchKernelGGL(k_tree_runs, dim3(1u << kRoundLevels), dim3(64u << (top - 2 * kRoundLevels)), 0, s, sum, mn, dirty, maxp, epoch, top);
-    return hipGetLastError();
-}
-
-hipError_t launch_tree_cap(float* sum, float* mn, int top, hipStream_t s) {
-    hipLaunchKernelGGL(k_tree_cap, dim3(1), dim3(64), 0, s, sum, mn, top);
     return hipGetLastError();
 }
 

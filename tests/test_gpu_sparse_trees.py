@@ -54,8 +54,8 @@ def test_every_node_above_the_entries(capacity, n):
 
 
 # (21 levels' own lines: fewer entries go by runs of leaves, more by tiles; and the most entries of 22 to 24 levels)
-@pytest.mark.parametrize("capacity,n", [((1 << 21) - 7, 8192), ((1 << 21) - 7, 8193), ((1 << 20) + 1, 20_000), (1 << 21, 32_768), (1 << 21, 32_769),
-                                        ((1 << 22) - 1, 4096), ((1 << 22) - 1, 4097), (1 << 22, 131_072), (1 << 22, 131_073),
+@pytest.mark.parametrize("capacity,n", [((1 << 21) - 7, 3072), ((1 << 21) - 7, 3073), ((1 << 20) + 1, 20_000), (1 << 21, 32_768), (1 << 21, 32_769),
+                                        ((1 << 22) - 1, 3072), ((1 << 22) - 1, 3073), (1 << 22, 131_072), (1 << 22, 131_073),
                                         ((1 << 23) - 1, 262_144), ((1 << 24) - 1, 262_144)])
 def test_where_the_entries_take_over(capacity, n):
     test_every_node_above_the_entries(capacity, n)
