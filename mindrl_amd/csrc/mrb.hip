@@ -456,15 +456,23 @@ void launch_gather_wide(dim3 grid, const int64_t* indices, int mode, int64_t cou
 }
 
 // Gather of n rows whose slots are given (indices), drawn from the generator (indices NULL,
-// fixed_slot < 0) or one fixed slot. Rows with a field of at least 1 KB go through the wide-row
-// kernel (a workgroup per row, all loads before the first store), narrow rows through the flat kernel.
+// fixed_slot < 0) or one fixed slot: by a kernel that numbers a field's granules over all rows, or one that
+// gives a row a workgroup or a wave.
 int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, int64_t count, uint64_t seed,
                 uint64_t calls, int64_t n, int64_t* out_indices, void* const* dst_fields, uint32_t* err,
                 hipStream_t s) {
     IoTable t;
     int rc = make_table(r, dst_fields, n, t);
     if (rc) return rc;
-    if (widest_field(r) >= 1024 && n <= (1ll << 24)) {
+    ShortIo io{};
+    const bool brief = fixed_slot < 0 && n <= 0xffffffffll && (out_indices ? short_io(out_indices, nullptr, t, io) : short_io(t, io));
+    const uint64_t most = most_granules(t);
+    // A workgroup per row is the faster one for some hundred rows of 4 KB and more, which are too few granules for four to a thread (workgroup per row /
+    // flat, us): 3.2 KB 64 rows 3.1 / 2.5, 1024 3.9 / 3.8; 7.5 KB 64 3.2 / 3.0, 512 4.0 / 4.2, 1024 5.3 / 5.5, 2048 8.8 / 8.5, 16,384 43 / 37; 28 KB 64 3.9 / 2.9,
+    // 128 4.3 / 3.6, 512 7.4 / 7.6 (given slots 5.7 / 6.3), 1024 12.5 / 11.7, 8192 63.5 / 58.7. (A wave per row: 1 KB 4096 rows 5.7 / 4.3, 2.4 KB 2048 5.4 / 4.8,
+    // 8192 11.8 / 10.8.) And it is what is asked for by row_split and row_wave, and for more than a brief launch's arguments hold the kernels that take a plan.
+    const bool wide = widest_field(r) >= 4096 && most >= 200000 && most <= 1u << 20;
+    if (widest_field(r) >= 1024 && n <= (1ll << 24) && (wide || !brief || r.row_split != 0 || r.row_wave != 0)) {
         const int mode = fixed_slot >= 0 ? kFromFixedSlot : (indices ? kFromIndices : kFromGenerator);
         WidePlan plan;
         dim3 grid;
@@ -488,9 +496,9 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
         return MRB_OK;
     }
     // a row of workgroups per field, as many as the field with the most granules needs
-    const uint32_t blocks = grid_for(most_granules(t));
-    if (ShortIo io{}; fixed_slot < 0 && n <= 0xffffffffll && (out_indices ? short_io(out_indices, nullptr, t, io) : short_io(t, io))) {
-        const hipError_t e = launch_short_gather(r.table, io, t.nfields, indices, count, seed, calls, n, blocks, out_indices != nullptr, s);
+    const uint32_t blocks = grid_for(most);
+    if (brief) {
+        const hipError_t e = launch_short_gather(r.table, io, t, indices, count, seed, calls, n, blocks, out_indices != nullptr, s);
         return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch k_short_gather: %s", hipGetErrorString(e));
     }
     hipLaunchKernelGGL(k_rows_gather, dim3(blocks, (uint32_t)t.nfields), dim3(kWG), 0, s, indices, fixed_slot, seed, calls,

@@ -12,7 +12,7 @@
 //
 // By value stay: more than kShortPointers matrices, matrices too far apart at an odd address, device-resident counters, single-row
 // reads, copies from another buffer's ring; the sampling kernels and the reservoir's push (3.35 / 3.40 and 2.8 / 2.9 when they
-// were tried: their row copies come last, so the table's trip is not hidden); and the gather of wide rows, which takes a plan
+// were tried: their row copies come last, so the table's trip is not hidden); and the gather with a workgroup or a wave to a row, which takes a plan
 // that a wave divides its lanes by (within 4 % of each other either way, 24,831-byte rows slower short).
 #pragma once
 #include <hip/hip_runtime.h>
@@ -69,6 +69,26 @@ __host__ __device__ inline uint32_t put_blocks(uint64_t granules, uint32_t threa
     uint64_t blocks = (granules + threads - 1) / threads;
     if (blocks > kPutFew) blocks = (blocks + kPutTrip - 1) / kPutTrip;
     return (uint32_t)(blocks < 16384 ? blocks : 16384);
+}
+
+// The field whose workgroups hold number `block` of those of all fields, one field's behind the other's; `block` is left as the number among
+// that field's, which are `blocks`. (The fields' sizes in one trip: with a dependent one for each, and four granules to a
+// thread of the small fields too, a gather of 4096 rows of 400 bytes in five fields took 6.0 us, with a granule to a thread 3.3.)
+__device__ __forceinline__ int field_of_block(const RowTable* __restrict__ table, uint64_t n, uint32_t& block, uint32_t& blocks) {
+    uint32_t units[kShortPointers];
+#pragma unroll
+    for (int f = 0; f < kShortPointers; ++f) units[f] = table->t.units[f];
+    const int nfields = table->t.nfields;
+    int at = 0;
+    blocks = put_blocks(n * units[0], kWG);
+#pragma unroll
+    for (int f = 1; f < kShortPointers; ++f)
+        if (at == f - 1 && f < nfields && block >= blocks) {
+            block -= blocks;
+            blocks = put_blocks(n * units[f], kWG);
+            at = f;
+        }
+    return at;
 }
 
 // The copy of a ring append, one field's n rows by workgroup `block` of `blocks` with `threads` threads each. (A row of
@@ -128,14 +148,63 @@ __device__ __forceinline__ void put_fields(const RowTable* __restrict__ table, c
         put_field(table, io, blockIdx.y, first_slot, n, block, blocks, kWG);
         return;
     }
-    int f = 0;
-    for (;;) {
-        blocks = put_blocks((uint64_t)n * table->t.units[f], kWG);
-        if (block < blocks || f + 1 == table->t.nfields) break;
-        block -= blocks;
-        ++f;
-    }
+    const int f = field_of_block(table, n, block, blocks);
     put_field(table, io, f, first_slot, n, block, blocks, kWG);
+}
+
+// Workgroups of a gather's largest field, a granule to a thread, from which on threads take four of the large fields and every field has its own
+// number of workgroups. A granule to a thread / four, us: 809 bytes, 8192 rows 5.1 / 5.4, 16,384 8.1 / 7.8; 1.6 KB 2048 3.9 / 4.3, 4096 5.5 / 5.2, 16,384 17.2 / 12.5;
+// 2.4 KB 2048 4.8 / 5.0, 4096 6.9 / 6.4, 16,384 19.7 / 17.1; 7.5 KB 16,384 62.6 / 37.3.
+constexpr uint32_t kGatherFew = 1024;
+
+// A gather of many granules, one field's n rows by workgroup `block` of `blocks`: as put_field, with the rows' slots given or drawn (see gather_body).
+template <int kPer>
+__device__ __forceinline__ void gather_field(const ShortRows& rows, int f, const int64_t* __restrict__ indices, int64_t count, uint64_t seed,
+                                             uint64_t calls, uint32_t block, uint32_t blocks) {
+    const uint32_t units = rows.units(f), vl = rows.vl(f), row_bytes = rows.row_bytes(f), stride = rows.stride(f);
+    const gbyte* const store = as_global((const uint8_t*)rows.store(f));
+    gbyte* const to = as_global(rows.io(f));
+    int64_t* const out_indices = rows.first && f == 0 ? reinterpret_cast<int64_t*>(rows.s.at(0)) : nullptr;
+    const uint64_t total = rows.granules(f);
+    for (uint64_t w = (uint64_t)block * kWG * kPer + threadIdx.x; w < total; w += (uint64_t)blocks * kWG * kPer) {
+        uint64_t row[kPer];
+        uint32_t unit[kPer];
+        int64_t slot[kPer];
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+            split_work(w + q * kWG < total ? w + q * kWG : w, units, row[q], unit[q]);  // (past the end: the thread's first again)
+            slot[q] = indices ? indices[row[q]] : rng_below(seed, calls, row[q], count);
+        }
+        bool outside = false;
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+            outside = outside || slot[q] < 0 || slot[q] >= count;
+            slot[q] = slot[q] < 0 ? 0 : slot[q] >= count ? (count > 0 ? count - 1 : 0) : slot[q];
+            if (out_indices && unit[q] == 0) out_indices[row[q]] = slot[q];
+        }
+        if (outside) atomicOr(rows.r->err, MRB_DERR_INDEX);
+        if (kPer > 1) {  // (granules of 16 bytes)
+            granule_t held[kPer];
+#pragma unroll
+            for (int q = 0; q < kPer; ++q)
+                held[q] = __builtin_nontemporal_load((const g16*)(store + (uint64_t)slot[q] * stride + granule_offset(unit[q], 4, row_bytes)));
+#pragma unroll
+            for (int q = 0; q < kPer; ++q) asm volatile("" : "+v"(held[q]));
+#pragma unroll
+            for (int q = 0; q < kPer; ++q)
+                if (w + q * kWG < total) *(g16*)(to + row[q] * row_bytes + granule_offset(unit[q], 4, row_bytes)) = held[q];
+        } else {
+            const uint32_t off = granule_offset(unit[0], vl, row_bytes);
+            copy_granule(to + row[0] * row_bytes + off, store + (uint64_t)slot[0] * stride + off, vl);
+        }
+    }
+}
+__device__ __forceinline__ void gather_fields(const ShortRows& rows, const int64_t* __restrict__ indices, int64_t count, uint64_t seed, uint64_t calls,
+                                              uint32_t block) {
+    uint32_t blocks;
+    const int f = field_of_block(rows.r, rows.n, block, blocks);
+    if (rows.vl(f) == 4 && rows.granules(f) > (uint64_t)kPutFew * kWG) gather_field<kPutTrip>(rows, f, indices, count, seed, calls, block, blocks);
+    else gather_field<1>(rows, f, indices, count, seed, calls, block, blocks);
 }
 
 // `blocks` of such a launch, and its grid behind (in x) `in_front` other workgroups. (t: the call's table.)
@@ -150,7 +219,7 @@ inline dim3 put_grid(const IoTable& t, uint32_t in_front, uint32_t& blocks) {
     return blocks ? dim3(in_front + blocks, (uint32_t)t.nfields) : dim3(in_front + all);
 }
 
-hipError_t launch_short_gather(const RowTable* table, const ShortIo& io, int nfields, const int64_t* indices, int64_t count, uint64_t seed,
+hipError_t launch_short_gather(const RowTable* table, const ShortIo& io, const IoTable& t, const int64_t* indices, int64_t count, uint64_t seed,
                                uint64_t calls, int64_t n, uint32_t blocks, bool with_indices, hipStream_t s);
 hipError_t launch_short_put(const RowTable* table, const ShortIo& io, const IoTable& t, int64_t first_slot, int64_t n, hipStream_t s);
 // (granules: the field's with the most)

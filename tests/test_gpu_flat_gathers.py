@@ -1,0 +1,49 @@
+"""Gathers that number the granules of a field over all rows: on both sides of the number from which on a thread takes four, of
+rows that went to other kernels before, in up to eight fields; drawn slots and given ones, some of them no slot of the buffer."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import random_rows, t2n, to_dev, torch_types
+
+pytestmark = pytest.mark.gpu
+
+F, U, L, B, H = np.float32, np.uint8, np.int64, np.bool_, np.float16
+
+
+@pytest.mark.parametrize("shapes,dtypes,batches", [
+    ([(1024,), (1,), (1,), (1,)], [U, L, F, B], (64, 4096, 4097, 9000)),          # 64 granules: 1024 workgroups, and more
+    ([(301,), (9,), (1,), (301,), (1,)], [F, F, F, F, B], (500, 3449, 3450)),      # two large fields, one of three granules
+    ([(1,), (2413,), (5,), (45,), (999,), (3, 3), (33,)], [B, U, F, H, U, U, L], (1700, 1737)),  # the first one small, all of odd sizes
+    ([(7500,)] + [(1,)] * 7, [U] * 8, (425, 426, 2230, 2236)),                     # eight fields; around those with a workgroup to a row
+    ([(28224,), (1,)], [U, L], (113, 114, 594, 595)),
+])
+@pytest.mark.parametrize("packed", [0, 4096])
+def test_flat_gathers(shapes, dtypes, batches, packed):
+    from mindrl_amd.core import UniformReplayBuffer
+    from oracle import orc
+    if packed and sum(int(np.prod(s)) * np.dtype(d).itemsize for s, d in zip(shapes, dtypes)) > 4096:
+        pytest.skip("rows too large to pack")
+    rng = np.random.default_rng(len(shapes))
+    cap = max(batches) + 50
+    for batch in batches:
+        g = UniformReplayBuffer(batch, cap, shapes, torch_types(dtypes), seed=4, packed_rows=packed)
+        c = orc.OracleUniform(cap, shapes, dtypes, seed=4)
+        new = random_rows(rng, cap - 30, shapes, dtypes)
+        g.insert(to_dev(new))
+        c.append(new, cap - 30)
+        idx, fields = g.sample_with_indices() if len(shapes) < 8 else (None, g.sample())
+        want_idx, want = c.sample(batch)
+        assert idx is None or np.array_equal(t2n(idx), want_idx), batch
+        assert all(np.array_equal(t2n(a), b) for a, b in zip(fields, want)), batch
+        given = rng.integers(0, cap - 30, batch)
+        fields = g.sample(torch.from_numpy(given).cuda())
+        assert all(np.array_equal(t2n(a), b[given]) for a, b in zip(fields, new)), batch
+        g.check()
+        given[batch // 2], given[-1] = cap - 30, -1
+        fields = g.sample(torch.from_numpy(given).cuda())
+        with pytest.raises(IndexError):
+            g.check()
+        given = np.clip(given, 0, cap - 31)
+        assert all(np.array_equal(t2n(a), b[given]) for a, b in zip(fields, new)), batch
+        g.destroy()
