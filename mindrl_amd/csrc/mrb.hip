@@ -468,9 +468,10 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
     const bool brief = fixed_slot < 0 && n <= 0xffffffffll && (out_indices ? short_io(out_indices, nullptr, t, io) : short_io(t, io));
     const uint64_t most = most_granules(t);
     // A workgroup per row is the faster one for some hundred rows of 4 KB and more, which are too few granules for four to a thread (workgroup per row /
-    // flat, us): 3.2 KB 64 rows 3.1 / 2.5, 1024 3.9 / 3.8; 7.5 KB 64 3.2 / 3.0, 512 4.0 / 4.2, 1024 5.3 / 5.5, 2048 8.8 / 8.5, 16,384 43 / 37; 28 KB 64 3.9 / 2.9,
-    // 128 4.3 / 3.6, 512 7.4 / 7.6 (given slots 5.7 / 6.3), 1024 12.5 / 11.7, 8192 63.5 / 58.7. (A wave per row: 1 KB 4096 rows 5.7 / 4.3, 2.4 KB 2048 5.4 / 4.8,
-    // 8192 11.8 / 10.8.) And it is what is asked for by row_split and row_wave, and for more than a brief launch's arguments hold the kernels that take a plan.
+    // flat, us): 3.2 KB 32 rows 3.0 / 2.4, 1024 3.9 / 3.7; 7.5 KB 32 3.1 / 2.8, 256 3.4 / 3.3, 512 4.0 / 4.2, 1024 5.3 / 5.5, 4096 15.2 / 14.1; 28 KB 32 3.7 / 2.7,
+    // 128 4.3 / 3.6, 512 7.4 / 7.6 (given slots 5.7 / 6.3), 2048 22.9 / 22.5. (A wave per row: 1 KB 2048 rows 4.9 / 3.6, 8192 7.6 / 6.1; 2.1 KB 8192
+    // 13.0 / 10.6; 2.4 KB 2048 5.3 / 4.7, 16,384 17.5 / 17.9.) And it is what is asked for by row_split and row_wave, and for more than a brief launch's
+    // arguments hold the kernels that take a plan.
     const bool wide = widest_field(r) >= 4096 && most >= 200000 && most <= 1u << 20;
     if (widest_field(r) >= 1024 && n <= (1ll << 24) && (wide || !brief || r.row_split != 0 || r.row_wave != 0)) {
         const int mode = fixed_slot >= 0 ? kFromFixedSlot : (indices ? kFromIndices : kFromGenerator);
@@ -692,12 +693,12 @@ int ride_alone_if_large(const UpdateArgs& a, PutArgs& put, hipStream_t s) {
     return MRB_OK;
 }
 
-// A push under at most 16 leaf tiles on a tree with rounds below its top is one launch of one workgroup, a wave per
+// A push under at most 16 leaf tiles on a tree with levels above them is one launch of one workgroup, a wave per
 // leaf tile (k_push_run; k_tree_fused where an update precedes it in the call): the number of those tiles, 0 where it
 // is not taken. (More than one tile per wave does not pay: the 16 waves of a workgroup share one compute unit's issue
 // slots, and a second tile costs a wave as much as the launch it would save; four cost twice as much.)
 uint32_t run_units(const Per& b, const UpdateArgs& a) {
-    if (a.nrounds == 0 || !b.fused || a.indices) return 0;
+    if (a.depth <= kRoundLevels || !b.fused || a.indices) return 0;
     uint64_t units;
     if (a.first_slot < 0) {
         units = push_units(a);  // the slots' start is only known on the device
@@ -793,7 +794,7 @@ constexpr int64_t kManyLeastTiles = 12;
 constexpr int kManyLeastDepth = 17;
 constexpr uint32_t kManyCopy = 1024;
 bool takes_push_many(const Per& b, int64_t first, int64_t n, bool with_priorities, uint32_t copy_blocks) {
-    if (b.device_counters || !b.fused || b.nrounds == 0 || first + n > b.rows.capacity) return false;
+    if (b.device_counters || !b.fused || b.depth <= kRoundLevels || first + n > b.rows.capacity) return false;
     const int64_t tiles = (first + n - 1) / kBlockNodes - first / kBlockNodes + 1;
     if (tiles > kManyMostTiles) return false;
     return with_priorities || tiles == 1 || tiles > kRunWaves || (tiles >= kManyLeastTiles && b.depth >= kManyLeastDepth) ||
@@ -1480,9 +1481,10 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
     // Only a call that overwrites rows of its own (more rows than capacity) needs a pass over all priorities.
     a.first_slot = b->device_counters ? -1 : first;
     a.n = n;
+    const bool run = run_units(*b, a) != 0;
     const int fold = !opt_priorities ? 0
-                     : (skip == 0 && nrows <= 1024 && !run_units(*b, a)) ? 1
-                     : (skip == 0 && a.nrounds > 0) ? 2 : 0;
+                     : (skip == 0 && nrows <= 1024 && !run) ? 1
+                     : (skip == 0 && (run || a.nrounds > 0)) ? 2 : 0;
     if (opt_priorities) {
         a.priorities = opt_priorities + skip;
         a.fold_max = fold;

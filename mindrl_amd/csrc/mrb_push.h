@@ -51,7 +51,7 @@ struct UpdateArgs {
 };
 
 // ---------------------------------------------------------------------------
-// A push under at most 16 leaf tiles on a tree of more than 12 levels, in ONE launch: a run of slots changes one path
+// A push under at most 16 leaf tiles on a tree of more than 8 levels, in ONE launch: a run of slots changes one path
 // of tiles - a wave rebuilds each leaf tile, then the tile eight levels up that holds their roots (two where the run
 // crosses its end, one more where it wraps around the ring), then the tile above that, up to the root. Which tiles
 // these are follows from the slots, so all of them are requested when the kernel starts: of their nodes only the
@@ -59,7 +59,8 @@ struct UpdateArgs {
 // memory and two to four rebuilds in a row (within one workgroup, whose waves share a compute unit: no fence), where
 // a launch per eight levels pays a launch, a trip and a rebuild for each. Measured, us per call before and now, plain /
 // with priorities: 64 rows into 2^24 leaves (three launches before) 12.0 / 10.6 and 3.8 / 5.6; 16 rows into 2^20 (one
-// launch that rebuilt the whole top) 4.2 / 6.5 and 3.8 / 5.3; 1024 rows into 2^21 4.8 / 7.4 and 4.3 / 5.6. With 4096
+// launch that rebuilt the whole top) 4.2 / 6.5 and 3.8 / 5.3; 1024 rows into 2^21 4.8 / 7.4 and 4.3 / 5.6; 64 rows into 2^12 (one workgroup that
+// rebuilt the whole tree) 4.3 / 6.2 and 2.6 / 3.4, into 2^9 3.6 / 5.6 and 2.4 / 3.2. With 4096
 // priorities the powers of one compute unit are the bound (5.6 / 8.7): k_push_many, which shares them out, takes pushes with
 // priorities where it can (takes_push_many). The row copy rides along as further workgroups of the
 // kernels that call this (k_push_run, k_short_push_run).

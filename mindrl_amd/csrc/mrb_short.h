@@ -153,8 +153,9 @@ __device__ __forceinline__ void put_fields(const RowTable* __restrict__ table, c
 }
 
 // Workgroups of a gather's largest field, a granule to a thread, from which on threads take four of the large fields and every field has its own
-// number of workgroups. A granule to a thread / four, us: 809 bytes, 8192 rows 5.1 / 5.4, 16,384 8.1 / 7.8; 1.6 KB 2048 3.9 / 4.3, 4096 5.5 / 5.2, 16,384 17.2 / 12.5;
-// 2.4 KB 2048 4.8 / 5.0, 4096 6.9 / 6.4, 16,384 19.7 / 17.1; 7.5 KB 16,384 62.6 / 37.3.
+// number of workgroups. A granule to a thread / four, us: 421 bytes 16,384 rows 6.5 / 6.8; 898 bytes 16,384 9.9 / 10.2, given slots 10.4 / 9.9; 809 bytes 8192 rows
+// 5.1 / 5.4, 16,384 8.1 / 7.8; 1.6 KB 2048 3.9 / 4.3, 4096 5.5 / 5.2, 16,384 17.2 / 12.5; 2.4 KB 2048 4.8 / 5.0, 4096 6.9 / 6.4, 16,384 19.7 / 17.1; 7.5 KB
+// 4096 20.5 / 13.9.
 constexpr uint32_t kGatherFew = 1024;
 
 // A gather of many granules, one field's n rows by workgroup `block` of `blocks`: as put_field, with the rows' slots given or drawn (see gather_body).

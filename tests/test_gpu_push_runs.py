@@ -99,3 +99,27 @@ def test_running_max_comes_from_the_pushed_priorities_alone(cap, device_counters
         assert np.float32(g.max_priority) == np.float32(c.max_priority) < np.float32(1.0), (cap, n)
         assert_tree_equal(g, c, "cap %d n %d" % (cap, n))
     g.destroy()
+
+
+# 8 levels, which one workgroup rebuilds whole, and 9 to 12: one to four levels above the leaf tiles
+@pytest.mark.parametrize("device_counters", [0, 1])
+@pytest.mark.parametrize("cap,starts", [(256, [0, 200]), (257, [0, 250]), (510, [255, 500]), (512, [0, 511]), (1000, [0, 513, 990]),
+                                        (2048, [255, 2040]), (2049, [1, 2000]), (4096, [0, 300, 4000])])
+def test_push_runs_on_small_trees(cap, starts, device_counters):
+    test_push_runs(cap, starts, device_counters)
+
+
+@pytest.mark.parametrize("cap", [257, 1000, 4096])
+def test_saved_small_trees(cap):
+    """A state that is loaded takes the way of a push of all slots."""
+    from mindrl_amd.core import PriorityReplayBuffer
+    rng = np.random.default_rng(cap)
+    a = PriorityReplayBuffer(0.6, cap, 8, SHAPES, torch_types(DTYPES), seed0=3)
+    b = PriorityReplayBuffer(0.6, cap, 8, SHAPES, torch_types(DTYPES), seed0=4)
+    for n in (2, cap // 2, cap):
+        a.insert(*to_dev(random_rows(rng, n, SHAPES, DTYPES)), priorities=torch.from_numpy(rng.pareto(1.5, n).astype(np.float32)).cuda())
+        b.load_state_dict(a.state_dict())
+        assert all(np.array_equal(x[1:], y[1:]) for x, y in zip(a.export_tree(), b.export_tree())) and a.max_priority == b.max_priority
+        a.check(), b.check()
+    a.destroy()
+    b.destroy()
