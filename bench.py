@@ -437,15 +437,14 @@ def bench_per(a):
     row_bytes = sum(r.buf._layout.bytes)
     levels = max(1, (r.capacity - 1).bit_length())
     # the library's own choice (mrb_per_sample): the LDS-top kernel for many narrow rows, else the wide-row kernel
-    lds_path = a.sample_path == 2 or (a.sample_path == 0 and batch >= 8192 and max(r.buf._layout.bytes) <= 256)
-    # (rows of at most 4 KB in 16-byte fields: the workgroup kernel with two copy waves, or, for launches of at least
-    # 2048 rows, the wave-per-row kernel)
+    lds_path = a.sample_path == 2 or (a.sample_path == 0 and batch >= 20480 and max(r.buf._layout.bytes) <= 256)
+    # (rows of at most 4 KB in 16-byte fields: the workgroup kernel with two copy waves; of thousands of rows, sixteen lanes to a stratum)
     wide_granules = sum(b // 16 for b in r.buf._layout.bytes if b % 16 == 0)
     narrow_bytes = sum(b for b in r.buf._layout.bytes if b % 16)
     if lds_path:
         kernel_name = "k_per_sample_lds"
-    elif wide_granules <= 256 and narrow_bytes <= 256 and batch >= 2048 and not a.row_split:
-        kernel_name = "k_per_sample_rows"
+    elif wide_granules <= 1280 and narrow_bytes <= 48 and batch >= 2048 and a.sample_path == 0 and not a.row_split:
+        kernel_name = "k_per_sample_lanes"
     elif wide_granules <= 256 and levels != 22 and not a.row_split:
         kernel_name = "k_per_sample_light"
     else:

@@ -168,7 +168,7 @@ __global__ __launch_bounds__(1024) void k_tree_range(const int64_t* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// Very large trees (22 levels and more) under a call that names few of their leaves (65,536 of 2^24): scanning every
+// Very large trees (21 levels and more) under a call that names few of their leaves (65,536 of 2^24): scanning every
 // 256-leaf tile would cost more in wave launches than the update itself, so the ENTRIES drive the lowest levels. A group
 // of 2^(g0-2) lanes (g0 = 4..6) takes one entry; if that entry owns its block of 2^g0 leaves (it holds the largest of
 // the block's stamps), the group replaces the leaves the stamps name, rebuilds the g0 levels above with tile_parents'
