@@ -259,6 +259,14 @@ __device__ __forceinline__ float lane_value(float x, uint32_t src_lane) {
 // its global loads and stores, which __syncthreads() would also wait for.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// Between LDS accesses of lanes of ONE wave that hand each other values: what stands before it is done before what stands behind
+// it. The device takes a wave's LDS accesses in order, so this is an order for the compiler and no instruction.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // The value lane ^ (1 << S) holds, S = 0..3, moved inside the register file (DPP) rather than through the
 // LDS crossbar a generic shuffle takes. For S = 2 and 3 the source is the mirrored lane of the 8- or 16-lane
 // group: it holds what lane ^ (1 << S) holds once the lanes of every aligned group of 2^S lanes agree, which

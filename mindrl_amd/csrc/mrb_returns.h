@@ -256,11 +256,13 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
             if (kQuad) *reinterpret_cast<f32x4*>(&s_x[buf][of][at]) = v[i];
         }
         if (kQuad) {
+            wave_lds_fence();
 #pragma unroll
             for (int i = 0; i < kPer; ++i)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) v[i][j] = s_x[buf][4 * quad + j][i * kSteps + step];
         }
+        wave_lds_fence();  // (the next chunk goes over what other lanes have read)
     };
     auto store = [&](int64_t c, const f32x4 (&v)[kPer], auto whole, int last) {
         char* const bo = reinterpret_cast<char*>(out + base_of(c) * cols);
