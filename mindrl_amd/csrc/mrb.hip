@@ -864,15 +864,28 @@ bool takes_range(const Per& b, int64_t n) {
     return !takes_range_one(b, n) && n <= (b.depth >= 21 ? 3072 : b.depth == 12 ? 8192 : 16384);
 }
 
-// Whether the entries drive the lowest levels of an update (launch_tree_sparse), with more than the 1024 that elect among themselves. The other ways
-// look at every tile of the tree, or at every entry in every workgroup. us per call, by tiles (up to 8193 entries by runs of leaves) / by entries, slots at random and,
-// behind the comma, one after the other:
-//   21 levels  3000 9.0 / 9.5, 10.1 / 8.6; 4096 9.6 / 9.5, 11.7 / 8.8; 8193 11.1 / 10.1, 16,384 14.9 / 11.4, 32,768 20.7 / 13.5, 10.9 / 9.5; 65,536 23.4 / 19.7,
-//              11.0 / 11.6; 131,072 27.9 / 29.0
-//   22 levels  2048 9.5 / 9.3, 3000 9.7 / 9.6, 10.7 / 8.8; 4096 10.7 / 9.7, 8192 13.2 / 10.2, 32,768 29.6 / 13.9, 131,072 38.7 / 32.0, 14.6 / 13.2; 200,000 43.3 / 43.0, 15.2 / 16.2
-//   23 levels  131,072 56 / 34, 262,144 66 / 56, 19.7 / 18.2; 524,288 83 / 95
-//   24 levels  131,072 93 / 36, 262,144 116 / 63, 27 / 18; 524,288 138 / 156; 25 levels  262,144 189 / 110, 524,288 235 / 173
-//   26 levels  524,288 368 / 338, 75 / 50; 1,048,576 458 / 599; deeper trees were not measured
+// Whether the entries drive the lowest levels of an update (launch_tree_sparse), with more than the 1024 that elect among themselves.
+// The other ways look at every entry in every workgroup (by runs of leaves: up to 3072 entries on 21 and 22 levels) or at every tile
+// of the tree. us per call, the other way / by entries, slots at random; in the order that a sample returns them; one after the
+// other; half of them and all of them the same:
+//   levels  entries    random         sample's       one by one     half           all
+//   21        3,073     9.2 /  9.6     8.5 /  9.3    10.8 /  8.8    10.0 /  9.2     9.6 /  8.1    by runs
+//   21        4,096     9.9 /  9.7     9.2 /  9.4    12.1 /  9.0    11.5 /  9.6    10.8 /  8.4    by runs
+//   21        8,192    11.8 / 10.4    11.6 /  9.9    12.2 /  9.1    16.2 / 10.9    15.0 /  9.1    by runs
+//   21       16,384    14.9 / 11.5    13.4 / 10.7    18.8 /  9.2    24.5 / 13.4    24.1 / 10.6    by runs
+//   22        3,073    10.1 /  9.8     9.5 /  9.6    11.2 /  8.9    11.1 /  9.3    10.4 /  8.2    by runs
+//   22        8,192    13.1 / 10.4    12.6 / 10.2    12.4 /  9.1    16.3 / 11.6    15.4 /  9.2    by runs
+// and by tiles / by entries, at random, one after the other:
+//   21       32,768    20.7 / 13.5                   10.9 /  9.5
+//   21       65,536    23.4 / 19.7                   11.0 / 11.6    (the line lies in front of what loses in one order)
+//   21      131,072    27.9 / 29.0
+//   22       32,768    29.6 / 13.9
+//   22      131,072    38.7 / 32.0                   14.6 / 13.2
+//   22      200,000    43.3 / 43.0                   15.2 / 16.2
+//   23      131,072      56 / 34;   262,144   66 / 56 and 19.7 / 18.2;   524,288   83 / 95
+//   24      131,072      93 / 36;   262,144  116 / 63 and 27 / 18;       524,288  138 / 156
+//   25      262,144     189 / 110;  524,288  235 / 173
+//   26      524,288     368 / 338 and 75 / 50;   1,048,576   458 / 599;   deeper trees were not measured
 bool takes_sparse(const Per& b, int64_t n) {
     const int share = b.depth == 22 || b.depth == 23 ? 5 : b.depth <= 25 ? 6 : b.depth == 26 ? 7 : 8;
     return b.s_g0 > 0 && n > kElectMax && n <= b.leaves >> share;

@@ -59,3 +59,48 @@ def test_every_node_above_the_entries(capacity, n):
                                         ((1 << 23) - 1, 262_144), ((1 << 24) - 1, 262_144)])
 def test_where_the_entries_take_over(capacity, n):
     test_every_node_above_the_entries(capacity, n)
+
+
+# entries of a wave bid for their leaf among themselves first: many of them on one leaf, on leaves that lie together, entries that
+# count for nothing behind those that do
+@pytest.mark.parametrize("capacity,n", [((1 << 14) - 1, 20_000), (1 << 20, 20_000), ((1 << 21) - 7, 3073), (1 << 21, 16_385), ((1 << 22) - 1, 8193), (1 << 24, 65_537)])
+def test_many_entries_on_few_leaves(capacity, n):
+    from mindrl_amd.core import PriorityReplayBuffer
+    rng = np.random.default_rng(n)
+    wild = rng.integers(0, capacity, n)
+    for idx in (np.full(n, capacity // 3), np.where(rng.random(n) < 0.5, capacity // 3, wild), np.sort(rng.integers(0, 100, n)) * (capacity // 100),
+                5 + np.arange(n) // 7 % capacity, 3 + rng.integers(0, 5, n) * 128 % capacity):
+        g = PriorityReplayBuffer(1.0, capacity, 4, [(1,)], [torch.uint8], seed0=1)
+        pr = (rng.pareto(1.5, n) + 1e-6).astype(np.float32)
+        bad = rng.random(n) < 0.3
+        bad[-3:] = True
+        given, at = np.where(bad & (np.arange(n) % 2 == 0), np.float32(-1), pr), np.where(bad & (np.arange(n) % 2 == 1), -1 - idx, idx)
+        g.update_priorities(torch.from_numpy(at).cuda(), torch.from_numpy(given).cuda())
+        sums, mins = g.export_tree()
+        for nodes, want_s, want_m in levels_above(capacity, idx[~bad], pr[~bad]):
+            assert np.array_equal(sums[nodes], want_s) and np.array_equal(mins[nodes], want_m), int(nodes[0]).bit_length() - 1
+        assert np.float32(g.max_priority) == max(pr[~bad].max(), np.float32(1.0))
+        with pytest.raises((IndexError, ValueError)):
+            g.check()
+        g.destroy()
+
+
+@pytest.mark.parametrize("capacity,n", [(1 << 20, 65_536), (1 << 21, 16_384), (1 << 22, 8192), (1 << 24, 65_536)])
+def test_many_entries_on_one_leaf_take_no_longer(capacity, n):
+    """One after the other their bids would take 11 ns each: 8 to 70 times as long as an update of as many leaves."""
+    from mindrl_amd.core import PriorityReplayBuffer
+    g = PriorityReplayBuffer(0.6, capacity, 4, [(1,)], [torch.uint8], seed0=1)
+    pr, took = torch.rand(n, device="cuda") + 0.01, []
+    for idx in (torch.randint(0, capacity, (n,), device="cuda"), torch.full((n,), capacity // 3, device="cuda")):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        best = []
+        for _ in range(5):
+            start.record()
+            for _ in range(20):
+                g.update_priorities(idx, pr)
+            end.record()
+            torch.cuda.synchronize()
+            best.append(start.elapsed_time(end))
+        took.append(min(best))
+    assert took[1] < 2.5 * took[0], took
+    g.destroy()
