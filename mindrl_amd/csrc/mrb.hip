@@ -2150,12 +2150,28 @@ static int discounted_return(const float* x, const uint8_t* done, float* end_val
     if (cols > (1ll << 31) || cols > (1ll << 40) / timesteps)
         return fail(MRB_EINVAL, "%lld columns of %lld steps exceed one call (at most 2^31 columns, 2^40 elements)",
                     (long long)cols, (long long)timesteps);
-    // A thread per column needs about 65 to 100 ns per step however few the columns (a trip to memory per 32 steps) and
-    // streams at up to 6 TB/s when there are many; chunks through LDS need 8 to 11 ns per step and stream at 4.8 TB/s.
-    // Measured, us per column / tiled: [20, 9000] 5.0 / 4.7, [32, 30001] 5.3 / 7.8; [64, 30000] 8.8 / 8.0, [64, 40000] 8.7 / 9.7, [48, 30001] 10.8 /
-    // 8.2; [100, 38000] 14.2 / 10.9, [200, 45000] 26.7 / 22.0, [128, 65536] 16.8 / 21.4, [200, 65536] 27.4 / 29.4; [256, 65536] 31.9 / 32.5, [300, 65536] 41.3 /
-    // 35.0, [1000, 65536] 123 / 113, [256, 80000] 38.0 / 40.5, [1000, 131072] 195 / 247.
-    const int64_t most = timesteps <= 32 ? 8192 : timesteps <= 64 ? 32768 : timesteps < 256 ? 40960 : 65536;
+    // A thread per column needs about 65 to 100 ns per step however few the columns (a trip to memory per 32 steps, and steps beyond a
+    // multiple of 32 cost it more) and streams at up to 6 TB/s when there are many; chunks of 64 steps through LDS need 8 to 11 ns per
+    // step and stream at 4.8 TB/s. So the line rises with the steps beyond a multiple of 32, and falls back behind 64. us, forward, per
+    // column / by chunks (backward the chunks gain up to 8 % on that):
+    //   steps           16,384         20,000         24,000         30,000         36,000         40,960    chunks are faster up to
+    //      20       4.8 /  5.0     4.9 /  5.6     4.9 /  6.6     5.0 /  7.8     5.1 /  8.9     5.1 /  9.7    16,000  (but the line is at 8192)
+    //      33       4.4 /  5.3     4.8 /  5.9     4.7 /  6.9     4.9 /  8.1     5.0 /  9.3     4.8 / 10.2    12,000
+    //      48       6.8 /  5.4     7.0 /  6.0     7.1 /  7.0     7.1 /  8.2     7.2 /  9.4     7.1 / 10.1    25,000
+    //      60       8.8 /  5.5     8.9 /  6.1     8.9 /  7.2     9.2 /  8.3     9.3 /  9.4     9.2 / 10.3    38,000
+    //      64       7.0 /  5.6     7.4 /  6.1     7.9 /  7.1     8.2 /  8.2     8.2 /  9.5     8.3 / 10.2    28,000  (backward 8.8 / 8.3 at 30,001)
+    //      65       7.3 /  6.1     7.7 /  6.7     8.0 /  7.8     8.3 /  9.2     8.4 / 10.6     8.5 / 11.5    25,000
+    //      80       9.4 /  6.1     9.9 /  6.8    10.0 /  7.9    10.6 /  9.3    11.1 / 10.6    10.3 / 11.4    38,000
+    // Beyond 95 steps the line is flat. 45,000 columns: 104 steps 14.4 / 13.2, 128 16.7 / 15.4, 192 23.8 / 19.9; 50,000: 14.7 / 13.7,
+    // 17.0 / 18.6, 24.4 / 23.5 (the line lies at 40,960, in front of what 128 steps lose and at the price of what 192 would gain);
+    // 65,536: 256 steps 31.6 / 29.7, 300 38.5 / 34.3, 1000 122 / 117; 81,920: 256 37.7 / 36.0, 300 46.8 / 41.5 (the line lies at 65,536).
+    const int64_t beyond = timesteps % 32;
+    const int64_t most = timesteps <= 32   ? 8192
+                         : timesteps < 64  ? 10000 + 900 * beyond
+                         : timesteps == 64 ? 31000
+                         : timesteps < 96  ? std::min<int64_t>(24000 + 900 * beyond, 40960)
+                         : timesteps < 256 ? 40960
+                                           : 65536;
     const bool per_column = cols > most;
     if (per_column) {
         hipLaunchKernelGGL(k_discounted_return, dim3(grid_exact((uint64_t)cols)), dim3(kWG), 0, s, x, done, end_value, out,

@@ -48,7 +48,9 @@ def test_return_and_gradient_bit_exact(shape):
 # half and whole, at either side of sixteen and eight steps; the lines between the kernels and the groups' widths
 EDGES = [(t, b, inner) for b, inner in ((5, 1), (3, 2), (4101, 1)) for t in (1, 16, 17, 32, 33, 48, 64, 96, 97, 128, 129, 192, 193, 256, 257, 320, 321, 385)]
 EDGES += [(33, 32768, 1), (33, 32769, 1), (64, 32769, 1), (65, 32769, 1), (65, 40961, 1), (127, 8193, 1), (128, 4097, 1), (127, 4097, 1),
-          (255, 40961, 1), (256, 40961, 1), (257, 65537, 1), (130, 2731, 3), (100, 5461, 3)]
+          (255, 40961, 1), (256, 40961, 1), (257, 65537, 1), (130, 2731, 3), (100, 5461, 3), (33, 10900, 1), (33, 10901, 1), (48, 24400, 1),
+          (48, 24401, 1), (63, 37900, 1), (63, 37901, 1), (64, 31000, 1), (64, 31001, 1), (65, 24900, 1), (65, 24901, 1), (95, 40960, 1),
+          (95, 40961, 1), (40, 5733, 3), (40, 5734, 3)]
 
 
 @pytest.mark.parametrize("shape", EDGES)
