@@ -1702,17 +1702,44 @@ static bool takes_lds(int64_t nbatch, int64_t batch, uint64_t rest, bool lanes) 
     const int64_t least = lanes ? (rest <= 16 ? 14336 : rest <= 40 ? 20480 : 12288) : (rest <= 16 ? 3072 : rest <= 64 ? 5120 : 12288);
     return rest <= 384 && batch >= fewest && rows >= least;
 }
-// Whether sixteen lanes to a stratum (k_per_sample_lanes) can take a sample, and from how many rows on they are the better ones. Workgroup per row
-// (k_per_sample_light) / lanes, us: 41 bytes 1024 rows 3.8 / 4.1, 1280 4.1 / 4.0; 153 bytes, 5 * 10^4 slots 1024 3.8 / 3.5, 10^5 3.85 / 3.9, 10^6 3.8 / 4.3;
-// 899 bytes in odd fields 1280 4.4 / 5.0, 1536 5.0 / 5.1; 1 KB 1536 4.75 / 5.0, 2048 6.4 / 5.1; 2.4 KB 1500 5.2 / 5.5, 2048 7.2 / 5.8; 13 KB 1024
-// 8.2 / 9.3, 2048 15.7 / 14.4; 20 KB 1024 13.8 / 13.8, 2048 23.2 / 20.8; 28 KB 2048 23.8 / 24.7, 4096 40.9 / 44.7. On 21 levels and more, whose walk takes
-// the workgroup longer: 153 bytes 1024 5.6 / 4.8, 521 bytes 5.4 / 4.7.
+// Whether sixteen lanes to a stratum (k_per_sample_lanes) can take a sample.
 static bool takes_lanes(const Per& b, const WidePlan& plan) {
     return b.rows.row_split == 0 && b.rows.row_wave == 0 && b.depth >= kLanesFewestLevels && plan.narrow_items <= kLanesMostNarrow &&
            plan.wide_items <= 1280;
 }
-static int64_t lanes_fewest_rows(int depth, uint32_t wide_items) {
-    return wide_items > 64 ? 2048 : depth >= 21 ? 1024 : wide_items <= 32 ? 1280 : 1536;
+// Whether they are faster than a workgroup to a row (k_per_sample_light, k_per_sample_wide). That one's time hardly depends on the row
+// but on how it walks the tree: on 20 levels in two groups of ten, which is its best, on 22 by the larger kernel, which is its worst.
+// us, it / lanes (byte images, masks and halves: 147 and 899 bytes; the others rows of floats):
+//   levels  row          1024 rows      1280           1536           1792           2048
+//   16      41 bytes     3.8 / 3.5      4.1 / 3.5      4.4 / 3.5      4.5 / 3.5      5.7 / 3.5
+//   16      521          3.8 / 4.0      4.1 / 4.0      4.5 / 4.0      4.8 / 4.0      6.1 / 4.1
+//   16      899          3.9 / 4.6      4.4 / 4.7      4.8 / 4.7      5.2 / 4.7      6.9 / 4.8
+//   18      41           3.8 / 4.0      4.1 / 4.0      4.5 / 4.0      4.7 / 4.0      6.1 / 4.0
+//   18      147          3.8 / 4.3      4.2 / 4.3      4.6 / 4.3      4.8 / 4.3      6.2 / 4.4      (1408: 4.5 / 4.3)
+//   18      899          4.0 / 5.0      4.4 / 5.0      4.9 / 5.0      5.3 / 5.1      7.0 / 5.1
+//   20      41           3.6 / 4.2      3.8 / 4.2      4.3 / 4.2      4.5 / 4.2      5.8 / 4.2
+//   20      147          3.6 / 4.6      3.9 / 4.6      4.4 / 4.6      4.6 / 4.6      5.9 / 4.6
+//   20      521          3.6 / 4.4      3.9 / 4.4      4.4 / 4.4      4.6 / 4.4      5.9 / 4.6
+//   20      899          4.0 / 5.1      4.4 / 5.1      4.7 / 5.1      5.1 / 5.2      6.7 / 5.3      (1920: 5.2 / 5.2)
+//   21      147          4.9 / 4.9      5.3 / 4.9      5.7 / 4.9      6.1 / 4.9      6.9 / 5.0      (768: 4.6 / 4.9; 41 bytes 4.6 / 4.6)
+//   21      899          5.2 / 5.3      5.8 / 5.4      6.2 / 5.4      6.6 / 5.5      7.7 / 5.6
+//   22      147          5.4 / 4.9      5.8 / 4.9      7.6 / 4.9      8.6 / 5.0      7.0 / 5.0      (768: 4.9 / 5.0, 521 bytes 4.9 / 4.6; 512: 4.5 / 4.6)
+//   24      41           4.5 / 4.8      5.0 / 4.8      5.3 / 4.8      5.5 / 4.8      6.9 / 4.8
+//   24      147          4.6 / 5.2      5.1 / 5.2      5.4 / 5.2      5.7 / 5.3      7.0 / 5.3
+//   26      41           4.7 / 5.4      5.2 / 5.4      5.6 / 5.5      5.8 / 5.5      7.1 / 5.5
+// Rows that waves carry whole (above a kilobyte): lanes from 2048 rows on, but not where their launch is more workgroups than the chip holds
+// at once and fills little of the second lot; both sides are in the table at lanes_strata (mrb_sample_lanes.hip).
+static bool lanes_better(int depth, uint32_t wide, uint32_t narrow, int64_t rows) {
+    if (wide > 64) {
+        if (rows < 2048) return false;
+        if (wide <= 192 || (wide > 256 && wide <= 512)) return true;
+        return wide <= 256 ? rows <= 4096 || rows >= 5632 : rows <= 2048 || (rows >= 3600 && rows <= 4096) || rows >= 6000;
+    }
+    const bool light = wide <= 16 && narrow <= 16;  // a granule and a byte to a lane: 0.2 us less
+    if (depth % kGroupMaxLevels == 0) return rows >= (light ? 1408 : wide <= 32 ? 1664 : 1920);
+    if (depth == 21 || depth == 22) return rows >= (depth == 22 || wide <= 32 ? 1024 : 1280);
+    if (depth < 18) return rows >= (wide <= 32 ? 1280 : 1536);
+    return rows >= (light ? 1280 : wide <= 32 ? 1408 : 1664);
 }
 static int lds_strata(int64_t rows, uint64_t rest) {
     if (rows <= 20480 && rest > 16) return 16;
@@ -1762,7 +1789,7 @@ static int per_sample_impl(Per* b, int64_t nbatch, int64_t batch, float beta, co
         dim3 grid;
         plan.nbatch = (uint32_t)nbatch;
         const bool lanes = !next && nbatch * batch >= 1024 && wide_plan(b->rows, t, nbatch * batch, plan, grid) && takes_lanes(*b, plan);
-        path = takes_lds(nbatch, batch, rest, lanes) ? 2 : lanes && nbatch * batch >= lanes_fewest_rows(b->depth, plan.wide_items) ? 3 : 1;
+        path = takes_lds(nbatch, batch, rest, lanes) ? 2 : lanes && lanes_better(b->depth, plan.wide_items, plan.narrow_items, nbatch * batch) ? 3 : 1;
         if (path == 3) {
             const hipError_t e = launch_per_sample_lanes(a, plan, nbatch, s);
             if (e != hipSuccess) return fail(MRB_EHIP, "launch k_per_sample_lanes: %s", hipGetErrorString(e));

@@ -295,17 +295,34 @@ int lanes_trips(int depth, int levels) { return (depth - levels + kLanesMost - 1
 // Staged levels: twelve, or as few of them as take no trip more, which are less to stage (17 levels, 8192 rows of 153 bytes: twelve
 // 5.0 us, nine 4.6; 16 levels, 1536 rows: 4.05 / 3.85; 22 levels, 4096 rows of 521 bytes: 5.5 / 5.3), but nine on 18 levels and
 // more, where the trips are to memory that is not in the cache.
-// Strata of a workgroup where a copy wave carries whole rows: enough workgroups for the chip's copies to be in flight first, then as
-// many strata as there may be, for the waves there are to dispatch. 16 / 8 / 4, us: 2.4 KB   2048 rows 7.6 / 6.0 / 5.8, 4096 8.7 / 7.7 /
-// 10.6, 8192 12.8 / 16.5 / 19.0; 1 KB   4096 rows 7.2 / 6.2 / 6.2, 8192 9.3 / 7.9 / 11.8; 7.5 KB   2048 rows 11.8 / 9.7 / 9.4,
-// 4096 16.5 / 17.2 / 19.1; 13 KB   4096 rows 25.1 / 24.6 / 27.0.
+// Strata of a workgroup where a copy wave carries whole rows: as few as leave the launch's workgroups on the chip all at once, then
+// as many as there may be, for the waves there are to dispatch. What the compute units hold, beyond which a launch takes a step (2304 rows
+// in the table's last three lines), is some 1024 workgroups of four strata, 768 of eight and 512 of sixteen where a lane holds two
+// granules; 768, 512 and 512 where it holds four; 512, 512 and 256 where it holds eight. 2 * 10^5 slots, us with 4 / 8 / 16 strata, and,
+// for comparison, a workgroup to a row:
+//   row         2048 rows                   2304                        3000                        4096                        5120                        8192
+//   1 KB      5.1 /  5.2 /  6.7,  6.4    5.4 /  5.7 /  6.8,  7.4    5.7 /  5.9 /  6.9,  7.6    6.1 /  6.2 /  7.2,  8.5    7.0 /  6.6 /  8.7,  9.6   11.6 /  7.9 /  9.4, 14.5
+//   2.4 KB    5.8 /  6.0 /  7.5,  7.1    6.4 /  6.7 /  7.7,  8.1    6.8 /  7.1 /  8.0,  8.4   10.6 /  7.7 /  8.7,  9.5   11.7 / 11.9 / 10.5, 11.1   18.9 / 16.4 / 12.5, 16.4
+//   4 KB      6.7 /  7.0 /  8.7,  7.5    7.3 /  7.7 /  8.9,  8.5    8.0 /  8.4 /  9.9,  8.9   12.3 /  9.6 / 11.2, 10.2   14.0 / 14.6 / 13.1, 11.9   21.7 / 19.7 / 16.4, 17.9
+//   7.5 KB    9.1 /  9.4 / 11.7, 10.4   14.3 / 12.9 / 12.0, 12.8   14.9 / 14.1 / 13.6, 14.3   18.9 / 17.1 / 16.3, 18.6   22.2 / 21.8 / 22.3, 22.4   31.8 / 29.1 / 26.3, 33.2
+//   13 KB    14.2 / 15.0 / 18.6, 15.7   20.9 / 19.8 / 19.1, 16.9   21.9 / 21.6 / 21.1, 21.1   26.8 / 24.6 / 24.8, 26.7   32.1 / 32.0 / 33.9, 31.9   45.6 / 42.5 / 41.8, 48.0
+//   20 KB    20.6 / 22.7 / 34.2, 22.9   30.6 / 31.8 / 34.9, 25.0   34.1 / 34.4 / 36.5, 30.9   40.5 / 37.4 / 38.8, 39.8   49.0 / 48.9 / 57.0, 47.8   (6000) 55.0 / 52.9 / 59.6, 55.0
+// (Where the workgroup to a row is the faster one, and the lines that keep the lanes away from it: lanes_better, mrb.hip.)
+static uint32_t lanes_strata(uint32_t wide, uint32_t rows) {
+    if (wide <= 64) return 16;  // sixteen lanes carry a row
+    if (wide <= 128) return rows <= 3072 ? 4 : rows <= 8192 ? 8 : 16;
+    if (wide <= 256) return rows <= 3072 ? 4 : rows <= 4096 ? 8 : 16;
+    if (wide <= 512) return rows <= 2048 ? 4 : rows > 4096 && rows <= 5120 ? 8 : 16;
+    return rows <= 2048 ? 4 : rows <= 6144 ? 8 : 16;
+}
+
 hipError_t launch_per_sample_lanes(const SampleArgs& a, const WidePlan& plan, int64_t nbatch, hipStream_t s) {
     const int most = a.depth >= 16 ? 12 : (a.depth - 4) / 3 * 3, fewest = a.depth >= 18 ? 9 : 3;
     int levels = most;
     while (levels > fewest && lanes_trips(a.depth, levels - 3) == lanes_trips(a.depth, most)) levels -= 3;
     const int trips = lanes_trips(a.depth, levels), trip = (a.depth - levels + trips - 1) / trips;
     const uint32_t nrows = (uint32_t)(nbatch * a.batch), w = plan.wide_items;
-    const uint32_t strata = w <= 64 ? 16 : nrows <= 3072 ? 4 : nrows <= (w <= 128 ? 8192u : 5120u) ? 8 : 16;
+    const uint32_t strata = lanes_strata(w, nrows);
     const SampleTail tail{a.mn, a.out_idx, a.out_w, a.err, a.size, a.beta};
     const int shape = a.depth | levels << 8 | trip << 16 | (a.size < 0 ? kLanesStored | (a.uniforms ? 0 : kLanesCounters) : 0);
     auto* kernel = w <= 16 ? k_per_sample_lanes<16, false, 1> : w <= 32 ? k_per_sample_lanes<16, false, 2> : k_per_sample_lanes<16, false, 4>;

@@ -60,7 +60,7 @@ def _compare(g, c, rng, batch, n, what):
 def test_trees(cap, device_counters):
     g, c, rng = _buffers("narrow", cap)
     g.set_option("device_counters", device_counters)
-    for batch in (1280, 1537):
+    for batch in (1280, 1665):
         _compare(g, c, rng, batch, 1, "%d leaves, batch %d" % (cap, batch))
     g.destroy()
 
@@ -68,8 +68,9 @@ def test_trees(cap, device_counters):
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,batches", [
     ("48", [(1280, 1), (1281, 1)]), ("16", [(1297, 1), (14_335, 1), (1, 1300), (431, 3)]), ("32", [(1280, 1), (20_479, 1)]),
-    ("64", [(1536, 1), (12_287, 1), (7, 221)]), ("65", [(2048, 1), (3073, 1), (8193, 1)]), ("129", [(2049, 1), (3073, 1), (5121, 1), (700, 3)]),
-    ("470", [(2051, 1), (3075, 1), (5125, 1)]), ("1280", [(2050, 1), (3073, 1), (5121, 1)])])
+    ("64", [(1536, 1), (12_287, 1), (7, 221)]), ("65", [(2048, 1), (3073, 1), (8193, 1)]),
+    ("129", [(2049, 1), (3073, 1), (4096, 1), (4097, 1), (5633, 1), (700, 3)]), ("470", [(2048, 1), (2051, 1), (4099, 1), (5125, 1)]),
+    ("1280", [(2048, 1), (2049, 1), (3601, 1), (4096, 1), (6001, 1), (6145, 1)])])
 @pytest.mark.parametrize("packed", [0, 4096])
 def test_rows(rows, batches, packed):
     g, c, rng = _buffers(rows, 1500, packed)
