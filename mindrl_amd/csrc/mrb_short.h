@@ -179,7 +179,7 @@ __device__ __forceinline__ void gather_field(const ShortRows& rows, int f, const
         bool outside = false;
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            outside = outside || slot[q] < 0 || slot[q] >= count;
+            outside = outside || (f == 0 && unit[q] == 0 && (slot[q] < 0 || slot[q] >= count));  // (one granule of a row: see gather_body)
             slot[q] = slot[q] < 0 ? 0 : slot[q] >= count ? (count > 0 ? count - 1 : 0) : slot[q];
             if (out_indices && unit[q] == 0) out_indices[row[q]] = slot[q];
         }

@@ -47,3 +47,34 @@ def test_flat_gathers(shapes, dtypes, batches, packed):
         given = np.clip(given, 0, cap - 31)
         assert all(np.array_equal(t2n(a), b[given]) for a, b in zip(fields, new)), batch
         g.destroy()
+
+
+def _time(call, n=20):
+    best = []
+    for _ in range(5):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(n):
+            call()
+        end.record()
+        torch.cuda.synchronize()
+        best.append(start.elapsed_time(end) / n)
+    return min(best)
+
+
+@pytest.mark.parametrize("shapes,dtypes,n", [([(28224,), (1,)], [U, L], 4096), ([(400,), (1,), (1,), (400,)], [F, F, F, F], 8192)])
+def test_rows_outside_are_flagged_once_each(shapes, dtypes, n):
+    """Flags go to one word, one atomic after the other, 11 ns each: one for each such row, not one for each of its granules, so a
+    batch of nothing but such rows takes the time of its atomics at most on top of its copy."""
+    from mindrl_amd.core import UniformReplayBuffer
+    rng = np.random.default_rng(3)
+    g = UniformReplayBuffer(n, 5000, shapes, torch_types(dtypes))
+    g.insert(to_dev(random_rows(rng, 5000, shapes, dtypes)))
+    good = torch.from_numpy(rng.integers(0, 5000, n)).cuda()
+    took = _time(lambda: g.sample(good))
+    g.check()
+    bad = _time(lambda: g.sample(good + 5000 * (1 + good % 2)))
+    with pytest.raises(IndexError):
+        g.check()
+    assert bad < took + 0.03 + n * 15e-6, (took, bad)  # (ms; two small kernels work out the slots)
+    g.destroy()
