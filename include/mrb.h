@@ -88,6 +88,8 @@ int mrb_version(void);
  *   "row_split"    least number of workgroups per row in the wide-row kernel (0 = auto, max 64)
  *   "row_wave"     prioritized buffers: the wave-per-row sample kernel (rows of at most 4 KB in 16-byte fields and 256
  *                  narrow bytes) is taken 0 = for launches of at least 2048 rows, 1 = whenever the rows fit it, 2 = never
+ *                  (0: or the sixteen-lane kernel in its place). Gathers of rows with a field of 1 KB and more: 0 = the
+ *                  kernel that is faster, 1 = from 2048 rows on a wave per row, 2 = a workgroup per row
  *   "sample_path"  prioritized buffers: 0 = choose by row size, 1 = wide-row kernel, 2 = LDS-top kernel
  *   "lds_levels"   prioritized buffers: tree levels staged in LDS by the LDS-top kernel (0 = auto, max 12)
  *   "device_counters" prioritized and uniform buffers: 1 = the ring position, the number of stored rows and the generator's

@@ -470,8 +470,8 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
     // A workgroup per row is the faster one for some hundred rows of 4 KB and more, which are too few granules for four to a thread (workgroup per row /
     // flat, us): 3.2 KB 32 rows 3.0 / 2.4, 1024 3.9 / 3.7; 7.5 KB 32 3.1 / 2.8, 256 3.4 / 3.3, 512 4.0 / 4.2, 1024 5.3 / 5.5, 4096 15.2 / 14.1; 28 KB 32 3.7 / 2.7,
     // 128 4.3 / 3.6, 512 7.4 / 7.6 (given slots 5.7 / 6.3), 2048 22.9 / 22.5. (A wave per row: 1 KB 2048 rows 4.9 / 3.6, 8192 7.6 / 6.1; 2.1 KB 8192
-    // 13.0 / 10.6; 2.4 KB 2048 5.3 / 4.7, 16,384 17.5 / 17.9.) And it is what is asked for by row_split and row_wave, and for more than a brief launch's
-    // arguments hold the kernels that take a plan.
+    // 13.0 / 10.6; 2.4 KB 2048 5.3 / 4.7, 16,384 17.5 / 17.9.) And row_split asks for it, as
+    // row_wave = 2 does, and row_wave = 1 for a wave per row; what a brief launch's arguments do not hold goes to the kernels that take a plan.
     const bool wide = widest_field(r) >= 4096 && most >= 200000 && most <= 1u << 20;
     if (widest_field(r) >= 1024 && n <= (1ll << 24) && (wide || !brief || r.row_split != 0 || r.row_wave != 0)) {
         const int mode = fixed_slot >= 0 ? kFromFixedSlot : (indices ? kFromIndices : kFromGenerator);
@@ -482,7 +482,7 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
         // Thousands of rows of up to 4 KB: a wave per row (3 KB, us, workgroup / wave: 1024 rows 6.2 / 6.7, 2048 7.5 / 6.8,
         // 8192 20.7 / 13.6; 1 KB: 2048 5.2 / 5.5, 4096 7.4 / 5.9).
         if (r.row_split == 0 && plan.split == 1 && plan.wide_items <= (uint32_t)kRowWaveInF * 64u && plan.narrow_items <= 256u &&
-            inflight != 0 && n >= kRowWaveMinRows) {
+            inflight != 0 && n >= kRowWaveMinRows && r.row_wave != 2) {
             hipLaunchKernelGGL(k_rows_gather_rows, dim3((uint32_t)((n + kRowWaveWG / 64 - 1) / (kRowWaveWG / 64))), dim3(kRowWaveWG),
                                0, s, indices, mode, count, fixed_slot, seed, calls, n, out_indices, err, plan);
             LAUNCH_CHECK("k_rows_gather_rows");

@@ -78,3 +78,22 @@ def test_rows_outside_are_flagged_once_each(shapes, dtypes, n):
         g.check()
     assert bad < took + 0.03 + n * 15e-6, (took, bad)  # (ms; two small kernels work out the slots)
     g.destroy()
+
+
+def _kernels(call):
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as p:
+        call()
+        torch.cuda.synchronize()
+    return [e.name for e in p.events()]
+
+
+@pytest.mark.parametrize("option,kernel", [(0, "k_short_gather"), (1, "k_rows_gather_rows"), (2, "k_rows_gather_wide")])
+def test_row_wave(option, kernel):
+    """1 asks for a wave to a row, 2 forbids it."""
+    from mindrl_amd.core import UniformReplayBuffer
+    g = UniformReplayBuffer(2048, 5000, [(1024,), (1,)], torch_types([U, L]))
+    g.insert(to_dev([np.zeros((5000, 1024), U), np.zeros((5000, 1), L)]))
+    g.set_option("row_wave", option)
+    g.sample()
+    assert any(kernel in name for name in _kernels(lambda: g.sample())), _kernels(lambda: g.sample())
+    g.destroy()
