@@ -467,13 +467,32 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
     ShortIo io{};
     const bool brief = fixed_slot < 0 && n <= 0xffffffffll && (out_indices ? short_io(out_indices, nullptr, t, io) : short_io(t, io));
     const uint64_t most = most_granules(t);
-    // A workgroup per row is the faster one for some hundred rows of 4 KB and more, which are too few granules for four to a thread (workgroup per row /
-    // flat, us): 3.2 KB 32 rows 3.0 / 2.4, 1024 3.9 / 3.7; 7.5 KB 32 3.1 / 2.8, 256 3.4 / 3.3, 512 4.0 / 4.2, 1024 5.3 / 5.5, 4096 15.2 / 14.1; 28 KB 32 3.7 / 2.7,
-    // 128 4.3 / 3.6, 512 7.4 / 7.6 (given slots 5.7 / 6.3), 2048 22.9 / 22.5. (A wave per row: 1 KB 2048 rows 4.9 / 3.6, 8192 7.6 / 6.1; 2.1 KB 8192
-    // 13.0 / 10.6; 2.4 KB 2048 5.3 / 4.7, 16,384 17.5 / 17.9.) And row_split asks for it, as
-    // row_wave = 2 does, and row_wave = 1 for a wave per row; what a brief launch's arguments do not hold goes to the kernels that take a plan.
-    const bool wide = widest_field(r) >= 4096 && most >= 200000 && most <= 1u << 20;
-    if (widest_field(r) >= 1024 && n <= (1ll << 24) && (wide || !brief || r.row_split != 0 || r.row_wave != 0)) {
+    // The flat kernel is the faster one but for some hundred rows of 4 KB and more, which are too few granules for four to a thread and
+    // go by a workgroup per row, and for more than 29 MB of rows that fill most of a wave, which go by a wave per row. us, that / flat
+    // (given slots in brackets):
+    //   workgroup per row    32 rows      120,000 granules       200,000                500,000 to 900,000      more
+    //     5 KB                            3.5 / 3.3 (3.0 / 3.1)  3.9 / 3.9 (3.2 / 3.7)
+    //     7.5 KB             3.1 / 2.8    3.4 / 3.3 (2.9 / 3.0)  3.8 / 3.8 (3.1 / 3.7)  5.3 / 5.5               4096 rows 15.0 / 13.9
+    //     12 KB                           3.7 / 2.9 (3.2 / 2.8)  4.1 / 3.5 (3.5 / 3.4)  7.1 / 7.6 (5.9 / 6.0)   2048 rows 12.0 / 11.5
+    //     28 KB              3.7 / 2.7    3.9 / 2.9 (3.2 / 2.8)  4.1 / 3.4 (3.4 / 3.4)  7.4 / 7.6 (5.7 / 6.3)   2048 rows 22.9 / 22.5
+    //   wave per row         2048 rows    8192                       12,000                     16,384
+    //     1 KB               4.9 / 3.5     7.7 /  6.2                10.2 /  7.5                12.3 /  9.2
+    //     2 KB (odd)                      11.5 /  9.1                15.5 / 12.1                19.3 / 16.3
+    //     2.4 KB             5.4 / 4.7    10.8 / 10.2                14.1 / 14.1 (13.9 / 14.2)  17.4 / 18.0
+    //     2.8 KB (odd)                    13.2 / 12.3                17.2 / 17.2 (17.1 / 16.8)  21.6 / 20.4
+    //     3.2 KB             5.7 / 5.1    12.4 / 11.7                15.8 / 15.9 (15.6 / 16.2)  20.5 / 20.8
+    //     3.6 KB                          13.0 / 12.9 (12.5 / 13.2)  17.1 / 18.1                22.5 / 23.4
+    //     4 KB               6.2 / 6.0    13.5 / 14.2 (13.6 / 14.5)  18.3 / 19.1                24.2 / 24.7
+    // And row_split asks for a workgroup per row, as row_wave = 2 does, and row_wave = 1 for a wave per row; what a brief launch's arguments do
+    // not hold goes to the kernels that take a plan.
+    int64_t granules = 0, narrow = 0;  // of a row: in fields of 16 bytes and more, and the bytes of the others
+    for (int f = 0; f < r.nfields; ++f) {
+        if (r.vec_log2[f] == 4) granules += r.units[f];
+        else narrow += r.bytes[f];
+    }
+    const bool by_workgroup = widest_field(r) >= 4096 && most >= 200000 && most <= 1u << 20;
+    const bool by_wave = granules >= 144 && granules <= kRowWaveInF * 64 && narrow <= 256 && n * granules >= 1800000;
+    if (widest_field(r) >= 1024 && n <= (1ll << 24) && (by_workgroup || by_wave || !brief || r.row_split != 0 || r.row_wave != 0)) {
         const int mode = fixed_slot >= 0 ? kFromFixedSlot : (indices ? kFromIndices : kFromGenerator);
         WidePlan plan;
         dim3 grid;

@@ -17,6 +17,8 @@ F, U, L, B, H = np.float32, np.uint8, np.int64, np.bool_, np.float16
     ([(1,), (2413,), (5,), (45,), (999,), (3, 3), (33,)], [B, U, F, H, U, U, L], (1700, 1737)),  # the first one small, all of odd sizes
     ([(7500,)] + [(1,)] * 7, [U] * 8, (425, 426, 2230, 2236)),                     # eight fields; around those with a workgroup to a row
     ([(28224,), (1,)], [U, L], (113, 114, 594, 595)),
+    ([(4096,), (1,)], [U, L], (7031, 7032)),                                       # around those with a wave to a row
+    ([(300,), (300,), (5, 51), (1,)], [F, F, U, B], (10_843, 10_844)),
 ])
 @pytest.mark.parametrize("packed", [0, 4096])
 def test_flat_gathers(shapes, dtypes, batches, packed):
