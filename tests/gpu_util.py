@@ -64,3 +64,11 @@ def random_rows(rng, n, shapes, dtypes):
 
 def to_dev(arrays):
     return [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in arrays]
+
+
+def kernels(call):
+    """Names of what a call launches."""
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as p:
+        call()
+        torch.cuda.synchronize()
+    return [e.name for e in p.events()]

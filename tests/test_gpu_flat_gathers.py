@@ -4,14 +4,14 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_util import random_rows, t2n, to_dev, torch_types
+from gpu_util import kernels, random_rows, t2n, to_dev, torch_types
 
 pytestmark = pytest.mark.gpu
 
 F, U, L, B, H = np.float32, np.uint8, np.int64, np.bool_, np.float16
 
 
-@pytest.mark.parametrize("shapes,dtypes,batches", [
+CASES = [
     ([(1024,), (1,), (1,), (1,)], [U, L, F, B], (64, 4096, 4097, 9000)),          # 64 granules: 1024 workgroups, and more
     ([(301,), (9,), (1,), (301,), (1,)], [F, F, F, F, B], (500, 3449, 3450)),      # two large fields, one of three granules
     ([(1,), (2413,), (5,), (45,), (999,), (3, 3), (33,)], [B, U, F, H, U, U, L], (1700, 1737)),  # the first one small, all of odd sizes
@@ -19,13 +19,18 @@ F, U, L, B, H = np.float32, np.uint8, np.int64, np.bool_, np.float16
     ([(28224,), (1,)], [U, L], (113, 114, 594, 595)),
     ([(4096,), (1,)], [U, L], (7031, 7032)),                                       # around those with a wave to a row
     ([(300,), (300,), (5, 51), (1,)], [F, F, U, B], (10_843, 10_844)),
-])
-@pytest.mark.parametrize("packed", [0, 4096])
-def test_flat_gathers(shapes, dtypes, batches, packed):
+]
+
+
+def _row(shapes, dtypes):
+    return sum(int(np.prod(s)) * np.dtype(d).itemsize for s, d in zip(shapes, dtypes))
+
+
+# (packed rows have at most 4096 bytes)
+@pytest.mark.parametrize("packed,shapes,dtypes,batches", [(0,) + c for c in CASES] + [(4096,) + c for c in CASES if _row(*c[:2]) <= 4096])
+def test_flat_gathers(packed, shapes, dtypes, batches):
     from mindrl_amd.core import UniformReplayBuffer
     from oracle import orc
-    if packed and sum(int(np.prod(s)) * np.dtype(d).itemsize for s, d in zip(shapes, dtypes)) > 4096:
-        pytest.skip("rows too large to pack")
     rng = np.random.default_rng(len(shapes))
     cap = max(batches) + 50
     for batch in batches:
@@ -82,13 +87,6 @@ def test_rows_outside_are_flagged_once_each(shapes, dtypes, n):
     g.destroy()
 
 
-def _kernels(call):
-    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as p:
-        call()
-        torch.cuda.synchronize()
-    return [e.name for e in p.events()]
-
-
 @pytest.mark.parametrize("option,kernel", [(0, "k_short_gather"), (1, "k_rows_gather_rows"), (2, "k_rows_gather_wide")])
 def test_row_wave(option, kernel):
     """1 asks for a wave to a row, 2 forbids it."""
@@ -97,5 +95,6 @@ def test_row_wave(option, kernel):
     g.insert(to_dev([np.zeros((5000, 1024), U), np.zeros((5000, 1), L)]))
     g.set_option("row_wave", option)
     g.sample()
-    assert any(kernel in name for name in _kernels(lambda: g.sample())), _kernels(lambda: g.sample())
+    ran = kernels(lambda: g.sample())
+    assert any(kernel in name for name in ran), ran
     g.destroy()
