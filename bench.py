@@ -384,6 +384,41 @@ class PerRun:
             self._lib.check(rc)
 
 
+def sample_kernel(field_bytes, capacity, rows, sample_path=0, row_split=0):
+    """The kernel that mrb_per_sample takes for one batch of `rows` rows: the rules of per_sample_impl (takes_lds, takes_lanes,
+    lanes_better) and sample_wide in mrb.hip. A field of 16 bytes and more is copied in granules of 16, a smaller one byte by byte."""
+    depth = max(0, (capacity - 1).bit_length())
+    wide = sum((b + 15) // 16 for b in field_bytes if b >= 16)
+    narrow = sum(b for b in field_bytes if b < 16)
+    granules = [(b + size - 1) // size for b in field_bytes for size in [min(16, 1 << (b.bit_length() - 1))]]
+    rest = sum(g for f, g in enumerate(granules) if f >= 4 or g > 1)
+    lanes = rows >= 1024 and not row_split and depth >= 7 and narrow <= 48 and wide <= 1280
+    path = sample_path
+    if path == 0:
+        least = ((14336 if rest <= 16 else 20480 if rest <= 40 else 12288) if lanes else
+                 3072 if rest <= 16 else 5120 if rest <= 64 else 12288)
+        if wide > 64:
+            better = rows >= 2048 and (wide <= 192 or 256 < wide <= 512 or
+                                       (rows <= 4096 or rows >= 5632 if wide <= 256 else
+                                        rows <= 2048 or 3600 <= rows <= 4096 or rows >= 6000))
+        elif depth % 10 == 0:
+            better = rows >= (1408 if wide <= 16 and narrow <= 16 else 1664 if wide <= 32 else 1920)
+        elif depth in (21, 22):
+            better = rows >= (1024 if depth == 22 or wide <= 32 else 1280)
+        elif depth < 18:
+            better = rows >= (1280 if wide <= 32 else 1536)
+        else:
+            better = rows >= (1280 if wide <= 16 and narrow <= 16 else 1408 if wide <= 32 else 1664)
+        path = 2 if rest <= 384 and rows >= max(least, 5 if rest <= 64 else 8) else 3 if lanes and better else 1
+    if path == 2 and rest <= 1 << 23:
+        return "k_per_sample_lds"
+    if path == 3:
+        return "k_per_sample_lanes"
+    if not row_split and wide <= 256 and narrow <= 256 and rows >= 2048:
+        return "k_per_sample_rows"
+    return "k_per_sample_light" if not row_split and wide <= 256 and depth != 22 else "k_per_sample_wide"
+
+
 def bench_per(a):
     """Configs 1, 3, 4, 5 (prioritized buffers)."""
     import torch
@@ -436,19 +471,7 @@ def bench_per(a):
 
     row_bytes = sum(r.buf._layout.bytes)
     levels = max(1, (r.capacity - 1).bit_length())
-    # the library's own choice (mrb_per_sample): the LDS-top kernel for many narrow rows, else the wide-row kernel
-    lds_path = a.sample_path == 2 or (a.sample_path == 0 and batch >= 20480 and max(r.buf._layout.bytes) <= 256)
-    # (rows of at most 4 KB in 16-byte fields: the workgroup kernel with two copy waves; of thousands of rows, sixteen lanes to a stratum)
-    wide_granules = sum(b // 16 for b in r.buf._layout.bytes if b % 16 == 0)
-    narrow_bytes = sum(b for b in r.buf._layout.bytes if b % 16)
-    if lds_path:
-        kernel_name = "k_per_sample_lds"
-    elif wide_granules <= 1280 and narrow_bytes <= 48 and batch >= 2048 and a.sample_path == 0 and not a.row_split:
-        kernel_name = "k_per_sample_lanes"
-    elif wide_granules <= 256 and levels != 22 and not a.row_split:
-        kernel_name = "k_per_sample_light"
-    else:
-        kernel_name = "k_per_sample_wide"
+    kernel_name = sample_kernel(r.buf._layout.bytes, r.capacity, batch, a.sample_path, a.row_split)
     if a.workload == "c3":
         # rows read + rows written + index (8) + weight (4): the gather-bound headline figure
         algo_bytes, formula = batch * (2 * row_bytes + 12), "batch * (2 * row_bytes + 12)"

@@ -144,6 +144,23 @@ def test_trees_that_were_never_filled():
     g.destroy()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cap", [(r, c) for r in sorted(ROWS) + ["49"] for c in (100, 20_000, 200_000, 1_000_000, (1 << 20) + 1, (1 << 22) - 5)])
+def test_the_benchmark_names_the_kernel_that_runs(rows, cap):
+    import bench
+    from mindrl_amd.core import PriorityReplayBuffer
+    shapes, dtypes = ROWS.get(rows, ([(49,)] + [(1,)] * 4 + [(9,)] * 5, [U] * 10))
+    if cap * sum(int(np.prod(s)) for s in shapes) > 1e9:
+        cap = 20_000
+    g = PriorityReplayBuffer(0.6, cap, 8, shapes, torch_types(dtypes), seed0=2)
+    g.insert(*to_dev(random_rows(np.random.default_rng(cap), 5, shapes, dtypes)))
+    for batch in (64, 1024, 1300, 1500, 2048, 2500, 4000, 5500, 6500, 13_000, 15_000, 21_000):
+        g._sample_size = batch
+        want, ran = bench.sample_kernel(g._layout.bytes, cap, batch), kernels(lambda: g.sample(0.4))
+        assert any(want in name for name in ran), (batch, want, ran)
+    g.destroy()
+
+
 def test_registers(tmp_path):
     """No scratch memory, and no more registers than leave a compute unit two workgroups of eight waves (one where a lane holds
     eight granules of two rows)."""
