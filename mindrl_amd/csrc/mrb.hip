@@ -403,11 +403,10 @@ int sample_wide(const RowStore& r, const SampleArgs& a, const IoTable& t, int64_
         LAUNCH_CHECK("k_per_sample_next");
         return MRB_OK;
     }
-    // Many rows of up to 4 KB in 16-byte fields and a handful of narrow bytes: a wave per row (k_per_sample_rows)
-    // instead of a workgroup per row. One wave does in a row what six do side by side, so a launch of few rows
-    // takes longer that way (config 4, 1024 rows of 521 B: 6.4 us against 5.5) and a launch of many less (4096
-    // rows: 9.2 us against 15.6; 16,384: 26 against 54): a sixth of the waves to dispatch. (`row_split` asks for
-    // the workgroup kernel.)
+    // Many rows of up to 4 KB in 16-byte fields and 49 to 256 narrow bytes (with fewer, sixteen lanes to a stratum have taken them):
+    // a wave per row (k_per_sample_rows) instead of a workgroup per row. One wave does in a row what six do side by side, so a launch
+    // of few rows takes longer that way and a launch of many less, for a sixth of the waves to dispatch (rows of 521 bytes, wave /
+    // workgroup: 1024 6.4 / 5.5 us, 4096 9.2 / 15.6, 16,384 26 / 54). (`row_split` asks for the workgroup kernel.)
     const int64_t nrows = nbatch * a.batch;
     if (r.row_split == 0 && r.row_wave != 2 && plan.split == 1 && plan.wide_items <= (uint32_t)kRowWaveInF * 64u &&
         plan.narrow_items <= 256u && (nrows >= kRowWaveMinRows || r.row_wave == 1)) {
@@ -861,23 +860,36 @@ UpdateArgs update_args(Per& b) {
 }
 
 // Most entries of an update that elect the last writer of each leaf among themselves (a wave per entry scans
-// the call's entries); larger calls take the stamp pass (2048 measured: config 4's update 14.0 us against 14.7 with the pass, at twice the waves and four times the comparisons: not taken).
+// the call's entries); larger calls take the stamp pass (2048 entries on 2^21 leaves 14.0 us against 14.7 with the pass, at twice
+// the waves and four times the comparisons: not taken).
 constexpr int64_t kElectMax = 1024;
 
-// Whether an update of few entries goes by runs of leaves in k_range_one, whose workgroups read the priorities with the indices and leave where
-// they have no entry, rather than in k_tree_range. us, 20 levels: 1024 entries 6.9 / 7.3, 1500 8.0 / 7.7, 4096 9.3 / 8.9, one after the other 1500 7.4 / 7.5, 3000
-// 9.4 / 9.7, 4096 10.8 / 11.3; 21 levels 512 6.4 / 7.1, 1024 7.5 / 7.5; 22 levels 1024 7.8 / 8.0. Trees of fewer than 8 levels have no whole tile, those of
-// more than 22 more than 256 runs.
+// Whether an update of few entries goes by runs of leaves in k_range_one, whose workgroups read the priorities with the indices and
+// leave where they have no entry, rather than in k_tree_range. us, k_range_one / k_tree_range:
+//   levels   entries   random         one by one
+//   20       1024       6.9 /  7.3
+//   20       1500       8.0 /  7.7     7.4 /  7.5
+//   20       3000                      9.4 /  9.7
+//   20       4096       9.3 /  8.9    10.8 / 11.3    (the line of 4096 is where these two take turns)
+//   21        512       6.4 /  7.1
+//   21       1024       7.5 /  7.5
+//   22       1024       7.8 /  8.0
+// Trees of fewer than 8 levels have no whole tile, those of more than 22 more than 256 runs.
 bool takes_range_one(const Per& b, int64_t n) {
     return b.fused && n <= (b.depth <= 20 ? kOneMostEntries : kElectMax) && b.depth >= 8 && b.depth <= 22;
 }
 
-// Whether an update of more entries goes by runs of leaves (launch_tree_range). Against what it would take
-// otherwise, us per call, before / by runs:
-//   most entries    12 levels, 8192 / 16,384: 10.0 / 11.4 against 9.6 / 13.8; 14 levels, 16,384 / 32,768: 11.7 / 12.5 against 11.2 / 16.7; 20 levels 14.4 / 15.4 against
-//                   14.1 / 18.7. On 21 levels and more what its entries drive is the other way: see takes_sparse.
-//   deepest tree    23 and 24 levels leave more than a tile above the runs and bring many runs without an entry: 2048
-//                   entries 14.9 / 15.9 against 14.9 / 23.3.
+// Whether an update of more entries goes by runs of leaves (launch_tree_range). us, by stamps and tiles / by runs:
+//   levels   entries
+//   12         8192    10.0 /  9.6
+//   12       16,384    11.4 / 13.8
+//   14       16,384    11.7 / 11.2
+//   14       32,768    12.5 / 16.7
+//   20       16,384    14.4 / 14.1
+//   20       32,768    15.4 / 18.7
+//   23         2048    14.9 / 14.9     (more than a tile above the runs, and many runs without an entry)
+//   24         2048    15.9 / 23.3
+// On 21 levels and more what its entries drive is the other way: see takes_sparse.
 bool takes_range(const Per& b, int64_t n) {
     if (!b.fused || b.depth < 12 || b.depth > 22) return false;
     return !takes_range_one(b, n) && n <= (b.depth >= 21 ? 3072 : b.depth == 12 ? 8192 : 16384);
@@ -910,10 +922,13 @@ bool takes_sparse(const Per& b, int64_t n) {
     return b.s_g0 > 0 && n > kElectMax && n <= b.leaves >> share;
 }
 
-// Where one workgroup's update alone (k_tree_wg) is faster than that. 1 / 16 / 64 / 96 / 128 entries, us, it against runs: 10 levels
-// 3.5 / 3.5 / 3.5 / 3.6 / 3.6 against 3.2 / 3.4 / 3.4 / 3.4 / 3.4; 11 levels 3.8 / 3.8 / 3.8 / 3.9 / 3.9 against 3.2 / 3.9 / 4.0 / 4.0 / 4.0; 12 levels
-// 4.1 / 4.2 / 4.3 / 4.6 / 4.7 against 4.4 / 4.7 / 4.7 / 4.7 / 4.7. 1 / 64 / 96 / 128: 13 levels 4.1 / 4.4 / 4.6 / 4.8 against 4.6 / 4.7 / 4.7 / 4.7; 14
-// levels 4.1 / 4.4 / 4.7 / 4.9 against 4.5 / 4.7 / 4.7 / 4.8.
+// Where one workgroup's update alone (k_tree_wg) is faster than that. us, k_tree_wg / by runs:
+//   levels   1 entry      16           64           96           128
+//   10       3.5 / 3.2    3.5 / 3.4    3.5 / 3.4    3.6 / 3.4    3.6 / 3.4
+//   11       3.8 / 3.2    3.8 / 3.9    3.8 / 4.0    3.9 / 4.0    3.9 / 4.0    (left to the runs with 10 levels)
+//   12       4.1 / 4.4    4.2 / 4.7    4.3 / 4.7    4.6 / 4.7    4.7 / 4.7
+//   13       4.1 / 4.6                 4.4 / 4.7    4.6 / 4.7    4.8 / 4.7
+//   14       4.1 / 4.5                 4.4 / 4.7    4.7 / 4.7    4.9 / 4.8
 bool takes_wg_rather(const Per& b, int64_t n) { return b.depth >= 12 && b.depth <= kWgMaxDepth && n <= 96; }
 
 // update_priorities on buffer b with `powered` (device f32[n]) as the scratch that holds the entries'
@@ -1712,10 +1727,21 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
 // the same (batches x rows of one): 8-byte rows, 10^6 slots 4096 x 1 6.6 / 20, 4096 x 2 11.0 / 20.6, 2048 x 4 10.9 / 12.1,
 // 2048 x 6 14.6 / 9.9, 1024 x 8 10.8 / 6.4; 521 bytes 2048 x 4 11.0 / 13.8, 4096 x 5 26 / 22; 3 KB 4096 x 3 21 / 30, 4096 x 6
 // 36 / 43, 2048 x 8 26 / 26. (A row above 4 KB takes a whole workgroup there: 6 KB 4096 x 3 46 / 43.)
-// `lanes`: whether sixteen lanes to a stratum could take it (takes_lanes), which is the better one up to (lanes / LDS-top, us) 8-byte rows 8192
-// 4.5 / 5.1, 16,384 6.0 / 5.3; 41 bytes 12,288 5.7 / 6.2, 16,384 6.8 / 6.2; 153 bytes 16,384 7.4 / 7.5, 32,768 13.0 / 9.0; 521 bytes 16,384 7.9 / 9.0,
-// 32,768 14.0 / 11.6; 899 bytes in odd fields 12,288 9.5 / 9.8, 16,384 14.2 / 10.8; 1 KB 12,000 10.9 against a wave's 18.9, 16,384 14.2 / 12.4; 2.4 KB
-// 16,384 22.9 / 21.5.
+// `lanes`: whether sixteen lanes to a stratum could take it (takes_lanes), which are the better ones longer than a wave is. us,
+// LDS-top / lanes:
+//   row        slots       8192 rows      10,240        12,288        14,336        16,384        18,000        20,480
+//   8 bytes    2 * 10^5     4.7 / 4.4     4.7 / 4.9     4.7 / 5.1     4.7 / 5.8
+//   8          10^6         5.1 / 4.5     5.3 / 4.9     5.2 / 5.1     5.3 / 5.8
+//   41         5 * 10^4     6.0 / 4.1     5.9 / 4.9     6.0 / 5.0     6.0 / 5.7     5.9 / 5.9     6.1 / 6.8     6.1 / 6.9
+//   41         4 * 10^6     6.8 / 5.5     7.0 / 6.4     7.0 / 6.5     7.0 / 7.8     7.0 / 7.9
+//   145        5 * 10^4     5.7 / 4.4     5.7 / 5.6     5.8 / 5.7     5.9 / 6.3     5.9 / 6.6
+//   145        10^6         6.9 / 5.3     7.2 / 6.1     7.3 / 6.2     7.3 / 7.1     7.5 / 7.3     7.8 / 9.6
+//   521        5 * 10^4     7.4 / 5.0     7.7 / 6.3     8.1 / 6.6     8.2 / 7.4     8.4 / 7.7     9.2 / 9.1     9.6 / 10.3
+//   521        4 * 10^6     9.2 / 6.0     9.8 / 7.3    10.2 / 7.7    10.7 / 9.0    10.9 / 9.2    11.6 / 11.3   11.8 / 11.8
+//   899        2 * 10^5                                 9.8 / 9.5                  10.8 / 14.2
+//   1 KB       2 * 10^5                                18.9 / 10.9 (a wave's)      12.4 / 14.2
+//   2.4 KB     2 * 10^5                                                            21.5 / 22.9
+// (Of rows with nothing but scalars the line, 14,336, is right for some trees and 5 % off for others.)
 static bool takes_lds(int64_t nbatch, int64_t batch, uint64_t rest, bool lanes) {
     const int64_t rows = nbatch * batch, fewest = rest <= 64 ? 5 : rest <= 256 ? 8 : 1;
     const int64_t least = lanes ? (rest <= 16 ? 14336 : rest <= 40 ? 20480 : 12288) : (rest <= 16 ? 3072 : rest <= 64 ? 5120 : 12288);

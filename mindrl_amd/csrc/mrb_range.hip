@@ -24,9 +24,11 @@ struct Trees {
 // four. What it pays is that every workgroup reads all indices (out of its L2: 16 KB for 2048 entries), which is why larger calls keep the
 // stamp pass (the rule, with both sides measured, is at takes_range).
 // A call is bound by its chain of trips - indices, priorities of a run's own, tiles, the roots' meeting -, not
-// by bytes. 2048 entries on 2^21 leaves 14.7 -> 8.6 us, and 8.4 with the meeting in the place of a
-// second launch (5000 on 2^20 9.5 -> 9.0, 5000 one after the other on 2^14 6.7 -> 6.5), which a host that is behind takes 2.7 us longer to issue. (Up to 1024 entries, up to
-// 4096 on at most 20 levels, k_range_one, whose workgroups read the priorities with the indices, is faster.)
+// by bytes. 2048 entries on 2^21 leaves 14.7 -> 8.6 us, and 8.4 with the meeting in the place of a second launch, which
+// a host that is behind takes 2.7 us longer to issue. (On the device: 5000 entries at random on 2^20 leaves 9.8 -> 9.3, on 2^18 8.3 -> 8.0, on 2^16
+// 7.5 and 7.5, on 2^14 7.6 -> 7.8; one after the other 6.5 -> 6.1 on 2^14, but 6.5 -> 6.8 on 2^15, 6.6 -> 7.0 on 2^16 and 6.7 -> 7.0 on 2^17, where
+// the few workgroups with entries come last and count in two steps.) Up to 1024 entries, up to 4096 on at most 20 levels, k_range_one,
+// whose workgroups read the priorities with the indices, is faster.
 // ---------------------------------------------------------------------------
 // (no argument for what the kernel can tell: see PutArgs::threads)
 __host__ __device__ constexpr int range_threads(int64_t n) { return n > 4096 ? 1024 : 512; }  // (256: 0.3 to 1.5 us more)

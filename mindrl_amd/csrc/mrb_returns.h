@@ -41,7 +41,7 @@ namespace mrb {
 // streams their second halves came from memory again (13.4 -> 12.5 us at [1000, 4096]). us before / now, forward and backward:
 //   [1000, 4096] 14.3 14.2 / 11.8 11.8, [1000, 32] 12.4 12.9 / 11.2 11.4, [2000, 3001] 27.6 27.7 / 20.9 21.1, [65, 4825] 5.3 5.4 / 4.4 4.5,
 //   [1000, 8192] 17.8 17.5 / 15.8 16.5, [2000, 8000] 28.5 29.1 / 28.4 29.2, [2000, 7501] 40.0 40.5 / 33.4 33.7, [1000, 16384] 30.2 30.8 / 28.7 28.5,
-//   [1011, 204, 3] 14.6 14.6 / 12.2 12.0, [1000, 3000, 3] 25.8 26.1 / 19.4 18.9; [4000, 8192], 300 MB that no cache holds, 57.0 56.0 / 54.4 57.6.
+//   [1011, 204, 3] 14.6 14.6 / 12.2 12.0, [1000, 3000, 3] 25.8 26.1 / 19.4 18.9; [4000, 8192], 300 MB that no cache holds, 56.6 55.7 / 52.9 54.5.
 // kCols is small so that a few thousand columns spread over all
 // compute units, several workgroups to each when there are more. The pad of four floats puts the sixteen columns'
 // 16-byte reads into different banks, and the movers' scalar writes likewise.

@@ -153,9 +153,15 @@ __device__ __forceinline__ void put_fields(const RowTable* __restrict__ table, c
 }
 
 // Workgroups of a gather's largest field, a granule to a thread, from which on threads take four of the large fields and every field has its own
-// number of workgroups. A granule to a thread / four, us: 421 bytes 16,384 rows 6.5 / 6.8; 898 bytes 16,384 9.9 / 10.2, given slots 10.4 / 9.9; 809 bytes 8192 rows
-// 5.1 / 5.4, 16,384 8.1 / 7.8; 1.6 KB 2048 3.9 / 4.3, 4096 5.5 / 5.2, 16,384 17.2 / 12.5; 2.4 KB 2048 4.8 / 5.0, 4096 6.9 / 6.4, 16,384 19.7 / 17.1; 7.5 KB
-// 4096 20.5 / 13.9.
+// number of workgroups. us, a granule to a thread / four, drawn slots (given ones in brackets):
+//   row          workgroups
+//   1.4 KB        656    4.2 / 4.4 (3.9 / 3.8)        421 bytes    1216    6.2 / 6.5 (5.8 / 5.6)
+//   1 KB          773    5.2 / 5.3 (5.2 / 4.9)        817          1219    6.7 / 6.6 (6.4 / 6.0)
+//   0.8 KB        832    5.4 / 5.4 (5.3 / 4.9)        2.4 KB       1216    6.7 / 6.4 (6.4 / 5.7)
+//   1 KB         1024    4.2 / 4.6 (3.9 / 3.7)        1.4 KB       1312    5.6 / 5.5 (5.3 / 4.4)
+//   1 KB         1056    6.2 / 6.1 (5.9 / 5.5)        898          1568    6.6 / 6.3 (6.4 / 5.7)
+//   898 bytes    1148    5.4 / 5.9 (5.3 / 5.3)        1 KB         1500    5.1 / 5.0 (4.7 / 4.1)
+//                                                     7.5 KB       7504   20.4 / 13.9 (19.3 / 14.0)
 constexpr uint32_t kGatherFew = 1024;
 
 // A gather of many granules, one field's n rows by workgroup `block` of `blocks`: as put_field, with the rows' slots given or drawn (see gather_body).
