@@ -153,16 +153,19 @@ __device__ __forceinline__ void put_fields(const RowTable* __restrict__ table, c
 }
 
 // Workgroups of a gather's largest field, a granule to a thread, from which on threads take four of the large fields and every field has its own
-// number of workgroups. us, a granule to a thread / four, drawn slots (given ones in brackets):
-//   row          workgroups
-//   1.4 KB        656    4.2 / 4.4 (3.9 / 3.8)        421 bytes    1216    6.2 / 6.5 (5.8 / 5.6)
-//   1 KB          773    5.2 / 5.3 (5.2 / 4.9)        817          1219    6.7 / 6.6 (6.4 / 6.0)
-//   0.8 KB        832    5.4 / 5.4 (5.3 / 4.9)        2.4 KB       1216    6.7 / 6.4 (6.4 / 5.7)
-//   1 KB         1024    4.2 / 4.6 (3.9 / 3.7)        1.4 KB       1312    5.6 / 5.5 (5.3 / 4.4)
-//   1 KB         1056    6.2 / 6.1 (5.9 / 5.5)        898          1568    6.6 / 6.3 (6.4 / 5.7)
-//   898 bytes    1148    5.4 / 5.9 (5.3 / 5.3)        1 KB         1500    5.1 / 5.0 (4.7 / 4.1)
-//                                                     7.5 KB       7504   20.4 / 13.9 (19.3 / 14.0)
-constexpr uint32_t kGatherFew = 1024;
+// number of workgroups; later for drawn slots, which each granule draws for itself. us, a granule to a thread / four:
+//   row         workgroups   given           drawn            row         workgroups   given           drawn
+//   1.8 KB        928        5.5 / 5.0       5.6 / 5.6        1.8 KB       1359         6.7 / 6.1       7.1 / 6.8
+//   1.1 KB       1008        4.6 / 4.1       5.0 / 5.1        1.1 KB       1476         5.9 / 5.1       6.1 / 6.1
+//   1 KB         1024        3.6 / 3.6       4.2 / 4.5        0.6 KB       1500         6.3 / 5.6       6.4 / 6.7
+//   1 KB (odd)   1024        4.2 / 4.0       4.5 / 4.9        1 KB         1546         7.2 / 6.8       7.6 / 7.7
+//   1.4 KB       1054        5.3 / 5.3       5.7 / 6.0        0.9 KB       1568         6.2 / 5.7       6.5 / 6.3
+//   0.9 KB       1148        5.4 / 5.2       5.5 / 5.9        1.3 KB       1898         5.5 / 4.5       6.0 / 5.7
+//   0.6 KB       1152        4.0 / 3.8       4.4 / 4.7        1 KB         2048         5.7 / 4.6       6.1 / 6.1
+//   0.4 KB       1216        5.9 / 5.7       6.4 / 6.6        0.9 KB       3136         9.6 / 9.2       9.8 / 10.2
+//   0.8 KB       1218        6.3 / 6.0       6.6 / 6.7        1.6 KB       3200         8.3 / 6.4       8.8 / 7.8
+//   1.3 KB       1296        4.2 / 3.9       4.7 / 4.9        7.5 KB       7504        19.3 / 14.0     20.4 / 13.9
+constexpr uint32_t kGatherFew = 1024, kGatherFewDrawn = 1312;
 
 // A gather of many granules, one field's n rows by workgroup `block` of `blocks`: as put_field, with the rows' slots given or drawn (see gather_body).
 template <int kPer>

@@ -12,7 +12,7 @@ F, U, L, B, H = np.float32, np.uint8, np.int64, np.bool_, np.float16
 
 
 CASES = [
-    ([(1024,), (1,), (1,), (1,)], [U, L, F, B], (64, 4096, 4097, 9000)),          # 64 granules: 1024 workgroups, and more
+    ([(1024,), (1,), (1,), (1,)], [U, L, F, B], (64, 4096, 4097, 5248, 5249, 9000)),  # 64 granules: 1024 workgroups (drawn: 1312), and more
     ([(301,), (9,), (1,), (301,), (1,)], [F, F, F, F, B], (500, 3449, 3450)),      # two large fields, one of three granules
     ([(1,), (2413,), (5,), (45,), (999,), (3, 3), (33,)], [B, U, F, H, U, U, L], (1700, 1737)),  # the first one small, all of odd sizes
     ([(7500,)] + [(1,)] * 7, [U] * 8, (425, 426, 2230, 2236)),                     # eight fields; around those with a workgroup to a row

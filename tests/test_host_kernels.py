@@ -7,7 +7,7 @@ import subprocess
 import pytest
 
 
-@pytest.mark.parametrize("source,count", [("mrb_range_one.hip", 10), ("mrb_short.hip", 4), ("mrb_push_many.hip", 3)])
+@pytest.mark.parametrize("source,count", [("mrb_range_one.hip", 10), ("mrb_short.hip", 5), ("mrb_push_many.hip", 3)])
 def test_kernels_use_no_scratch_memory(source, count, tmp_path):
     from mindrl_amd import build
     out = tmp_path / "kernels.s"
