@@ -26,7 +26,7 @@ struct Trees {
 // A call is bound by its chain of trips - indices, priorities of a run's own, tiles, the roots' meeting -, not
 // by bytes. 2048 entries on 2^21 leaves 14.7 -> 8.6 us, and 8.4 with the meeting in the place of a second launch, which
 // a host that is behind takes 2.7 us longer to issue. (On the device: 5000 entries at random on 2^20 leaves 9.8 -> 9.3, on 2^18 8.3 -> 8.0, on 2^16
-// 7.5 and 7.5, on 2^14 7.6 -> 7.8; one after the other 6.5 -> 6.1 on 2^14, but 6.5 -> 6.8 on 2^15, 6.6 -> 7.0 on 2^16 and 6.7 -> 7.0 on 2^17, where
+// 7.5 and 7.5, on 2^14 7.6 -> 7.8 and 12,000 10.0 -> 10.4; one after the other 6.5 -> 6.1 on 2^14, but 6.5 -> 6.8 on 2^15, 6.6 -> 7.0 on 2^16 and 6.7 -> 7.0 on 2^17, where
 // the few workgroups with entries come last and count in two steps.) Up to 1024 entries, up to 4096 on at most 20 levels, k_range_one,
 // whose workgroups read the priorities with the indices, is faster.
 // ---------------------------------------------------------------------------
