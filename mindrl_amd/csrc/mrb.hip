@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "mrb_kernels.h"
+#include "mrb_launch.h"
 #include "mrb_meet.h"
 #include "mrb_push_many.h"
 #include "mrb_range.h"
@@ -265,7 +266,7 @@ int rows_put(const RowStore& r, const void* const* src, int64_t skip, int64_t n,
         const hipError_t e = launch_short_put(r.table, io, p.t, first_slot, n, s);
         return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch k_short_put: %s", hipGetErrorString(e));
     }
-    hipLaunchKernelGGL(k_rows_put, dim3(p.blocks), dim3(kWG), 0, s, p);
+    launch_kernel(k_rows_put, dim3(p.blocks), dim3(kWG), 0, s, p);
     LAUNCH_CHECK("k_rows_put");
     return MRB_OK;
 }
@@ -334,8 +335,8 @@ inline uint32_t wide_threads(const WidePlan& plan) { return plan.narrow_items ? 
 template <int kInF, bool kTen, bool kOneWide>
 void launch_sample_wide(dim3 grid, const SampleArgs& a, const WidePlan& plan, hipStream_t s) {
     const SampleTail tail{a.mn, a.out_idx, a.out_w, a.err, a.size, a.beta};
-    hipLaunchKernelGGL((k_per_sample_wide<kInF, kTen, kOneWide>), grid, dim3(wide_threads(plan)), 0, s, a.sum, a.uniforms, a.depth,
-                       groups_word(a, plan.nbatch), (int)a.batch, (uint32_t)a.capacity, a.seed, a.calls, tail, plan);
+    launch_kernel((k_per_sample_wide<kInF, kTen, kOneWide>), grid, dim3(wide_threads(plan)), 0, s, a.sum, a.uniforms, a.depth,
+                  groups_word(a, plan.nbatch), (int)a.batch, (uint32_t)a.capacity, a.seed, a.calls, tail, plan);
 }
 
 template <int kInF>
@@ -358,8 +359,8 @@ constexpr int64_t kRowWaveMinRows = 2048;  // fewest rows of a launch that go to
 template <int kInF, bool kTen, bool kOneWide>
 void launch_sample_next(dim3 grid, const SampleArgs& a, const WidePlan& plan, const NextPlan& nx, hipStream_t s) {
     const SampleTail tail{a.mn, a.out_idx, a.out_w, a.err, a.size, a.beta};
-    hipLaunchKernelGGL((k_per_sample_next<kInF, kTen, kOneWide>), grid, dim3(wide_threads(plan)), 0, s, a.sum, a.uniforms, a.depth,
-                       groups_word(a, 1), (int)a.batch, (uint32_t)a.capacity, a.seed, a.calls, tail, plan, nx);
+    launch_kernel((k_per_sample_next<kInF, kTen, kOneWide>), grid, dim3(wide_threads(plan)), 0, s, a.sum, a.uniforms, a.depth,
+                  groups_word(a, 1), (int)a.batch, (uint32_t)a.capacity, a.seed, a.calls, tail, plan, nx);
 }
 
 template <int kInF>
@@ -414,11 +415,11 @@ int sample_wide(const RowStore& r, const SampleArgs& a, const IoTable& t, int64_
         const uint32_t blocks = (uint32_t)((nrows + kRowWaveWG / 64 - 1) / (kRowWaveWG / 64));
         const uint32_t packed = groups_word(a, plan.nbatch);
         if (a.depth > 0 && a.depth % kGroupMaxLevels == 0)
-            hipLaunchKernelGGL((k_per_sample_rows<true>), dim3(blocks), dim3(kRowWaveWG), 0, s, a.sum, a.uniforms, a.depth, packed,
-                               (int)a.batch, (uint32_t)a.capacity, a.seed, a.calls, nrows, tail, plan);
+            launch_kernel((k_per_sample_rows<true>), dim3(blocks), dim3(kRowWaveWG), 0, s, a.sum, a.uniforms, a.depth, packed,
+                          (int)a.batch, (uint32_t)a.capacity, a.seed, a.calls, nrows, tail, plan);
         else
-            hipLaunchKernelGGL((k_per_sample_rows<false>), dim3(blocks), dim3(kRowWaveWG), 0, s, a.sum, a.uniforms, a.depth, packed,
-                               (int)a.batch, (uint32_t)a.capacity, a.seed, a.calls, nrows, tail, plan);
+            launch_kernel((k_per_sample_rows<false>), dim3(blocks), dim3(kRowWaveWG), 0, s, a.sum, a.uniforms, a.depth, packed,
+                          (int)a.batch, (uint32_t)a.capacity, a.seed, a.calls, nrows, tail, plan);
         LAUNCH_CHECK("k_per_sample_rows");
         return MRB_OK;
     }
@@ -429,8 +430,8 @@ int sample_wide(const RowStore& r, const SampleArgs& a, const IoTable& t, int64_
         const dim3 threads(plan.narrow_items ? (uint32_t)kLightWG : (uint32_t)kLightWG - 64u);
         const bool ten = a.depth > 0 && a.depth % kGroupMaxLevels == 0, one = plan.nwide == 1;
 #define MRB_LAUNCH_LIGHT(T, O)                                                                                         \
-    hipLaunchKernelGGL((k_per_sample_light<T, O>), grid, threads, 0, s, a.sum, a.uniforms, a.depth, packed, (int)a.batch, \
-                       (uint32_t)a.capacity, a.seed, a.calls, tail, plan)
+    launch_kernel((k_per_sample_light<T, O>), grid, threads, 0, s, a.sum, a.uniforms, a.depth, packed, (int)a.batch, \
+                  (uint32_t)a.capacity, a.seed, a.calls, tail, plan)
         if (ten) { if (one) MRB_LAUNCH_LIGHT(true, true); else MRB_LAUNCH_LIGHT(true, false); }
         else { if (one) MRB_LAUNCH_LIGHT(false, true); else MRB_LAUNCH_LIGHT(false, false); }
 #undef MRB_LAUNCH_LIGHT
@@ -447,11 +448,11 @@ template <int kInF>
 void launch_gather_wide(dim3 grid, const int64_t* indices, int mode, int64_t count, int64_t fixed_slot, uint64_t seed,
                         uint64_t calls, int64_t* out_indices, uint32_t* err, const WidePlan& plan, hipStream_t s) {
     if (plan.nwide == 1)
-        hipLaunchKernelGGL((k_rows_gather_wide<kInF, true>), grid, dim3(wide_threads(plan)), 0, s, indices, mode, count, fixed_slot, seed,
-                           calls, out_indices, err, plan);
+        launch_kernel((k_rows_gather_wide<kInF, true>), grid, dim3(wide_threads(plan)), 0, s, indices, mode, count, fixed_slot, seed,
+                      calls, out_indices, err, plan);
     else
-        hipLaunchKernelGGL((k_rows_gather_wide<kInF, false>), grid, dim3(wide_threads(plan)), 0, s, indices, mode, count, fixed_slot, seed,
-                           calls, out_indices, err, plan);
+        launch_kernel((k_rows_gather_wide<kInF, false>), grid, dim3(wide_threads(plan)), 0, s, indices, mode, count, fixed_slot, seed,
+                      calls, out_indices, err, plan);
 }
 
 // Gather of n rows whose slots are given (indices), drawn from the generator (indices NULL,
@@ -501,8 +502,8 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
         // 8192 20.7 / 13.6; 1 KB: 2048 5.2 / 5.5, 4096 7.4 / 5.9).
         if (r.row_split == 0 && plan.split == 1 && plan.wide_items <= (uint32_t)kRowWaveInF * 64u && plan.narrow_items <= 256u &&
             inflight != 0 && n >= kRowWaveMinRows && r.row_wave != 2) {
-            hipLaunchKernelGGL(k_rows_gather_rows, dim3((uint32_t)((n + kRowWaveWG / 64 - 1) / (kRowWaveWG / 64))), dim3(kRowWaveWG),
-                               0, s, indices, mode, count, fixed_slot, seed, calls, n, out_indices, err, plan);
+            launch_kernel(k_rows_gather_rows, dim3((uint32_t)((n + kRowWaveWG / 64 - 1) / (kRowWaveWG / 64))), dim3(kRowWaveWG),
+                          0, s, indices, mode, count, fixed_slot, seed, calls, n, out_indices, err, plan);
             LAUNCH_CHECK("k_rows_gather_rows");
             return MRB_OK;
         }
@@ -520,8 +521,8 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
         const hipError_t e = launch_short_gather(r.table, io, t, indices, count, seed, calls, n, blocks, out_indices != nullptr, s);
         return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch k_short_gather: %s", hipGetErrorString(e));
     }
-    hipLaunchKernelGGL(k_rows_gather, dim3(blocks, (uint32_t)t.nfields), dim3(kWG), 0, s, indices, fixed_slot, seed, calls,
-                       count, out_indices, err, r.capacity, blocks, t);
+    launch_kernel(k_rows_gather, dim3(blocks, (uint32_t)t.nfields), dim3(kWG), 0, s, indices, fixed_slot, seed, calls,
+                  count, out_indices, err, r.capacity, blocks, t);
     LAUNCH_CHECK("k_rows_gather");
     return MRB_OK;
 }
@@ -704,7 +705,7 @@ uint32_t push_units(const UpdateArgs& a) {
 constexpr uint32_t kRideWithCounters = 64;
 int ride_alone_if_large(const UpdateArgs& a, PutArgs& put, hipStream_t s) {
     if (a.advance && put.blocks > kRideWithCounters) {
-        hipLaunchKernelGGL(k_rows_put, dim3(put.blocks), dim3(kWG), 0, s, put);
+        launch_kernel(k_rows_put, dim3(put.blocks), dim3(kWG), 0, s, put);
         LAUNCH_CHECK("k_rows_put");
         put.blocks = 0;
     }
@@ -740,7 +741,7 @@ int tree_rebuild(Per& b, UpdateArgs a, hipStream_t s, const PutArgs* ride = null
         if (a.full_top) {
             // (the update's launch before this one has carried the row copy)
             a.readers = 1;
-            hipLaunchKernelGGL(k_tree_fused, dim3(1), dim3(kFusedWG), 0, s, a, (uint32_t)(a.first_slot / kBlockNodes), units);
+            launch_kernel(k_tree_fused, dim3(1), dim3(kFusedWG), 0, s, a, (uint32_t)(a.first_slot / kBlockNodes), units);
             LAUNCH_CHECK("k_tree_fused");
             return MRB_OK;
         }
@@ -752,7 +753,7 @@ int tree_rebuild(Per& b, UpdateArgs a, hipStream_t s, const PutArgs* ride = null
             return e == hipSuccess ? MRB_OK : fail(MRB_EHIP, "launch k_short_push_run: %s", hipGetErrorString(e));
         }
         a.readers = 1 + put.blocks;  // (a.advance != 0: this one launch also moves the device's counters on)
-        hipLaunchKernelGGL(k_push_run, dim3(1 + put.blocks), dim3(threads), 0, s, a, units, put);
+        launch_kernel(k_push_run, dim3(1 + put.blocks), dim3(threads), 0, s, a, units, put);
         LAUNCH_CHECK("k_push_run");
         return MRB_OK;
     }
@@ -780,8 +781,8 @@ int tree_rebuild(Per& b, UpdateArgs a, hipStream_t s, const PutArgs* ride = null
         const PutArgs& put = (r == 0 && ride) ? *ride : none;
         if (r == 0 && a.inline_election) tiles = (a.n > kPairedAbove ? 2u : 1u) * (uint32_t)a.n;  // one or two waves per entry (see k_tree_update)
         a.tile_blocks = (tiles + 3) / 4;
-        hipLaunchKernelGGL(k_tree_update, dim3(a.tile_blocks + put.blocks), dim3(kWG), 0, s, a.indices, a.priorities, a.sum, a.mn,
-                           a.n, a.capacity, r | a.lo[r] << 8 | a.g[r] << 16, a.alpha, a, tile_base, put);
+        launch_kernel(k_tree_update, dim3(a.tile_blocks + put.blocks), dim3(kWG), 0, s, a.indices, a.priorities, a.sum, a.mn,
+                      a.n, a.capacity, r | a.lo[r] << 8 | a.g[r] << 16, a.alpha, a, tile_base, put);
         LAUNCH_CHECK("k_tree_update");
     }
     PutArgs put = (a.nrounds == 0 && ride) ? *ride : none;
@@ -790,7 +791,7 @@ int tree_rebuild(Per& b, UpdateArgs a, hipStream_t s, const PutArgs* ride = null
     // the top is the call's last launch: it moves the device's counters on (a.advance != 0); only when it is also
     // the first do its workgroups read the ring position
     a.readers = a.nrounds == 0 ? 1 + put.blocks : 0;
-    hipLaunchKernelGGL(k_tree_top, dim3(1 + put.blocks), dim3(kTopWG), 0, s, a, put);
+    launch_kernel(k_tree_top, dim3(1 + put.blocks), dim3(kTopWG), 0, s, a, put);
     LAUNCH_CHECK("k_tree_top");
     return MRB_OK;
 }
@@ -798,7 +799,7 @@ int tree_rebuild(Per& b, UpdateArgs a, hipStream_t s, const PutArgs* ride = null
 // Zero-fills `bytes` (a multiple of 4) of device memory with a kernel.
 void fill_zero(void* p, size_t bytes, hipStream_t s) {
     const uint64_t n = bytes / sizeof(float);
-    hipLaunchKernelGGL(k_fill_f32, dim3(grid_for(n)), dim3(kWG), 0, s, static_cast<float*>(p), 0.0f, n);
+    launch_kernel(k_fill_f32, dim3(grid_for(n)), dim3(kWG), 0, s, static_cast<float*>(p), 0.0f, n);
 }
 
 // A push whose leaf tiles are rebuilt by several workgroups, or whose powers one shares out over its threads (k_push_many): with
@@ -978,14 +979,14 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
     if (!sparse && b->fused && n <= kWgBestEntries && b->depth >= 2 && b->depth <= kWgMaxDepth) {
         // (65 to 128 entries: 1024 threads, eight per entry - the kernel's one-step path below the staged top)
         const uint32_t threads = n > 64 && n <= 128 ? 1024u : n <= kWgMinThreads ? (uint32_t)kWgMinThreads : (uint32_t)((n + 63) / 64 * 64);
-        hipLaunchKernelGGL(k_tree_wg, dim3(1), dim3(threads), 0, s, a.indices, a.priorities, a.sum, a.mn, a.maxp, (int)a.n,
-                           a.depth | (int)threads << 8, (int)a.capacity, a.alpha);
+        launch_kernel(k_tree_wg, dim3(1), dim3(threads), 0, s, a.indices, a.priorities, a.sum, a.mn, a.maxp, (int)a.n,
+                      a.depth | (int)threads << 8, (int)a.capacity, a.alpha);
         LAUNCH_CHECK("k_tree_wg");
         return MRB_OK;
     }
     // At most 64 entries on a very deep tree: one wave walks the entries' paths, leaves to root, in one launch (k_tree_paths).
     if (!sparse && b->fused && n <= kPathEntries && b->depth <= kPathMaxDepth) {
-        hipLaunchKernelGGL(k_tree_paths, dim3(1), dim3(64), 0, s, a);
+        launch_kernel(k_tree_paths, dim3(1), dim3(64), 0, s, a);
         LAUNCH_CHECK("k_tree_paths");
         return MRB_OK;
     }
@@ -995,8 +996,8 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
         a.inline_election = 1;
         return tree_rebuild(*b, a, s);
     }
-    hipLaunchKernelGGL(k_update_stamp, dim3(grid_exact((uint64_t)n)), dim3(kWG), 0, s, a.indices, a.priorities, a.stamp, a.powered, a.maxp,
-                       (uint32_t)a.n, (uint32_t)a.capacity, a.epoch, a.alpha, !sparse && a.nrounds ? a.dirty[0] : nullptr, a.g[0]);
+    launch_kernel(k_update_stamp, dim3(grid_exact((uint64_t)n)), dim3(kWG), 0, s, a.indices, a.priorities, a.stamp, a.powered, a.maxp,
+                  (uint32_t)a.n, (uint32_t)a.capacity, a.epoch, a.alpha, !sparse && a.nrounds ? a.dirty[0] : nullptr, a.g[0]);
     LAUNCH_CHECK("k_update_stamp");
     if (!sparse) return tree_rebuild(*b, a, s);
     const auto checked = [](hipError_t e, const char* name) {
@@ -1009,8 +1010,8 @@ int per_update(Per& pb, const int64_t* indices, const float* priorities, int64_t
     for (int r = 0; r < last; ++r) {
         const uint32_t tiles = (1u << b->s_lo[r]) / kBlockNodes;
         a.tile_blocks = (tiles + 3) / 4;
-        hipLaunchKernelGGL(k_tree_update, dim3(a.tile_blocks), dim3(kWG), 0, s, a.indices, a.priorities, a.sum, a.mn, a.n,
-                           a.capacity, r | a.lo[r] << 8 | a.g[r] << 16, a.alpha, a, 0u, PutArgs{});
+        launch_kernel(k_tree_update, dim3(a.tile_blocks), dim3(kWG), 0, s, a.indices, a.priorities, a.sum, a.mn, a.n,
+                      a.capacity, r | a.lo[r] << 8 | a.g[r] << 16, a.alpha, a, 0u, PutArgs{});
         LAUNCH_CHECK("k_tree_update");
     }
     return checked(launch_tree_runs(a.sum, a.mn, a.dirty[last], a.maxp, a.lo[last], a.epoch, s), "k_tree_runs");
@@ -1047,12 +1048,12 @@ int counters_from_device(Urb& b) {
     return MRB_OK;
 }
 int counters_advance(Urb& b, int64_t rows, int64_t calls, hipStream_t s) {
-    hipLaunchKernelGGL(k_urb_advance, dim3(1), dim3(64), 0, s, b.counters, rows, b.rows.capacity, calls);
+    launch_kernel(k_urb_advance, dim3(1), dim3(64), 0, s, b.counters, rows, b.rows.capacity, calls);
     LAUNCH_CHECK("k_urb_advance");
     return MRB_OK;
 }
 int counters_advance(Per& b, int64_t pushed, int64_t calls, hipStream_t s) {
-    hipLaunchKernelGGL(k_counters_advance, dim3(1), dim3(64), 0, s, b.counters, pushed, b.rows.capacity, calls);
+    launch_kernel(k_counters_advance, dim3(1), dim3(64), 0, s, b.counters, pushed, b.rows.capacity, calls);
     LAUNCH_CHECK("k_counters_advance");
     return MRB_OK;
 }
@@ -1083,12 +1084,12 @@ int res_push_by_stamps(Res& b, const IoTable& t, int64_t nrows, bool elect, hipS
             LAUNCH_CHECK("k_fill_f32");
             b.epoch += 1;
         }
-        hipLaunchKernelGGL(k_res_elect, dim3(grid_exact((uint64_t)nrows)), dim3(kWG), 0, s, b.stamp, b.total, nrows,
-                           cap, b.seed, (uint32_t)b.epoch);
+        launch_kernel(k_res_elect, dim3(grid_exact((uint64_t)nrows)), dim3(kWG), 0, s, b.stamp, b.total, nrows,
+                      cap, b.seed, (uint32_t)b.epoch);
         LAUNCH_CHECK("k_res_elect");
     }
-    hipLaunchKernelGGL(k_res_put, dim3(grid_for(t.prefix[t.nfields])), dim3(kWG), 0, s, t,
-                       elect ? b.stamp : nullptr, b.total, cap, b.seed, (uint32_t)b.epoch);
+    launch_kernel(k_res_put, dim3(grid_for(t.prefix[t.nfields])), dim3(kWG), 0, s, t,
+                  elect ? b.stamp : nullptr, b.total, cap, b.seed, (uint32_t)b.epoch);
     LAUNCH_CHECK("k_res_put");
     return MRB_OK;
 }
@@ -1206,7 +1207,7 @@ int mrb_urb_append(int64_t h, const void* const* src_fields, int64_t nrows, void
         if (rc) return rc;
         p.first_slot = -1;
         p.src_first = reinterpret_cast<int64_t>(b->counters);
-        hipLaunchKernelGGL(k_rows_put, dim3(p.blocks), dim3(kWG), 0, s, p);
+        launch_kernel(k_rows_put, dim3(p.blocks), dim3(kWG), 0, s, p);
         LAUNCH_CHECK("k_rows_put");
         urb_advance(*b, nrows);
         return counters_advance(*b, nrows, 0, s);
@@ -1253,7 +1254,7 @@ int mrb_urb_append_from(int64_t h, int64_t src, int64_t first_logical, int64_t n
     p.src_first = (src_first + skip) % from->rows.capacity;
     p.blocks = grid_for(p.t.prefix[p.t.nfields]);
     p.threads = kWG;
-    hipLaunchKernelGGL(k_rows_put, dim3(p.blocks), dim3(kWG), 0, static_cast<hipStream_t>(stream), p);
+    launch_kernel(k_rows_put, dim3(p.blocks), dim3(kWG), 0, static_cast<hipStream_t>(stream), p);
     LAUNCH_CHECK("k_rows_put");
     urb_advance(*b, n);
     return MRB_OK;
@@ -1273,8 +1274,8 @@ int mrb_urb_get_item(int64_t h, int64_t logical_index, void* const* dst_fields, 
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (b->device_counters) {
         // count and head are read on the device: the slot is worked out there and the gather takes it as a given index
-        hipLaunchKernelGGL(k_urb_slots, dim3(1), dim3(kWG), 0, s, b->slots, b->seed, b->counters, (int64_t)1, logical_index, 1,
-                           b->err);
+        launch_kernel(k_urb_slots, dim3(1), dim3(kWG), 0, s, b->slots, b->seed, b->counters, (int64_t)1, logical_index, 1,
+                      b->err);
         LAUNCH_CHECK("k_urb_slots");
         return gather_rows(b->rows, b->slots, -1, b->rows.capacity, b->seed, b->calls, 1, nullptr, dst_fields, b->err, s);
     }
@@ -1305,8 +1306,8 @@ int mrb_urb_sample(int64_t h, int64_t n, int64_t* out_indices, void* const* dst_
         // takes them as given indices, and the call counter moves on there
         if (n > kUrbDrawMax)
             return fail(MRB_ESTATE, "with device_counters a sample takes at most %lld rows", (long long)kUrbDrawMax);
-        hipLaunchKernelGGL(k_urb_slots, dim3(grid_exact((uint64_t)n)), dim3(kWG), 0, s, b->slots, b->seed, b->counters, n,
-                           (int64_t)0, 0, b->err);
+        launch_kernel(k_urb_slots, dim3(grid_exact((uint64_t)n)), dim3(kWG), 0, s, b->slots, b->seed, b->counters, n,
+                      (int64_t)0, 0, b->err);
         LAUNCH_CHECK("k_urb_slots");
         int rc = gather_rows(b->rows, b->slots, -1, b->rows.capacity, b->seed, b->calls, n, out_indices, dst_fields, b->err, s);
         if (rc) return rc;
@@ -1451,7 +1452,7 @@ int mrb_per_create(int64_t capacity, float alpha, int nfields, const int64_t* fi
             HIP_TRY(hipMemset(b->s_dirty[r], 0, nblocks * sizeof(uint32_t)));
         }
     }
-    hipLaunchKernelGGL(k_fill_f32, dim3(grid_for(nodes)), dim3(kWG), 0, nullptr, b->mn, FLT_MAX, (uint64_t)nodes);
+    launch_kernel(k_fill_f32, dim3(grid_for(nodes)), dim3(kWG), 0, nullptr, b->mn, FLT_MAX, (uint64_t)nodes);
     LAUNCH_CHECK("k_fill_f32");
     const float one_then_zero[4] = {1.0f, 0.0f, 0.0f, 0.0f};  // the running max; the max a push in progress has seen
     HIP_TRY(hipMemcpy(b->maxp, one_then_zero, sizeof(one_then_zero), hipMemcpyHostToDevice));
@@ -1501,7 +1502,7 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
             const hipError_t e = launch_short_put(b->rows.table, io, put.t, first, n, s);
             if (e != hipSuccess) return fail(MRB_EHIP, "launch k_short_put: %s", hipGetErrorString(e));
         } else {
-            hipLaunchKernelGGL(k_rows_put, dim3(put.blocks), dim3(kWG), 0, s, put);
+            launch_kernel(k_rows_put, dim3(put.blocks), dim3(kWG), 0, s, put);
             LAUNCH_CHECK("k_rows_put");
         }
         put.blocks = 0;
@@ -1511,8 +1512,8 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
         const uint32_t waves = (lead->a.n > kPairedAbove ? 2u : 1u) * (uint32_t)lead->a.n;
         UpdateArgs la = lead->a;
         la.tile_blocks = (waves + 3) / 4;
-        hipLaunchKernelGGL(k_tree_update, dim3(la.tile_blocks + put.blocks), dim3(kWG), 0, s, la.indices, la.priorities, la.sum,
-                           la.mn, la.n, la.capacity, 0 | la.lo[0] << 8 | la.g[0] << 16, la.alpha, la, 0u, put);
+        launch_kernel(k_tree_update, dim3(la.tile_blocks + put.blocks), dim3(kWG), 0, s, la.indices, la.priorities, la.sum,
+                      la.mn, la.n, la.capacity, 0 | la.lo[0] << 8 | la.g[0] << 16, la.alpha, la, 0u, put);
         LAUNCH_CHECK("k_tree_update");
         put.blocks = 0;
     }
@@ -1547,9 +1548,9 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
                                                        a.alpha, opt_priorities, most_granules(put.t), s);
             if (e != hipSuccess) return fail(MRB_EHIP, "launch k_short_push_one: %s", hipGetErrorString(e));
         } else {
-            hipLaunchKernelGGL(b->device_counters ? k_push_one<true> : k_push_one<false>, dim3(1 + put.blocks), dim3(kWG), 0, s,
-                               a.sum, a.mn, a.maxp, a.first_slot, a.capacity, a.leaves, a.depth, a.alpha, opt_priorities, a.err, put,
-                               a.advance, 1 + put.blocks * (kWG / 64));
+            launch_kernel(b->device_counters ? k_push_one<true> : k_push_one<false>, dim3(1 + put.blocks), dim3(kWG), 0, s,
+                          a.sum, a.mn, a.maxp, a.first_slot, a.capacity, a.leaves, a.depth, a.alpha, opt_priorities, a.err, put,
+                          a.advance, 1 + put.blocks * (kWG / 64));
             LAUNCH_CHECK("k_push_one");
         }
         b->pushes += nrows;
@@ -1562,8 +1563,8 @@ static int per_push(Per* b, const void* const* src_fields, int64_t nrows, const 
         a.priorities = opt_priorities;
         a.n = nrows;
         // (no indices: nothing to elect, the priorities are looked at and folded into the running max)
-        hipLaunchKernelGGL(k_update_stamp, dim3(grid_exact((uint64_t)nrows)), dim3(kWG), 0, s, a.indices, a.priorities, a.stamp, a.powered, a.maxp,
-                           (uint32_t)a.n, (uint32_t)a.capacity, a.epoch, a.alpha, static_cast<uint32_t*>(nullptr), 0);
+        launch_kernel(k_update_stamp, dim3(grid_exact((uint64_t)nrows)), dim3(kWG), 0, s, a.indices, a.priorities, a.stamp, a.powered, a.maxp,
+                      (uint32_t)a.n, (uint32_t)a.capacity, a.epoch, a.alpha, static_cast<uint32_t*>(nullptr), 0);
         LAUNCH_CHECK("k_update_stamp");
     }
     b->pushes += nrows;
@@ -1678,15 +1679,15 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
         const uint32_t threads = n > 64 && n <= 128 ? 1024u : n <= kWgMinThreads ? (uint32_t)kWgMinThreads : (uint32_t)((n + 63) / 64 * 64);
                 a.readers = 1 + put.blocks * (threads / 64);
                 put.threads = threads;
-                hipLaunchKernelGGL(b->device_counters ? k_tree_wg_push<true> : k_tree_wg_push<false>, dim3(1 + put.blocks),
-                                   dim3(threads), 0, s, a.indices, a.priorities, a.sum, a.mn, a.maxp, (int)a.n,
-                                   a.depth | (int)threads << 8,
-                                   (int)a.capacity, a.alpha, a, slot, opt_push_priorities, put);
+                launch_kernel(b->device_counters ? k_tree_wg_push<true> : k_tree_wg_push<false>, dim3(1 + put.blocks),
+                              dim3(threads), 0, s, a.indices, a.priorities, a.sum, a.mn, a.maxp, (int)a.n,
+                              a.depth | (int)threads << 8,
+                              (int)a.capacity, a.alpha, a, slot, opt_push_priorities, put);
                 LAUNCH_CHECK("k_tree_wg_push");
             } else {
                 a.readers = 1 + put.blocks * (kWG / 64);
-                hipLaunchKernelGGL(b->device_counters ? k_tree_paths_push<true> : k_tree_paths_push<false>, dim3(1 + put.blocks),
-                                   dim3(kWG), 0, s, a, slot, opt_push_priorities, put);
+                launch_kernel(b->device_counters ? k_tree_paths_push<true> : k_tree_paths_push<false>, dim3(1 + put.blocks),
+                              dim3(kWG), 0, s, a, slot, opt_push_priorities, put);
                 LAUNCH_CHECK("k_tree_paths_push");
             }
             b->pushes += 1;
@@ -1923,9 +1924,9 @@ int mrb_per_update_push_sample(int64_t h, const int64_t* indices, const float* p
             const bool wide = n > 64 && n <= 128;  // 1024 threads, eight per entry (see k_tree_wg)
             auto* const kernel = b->device_counters ? (wide ? k_tree_wg_push_sample<true, 1024> : k_tree_wg_push_sample<true, kStepThreads>)
                                                     : (wide ? k_tree_wg_push_sample<false, 1024> : k_tree_wg_push_sample<false, kStepThreads>);
-            hipLaunchKernelGGL(kernel, dim3(1), dim3(wide ? 1024 : kStepThreads), 0, s, indices, priorities, b->sum, b->mn, a.maxp,
-                               (int)(cap << 16 | (b->device_counters ? 0 : first)), (int)(n << 18 | batch << 8) | b->depth, a.alpha,
-                               late);
+            launch_kernel(kernel, dim3(1), dim3(wide ? 1024 : kStepThreads), 0, s, indices, priorities, b->sum, b->mn, a.maxp,
+                          (int)(cap << 16 | (b->device_counters ? 0 : first)), (int)(n << 18 | batch << 8) | b->depth, a.alpha,
+                          late);
             LAUNCH_CHECK("k_tree_wg_push_sample");
             b->pushes += 1;
             b->size = late.size;
@@ -2046,8 +2047,8 @@ int mrb_res_push(int64_t h, const void* const* src_fields, int64_t nrows, void* 
     int64_t per_row = 0;
     for (int f = 0; f < t.nfields; ++f) per_row += t.units[f];
     if (const int rows = elect ? res_rows_per_workgroup(nrows, per_row, cap) : 0) {
-        hipLaunchKernelGGL(k_res_push, dim3((uint32_t)((nrows + rows - 1) / rows)), dim3(kResWG), 0, s, b->total, cap, b->seed,
-                           (int)nrows, rows, t.nfields, (uint32_t)per_row, t);
+        launch_kernel(k_res_push, dim3((uint32_t)((nrows + rows - 1) / rows)), dim3(kResWG), 0, s, b->total, cap, b->seed,
+                      (int)nrows, rows, t.nfields, (uint32_t)per_row, t);
         LAUNCH_CHECK("k_res_push");
     } else {
         rc = res_push_by_stamps(*b, t, nrows, elect, s);
@@ -2170,9 +2171,9 @@ int mrb_per_load_leaves(int64_t h, const float* leaves, int64_t n, float max_pri
     hipStream_t s = static_cast<hipStream_t>(stream);
     const size_t nodes = 2 * (size_t)b->leaves;
     fill_zero(b->sum, nodes * sizeof(float), s);
-    hipLaunchKernelGGL(k_fill_f32, dim3(grid_for(nodes)), dim3(kWG), 0, s, b->mn, FLT_MAX, (uint64_t)nodes);
+    launch_kernel(k_fill_f32, dim3(grid_for(nodes)), dim3(kWG), 0, s, b->mn, FLT_MAX, (uint64_t)nodes);
     LAUNCH_CHECK("k_fill_f32");
-    hipLaunchKernelGGL(k_fill_f32, dim3(1), dim3(kWG), 0, s, b->maxp, max_priority, (uint64_t)1);
+    launch_kernel(k_fill_f32, dim3(1), dim3(kWG), 0, s, b->maxp, max_priority, (uint64_t)1);
     LAUNCH_CHECK("k_fill_f32");
     if (n == 0) return MRB_OK;
     int rc = next_epoch(*b, s);
@@ -2191,7 +2192,7 @@ int mrb_per_load_leaves(int64_t h, const float* leaves, int64_t n, float max_pri
 int mrb_bench_launch(int kind, void* dst, const void* src, int64_t bytes, void* stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (kind == 0) {
-        hipLaunchKernelGGL(k_nothing, dim3(1), dim3(64), 0, s);
+        launch_kernel(k_nothing, dim3(1), dim3(64), 0, s);
         LAUNCH_CHECK("k_nothing");
         return MRB_OK;
     }
@@ -2246,8 +2247,8 @@ static int discounted_return(const float* x, const uint8_t* done, float* end_val
                                            : 65536;
     const bool per_column = cols > most;
     if (per_column) {
-        hipLaunchKernelGGL(k_discounted_return, dim3(grid_exact((uint64_t)cols)), dim3(kWG), 0, s, x, done, end_value, out,
-                           timesteps, batch, inner, gamma, kBack ? 1 : 0);
+        launch_kernel(k_discounted_return, dim3(grid_exact((uint64_t)cols)), dim3(kWG), 0, s, x, done, end_value, out,
+                      timesteps, batch, inner, gamma, kBack ? 1 : 0);
         LAUNCH_CHECK("k_discounted_return");
         return MRB_OK;
     }

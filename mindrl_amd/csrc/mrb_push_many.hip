@@ -1,6 +1,7 @@
 #include "mrb_push_many.h"
 
 #include "../../include/mrb.h"
+#include "mrb_launch.h"
 #include "mrb_meet.h"
 #include "mrb_push.h"
 #include "mrb_tree.h"
@@ -287,8 +288,8 @@ hipError_t launch_push_many(const RowTable* table, const ShortIo& io, const IoTa
     auto* kernel = k_push_many<4, false>;
     if (per == 1) kernel = k_push_many<1, false>;
     if (tiles == 1) kernel = k_push_many<1, true>;
-    hipLaunchKernelGGL(kernel, grid, dim3(kWG), 0, s, sum, mn, maxp,
-                       priorities, table, (uint32_t)first_slot, (uint32_t)n, (uint32_t)depth | groups << 8, alpha, blocks, io);
+    launch_kernel(kernel, grid, dim3(kWG), 0, s, sum, mn, maxp,
+                  priorities, table, (uint32_t)first_slot, (uint32_t)n, (uint32_t)depth | groups << 8, alpha, blocks, io);
     return hipGetLastError();
 }
 

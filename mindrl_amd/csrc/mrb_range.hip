@@ -1,6 +1,7 @@
 #include "mrb_range.h"
 
 #include "../../include/mrb.h"
+#include "mrb_launch.h"
 #include "mrb_meet.h"
 #include "mrb_rows.h"
 #include "mrb_tree.h"
@@ -317,7 +318,7 @@ hipError_t launch_tree_range(const int64_t* indices, const float* priorities, in
     const int w = tree_range_levels(depth);
     const dim3 grid((uint32_t)((capacity + ((int64_t)1 << w) - 1) >> w)), threads(range_threads(n));
     auto* const kernel = w <= 10 ? k_tree_range<10> : w <= 12 ? k_tree_range<12> : w == 13 ? k_tree_range<13> : k_tree_range<14>;
-    hipLaunchKernelGGL(kernel, grid, threads, 0, s, indices, priorities, sum, mn, maxp, (int)n, (int)capacity, depth | w << 8, alpha);
+    launch_kernel(kernel, grid, threads, 0, s, indices, priorities, sum, mn, maxp, (int)n, (int)capacity, depth | w << 8, alpha);
     return hipGetLastError();
 }
 
@@ -325,13 +326,13 @@ hipError_t launch_tree_sparse(const int64_t* indices, const unsigned long long* 
                               uint32_t* dirty, int64_t n, int64_t capacity, int depth, int g0, int g_dirty, uint32_t epoch,
                               hipStream_t s) {
     const dim3 grid((uint32_t)(((n << (g0 - 2)) + kSparseWG - 1) / kSparseWG));
-    hipLaunchKernelGGL(g0 == 4 ? k_tree_sparse<4> : k_tree_sparse<0>, grid, dim3(kSparseWG), 0, s, indices, stamp, powered, sum, mn, dirty, (int)n, (uint32_t)capacity,
-                       epoch, depth | g0 << 8 | g_dirty << 16);
+    launch_kernel(g0 == 4 ? k_tree_sparse<4> : k_tree_sparse<0>, grid, dim3(kSparseWG), 0, s, indices, stamp, powered, sum, mn, dirty, (int)n, (uint32_t)capacity,
+                  epoch, depth | g0 << 8 | g_dirty << 16);
     return hipGetLastError();
 }
 
 hipError_t launch_tree_runs(float* sum, float* mn, const uint32_t* dirty, float* maxp, int top, uint32_t epoch, hipStream_t s) {
-    hipLaunchKernelGGL(k_tree_runs, dim3(1u << kRoundLevels), dim3(64u << (top - 2 * kRoundLevels)), 0, s, sum, mn, dirty, maxp, epoch, top);
+    launch_kernel(k_tree_runs, dim3(1u << kRoundLevels), dim3(64u << (top - 2 * kRoundLevels)), 0, s, sum, mn, dirty, maxp, epoch, top);
     return hipGetLastError();
 }
 

@@ -1,6 +1,7 @@
 #include "mrb_range_one.h"
 
 #include "../../include/mrb.h"
+#include "mrb_launch.h"
 #include "mrb_meet.h"
 #include "mrb_tree.h"
 
@@ -290,8 +291,8 @@ hipError_t launch_range_one(const int64_t* indices, const float* priorities, int
         if (w > 12) return hipErrorInvalidValue;  // (more than 20 levels: not taken, see takes_range_one)
         kernel = w <= 10 ? k_range_one<10, kOneMany> : k_range_one<12, kOneMany>;
     }
-    hipLaunchKernelGGL(kernel, dim3(runs_of(capacity, w)), dim3(kOneWG), 0, s, indices, priorities, sum, mn, maxp, (int)n, (int)capacity,
-                       depth | w << 8, alpha);
+    launch_kernel(kernel, dim3(runs_of(capacity, w)), dim3(kOneWG), 0, s, indices, priorities, sum, mn, maxp, (int)n, (int)capacity,
+                  depth | w << 8, alpha);
     return hipGetLastError();
 }
 
@@ -303,8 +304,8 @@ hipError_t launch_range_one_push(const int64_t* indices, const float* priorities
     ride.blocks = (put.blocks * kWG + kOneWG - 1) / kOneWG;
     ride.threads = kOneWG;
     auto* const kernel = w <= 10 ? k_range_one_push<10> : w <= 12 ? k_range_one_push<12> : w == 13 ? k_range_one_push<13> : k_range_one_push<14>;
-    hipLaunchKernelGGL(kernel, dim3(runs + ride.blocks), dim3(kOneWG), 0, s, indices, priorities, sum, mn, maxp, (int)n, (int)capacity,
-                       depth | w << 8, alpha, runs, push, ride);
+    launch_kernel(kernel, dim3(runs + ride.blocks), dim3(kOneWG), 0, s, indices, priorities, sum, mn, maxp, (int)n, (int)capacity,
+                  depth | w << 8, alpha, runs, push, ride);
     return hipGetLastError();
 }
 

@@ -1,5 +1,6 @@
 // The instantiations of k_discounted_return_tiled and the rule that chooses among them.
 #include "mrb_returns.h"
+#include "mrb_launch.h"
 
 namespace mrb {
 
@@ -10,11 +11,11 @@ void launch(bool back, const float* x, const uint8_t* done, float* end_value, fl
             int64_t inner, float gamma, hipStream_t s) {
     const dim3 grid((uint32_t)((batch * inner + kCols - 1) / kCols)), threads(64 + kMovers);
     if (back)
-        hipLaunchKernelGGL((k_discounted_return_tiled<true, kQuad, kCols, kMovers>), grid, threads, 0, s, x, done, end_value, out,
-                           timesteps, batch, inner, gamma);
+        launch_kernel((k_discounted_return_tiled<true, kQuad, kCols, kMovers>), grid, threads, 0, s, x, done, end_value, out,
+                      timesteps, batch, inner, gamma);
     else
-        hipLaunchKernelGGL((k_discounted_return_tiled<false, kQuad, kCols, kMovers>), grid, threads, 0, s, x, done, end_value, out,
-                           timesteps, batch, inner, gamma);
+        launch_kernel((k_discounted_return_tiled<false, kQuad, kCols, kMovers>), grid, threads, 0, s, x, done, end_value, out,
+                      timesteps, batch, inner, gamma);
 }
 
 }  // namespace

@@ -1,5 +1,6 @@
 // Samples of thousands of rows, sixteen lanes to a stratum: the kernel and its launch.
 #include "mrb_samples.h"
+#include "mrb_launch.h"
 
 namespace mrb {
 
@@ -331,8 +332,8 @@ hipError_t launch_per_sample_lanes(const SampleArgs& a, const WidePlan& plan, in
         else if (strata == 8) kernel = w <= 128 ? k_per_sample_lanes<8, true, 2> : w <= 256 ? k_per_sample_lanes<8, true, 4> : k_per_sample_lanes<8, true, 8>;
         else kernel = w <= 128 ? k_per_sample_lanes<16, true, 2> : w <= 256 ? k_per_sample_lanes<16, true, 4> : k_per_sample_lanes<16, true, 8>;
     }
-    hipLaunchKernelGGL(kernel, dim3((nrows + strata - 1) / strata), dim3(kLanes * strata + 64 * kLanesCopyWaves), (size_t)(5 << levels) + 8, s,
-                       a.sum, a.uniforms, a.mn, shape, (uint32_t)a.batch, nrows, (uint32_t)a.capacity, a.seed, a.calls, tail, plan);
+    launch_kernel(kernel, dim3((nrows + strata - 1) / strata), dim3(kLanes * strata + 64 * kLanesCopyWaves), (size_t)(5 << levels) + 8, s,
+                  a.sum, a.uniforms, a.mn, shape, (uint32_t)a.batch, nrows, (uint32_t)a.capacity, a.seed, a.calls, tail, plan);
     return hipGetLastError();
 }
 

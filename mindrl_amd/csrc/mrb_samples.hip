@@ -1,5 +1,6 @@
 // Samples of thousands of rows: the LDS-top kernel and its launch.
 #include "mrb_samples.h"
+#include "mrb_launch.h"
 
 namespace mrb {
 
@@ -163,8 +164,8 @@ hipError_t launch_per_sample_lds(const SampleArgs& a, const IoTable& t, int64_t 
                          : strata == 32 ? k_per_sample_lds<32>
                          : strata == 64 ? k_per_sample_lds<64>
                                         : k_per_sample_lds<256>;
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)((a.batch + strata - 1) / strata), (uint32_t)nbatch), dim3(kLdsWG), lds, s, a.sum,
-                       a.uniforms, a.mn, a.depth, levels, (int)a.batch, a.beta, a.seed, a.calls, rest, a, t);
+    launch_kernel(kernel, dim3((uint32_t)((a.batch + strata - 1) / strata), (uint32_t)nbatch), dim3(kLdsWG), lds, s, a.sum,
+                  a.uniforms, a.mn, a.depth, levels, (int)a.batch, a.beta, a.seed, a.calls, rest, a, t);
     return hipGetLastError();
 }
 

@@ -1,6 +1,7 @@
 #include "mrb_short.h"
 
 #include "mrb_gather.h"
+#include "mrb_launch.h"
 
 namespace mrb {
 
@@ -71,26 +72,26 @@ hipError_t launch_short_gather(const RowTable* table, const ShortIo& io, const I
     if (blocks > (indices ? kGatherFew : kGatherFewDrawn)) {
         dim3 grid(0);
         for (int f = 0; f < t.nfields; ++f) grid.x += put_blocks(t.prefix[f + 1] - t.prefix[f], kWG);
-        hipLaunchKernelGGL(k_short_gather_many, grid, dim3(kWG), 0, s, table, indices, seed, calls, (uint32_t)count, (uint32_t)n, with_indices ? 1 : 0, io);
+        launch_kernel(k_short_gather_many, grid, dim3(kWG), 0, s, table, indices, seed, calls, (uint32_t)count, (uint32_t)n, with_indices ? 1 : 0, io);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(k_short_gather, dim3(blocks, (uint32_t)t.nfields), dim3(kWG), 0, s, table, indices, seed, calls, (uint32_t)count, (uint32_t)n,
-                       blocks, with_indices ? 1 : 0, io);
+    launch_kernel(k_short_gather, dim3(blocks, (uint32_t)t.nfields), dim3(kWG), 0, s, table, indices, seed, calls, (uint32_t)count, (uint32_t)n,
+                  blocks, with_indices ? 1 : 0, io);
     return hipGetLastError();
 }
 
 hipError_t launch_short_put(const RowTable* table, const ShortIo& io, const IoTable& t, int64_t first_slot, int64_t n, hipStream_t s) {
     uint32_t blocks;
     const dim3 grid = put_grid(t, 0, blocks);
-    hipLaunchKernelGGL(k_short_put, grid, dim3(kWG), 0, s, table, (uint32_t)first_slot, (uint32_t)n, blocks, io);
+    launch_kernel(k_short_put, grid, dim3(kWG), 0, s, table, (uint32_t)first_slot, (uint32_t)n, blocks, io);
     return hipGetLastError();
 }
 
 hipError_t launch_short_push_one(const RowTable* table, const ShortIo& io, int nfields, float* sum, float* mn, float* maxp, int64_t first_slot,
                                  int depth, float alpha, const float* priority, uint64_t granules, hipStream_t s) {
     const uint32_t blocks = put_blocks(granules, kWG);
-    hipLaunchKernelGGL(k_short_push_one, dim3(1 + blocks, (uint32_t)nfields), dim3(kWG), 0, s, sum, mn, maxp, table, priority,
-                       (uint32_t)first_slot, depth, alpha, blocks, io);
+    launch_kernel(k_short_push_one, dim3(1 + blocks, (uint32_t)nfields), dim3(kWG), 0, s, sum, mn, maxp, table, priority,
+                  (uint32_t)first_slot, depth, alpha, blocks, io);
     return hipGetLastError();
 }
 
@@ -98,8 +99,8 @@ hipError_t launch_short_push_run(const RowTable* table, const ShortIo& io, int n
                                  uint32_t threads, hipStream_t s) {
     const uint32_t plan = (uint32_t)a.depth | units << 8 | (threads == (uint32_t)kFusedWG ? 1u << 16 : 0u) | (a.fold_max ? 1u << 17 : 0u);
     const uint32_t blocks = put_blocks(granules, threads);
-    hipLaunchKernelGGL(k_short_push_run, dim3(1 + blocks, (uint32_t)nfields), dim3(threads), 0, s, a.sum, a.mn, a.maxp, a.priorities, table,
-                       (uint32_t)a.first_slot, (uint32_t)a.n, plan, a.alpha, (uint32_t)a.capacity, blocks, io);
+    launch_kernel(k_short_push_run, dim3(1 + blocks, (uint32_t)nfields), dim3(threads), 0, s, a.sum, a.mn, a.maxp, a.priorities, table,
+                  (uint32_t)a.first_slot, (uint32_t)a.n, plan, a.alpha, (uint32_t)a.capacity, blocks, io);
     return hipGetLastError();
 }
 
