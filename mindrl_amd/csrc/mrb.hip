@@ -299,6 +299,7 @@ int wide_plan(const RowStore& r, const IoTable& t, int64_t n, WidePlan& plan, di
         plan.f[q].first = items;
         items += wide ? r.units[i] : t.row_bytes[i];
     }
+    plan.through = stores_through(batch_bytes(t));
     const uint32_t per_wg = (uint32_t)kMaxInFlight * kCopyThreads;
     uint32_t split = (plan.wide_items + per_wg - 1) / per_wg;
     if (r.row_split > (int64_t)split) split = (uint32_t)r.row_split;
@@ -394,6 +395,7 @@ int sample_wide(const RowStore& r, const SampleArgs& a, const IoTable& t, int64_
         const uint32_t per_wg = (uint32_t)kMaxInFlight * kCopyThreads;
         const uint32_t split = (nx.plan.wide_items + per_wg - 1) / per_wg;
         nx.plan.split = (int)split;
+        plan.through = nx.plan.through = stores_through(batch_bytes(t) + (uint64_t)a.batch * r.bytes[f]);
         nx.plan.share = (nx.plan.wide_items + split - 1) / split;
         if (split > 65535u) return fail(MRB_EINVAL, "field %d is too wide for one launch", f);
         if (split > grid.y) grid.y = split;

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/mrb.h"
 #include "mrb_device.h"
 
@@ -374,7 +376,7 @@ struct WidePlan {
     uint32_t narrow_items;  // bytes of narrow fields per row
     int nwide, nnarrow;     // fields of each kind
     uint32_t nbatch;        // host side only: batches in the launch
-    uint32_t pad;
+    uint32_t through;       // whether the batch is stored through the L2 (see store_granule)
     WideField f[MRB_MAX_FIELDS];  // the wide fields first, then the narrow ones
 };
 
@@ -396,6 +398,32 @@ constexpr int kMaxInFlight = 8;             // most granules a copy thread holds
 constexpr int kFastWide = 2;                // wide fields whose table entries are fetched unconditionally, in one round
 
 using g16 = MRB_GLOBAL granule16_u;
+
+// A granule of a batch, or (kThrough) of a large one: stored through the die's L2 into memory at once. What lies changed in the eight
+// dies' caches (4 MB each) when a kernel ends is written out then, with nothing else going on; a large batch's stores had better be on
+// their way while rows are still being read. The memory's own cache keeps them either way, and a read of the batch right behind is not
+// slower (220 MB: sampled and read 128 us as before, 124 so), as it is behind non-temporal stores (149).
+// Smaller batches are faster left in the L2. us, L2 / through, by MB of the batch:
+//                                       14            16            20             24             32             48             64             220
+//   sample, 28 KB rows               9.3 /  9.2    9.7 / 10.0    10.8 / 10.4    12.5 / 11.8    15.0 / 14.3    21.6 / 19.9    26.9 / 24.5    88.0 / 84.0
+//   uniform gather, 28 KB            9.0 /  8.9    9.0 /  9.5    10.2 / 10.0    11.6 / 11.2    14.3 / 13.5    19.8 / 18.1    25.2 / 23.1
+//   uniform gather, 7.5 KB           8.7 /  8.7    9.4 /  9.3    10.7 / 10.8    12.3 / 12.2    15.3 / 14.5    21.1 / 19.6    26.4 / 25.0
+//   uniform gather, 4 KB             7.9 /  8.2    8.5 /  8.6    10.2 / 10.1    11.6 / 11.4    13.8 / 13.2    19.3 / 18.0    24.7 / 22.8
+//   uniform gather, 2.4 KB           8.3 /  8.7    9.3 /  9.4    10.9 / 10.7    12.5 / 12.0    15.5 / 15.5
+// (k_per_sample_lanes, whose lanes store pieces of many rows at once, is slower so at every size: 7.5 KB 32.2 / 35.8 with 64 MB.)
+template <bool kThrough>
+__device__ __forceinline__ void store_granule(g16* to, granule_t v) {
+    // (an instruction for which there is no builtin with an address to a lane; the s_nop keeps v as it is until the store has read it)
+    if (kThrough) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(to), "v"(v) : "memory");
+    else *to = v;
+}
+constexpr uint64_t kThroughBytes = 20ull << 20;
+inline uint64_t batch_bytes(const IoTable& t) {
+    uint64_t bytes = 0;
+    for (int f = 0; f < t.nfields; ++f) bytes += (t.prefix[f + 1] - t.prefix[f]) << t.vec_log2[f];
+    return bytes;
+}
+inline bool stores_through(uint64_t bytes) { return bytes > kThroughBytes; }
 
 constexpr int kNarrowInF = 2;  // narrow bytes a thread of the first copy wave holds beside its wide granules
 
@@ -576,13 +604,16 @@ struct CopyWork {
             // next to its conditional store, behind the other stores' waits)
 #pragma unroll
             for (int j = 0; j < kInF; ++j) asm volatile("" : "+v"(held[j]));
+            auto store = [&](auto through) {
 #pragma unroll
-            for (int j = 0; j < kInF; ++j) {
-                if (live & (1u << j)) {
-                    if (kOneWide) *(g16*)(as_global(dst0) + off[j]) = held[j];
-                    else *dst[j < (kOneWide ? 1 : kInF) ? j : 0] = held[j];
-                }
-            }
+                for (int j = 0; j < kInF; ++j)
+                    if (live & (1u << j)) {
+                        if (kOneWide) store_granule<decltype(through)::value>((g16*)(as_global(dst0) + off[j]), held[j]);
+                        else store_granule<decltype(through)::value>(dst[j < (kOneWide ? 1 : kInF) ? j : 0], held[j]);
+                    }
+            };
+            if (plan.through) store(std::true_type{});  // uniform
+            else store(std::false_type{});
         }
         if (narrow) nw.store(slot, nheld, plan, lane);
     }

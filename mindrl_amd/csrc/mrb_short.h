@@ -168,7 +168,7 @@ __device__ __forceinline__ void put_fields(const RowTable* __restrict__ table, c
 constexpr uint32_t kGatherFew = 1024, kGatherFewDrawn = 1312;
 
 // A gather of many granules, one field's n rows by workgroup `block` of `blocks`: as put_field, with the rows' slots given or drawn (see gather_body).
-template <int kPer>
+template <int kPer, bool kThrough = false>
 __device__ __forceinline__ void gather_field(const ShortRows& rows, int f, const int64_t* __restrict__ indices, int64_t count, uint64_t seed,
                                              uint64_t calls, uint32_t block, uint32_t blocks) {
     const uint32_t units = rows.units(f), vl = rows.vl(f), row_bytes = rows.row_bytes(f), stride = rows.stride(f);
@@ -202,7 +202,7 @@ __device__ __forceinline__ void gather_field(const ShortRows& rows, int f, const
             for (int q = 0; q < kPer; ++q) asm volatile("" : "+v"(held[q]));
 #pragma unroll
             for (int q = 0; q < kPer; ++q)
-                if (w + q * kWG < total) *(g16*)(to + row[q] * row_bytes + granule_offset(unit[q], 4, row_bytes)) = held[q];
+                if (w + q * kWG < total) store_granule<kThrough>((g16*)(to + row[q] * row_bytes + granule_offset(unit[q], 4, row_bytes)), held[q]);
         } else {
             const uint32_t off = granule_offset(unit[0], vl, row_bytes);
             copy_granule(to + row[0] * row_bytes + off, store + (uint64_t)slot[0] * stride + off, vl);
@@ -210,10 +210,12 @@ __device__ __forceinline__ void gather_field(const ShortRows& rows, int f, const
     }
 }
 __device__ __forceinline__ void gather_fields(const ShortRows& rows, const int64_t* __restrict__ indices, int64_t count, uint64_t seed, uint64_t calls,
-                                              uint32_t block) {
+                                              uint32_t block, bool through) {
     uint32_t blocks;
     const int f = field_of_block(rows.r, rows.n, block, blocks);
-    if (rows.vl(f) == 4 && rows.granules(f) > (uint64_t)kPutFew * kWG) gather_field<kPutTrip>(rows, f, indices, count, seed, calls, block, blocks);
+    const bool many = rows.vl(f) == 4 && rows.granules(f) > (uint64_t)kPutFew * kWG;
+    if (many && through) gather_field<kPutTrip, true>(rows, f, indices, count, seed, calls, block, blocks);
+    else if (many) gather_field<kPutTrip>(rows, f, indices, count, seed, calls, block, blocks);
     else gather_field<1>(rows, f, indices, count, seed, calls, block, blocks);
 }
 

@@ -17,8 +17,8 @@ __global__ __launch_bounds__(kWG) void k_short_gather(const RowTable* __restrict
 // The same for many granules: four to a thread of the large fields, each field its own workgroups. (A kernel of its own: in one with the
 // other, whose threads need 18 registers, they had 46, and 16,384 drawn rows of 899 bytes, a granule to a thread, took 10.4 us for 9.8.)
 __global__ __launch_bounds__(kWG) void k_short_gather_many(const RowTable* __restrict__ table, const int64_t* __restrict__ indices, uint64_t seed,
-                                                           uint64_t calls, uint32_t count, uint32_t n, int with_indices, ShortIo io) {
-    gather_fields(ShortRows{table, io, n, with_indices}, indices, count, seed, calls, blockIdx.x);
+                                                           uint64_t calls, uint32_t count, uint32_t n, int flags, ShortIo io) {
+    gather_fields(ShortRows{table, io, n, flags & 1}, indices, count, seed, calls, blockIdx.x, flags & 2);
 }
 
 __global__ __launch_bounds__(kWG) void k_short_put(const RowTable* __restrict__ table, uint32_t first_slot, uint32_t n, uint32_t blocks,
@@ -72,7 +72,8 @@ hipError_t launch_short_gather(const RowTable* table, const ShortIo& io, const I
     if (blocks > (indices ? kGatherFew : kGatherFewDrawn)) {
         dim3 grid(0);
         for (int f = 0; f < t.nfields; ++f) grid.x += put_blocks(t.prefix[f + 1] - t.prefix[f], kWG);
-        launch_kernel(k_short_gather_many, grid, dim3(kWG), 0, s, table, indices, seed, calls, (uint32_t)count, (uint32_t)n, with_indices ? 1 : 0, io);
+        launch_kernel(k_short_gather_many, grid, dim3(kWG), 0, s, table, indices, seed, calls, (uint32_t)count, (uint32_t)n,
+                      (with_indices ? 1 : 0) | (stores_through(batch_bytes(t)) ? 2 : 0), io);
         return hipGetLastError();
     }
     launch_kernel(k_short_gather, dim3(blocks, (uint32_t)t.nfields), dim3(kWG), 0, s, table, indices, seed, calls, (uint32_t)count, (uint32_t)n,
