@@ -30,3 +30,19 @@ def test_kernels_use_no_scratch_memory(source, count, tmp_path):
         # the election words, a root of each tree and a mark per tile, a mark per run and a word per wave
         leaves = 1 << int(runs.group(1))
         assert 0 <= lds - (8 * leaves + 12 * (leaves // 256)) <= 1088, (name, lds)
+
+
+@pytest.mark.parametrize("source", ["mrb.hip", "mrb_short.hip"])
+def test_stores_written_in_assembly_keep_their_registers(source, tmp_path):
+    """A 16-byte store's registers may be written two wait states behind it, which the compiler does not look after in inline assembly."""
+    from mindrl_amd import build
+    out = tmp_path / "kernels.s"
+    flags = [f for f in build.HIPCC_FLAGS if f not in ("-shared", "-fPIC")]
+    res = subprocess.run(["/opt/rocm/bin/hipcc"] + flags + ["--cuda-device-only", "-S", "-o", str(out), os.path.join(build.CSRC, source)],
+                         stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert res.returncode == 0, res.stdout
+    written = re.findall(r";;#ASMSTART\n(.*?);;#ASMEND", out.read_text(), re.S)
+    stores = [text for text in written if "store_dwordx4" in text]
+    assert stores
+    for text in stores:
+        assert re.search(r"store_dwordx4 [^\n]*\n\s*s_nop ([1-9])", text), text
