@@ -259,6 +259,16 @@ __device__ __forceinline__ float lane_value(float x, uint32_t src_lane) {
 // its global loads and stores, which __syncthreads() would also wait for.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// Stores 16 bytes, or 4, through the die's L2 into memory at once (and into the memory's cache): an instruction for which there is no
+// builtin with 16 bytes at an address to a lane. A vector instruction may write the registers of a store of more than 8 bytes two wait
+// states behind it: the compiler sees to that for its own stores, the s_nop here. With one, values of the next addresses were stored.
+template <typename V>
+__device__ __forceinline__ void store_through(void* to, V v) {
+    static_assert(sizeof(V) == 16 || sizeof(V) == 4, "four words or one");
+    if constexpr (sizeof(V) == 16) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(to), "v"(v) : "memory");
+    else asm volatile("global_store_dword %0, %1, off sc1" ::"v"(to), "v"(v) : "memory");
+}
+
 // Between LDS accesses of lanes of ONE wave that hand each other values: what stands before it is done before what stands behind
 // it. The device takes a wave's LDS accesses in order, so this is an order for the compiler and no instruction.
 __device__ __forceinline__ void wave_lds_fence() {

@@ -42,6 +42,12 @@ namespace mrb {
 //   [1000, 4096] 14.3 14.2 / 11.8 11.8, [1000, 32] 12.4 12.9 / 11.2 11.4, [2000, 3001] 27.6 27.7 / 20.9 21.1, [65, 4825] 5.3 5.4 / 4.4 4.5,
 //   [1000, 8192] 17.8 17.5 / 15.8 16.5, [2000, 8000] 28.5 29.1 / 28.4 29.2, [2000, 7501] 40.0 40.5 / 33.4 33.7, [1000, 16384] 30.2 30.8 / 28.7 28.5,
 //   [1011, 204, 3] 14.6 14.6 / 12.2 12.0, [1000, 3000, 3] 25.8 26.1 / 19.4 18.9; [4000, 8192], 300 MB that no cache holds, 56.6 55.7 / 52.9 54.5.
+// Up to 32 MB of results are stored through the L2 at once. What a non-temporal store leaves of a 128-byte line that two groups share is
+// written twice, and a plain one's lines are written when the kernel ends; but more of them push the inputs out of the memory's
+// cache. us, non-temporal / plain / through: [135, 52] 4.6 / 4.0 / 4.1, [353, 444] 6.3 / 5.9 / 6.0, [1494, 290] 16.6 / 16.4 / 16.1, [128, 5000] 4.7 / - / 4.3,
+// [200, 8000] 6.0 / 6.3 / 5.6, [1000, 4096] 11.9 / 13.1 / 11.6, [2000, 3001] 21.0 / 21.7 / 20.3, [1000, 2500, 3] 15.0 / - / 13.9, [1000, 8192] 15.9 / - / 15.7;
+// [4000, 4096] 37.7 / - / 37.4, [2000, 7501] 28.3 / - / 28.5, [3000, 1365, 3] 29.2 / - / 31.8, [2000, 2700, 3] 25.8 / - / 27.1, [8000, 4096] 72.6 / - / 82.6. And with
+// sixty-four columns [1000, 16384] 23.4 / 24.1 / 23.5, [1000, 24000] 36.6 / - / 37.9, [1000, 32768] 44.6 / - / 56.4.
 // kCols is small so that a few thousand columns spread over all
 // compute units, several workgroups to each when there are more. The pad of four floats puts the sixteen columns'
 // 16-byte reads into different banks, and the movers' scalar writes likewise.
@@ -58,10 +64,16 @@ constexpr int kDrChunk = 64;  // steps
 constexpr int kDrAhead = 3;   // chunks on their way from memory at any time
 constexpr int kDrBuffers = 3;
 constexpr int kDrPitch = kDrChunk + 4;
+constexpr int64_t kDrThrough = 8 << 20;  // results up to which they are stored through the L2 (sixteen and thirty-two columns)
 
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));      // four floats at any float's address
 typedef uint32_t u32_u __attribute__((aligned(1)));                         // four flags at any address
 #define MRB_GLOBAL __attribute__((address_space(1)))
+
+#ifndef __HIP__  // the CPU, where a test runs these kernels
+template <typename V>
+inline void store_through(void* to, V v) { memcpy(to, &v, sizeof(v)); }
+#endif
 
 template <bool kBack, bool kQuad, int kCols, int kMovers>
 __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
@@ -77,6 +89,7 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
     __shared__ float s_x[kDrBuffers][kCols][kDrPitch];  // a step's value in, its result out
     __shared__ float s_f[kDrBuffers][kCols][kDrPitch];  // its factor (1 - done) * gamma
     const int64_t cols = batch * inner;
+    const bool through = kCols < 64 && timesteps * cols <= kDrThrough;
     // Workgroups are dealt to the chip's eight dies in turn, and each die has its own L2. Neighbouring column groups
     // share cache lines (a group's flags of a step are kCols bytes), so they go to the SAME die.
     const uint32_t groups = (uint32_t)((cols + kCols - 1) / kCols), per = groups >> 3, more = groups & 7u, die = blockIdx.x & 7u;
@@ -264,20 +277,32 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
         }
         wave_lds_fence();  // (the next chunk goes over what other lanes have read)
     };
-    auto store = [&](int64_t c, const f32x4 (&v)[kPer], auto whole, int last) {
+    auto store_as = [&](auto how, int64_t c, const f32x4 (&v)[kPer], auto whole, int last) {
+        constexpr bool kThrough = decltype(how)::value;
         char* const bo = reinterpret_cast<char*>(out + base_of(c) * cols);
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             const int k = i * kSteps + step;
             if (kQuad) {
-                if (decltype(whole)::value || k <= last) __builtin_nontemporal_store(v[i], reinterpret_cast<f32x4_u*>(bo + (row_of(k, last) * row_x + off_x)));
+                if (decltype(whole)::value || k <= last) {
+                    char* const to = bo + (row_of(k, last) * row_x + off_x);
+                    if (kThrough) store_through(to, v[i]);
+                    else __builtin_nontemporal_store(v[i], reinterpret_cast<f32x4_u*>(to));
+                }
             } else {
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    if (decltype(whole)::value || k + j <= last)
-                        __builtin_nontemporal_store(v[i][j], reinterpret_cast<float*>(bo + (row_of(k + j, last) * row_x + off_x)));
+                    if (decltype(whole)::value || k + j <= last) {
+                        char* const to = bo + (row_of(k + j, last) * row_x + off_x);
+                        if (kThrough) store_through(to, (float)v[i][j]);
+                        else __builtin_nontemporal_store(v[i][j], reinterpret_cast<float*>(to));
+                    }
             }
         }
+    };
+    auto store = [&](int64_t c, const f32x4 (&v)[kPer], auto whole, int last) {
+        if (through) store_as(std::true_type{}, c, v, whole, last);  // uniform
+        else store_as(std::false_type{}, c, v, whole, last);
     };
     const int end = last_of(nchunks - 1);  // the last chunk's last step
 #pragma unroll

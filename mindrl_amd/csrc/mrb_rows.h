@@ -413,10 +413,7 @@ using g16 = MRB_GLOBAL granule16_u;
 // (k_per_sample_lanes, whose lanes store pieces of many rows at once, is slower so at every size: 7.5 KB 32.2 / 35.8 with 64 MB.)
 template <bool kThrough>
 __device__ __forceinline__ void store_granule(g16* to, granule_t v) {
-    // (An instruction for which there is no builtin with an address to a lane. A vector instruction may write the registers of a store of
-    // more than 8 bytes two wait states behind it: the compiler sees to that for its own stores, the s_nop here. With one, values of the
-    // next addresses were stored.)
-    if (kThrough) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(to), "v"(v) : "memory");
+    if (kThrough) store_through((void*)to, v);
     else *to = v;
 }
 constexpr uint64_t kThroughBytes = 20ull << 20;

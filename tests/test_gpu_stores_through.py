@@ -100,3 +100,27 @@ def test_replayed():
         seen.append(out[0].clone())
     assert not torch.equal(seen[0], seen[1])
     b.destroy()
+
+
+@pytest.mark.parametrize("shape", [(192, 8192, 1), (1024, 8192, 1), (1025, 8192, 1), (2049, 4095, 1), (2047, 1365, 3), (1025, 2730, 3), (7, 3, 1)])
+def test_returns(shape):
+    """Returns and their gradient on both sides of the size up to which they are stored so, bit for bit: the recurrence, an operation
+    at a time."""
+    from mindrl_amd.utils import DiscountedReturn
+    rng = np.random.default_rng(shape[0])
+    x, w = [rng.normal(size=shape).astype(np.float32) for _ in range(2)]
+    done, value = rng.random(shape[:2]) < 0.03, rng.normal(size=shape[1:]).astype(np.float32)
+    c = ((np.float32(1) - done.astype(np.float32)) * np.float32(0.97))[..., None]
+    want, last = np.empty_like(x), value
+    for t in reversed(range(shape[0])):
+        want[t] = last = x[t] + c[t] * last
+    grad, last = np.empty_like(x), np.zeros_like(value)
+    for t in range(shape[0]):
+        grad[t] = last = w[t] + (c[t - 1] * last if t else 0)
+    X, V = [torch.from_numpy(a).cuda().requires_grad_(True) for a in (x, value)]
+    for _ in range(2):
+        out = DiscountedReturn(0.97, need_bprop=True)(X, torch.from_numpy(done).cuda(), V)
+        gx, gv = torch.autograd.grad(out, (X, V), torch.from_numpy(w).cuda())
+        assert np.array_equal(out.detach().cpu().numpy(), want)
+        assert np.array_equal(gx.cpu().numpy(), grad)
+        assert np.array_equal(gv.cpu().numpy(), c[-1] * grad[-1])

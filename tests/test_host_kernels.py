@@ -32,7 +32,7 @@ def test_kernels_use_no_scratch_memory(source, count, tmp_path):
         assert 0 <= lds - (8 * leaves + 12 * (leaves // 256)) <= 1088, (name, lds)
 
 
-@pytest.mark.parametrize("source", ["mrb.hip", "mrb_short.hip"])
+@pytest.mark.parametrize("source", ["mrb.hip", "mrb_short.hip", "mrb_returns.hip"])
 def test_stores_written_in_assembly_keep_their_registers(source, tmp_path):
     """A 16-byte store's registers may be written two wait states behind it, which the compiler does not look after in inline assembly."""
     from mindrl_amd import build
