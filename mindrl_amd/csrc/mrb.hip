@@ -24,6 +24,7 @@
 #include "mrb_returns.h"
 #include "mrb_samples.h"
 #include "mrb_short.h"
+#include "mrb_silent.h"
 #include "../../include/mrb_more.h"
 
 namespace {
@@ -1853,6 +1854,7 @@ static int per_sample_impl(Per* b, int64_t nbatch, int64_t batch, float beta, co
     } else if (path == 2) {
         int levels = b->lds_levels > 0 ? (int)b->lds_levels : 9;
         if (levels > b->depth) levels = b->depth;
+        if (has_silent(b->depth)) levels = std::min(levels, b->depth - kSilentLevels - 1);
         const hipError_t e = launch_per_sample_lds(a, t, nbatch, lds_strata(nbatch * batch, rest), levels, (uint32_t)rest, s);
         if (e != hipSuccess) return fail(MRB_EHIP, "launch k_per_sample_lds: %s", hipGetErrorString(e));
     }
@@ -1971,6 +1973,16 @@ int mrb_per_export_tree(int64_t h, float* sum_heap, float* min_heap, int64_t* le
     hipStream_t s = static_cast<hipStream_t>(stream);
     const size_t bytes = 2 * (size_t)b->leaves * sizeof(float);
     HIP_TRY(hipStreamSynchronize(s));
+    if (has_silent(b->depth) && (sum_heap || min_heap)) {
+        // (whatever device is current, as for the copies; what the caller has queued is done)
+        int device = 0;
+        HIP_TRY(hipGetDevice(&device));
+        if (device != b->device) HIP_TRY(hipSetDevice(b->device));
+        hipError_t e = launch_tree_silent(b->sum, b->mn, b->leaves, nullptr);
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+        if (device != b->device) (void)hipSetDevice(device);
+        if (e != hipSuccess) return fail(MRB_EHIP, "launch k_tree_silent: %s", hipGetErrorString(e));
+    }
     if (sum_heap) HIP_TRY(hipMemcpy(sum_heap, b->sum, bytes, hipMemcpyDeviceToHost));
     if (min_heap) HIP_TRY(hipMemcpy(min_heap, b->mn, bytes, hipMemcpyDeviceToHost));
     if (leaves) *leaves = b->leaves;

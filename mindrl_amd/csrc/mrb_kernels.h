@@ -845,7 +845,7 @@ __device__ __forceinline__ void tile_round(const UpdateArgs& a, int lo, int g, u
         const float q = wave_max(largest);
         if (lane == 0 && q > 0.0f) raise_max(a.maxp_next, q);
     }
-    tile_parents(a, g, first, lane, active, vs, vm, root_s, root_m);
+    tile_parents(a, g, first, lane, active, vs, vm, root_s, root_m, leaf_level && has_silent(a.depth));
     if (rebuilt) *rebuilt = __any(active);
 }
 
@@ -990,7 +990,7 @@ __device__ __forceinline__ void entry_finish(const UpdateArgs& a, int g, uint32_
     }
     const uint32_t off = tile * kBlockNodes + 4 * lane;  // this lane's first leaf
     if (active && dirty_out && (off & ((1u << g) - 1)) == 0) dirty_out[(off >> g) >> g_next] = a.epoch;
-    tile_parents(a, g, first, lane, active, vs, vm);
+    tile_parents(a, g, first, lane, active, vs, vm, nullptr, nullptr, has_silent(a.depth));
 }
 
 // One wave per entry. The loads are kept apart from what they do not depend on: the entry, the first entries
@@ -1363,11 +1363,17 @@ __device__ __forceinline__ void tree_paths_body(const UpdateArgs& a) {
     uint32_t v = (uint32_t)a.leaves + leaf;  // heap index of the node this lane carries
     // siblings along the path, as memory holds them (level L's in [L - 1])
     float sib_s[kPathMaxDepth], sib_m[kPathMaxDepth];
+    SilentNode under[kSilentLevels]{};  // of the siblings 1, 2, 3 levels above the leaves, where those are silent
+    const bool silent = has_silent(a.depth);
+    if (silent && act) {
+#pragma unroll
+        for (int up = 1; up <= kSilentLevels; ++up) under[up - 1].request(a.sum, a.mn, (v >> up) ^ 1u, up);
+    }
 #pragma unroll
     for (int L = kPathMaxDepth; L >= 1; --L) {
         sib_s[L - 1] = 0.0f;
         sib_m[L - 1] = 0.0f;
-        if (L <= a.depth && act) {
+        if (L <= a.depth && act && !(silent && L < a.depth && L >= a.depth - kSilentLevels)) {
             const uint32_t node = (v >> (a.depth - L)) ^ 1u;
             sib_s[L - 1] = a.sum[node];
             sib_m[L - 1] = a.mn[node];
@@ -1378,6 +1384,9 @@ __device__ __forceinline__ void tree_paths_body(const UpdateArgs& a) {
     const float q = mine ? powf_det(p_here, a.alpha) : 0.0f;
     const float qmax = wave_max(q);
     if (lane == 0 && qmax > 0.0f) raise_max(a.maxp, qmax);
+    float under_s[kSilentLevels], under_m[kSilentLevels];
+#pragma unroll
+    for (int up = 1; up <= kSilentLevels; ++up) under[up - 1].take((v >> up) ^ 1u, up, under_s[up - 1], under_m[up - 1]);
     float cs = q, cm = q;
     if (act) {
         a.sum[v] = cs;
@@ -1394,7 +1403,15 @@ __device__ __forceinline__ void tree_paths_body(const UpdateArgs& a) {
             const uint32_t nv = (uint32_t)__shfl((int)v, src);
             const float ns = __shfl(cs, src), nm = __shfl(cm, src);
             const bool met = act && nb >= 0 && nv == (v ^ 1u);  // the other child is another entry's node
-            const float os = met ? ns : sib_s[L - 1], om = met ? nm : sib_m[L - 1];
+            float was_s = sib_s[L - 1], was_m = sib_m[L - 1];
+            if (silent) {  // uniform, as what follows
+#pragma unroll
+                for (int up = 1; up <= kSilentLevels; ++up) {
+                    was_s = L == a.depth - up ? under_s[up - 1] : was_s;
+                    was_m = L == a.depth - up ? under_m[up - 1] : was_m;
+                }
+            }
+            const float os = met ? ns : was_s, om = met ? nm : was_m;
             cs = left ? cs + os : os + cs;
             cm = left ? fminf(cm, om) : fminf(om, cm);
             v >>= 1;
@@ -1501,6 +1518,7 @@ constexpr int kWgTopNodes = 2 << kWgTopLevels;    // 4096 (node 0 does not exist
 constexpr int kWgSlotsLog2 = 11;
 constexpr int kWgSlots = 1 << kWgSlotsLog2;       // slots per hash table: twice the most entries
 constexpr int kWgMaxDepth = 14;                  // deepest tree the kernel is compiled for
+static_assert(kWgMaxDepth < kSilentDepth, "it reads every level");
 constexpr int kWgBestEntries = 384;              // most entries it is taken for (one launch by runs of leaves beats it long before: takes_wg_rather)
 constexpr int kWgHashSteps = (kWgMaxDepth - kWgTopLevels + 1) / 2;  // most two-level steps below the staged top
 constexpr int kWgTopSteps = (kWgTopLevels + 1) / 2;
@@ -1981,8 +1999,8 @@ __global__ __launch_bounds__(kWgMaxEntries) void k_tree_wg_push(MRB_WG_LEAD_PARA
             slot = ((int64_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) |
                    (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
         }
-        push_one_walk<true>(a.sum, a.mn, a.maxp, slot, a.capacity, a.leaves, a.depth, a.alpha, priority, a.err, threadIdx.x,
-                            none, false, false, 0);
+        push_one_levels<true, false>(a.sum, a.mn, a.maxp, slot, a.capacity, a.leaves, a.depth, a.alpha, priority, a.err, threadIdx.x,
+                                     none, false, false, 0);  // (these trees have no silent levels)
     } else if (keeper) {
         counters_settle(t, a.err, a.advance, a.capacity, a.readers, threadIdx.x & 63u);
     }

@@ -164,7 +164,7 @@ __device__ __forceinline__ void push_run_body(const UpdateArgs& a, uint32_t unit
             *reinterpret_cast<float4*>(a.mn + leaf_first + 4 * lane) = lm;
         }
         if (a.fold_max) largest = wave_max(largest);
-        tile_parents(a, kRoundLevels, leaf_first, lane, true, ls, lm, &rs, &rm);
+        tile_parents(a, kRoundLevels, leaf_first, lane, true, ls, lm, &rs, &rm, has_silent(a.depth));
     }
     if (lane == 0) s_largest[wave] = largest;
 #pragma unroll
@@ -231,19 +231,23 @@ constexpr int kPushOneMaxDepth = 30;
 // `taken`: this launch moves the device's counters on, `ticket` holds them as the caller took them - the position is theirs,
 // and, unless the caller has reported already (`report`), the wave's report (see counters_report) goes out behind the
 // walk's own requests, so that nothing the walk waits for queues up behind the atomic.
-template <bool kAfterUpdate>
-__device__ __forceinline__ void push_one_walk(float* sum, float* mn, float* maxp, int64_t first_slot,
-                                              int64_t capacity, int64_t leaves, int depth, float alpha,
-                                              const float* priority, uint32_t* err, uint32_t lane,
-                                              CounterTicket& ticket, bool taken, bool report, uint32_t readers) {
+// kSilent (has_silent(depth)): lanes 32 to 47 bring the sixteen leaves around the row's instead of the siblings on the levels above the
+// leaves, and four butterflies go from the leaf to the node four levels up, which need not write what lies between.
+template <bool kAfterUpdate, bool kSilent>
+__device__ __forceinline__ void push_one_levels(float* sum, float* mn, float* maxp, int64_t first_slot, int64_t capacity, int64_t leaves,
+                                                int depth, float alpha, const float* priority, uint32_t* err, uint32_t lane,
+                                                CounterTicket& ticket, bool taken, bool report, uint32_t readers) {
     // negative: the ring position is on the device (see Counters)
     const int64_t slot = taken             ? ticket_position(ticket, capacity)
                          : first_slot >= 0 ? first_slot
                                            : ring_position(counters_behind(err), capacity);
     const uint32_t v = (uint32_t)leaves + (uint32_t)slot;
+    constexpr int kStart = kSilent ? kSilentLevels + 1 : 0;  // levels above the leaves that the walk starts from
+    const int top = depth - kStart;
     float sib_s = 0.0f, sib_m = 0.0f;
-    if (lane >= 1 && lane <= (uint32_t)depth) {
-        const uint32_t node = (v >> ((uint32_t)depth - lane)) ^ 1u;
+    const bool leaf_lane = kSilent && lane >> 4 == 2u;
+    if ((lane >= 1 && lane <= (uint32_t)top) || leaf_lane) {
+        const uint32_t node = leaf_lane ? (v & ~15u) + (lane & 15u) : (v >> (((uint32_t)depth - lane) & 31u)) ^ 1u;
         sib_s = sum[node];
         sib_m = mn[node];
     }
@@ -263,9 +267,29 @@ __device__ __forceinline__ void push_one_walk(float* sum, float* mn, float* maxp
         sum[node] = cs;
         mn[node] = cm;
     }
+    if (kSilent) {
+        static_assert(!kSilent || kStart == 4, "sixteen leaves");
+        const bool own = lane == 32u + (v & 15u);
+        float s = own ? q : sib_s, m = own ? q : sib_m;
+        s = s + butterfly_peer<0>(s);
+        m = fminf(m, butterfly_peer<0>(m));
+        s = s + butterfly_peer<1>(s);
+        m = fminf(m, butterfly_peer<1>(m));
+        s = s + butterfly_peer<2>(s);
+        m = fminf(m, butterfly_peer<2>(m));
+        s = s + butterfly_peer<3>(s);
+        m = fminf(m, butterfly_peer<3>(m));
+        cs = lane_value(s, 32);
+        cm = lane_value(m, 32);
+        node = v >> kStart;
+        if (lane == 0) {
+            sum[node] = cs;
+            mn[node] = cm;
+        }
+    }
 #pragma unroll
-    for (int L = kPushOneMaxDepth; L >= 1; --L) {
-        if (L <= depth) {  // wave-uniform
+    for (int L = kPushOneMaxDepth - kStart; L >= 1; --L) {
+        if (L <= top) {  // wave-uniform
             const float os = lane_value(sib_s, L), om = lane_value(sib_m, L);
             const bool right = (node & 1u) != 0;
             cs = right ? os + cs : cs + os;
@@ -279,6 +303,15 @@ __device__ __forceinline__ void push_one_walk(float* sum, float* mn, float* maxp
     }
     // last: the leaf has read the running max as the call found it
     if (given && lane == 0 && q > 0.0f) raise_max(maxp, q);
+}
+template <bool kAfterUpdate>
+__device__ __forceinline__ void push_one_walk(float* sum, float* mn, float* maxp, int64_t first_slot, int64_t capacity, int64_t leaves,
+                                              int depth, float alpha, const float* priority, uint32_t* err, uint32_t lane,
+                                              CounterTicket& ticket, bool taken, bool report, uint32_t readers) {
+    if (has_silent(depth))  // uniform
+        push_one_levels<kAfterUpdate, true>(sum, mn, maxp, first_slot, capacity, leaves, depth, alpha, priority, err, lane, ticket, taken, report, readers);
+    else
+        push_one_levels<kAfterUpdate, false>(sum, mn, maxp, first_slot, capacity, leaves, depth, alpha, priority, err, lane, ticket, taken, report, readers);
 }
 
 }  // namespace mrb

@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kWG) void k_push_many(float* sum, float* mn, float*
             *reinterpret_cast<float4*>(sum + leaf_first + 4 * lane) = ls;
             *reinterpret_cast<float4*>(mn + leaf_first + 4 * lane) = lm;
         }
-        tile_parents(trees, kRoundLevels, leaf_first, lane, true, ls, lm, &rs, &rm);
+        tile_parents(trees, kRoundLevels, leaf_first, lane, true, ls, lm, &rs, &rm, has_silent(depth));
         if (lane == 0 && !kAlone) {
             const unsigned long long number = (unsigned long long)tag << 32;
             __hip_atomic_store(&m->root[unit][0], number | __float_as_uint(rs), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -149,7 +149,7 @@ __global__ __launch_bounds__(1024) void k_tree_range(const int64_t* __restrict__
             *reinterpret_cast<float4*>(mn + first + 4 * lane) = lm;
         }
         float rs, rm;
-        tile_parents(trees, kRoundLevels, first, lane, true, ls, lm, &rs, &rm);
+        tile_parents(trees, kRoundLevels, first, lane, true, ls, lm, &rs, &rm, has_silent(depth));
         if (lane == 0) {
             s_rs[t] = rs;
             s_rm[t] = rm;
@@ -176,12 +176,13 @@ __global__ __launch_bounds__(1024) void k_tree_range(const int64_t* __restrict__
 // of 2^(g0-2) lanes (g0 = 4..6) takes one entry; if that entry owns its block of 2^g0 leaves (it holds the largest of
 // the block's stamps), the group replaces the leaves the stamps name, rebuilds the g0 levels above with tile_parents'
 // operations and marks the tile of the next round.
-// What bounds it: trips to memory that nothing is cached for, and some ten lines per entry written in part. The block's
+// What bounds it: trips to memory that nothing is cached for, and four lines per entry written in part (ten with the silent levels, and
+// that bound it: see kSilentLevels). The block's
 // stamps, its nodes and the entry's own power are therefore requested together, as soon as the index is there, whether
 // or not the entry turns out to own the block (nearly every one does), and the arguments are preloaded: two trips where
 // there were five (arguments, index and priority, stamps, nodes, powers). An owner stores all leaves of its block, 64
-// bytes of a line instead of the pieces that changed. 65,536 entries on 2^24 leaves that no cache holds: 19.2 -> 17.7 us,
-// of which the 0.5 million partial lines of the levels between are the rest.
+// bytes of a line instead of the pieces that changed. 65,536 entries on 2^24 leaves that no cache holds, this launch by itself: 19.2 -> 17.7 us,
+// without the silent levels some 5 less.
 // ---------------------------------------------------------------------------
 constexpr int kSparseWG = 256;
 
@@ -191,7 +192,7 @@ __device__ __forceinline__ void sparse_step(const Trees& a, int g0, uint32_t fir
     if (S < g0 - 2) {  // uniform
         cs = cs + butterfly_peer<S>(cs);
         cm = fminf(cm, butterfly_peer<S>(cm));
-        if (active && (sub & ((2u << S) - 1)) == 0) {
+        if (S >= kSilentLevels - 2 && active && (sub & ((2u << S) - 1)) == 0) {
             a.sum[(first >> (3 + S)) + (sub >> (S + 1))] = cs;
             a.mn[(first >> (3 + S)) + (sub >> (S + 1))] = cm;
         }
@@ -250,13 +251,7 @@ __global__ __launch_bounds__(kSparseWG) void k_tree_sparse(const int64_t* __rest
     }
     const float s0 = vs.x + vs.y, s1 = vs.z + vs.w;
     const float m0 = fminf(vm.x, vm.y), m1 = fminf(vm.z, vm.w);
-    float cs = s0 + s1, cm = fminf(m0, m1);
-    if (active) {
-        *reinterpret_cast<float2*>(sum + (first >> 1) + 2 * sub) = make_float2(s0, s1);
-        *reinterpret_cast<float2*>(mn + (first >> 1) + 2 * sub) = make_float2(m0, m1);
-        sum[(first >> 2) + sub] = cs;
-        mn[(first >> 2) + sub] = cm;
-    }
+    float cs = s0 + s1, cm = fminf(m0, m1);  // (the levels up to kSilentLevels are silent: these trees have 21 levels and more)
     sparse_step<0>(trees, g0, first, sub, active, cs, cm);
     sparse_step<1>(trees, g0, first, sub, active, cs, cm);
     sparse_step<2>(trees, g0, first, sub, active, cs, cm);

@@ -226,7 +226,7 @@ __device__ __forceinline__ void range_one(const int64_t* __restrict__ indices, c
             *reinterpret_cast<float4*>(mn + first + 4 * lane) = lm;
         }
         float rs, rm;
-        tile_parents(trees, kRoundLevels, first, lane, true, ls, lm, &rs, &rm);
+        tile_parents(trees, kRoundLevels, first, lane, true, ls, lm, &rs, &rm, has_silent(depth));
         if (lane == 0) {
             s_rs[t] = rs;
             s_rm[t] = rm;

@@ -97,12 +97,12 @@ __global__ __launch_bounds__(kLdsWG) void k_per_sample_lds(const float* __restri
         // Below the staged levels every dependent load brings up to five levels at once: the 32 (16, 8,
         // 4, 2) descendants of `node` five (four, ... one) levels down are 128 (64, ... 8) contiguous,
         // aligned bytes - a whole cache line in the first case; the levels between are rebuilt with
-        // the additions the tree was built with. The remaining levels are taken five at a time, except
-        // that seven are split 4 + 3 (5 + 1 + 1 would be a load more).
+        // the additions the tree was built with. The remaining levels are taken five at a time, and so that the last load brings
+        // four at least (the levels it would start from otherwise may be silent, see kSilentLevels): eight are 4 + 4, seven 3 + 4, six 2 + 4.
         float picked = depth <= lds_levels ? s_top[node] : 0.0f;
         while (d < depth) {  // wave-uniform
             const int rest = depth - d;
-            const int g = rest >= 5 ? (rest == 7 ? 4 : 5) : rest;
+            const int g = rest <= 5 ? rest : rest <= 8 ? rest - 4 : 5;
             node = descend_group(sum, node, g, mass, picked);
             d += g;
         }
