@@ -161,11 +161,14 @@ __device__ __forceinline__ float4 powf_det_x4(float4 x4, float a) {
 __device__ __attribute__((noinline)) float powf_det_call(float x, float a) { return powf_det(x, a); }
 
 // Counter-based generator: one 64-bit mix of (seed, call counter, draw number).
-__device__ __forceinline__ uint64_t rng_u64(uint64_t seed, uint64_t counter, uint64_t k) {
-    uint64_t z = seed + 0x9E3779B97F4A7C15ULL * ((counter << 32) + k + 1ULL);
+__device__ __forceinline__ uint64_t rng_mix(uint64_t z) {
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
     return z ^ (z >> 31);
+}
+constexpr uint64_t kRngStep = 0x9E3779B97F4A7C15ULL;  // from one draw number's word to the next one's, before it is mixed
+__device__ __forceinline__ uint64_t rng_u64(uint64_t seed, uint64_t counter, uint64_t k) {
+    return rng_mix(seed + kRngStep * ((counter << 32) + k + 1ULL));
 }
 // 24 random bits -> float in [0, 1).
 __device__ __forceinline__ float rng_uniform(uint64_t seed, uint64_t counter, uint64_t k) {
@@ -174,6 +177,10 @@ __device__ __forceinline__ float rng_uniform(uint64_t seed, uint64_t counter, ui
 // Integer in [0, bound): high half of the 128-bit product.
 __device__ __forceinline__ int64_t rng_below(uint64_t seed, uint64_t counter, uint64_t k, int64_t bound) {
     return (int64_t)__umul64hi(rng_u64(seed, counter, k), (uint64_t)bound);
+}
+// The integer that rng_below makes of a mixed word z, for a bound of 32 bits: two multiplications instead of four.
+__device__ __forceinline__ uint32_t below_32(uint64_t z, uint32_t bound) {
+    return (uint32_t)(((z >> 32) * bound + ((uint64_t)(uint32_t)z * bound >> 32)) >> 32);
 }
 
 // ---------------------------------------------------------------------------

@@ -75,6 +75,8 @@ __global__ __launch_bounds__(kWG) void k_res_put(IoTable t, const unsigned long 
 // from memory while it draws.
 // What bounds it: the launch, two trips to memory (the arguments, the rows) and a thread's nrows / 512 draws.
 // A call in two launches / in this one, us: 512 rows of 96 bytes 7.3 / 3.9, 4096 7.2 / 5.7, 1024 rows of 28 KB 10.0 / 8.5.
+// A draw is multiplications: a thread's draws a fixed step apart and 32-bit bounds leave 8 of 13 quarter-rate ones (4096 rows 5.6 -> 5.25,
+// 8192 7.05 -> 6.5, 256 3.35 as before).
 constexpr int kResWG = 512;
 constexpr int kResMaxRows = 64;    // most rows of a workgroup
 constexpr int kResAhead = 2;       // granules of a thread that are on their way while it draws
@@ -139,12 +141,21 @@ __global__ __launch_bounds__(kResWG) void k_res_push(int64_t total, int64_t capa
         if (at[q].row >= 0) held[q].load(at[q].from, at[q].vl);
     }
     lds_barrier();
-#pragma unroll 4
-    for (int j = first + 1 + tid; j < nrows; j += kResWG) {
-        const int64_t slot = reservoir_slot(total + j, capacity, seed);
+    auto look = [&](int j, int64_t slot) {
         int i = slot >= 0 ? s_head[bucket_of(slot)] : -1;
         for (; i >= 0; i = s_next[i])
             if (s_slot[i] == slot && first + i < j) s_replaced[i] = 1;
+    };
+    if (total + nrows < 0xffffffffll) {  // (uniform) reservoir_slot for 32 bits, with a thread's draws a fixed step apart
+        uint64_t word = seed + kRngStep * (uint64_t)(total + first + 2 + tid);
+#pragma unroll 4
+        for (int j = first + 1 + tid; j < nrows; j += kResWG, word += kRngStep * kResWG) {
+            const uint32_t row = (uint32_t)(total + j), r = row < capacity ? row : below_32(rng_mix(word), row + 1);
+            look(j, r < capacity ? (int64_t)r : -1);
+        }
+    } else {
+#pragma unroll 4
+        for (int j = first + 1 + tid; j < nrows; j += kResWG) look(j, reservoir_slot(total + j, capacity, seed));
     }
     lds_barrier();
 #pragma unroll
