@@ -1,0 +1,211 @@
+// Samples of thousands of rows: the LDS-top kernels' body (no kernels here).
+#pragma once
+#include <type_traits>
+
+#include "mrb_samples.h"
+
+namespace mrb {
+
+// ---------------------------------------------------------------------------
+// PER sample, many narrow rows: one workgroup per kStrata strata. The top
+// `lds_levels` levels of the sum tree (nodes [1, 2 << lds_levels)) are staged
+// in LDS once per workgroup, so each thread's descent reads HBM/L2 only for
+// the levels below; then the workgroup gathers its rows with coalesced
+// writes. Same outputs, bit for bit, as k_per_sample_wide.
+// What bounds it: a chain of trips (the arguments and the top, the descent's two or three, the rows), and, with few
+// workgroups, the compute units that have none: 256 strata to a workgroup used 64 of them for a batch of 16,384. The
+// rows' granules are numbered over all fields and four to a thread are in flight at once; field by field every field was
+// a trip of its own. 16,384 rows of
+// 153 bytes 17.1 -> 7.9 us, 13,764 of 139 bytes 15.8 -> 8.1, 16,384 of 521 bytes 35 -> 11.1.
+// ---------------------------------------------------------------------------
+// sum .. calls repeat members of `a` as plain leading parameters: those are preloaded into scalar
+// registers, so the staging loads go out when the wave starts instead of a round trip to the
+// kernel-argument segment later.
+// kLarge: fields that bring every thread eight granules and more are copied by themselves, four granules of a thread in flight: what a
+// granule's field is need not be looked up for each, and where it lies is a multiplication instead of a division - these kernels, not the
+// memory, were what bounded large rows. Batches of more than 20 MB are stored through the L2 (store_granule). us, all by the lookup / so:
+//   row       1 x 12,288 rows   1 x 16,384     2 x 12,288     5 x 8192       5 x 16,384     1 x 65,536
+//   1 KB                                                                     36.6 / 30.9    31.7 / 25.8
+//   2.4 KB                                     32.8 / 25.4    47.0 / 42.2    87.3 / 84.9    73.5 / 69.2
+//   3 KB      23.8 / 20.3       28.0 / 24.9    42.2 / 31.8   (61.6 / 66.0   114.4 / 132     96.4 / 106.5)
+//   4 KB      26.4 / 21.3       34.1 / 26.5    49.8 / 42.5    74.5 / 70.7                   115.1 / 106.4
+//   6 KB      38.8 / 27.6       46.2 / 38.4    70.2 / 62.5   102.0 / 100.5
+// (3 KB: rows of no whole granules, which lose in brackets: kLargeOdd. With ordinary loads 2.4 KB 28.6, 45.1, 3 KB 41.6, 65.5, 4 KB 45.4, 71.2.)
+// ---------------------------------------------------------------------------
+constexpr int kLargeTrip = 4;
+constexpr uint64_t kLargeOdd = 96ull << 20;  // bytes of a batch up to which rows of no whole granules are copied so
+inline bool large_field(const IoTable& t, int f, int strata, uint64_t bytes) {
+    return t.vec_log2[f] == 4 && t.units[f] * (uint64_t)strata >= (uint64_t)(2 * kLargeTrip * kWG) && t.units[f] <= 1u << 14 &&
+           (t.row_bytes[f] % 16 == 0 || bytes <= kLargeOdd);
+}
+__device__ __forceinline__ uint8_t* uniform_pointer(uint8_t* p) {
+    const uint64_t v = (uint64_t)p;
+    return (uint8_t*)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)v));
+}
+
+// rest: granules of a row in the other fields. large (kLarge): a bit for each field that is large; bit 31: store through the L2. blockIdx.y:
+// the batch, of several that are drawn at once (each stratified on its own, with the generator's next call counter).
+template <int kStrata, bool kLarge>
+__device__ __forceinline__ void sample_lds(const float* __restrict__ sum, const float* __restrict__ uniforms, const float* __restrict__ mn, int depth,
+                                           int lds_levels, int batch, float beta, uint64_t seed, uint64_t calls, uint32_t rest, uint32_t large,
+                                           const SampleArgs& a, const IoTable& t) {
+    extern __shared__ float s_top[];  // [2 << lds_levels] floats, then kStrata + 1 int64: the slots, the number of stored rows
+    __shared__ float s_max_w;
+    // the field table (see k_res_push); units: of the fields that make up `rest`
+    __shared__ uint8_t *s_io[MRB_MAX_FIELDS], *s_store[MRB_MAX_FIELDS];
+    __shared__ uint32_t s_bytes[MRB_MAX_FIELDS], s_stride[MRB_MAX_FIELDS], s_units[MRB_MAX_FIELDS], s_vl[MRB_MAX_FIELDS];
+    __shared__ uint32_t s_large[kLarge ? MRB_MAX_FIELDS : 1];  // granules of a row of a large field, else 0
+    const uint32_t ntop = 2u << lds_levels;
+    int64_t* s_slot = reinterpret_cast<int64_t*>(s_top + (ntop < 4 ? 4 : ntop));
+    const int64_t row0 = (int64_t)blockIdx.y * batch;  // the batch's first row of the call's
+    const int64_t k0 = (int64_t)blockIdx.x * kStrata;
+    const int64_t k = threadIdx.x < kStrata ? k0 + threadIdx.x : batch;
+    if (threadIdx.x >= kWG) {
+        const int f = (int)threadIdx.x - kWG;
+        if (f < t.nfields) {
+            s_io[f] = t.io[f];
+            s_store[f] = t.store[f];
+            s_bytes[f] = t.row_bytes[f];
+            s_stride[f] = t.stride[f];
+            s_units[f] = (f < kLdsOwn && t.units[f] == 1) || (kLarge && large >> f & 1u) ? 0 : t.units[f];
+            if (kLarge) s_large[f] = large >> f & 1u ? t.units[f] : 0;
+            s_vl[f] = t.vec_log2[f];
+        }
+        // The helper wave: the weights' common denominator (pmin / total * size)^-beta, once per
+        // workgroup, off the strata's path (two loads and a power: as long as staging the top).
+        // (the number of stored rows: the argument, or read from the device when the counters live there)
+        if (threadIdx.x == kWG) s_slot[kStrata] = a.size >= 0 ? a.size : counters_behind(a.err)[kCntSize];
+        __syncthreads();
+        if (threadIdx.x == kWG) s_max_w = powf_det(mn[1] / sum[1] * (float)s_slot[kStrata], -beta);
+        __syncthreads();
+        return;
+    }
+    // the stratum's draw is requested together with the top of the tree
+    float u = 0.0f;
+    if (k < batch && uniforms) u = uniforms[row0 + k];
+    if (ntop >= 4) {
+        for (uint32_t i = threadIdx.x * 4; i < ntop; i += kWG * 4)
+            *reinterpret_cast<float4*>(s_top + i) = *reinterpret_cast<const float4*>(sum + i);
+    } else if (threadIdx.x < ntop) {
+        s_top[threadIdx.x] = sum[threadIdx.x];
+    }
+    __syncthreads();
+    AnyGranule own[kLdsOwn];
+    float weight = 0.0f;
+    if (k < batch) {
+        const float total = s_top[1];
+        if (!uniforms) u = rng_uniform(seed, generator_calls(uniforms, calls, a.size, a.err) + blockIdx.y, (uint64_t)k);
+        float mass = (u + (float)k) * (total / (float)batch);  // each operation rounded once
+        uint32_t node = 1;
+        int d = 0;
+        // through the staged levels three at a time: the eight descendants of `node` three levels down are 32
+        // contiguous, aligned bytes of LDS - one read instead of three dependent ones -, the two levels between
+        // are rebuilt with the additions the tree was built with
+        for (; d + 3 <= lds_levels; d += 3) {
+            const float4 lo = *reinterpret_cast<const float4*>(s_top + ((size_t)node << 3));
+            const float4 hi = *reinterpret_cast<const float4*>(s_top + ((size_t)node << 3) + 4);
+            float unused;
+            node = (node << 3) + walk8(lo, hi, mass, unused);
+        }
+        for (; d < lds_levels; ++d) {
+            const float left = s_top[2 * node];
+            if (mass <= left) {
+                node = 2 * node;
+            } else {
+                mass -= left;
+                node = 2 * node + 1;
+            }
+        }
+        // Below the staged levels every dependent load brings up to five levels at once: the 32 (16, 8,
+        // 4, 2) descendants of `node` five (four, ... one) levels down are 128 (64, ... 8) contiguous,
+        // aligned bytes - a whole cache line in the first case; the levels between are rebuilt with
+        // the additions the tree was built with. The remaining levels are taken five at a time, and so that the last load brings
+        // four at least (the levels it would start from otherwise may be silent, see kSilentLevels): eight are 4 + 4, seven 3 + 4, six 2 + 4.
+        float picked = depth <= lds_levels ? s_top[node] : 0.0f;
+        while (d < depth) {  // wave-uniform
+            const int rest = depth - d;
+            const int g = rest <= 5 ? rest : rest <= 8 ? rest - 4 : 5;
+            node = descend_group(sum, node, g, mass, picked);
+            d += g;
+        }
+        const int64_t idx = (int64_t)node - ((int64_t)1 << depth);
+        const int64_t slot = idx < a.capacity ? idx : a.capacity - 1;
+        // the row's scalar fields are requested now, before the weight's arithmetic and the barrier
+#pragma unroll
+        for (int f = 0; f < kLdsOwn; ++f)
+            if (f < t.nfields && t.units[f] == 1)
+                own[f].load(as_global(t.store[f]) + (uint64_t)slot * t.stride[f], t.vec_log2[f]);
+        a.out_idx[row0 + k] = idx;
+        const int64_t size = s_slot[kStrata];  // left there by the helper wave before the first barrier
+        weight = powf_det(picked / total * (float)size, -beta);
+        sample_flags(a, total, idx, size);
+        s_slot[threadIdx.x] = slot;
+    }
+    __syncthreads();
+    const uint32_t rows = (uint32_t)((batch - k0) < kStrata ? (batch - k0) : kStrata);
+    if (k < batch) {
+        a.out_w[row0 + k] = weight / s_max_w;
+#pragma unroll
+        for (int f = 0; f < kLdsOwn; ++f)
+            if (f < t.nfields && t.units[f] == 1)
+                own[f].store(as_global(t.io[f]) + (uint64_t)(row0 + k) * t.row_bytes[f], t.vec_log2[f]);
+    }
+    // the other granules, coalesced over the workgroup's rows: of large fields field by field,
+    for (int f = 0; kLarge && f < t.nfields; ++f) {
+        const uint32_t units = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_large[f]);
+        if (units == 0) continue;
+        const uint32_t bytes = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_bytes[f]), stride = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_stride[f]);
+        const gbyte* const store = as_global((const uint8_t*)uniform_pointer(s_store[f]));
+        gbyte* const io = as_global(uniform_pointer(s_io[f])) + (uint64_t)(row0 + k0) * bytes;
+        const uint32_t work = rows * units;
+        const float inverse = 1.0f / (float)units;
+        for (uint32_t base = threadIdx.x; base < work; base += kLargeTrip * kWG) {
+            granule_t held[kLargeTrip];
+            gbyte* to[kLargeTrip];
+#pragma unroll
+            for (int q = 0; q < kLargeTrip; ++q) {
+                const uint32_t w = base + q * kWG < work ? base + q * kWG : base;  // (past the end: the thread's first again)
+                uint32_t r = (uint32_t)((float)w * inverse), unit = w - r * units;  // (within one of the quotient: w is below 2^23)
+                if ((int)unit < 0) r -= 1, unit += units;
+                if (unit >= units) r += 1, unit -= units;
+                const uint32_t off = granule_offset(unit, 4, bytes);
+                held[q] = __builtin_nontemporal_load((const g16*)(store + (uint64_t)s_slot[r] * stride + off));
+                to[q] = io + (r * bytes + off);
+            }
+#pragma unroll
+            for (int q = 0; q < kLargeTrip; ++q) asm volatile("" : "+v"(held[q]));
+            auto store_all = [&](auto through) {
+#pragma unroll
+                for (int q = 0; q < kLargeTrip; ++q)
+                    if (base + q * kWG < work) store_granule<decltype(through)::value>((g16*)to[q], held[q]);
+            };
+            if (large >> 31) store_all(std::true_type{});  // uniform
+            else store_all(std::false_type{});
+        }
+    }
+    // of the others field by field and row by row
+    const uint32_t work = rows * rest;
+    for (uint32_t base = threadIdx.x; base < work; base += kLargeTrip * kWG) {
+        gbyte* to[kLargeTrip];
+        uint32_t vl[kLargeTrip];
+        AnyGranule held[kLargeTrip];
+#pragma unroll
+        for (int q = 0; q < kLargeTrip; ++q) {
+            uint32_t w = base + (uint32_t)q * kWG;
+            to[q] = nullptr;
+            if (w >= work) continue;
+            int f = 0;
+            while (w >= rows * s_units[f]) w -= rows * s_units[f++];  // (ends at a field of `rest`: w is below their total)
+            const uint32_t units = s_units[f], r = w / units;
+            vl[q] = s_vl[f];
+            const uint32_t off = granule_offset(w - r * units, vl[q], s_bytes[f]);
+            held[q].load(as_global(s_store[f]) + (uint64_t)s_slot[r] * s_stride[f] + off, vl[q]);
+            to[q] = as_global(s_io[f]) + (uint64_t)(row0 + k0 + r) * s_bytes[f] + off;
+        }
+#pragma unroll
+        for (int q = 0; q < kLargeTrip; ++q)
+            if (to[q]) held[q].store(to[q], vl[q]);
+    }
+}
+
+}  // namespace mrb

@@ -9,6 +9,10 @@ namespace mrb {
 hipError_t launch_per_sample_lds(const SampleArgs& a, const IoTable& t, int64_t nbatch, int strata, int levels, uint32_t rest,
                                  hipStream_t s);
 
+// The same where some fields are large (a bit for each, and bit 31 to store through the L2; rest: of the others). launch_per_sample_lds calls it.
+hipError_t launch_per_sample_lds_large(const SampleArgs& a, const IoTable& t, int64_t nbatch, int strata, int levels, uint32_t rest, uint32_t large,
+                                       size_t lds, hipStream_t s);
+
 // The same by sixteen lanes for each stratum: trees of at least kLanesFewestLevels levels, rows of at most kLanesMostNarrow bytes in
 // narrow fields.
 constexpr int kLanesFewestLevels = 7;
