@@ -70,11 +70,6 @@ typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));      // f
 typedef uint32_t u32_u __attribute__((aligned(1)));                         // four flags at any address
 #define MRB_GLOBAL __attribute__((address_space(1)))
 
-#ifndef __HIP__  // the CPU, where a test runs these kernels
-template <typename V>
-inline void store_through(void* to, V v) { memcpy(to, &v, sizeof(v)); }
-#endif
-
 template <bool kBack, bool kQuad, int kCols, int kMovers>
 __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
     const float* __restrict__ x, const uint8_t* __restrict__ done, float* __restrict__ end_value, float* __restrict__ out,

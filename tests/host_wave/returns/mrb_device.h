@@ -106,5 +106,7 @@ namespace mrb {
 
 inline void lds_barrier() { sim::wait(2); }
 inline void wave_lds_fence() { sim::wait(1); }
+template <typename V>
+inline void store_through(void* to, V v) { memcpy(to, &v, sizeof(v)); }
 
 }  // namespace mrb
