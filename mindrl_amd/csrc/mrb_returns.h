@@ -48,6 +48,10 @@ namespace mrb {
 // [200, 8000] 6.0 / 6.3 / 5.6, [1000, 4096] 11.9 / 13.1 / 11.6, [2000, 3001] 21.0 / 21.7 / 20.3, [1000, 2500, 3] 15.0 / - / 13.9, [1000, 8192] 15.9 / - / 15.7;
 // [4000, 4096] 37.7 / - / 37.4, [2000, 7501] 28.3 / - / 28.5, [3000, 1365, 3] 29.2 / - / 31.8, [2000, 2700, 3] 25.8 / - / 27.1, [8000, 4096] 72.6 / - / 82.6. And with
 // sixty-four columns [1000, 16384] 23.4 / 24.1 / 23.5, [1000, 24000] 36.6 / - / 37.9, [1000, 32768] 44.6 / - / 56.4.
+// A single group shares no line, and who reads its results next finds them in the L2 they went through only where they may stay: as
+// non-temporal ones. us, non-temporal / through, alone and with the maximum over the steps behind it: [20, 1] 3.14 / 3.33, 5.9 / 6.3,
+// [64, 8] 3.01 / 3.04, 10.7 / 13.3, [128, 8] 3.51 / 3.56, 15.5 / 22.0, [1000, 16] 11.2 / 11.1, 17.6 / 18.8; of several groups [20, 17] 3.14 / 2.92, 7.3 / 6.8,
+// [128, 17] 3.94 / 3.55, 20.3 / 15.4, [128, 128] 3.63 / 3.66, 12.5 / 11.1, [1000, 100] 11.9 / 11.5, 36.1 / 29.5.
 // kCols is small so that a few thousand columns spread over all
 // compute units, several workgroups to each when there are more. The pad of four floats puts the sixteen columns'
 // 16-byte reads into different banks, and the movers' scalar writes likewise.
@@ -64,7 +68,7 @@ constexpr int kDrChunk = 64;  // steps
 constexpr int kDrAhead = 3;   // chunks on their way from memory at any time
 constexpr int kDrBuffers = 3;
 constexpr int kDrPitch = kDrChunk + 4;
-constexpr int64_t kDrThrough = 8 << 20;  // results up to which they are stored through the L2 (sixteen and thirty-two columns)
+constexpr int64_t kDrThrough = 8 << 20;  // results of several groups up to which they are stored through the L2 (sixteen and thirty-two columns)
 
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));      // four floats at any float's address
 typedef uint32_t u32_u __attribute__((aligned(1)));                         // four flags at any address
@@ -84,7 +88,7 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
     __shared__ float s_x[kDrBuffers][kCols][kDrPitch];  // a step's value in, its result out
     __shared__ float s_f[kDrBuffers][kCols][kDrPitch];  // its factor (1 - done) * gamma
     const int64_t cols = batch * inner;
-    const bool through = kCols < 64 && timesteps * cols <= kDrThrough;
+    const bool through = kCols < 64 && timesteps * cols <= (cols > kCols ? kDrThrough : 0);
     // Workgroups are dealt to the chip's eight dies in turn, and each die has its own L2. Neighbouring column groups
     // share cache lines (a group's flags of a step are kCols bytes), so they go to the SAME die.
     const uint32_t groups = (uint32_t)((cols + kCols - 1) / kCols), per = groups >> 3, more = groups & 7u, die = blockIdx.x & 7u;

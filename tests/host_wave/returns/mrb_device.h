@@ -106,7 +106,11 @@ namespace mrb {
 
 inline void lds_barrier() { sim::wait(2); }
 inline void wave_lds_fence() { sim::wait(1); }
+inline int64_t g_through = 0;  // results that were stored so
 template <typename V>
-inline void store_through(void* to, V v) { memcpy(to, &v, sizeof(v)); }
+inline void store_through(void* to, V v) {
+    memcpy(to, &v, sizeof(v));
+    g_through += sizeof(v) / 4;
+}
 
 }  // namespace mrb
