@@ -300,7 +300,6 @@ int wide_plan(const RowStore& r, const IoTable& t, int64_t n, WidePlan& plan, di
         plan.f[q].first = items;
         items += wide ? r.units[i] : t.row_bytes[i];
     }
-    plan.through = stores_through(batch_bytes(t));
     const uint32_t per_wg = (uint32_t)kMaxInFlight * kCopyThreads;
     uint32_t split = (plan.wide_items + per_wg - 1) / per_wg;
     if (r.row_split > (int64_t)split) split = (uint32_t)r.row_split;
@@ -380,6 +379,7 @@ int sample_wide(const RowStore& r, const SampleArgs& a, const IoTable& t, int64_
     plan.nbatch = (uint32_t)nbatch;
     const int inflight = wide_plan(r, t, nbatch * a.batch, plan, grid);
     if (inflight == 0) return MRB_EINVAL;
+    plan.through = stores_through(batch_bytes(t), kThroughSample);
     if (next) {
         // the second layer of workgroups: one wide field, split like a row of its own
         NextPlan nx{};
@@ -396,8 +396,9 @@ int sample_wide(const RowStore& r, const SampleArgs& a, const IoTable& t, int64_
         const uint32_t per_wg = (uint32_t)kMaxInFlight * kCopyThreads;
         const uint32_t split = (nx.plan.wide_items + per_wg - 1) / per_wg;
         nx.plan.split = (int)split;
-        plan.through = nx.plan.through = stores_through(batch_bytes(t) + (uint64_t)a.batch * r.bytes[f]);
         nx.plan.share = (nx.plan.wide_items + split - 1) / split;
+        plan.through = nx.plan.through =
+            stores_through(batch_bytes(t) + (uint64_t)a.batch * r.bytes[f], kThroughSample);
         if (split > 65535u) return fail(MRB_EINVAL, "field %d is too wide for one launch", f);
         if (split > grid.y) grid.y = split;
         grid.z = 2;
@@ -501,6 +502,7 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
         dim3 grid;
         plan.nbatch = 1;
         const int inflight = wide_plan(r, t, n, plan, grid);
+        plan.through = stores_through(batch_bytes(t), kThroughGather);
         // Thousands of rows of up to 4 KB: a wave per row (3 KB, us, workgroup / wave: 1024 rows 6.2 / 6.7, 2048 7.5 / 6.8,
         // 8192 20.7 / 13.6; 1 KB: 2048 5.2 / 5.5, 4096 7.4 / 5.9).
         if (r.row_split == 0 && plan.split == 1 && plan.wide_items <= (uint32_t)kRowWaveInF * 64u && plan.narrow_items <= 256u &&

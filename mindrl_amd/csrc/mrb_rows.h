@@ -401,28 +401,41 @@ using g16 = MRB_GLOBAL granule16_u;
 
 // A granule of a batch, or (kThrough) of a large one: stored through the die's L2 into memory at once. What lies changed in the eight
 // dies' caches (4 MB each) when a kernel ends is written out then, with nothing else going on; a large batch's stores had better be on
-// their way while rows are still being read. The memory's own cache keeps them either way, and a read of the batch right behind is not
-// slower (220 MB: sampled and read 128 us as before, 124 so), as it is behind non-temporal stores (149).
-// Smaller batches are faster left in the L2. us, L2 / through, by MB of the batch:
+// their way while rows are still being read. The memory's own cache keeps them either way, as it does not behind non-temporal stores
+// (220 MB sampled and read 128 us, 124 so, 149 with those). us, L2 / through, by MB of the batch:
 //                                       14            16            20             24             32             48             64             220
 //   sample, 28 KB rows               9.3 /  9.2    9.7 / 10.0    10.8 / 10.4    12.5 / 11.8    15.0 / 14.3    21.6 / 19.9    26.9 / 24.5    88.0 / 84.0
 //   uniform gather, 28 KB            9.0 /  8.9    9.0 /  9.5    10.2 / 10.0    11.6 / 11.2    14.3 / 13.5    19.8 / 18.1    25.2 / 23.1
 //   uniform gather, 7.5 KB           8.7 /  8.7    9.4 /  9.3    10.7 / 10.8    12.3 / 12.2    15.3 / 14.5    21.1 / 19.6    26.4 / 25.0
 //   uniform gather, 4 KB             7.9 /  8.2    8.5 /  8.6    10.2 / 10.1    11.6 / 11.4    13.8 / 13.2    19.3 / 18.0    24.7 / 22.8
 //   uniform gather, 2.4 KB           8.3 /  8.7    9.3 /  9.4    10.9 / 10.7    12.5 / 12.0    15.5 / 15.5
-// (k_per_sample_lanes, whose lanes store pieces of many rows at once, is slower so at every size: 7.5 KB 32.2 / 35.8 with 64 MB.)
+// But a batch is read next, and what the dies' caches (32 MB together) hold of a gather's is found there, so the line of gathers lies where
+// about as many readers gain as lose. The call and a reader behind it, us, L2 / through (a product with 64 or 256 columns, a copy into bf16):
+//   MB                                                    22              26              34              40              48              64
+//   gather, 2.4 KB, f32 x 64                         32.1 / 36.9     31.6 / 37.6     32.8 / 34.4     46.1 / 45.5     49.9 / 48.6     52.2 / 51.5
+//   gather, 2.4 KB, bf16 x 256                       38.4 / 42.0     39.3 / 42.7     41.1 / 42.4     46.7 / 48.3     49.6 / 50.7     56.6 / 55.1
+//   gather, 4 KB, f32 x 64                           29.5 / 34.0     29.4 / 34.7     36.9 / 38.2     38.0 / 38.9     40.1 / 40.8     45.8 / 45.5
+//   gather, 7.5 KB, f32 x 64                         33.7 / 37.8     33.5 / 39.0     40.0 / 43.9     41.9 / 43.8     44.6 / 45.8     63.0 / 62.4
+//   gather, 1 KB, bf16 x 256                         29.1 / 32.2     30.8 / 33.0     35.3 / 37.6     37.4 / 38.6     44.6 / 45.0     50.7 / 49.8
+//   gather, 28 KB, u8 to bf16                        51.9 / 51.0     59.2 / 58.4     73.5 / 72.6     85.4 / 83.8    100.4 / 98.6    130.3 / 128.0
+//   sample, 28 KB, u8 to bf16                        52.4 / 51.0     59.1 / 57.9     74.1 / 73.1     87.5 / 85.9    102.0 / 100.6   132.2 / 129.7
+//   sample, 28 KB, bf16 x 256                        66.3 / 66.1     67.3 / 67.4     75.0 / 74.9     79.0 / 77.6     82.4 / 81.0     96.6 / 94.6
+//   sample, 1 KB (k_per_sample_lds_large), f32 x 64  35.3 / 34.2     30.0 / 29.5     50.9 / 49.9     52.8 / 51.9     47.4 / 45.7     53.0 / 51.0
+// (A sample with a mere maximum of each row behind it, 24 MB 26.7 / 27.3, 32 MB 28.5 / 28.7, 48 MB 35.3 / 33.9.)
+// Not stored so are single rows, rows of few granules, and those of k_per_sample_rows, of k_per_sample_lds and of k_per_sample_lanes
+// (whose lanes store pieces of many rows at once and are slower so at every size: 7.5 KB 32.2 / 35.8 with 64 MB).
 template <bool kThrough>
 __device__ __forceinline__ void store_granule(g16* to, granule_t v) {
     if (kThrough) store_through((void*)to, v);
     else *to = v;
 }
-constexpr uint64_t kThroughBytes = 20ull << 20;
+constexpr uint64_t kThroughSample = 20ull << 20, kThroughGather = 40ull << 20;  // bytes of a batch from which on it is stored so
 inline uint64_t batch_bytes(const IoTable& t) {
     uint64_t bytes = 0;
     for (int f = 0; f < t.nfields; ++f) bytes += (t.prefix[f + 1] - t.prefix[f]) << t.vec_log2[f];
     return bytes;
 }
-inline bool stores_through(uint64_t bytes) { return bytes > kThroughBytes; }
+inline bool stores_through(uint64_t bytes, uint64_t from) { return bytes > from; }
 
 constexpr int kNarrowInF = 2;  // narrow bytes a thread of the first copy wave holds beside its wide granules
 

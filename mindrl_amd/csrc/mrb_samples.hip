@@ -28,7 +28,7 @@ hipError_t launch_per_sample_lds(const SampleArgs& a, const IoTable& t, int64_t 
         smaller -= t.units[f];
     }
     const size_t lds = ntop * sizeof(float) + ((size_t)strata + 1) * sizeof(int64_t);
-    if (large) return launch_per_sample_lds_large(a, t, nbatch, strata, levels, smaller, large | (stores_through(bytes) ? 1u << 31 : 0u), lds, s);
+    if (large) return launch_per_sample_lds_large(a, t, nbatch, strata, levels, smaller, large | (stores_through(bytes, kThroughSample) ? 1u << 31 : 0u), lds, s);
     auto* const kernel = strata == 16   ? k_per_sample_lds<16>
                          : strata == 32 ? k_per_sample_lds<32>
                          : strata == 64 ? k_per_sample_lds<64>

@@ -73,7 +73,7 @@ hipError_t launch_short_gather(const RowTable* table, const ShortIo& io, const I
         dim3 grid(0);
         for (int f = 0; f < t.nfields; ++f) grid.x += put_blocks(t.prefix[f + 1] - t.prefix[f], kWG);
         launch_kernel(k_short_gather_many, grid, dim3(kWG), 0, s, table, indices, seed, calls, (uint32_t)count, (uint32_t)n,
-                      (with_indices ? 1 : 0) | (stores_through(batch_bytes(t)) ? 2 : 0), io);
+                      (with_indices ? 1 : 0) | (stores_through(batch_bytes(t), kThroughGather) ? 2 : 0), io);
         return hipGetLastError();
     }
     launch_kernel(k_short_gather, dim3(blocks, (uint32_t)t.nfields), dim3(kWG), 0, s, table, indices, seed, calls, (uint32_t)count, (uint32_t)n,

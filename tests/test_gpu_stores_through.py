@@ -1,4 +1,4 @@
-"""Batches on both sides of the size from which their rows are stored through the caches (store_granule, mrb_rows.h), by each of the
+"""Batches on both sides of the sizes from which their rows are stored through the caches (store_granule, mrb_rows.h), by each of the
 kernels that do so: a workgroup to a row with one and with several large fields, the same with the next observation, a wave to a
 row, and granules numbered over all rows. Rows against the buffer's own at the returned slots, byte for byte, also of calls replayed
 from a graph into tensors that have been cleared."""
@@ -10,7 +10,7 @@ from gpu_util import random_rows, to_dev, torch_types
 
 pytestmark = pytest.mark.gpu
 
-LINE = 20 << 20
+LINE, GATHERS_LINE = 20 << 20, 40 << 20
 ROWS = {  # (the second field: a slot number)
     "frames": ([(84, 84, 4), (1,), (1,)], [np.uint8, np.int64, np.float32]),
     "odd": ([(48, 51, 3), (1,), (307,), (1,), (9,)], [np.uint8, np.int64, np.float32, np.bool_, np.float16]),
@@ -43,8 +43,8 @@ def filled(make, rows, cap, insert):
 def test_uniform(rows):
     from mindrl_amd.core import UniformReplayBuffer
     size = row_bytes(*ROWS[rows])
-    cap = LINE // size * 3 // 2 + 5
-    for n in (LINE // size, LINE // size + 1, cap):
+    cap = GATHERS_LINE // size * 5 // 4 + 5
+    for n in (LINE // size, LINE // size + 1, GATHERS_LINE // size, GATHERS_LINE // size + 1, cap):
         b, new = filled(lambda s, t: UniformReplayBuffer(n, cap, s, t, seed=3), rows, cap, lambda b, new: b.insert(new))
         for _ in range(2):
             slots, out = b.sample_with_indices()
