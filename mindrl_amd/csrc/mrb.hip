@@ -379,7 +379,7 @@ int sample_wide(const RowStore& r, const SampleArgs& a, const IoTable& t, int64_
     plan.nbatch = (uint32_t)nbatch;
     const int inflight = wide_plan(r, t, nbatch * a.batch, plan, grid);
     if (inflight == 0) return MRB_EINVAL;
-    plan.through = stores_through(batch_bytes(t), kThroughSample);
+    plan.through = stores_through(batch_bytes(t), kThroughSample, whole_pieces(plan));
     if (next) {
         // the second layer of workgroups: one wide field, split like a row of its own
         NextPlan nx{};
@@ -398,7 +398,7 @@ int sample_wide(const RowStore& r, const SampleArgs& a, const IoTable& t, int64_
         nx.plan.split = (int)split;
         nx.plan.share = (nx.plan.wide_items + split - 1) / split;
         plan.through = nx.plan.through =
-            stores_through(batch_bytes(t) + (uint64_t)a.batch * r.bytes[f], kThroughSample);
+            stores_through(batch_bytes(t) + (uint64_t)a.batch * r.bytes[f], kThroughSample, whole_pieces(plan) && whole_pieces(nx.plan));
         if (split > 65535u) return fail(MRB_EINVAL, "field %d is too wide for one launch", f);
         if (split > grid.y) grid.y = split;
         grid.z = 2;
@@ -502,7 +502,7 @@ int gather_rows(const RowStore& r, const int64_t* indices, int64_t fixed_slot, i
         dim3 grid;
         plan.nbatch = 1;
         const int inflight = wide_plan(r, t, n, plan, grid);
-        plan.through = stores_through(batch_bytes(t), kThroughGather);
+        plan.through = stores_through(batch_bytes(t), kThroughGather, whole_pieces(plan));
         // Thousands of rows of up to 4 KB: a wave per row (3 KB, us, workgroup / wave: 1024 rows 6.2 / 6.7, 2048 7.5 / 6.8,
         // 8192 20.7 / 13.6; 1 KB: 2048 5.2 / 5.5, 4096 7.4 / 5.9).
         if (r.row_split == 0 && plan.split == 1 && plan.wide_items <= (uint32_t)kRowWaveInF * 64u && plan.narrow_items <= 256u &&

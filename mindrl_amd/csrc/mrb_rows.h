@@ -422,6 +422,19 @@ using g16 = MRB_GLOBAL granule16_u;
 //   sample, 28 KB, bf16 x 256                        66.3 / 66.1     67.3 / 67.4     75.0 / 74.9     79.0 / 77.6     82.4 / 81.0     96.6 / 94.6
 //   sample, 1 KB (k_per_sample_lds_large), f32 x 64  35.3 / 34.2     30.0 / 29.5     50.9 / 49.9     52.8 / 51.9     47.4 / 45.7     53.0 / 51.0
 // (A sample with a mere maximum of each row behind it, 24 MB 26.7 / 27.3, 32 MB 28.5 / 28.7, 48 MB 35.3 / 33.9.)
+// And where a wave's store ends in the middle of 64 bytes, the rest of them comes later, from another wave: what is more than
+// the memory's cache (256 MB, of which the batch's readers and the rows take their part) is then written to memory in pieces. us, L2 / through:
+//                                                   128 MB          180 MB          256 MB           360 MB          460 MB          920 MB
+//   sample, 28,224 bytes                                                                            136 / 129       169 / 161       332 / 313
+//   sample, 28,192                                                                                  142 / 139       171 / 194       334 / 397
+//   sample, 40,000 (two workgroups, 20,000 each)                                                    155 / 152       192 / 205       385 / 415
+//   sample, 28,225, and a copy behind it            93 /  92       144 / 143       224 / 235
+//   gather, 7488 (k_short_gather_many)                                                              136 / 129       174 / 165       350 / 333
+//   gather, 7500                                                                                    153 / 146       187 / 210       385 / 438
+//   gather, 1500, and a copy behind it              85 /  83       136 / 133       217 / 226
+//   gather, 2432 (k_rows_gather_rows)                                                               137 / 128       176 / 165       346 / 323
+//   gather, 2400                                                                                    153 / 145       183 / 194       358 / 395
+// So such batches are stored so up to 160 MB, others without an end (measured up to 1.8 GB: sample, 28,224 bytes 690 / 659).
 // Not stored so are single rows, rows of few granules, and those of k_per_sample_rows, of k_per_sample_lds and of k_per_sample_lanes
 // (whose lanes store pieces of many rows at once and are slower so at every size: 7.5 KB 32.2 / 35.8 with 64 MB).
 template <bool kThrough>
@@ -430,12 +443,21 @@ __device__ __forceinline__ void store_granule(g16* to, granule_t v) {
     else *to = v;
 }
 constexpr uint64_t kThroughSample = 20ull << 20, kThroughGather = 40ull << 20;  // bytes of a batch from which on it is stored so
+constexpr uint64_t kThroughBroken = 160ull << 20;                                // and up to which, where waves' stores end within 64 bytes
 inline uint64_t batch_bytes(const IoTable& t) {
     uint64_t bytes = 0;
     for (int f = 0; f < t.nfields; ++f) bytes += (t.prefix[f + 1] - t.prefix[f]) << t.vec_log2[f];
     return bytes;
 }
-inline bool stores_through(uint64_t bytes, uint64_t from) { return bytes > from; }
+// Whether a wave's stores are whole pieces of 64 bytes: of the rows, or parts of rows, that a plan's workgroups or waves write, or of a field
+// whose granules are numbered over all rows.
+inline bool whole_pieces(const WidePlan& plan) {
+    bool whole = plan.split == 1 || plan.share % 4 == 0;
+    for (int q = 0; q < plan.nwide; ++q) whole = whole && (((uint64_t)plan.f[q].dst | plan.f[q].rb) & 63) == 0;
+    return whole;
+}
+inline bool whole_pieces(const IoTable& t, int f) { return ((uint64_t)t.io[f] & 63) == 0 && t.row_bytes[f] % 16 == 0; }
+inline bool stores_through(uint64_t bytes, uint64_t from, bool whole) { return bytes > from && (whole || bytes <= kThroughBroken); }
 
 constexpr int kNarrowInF = 2;  // narrow bytes a thread of the first copy wave holds beside its wide granules
 

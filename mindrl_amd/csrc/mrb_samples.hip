@@ -22,13 +22,15 @@ hipError_t launch_per_sample_lds(const SampleArgs& a, const IoTable& t, int64_t 
     const uint32_t ntop = (2u << levels) < 4 ? 4 : (2u << levels);
     const uint64_t bytes = batch_bytes(t);
     uint32_t large = 0, smaller = rest;
+    bool whole = true;
     for (int f = 0; f < t.nfields; ++f) {
         if (!large_field(t, f, strata, bytes)) continue;
         large |= 1u << f;
         smaller -= t.units[f];
+        whole = whole && whole_pieces(t, f);
     }
     const size_t lds = ntop * sizeof(float) + ((size_t)strata + 1) * sizeof(int64_t);
-    if (large) return launch_per_sample_lds_large(a, t, nbatch, strata, levels, smaller, large | (stores_through(bytes, kThroughSample) ? 1u << 31 : 0u), lds, s);
+    if (large) return launch_per_sample_lds_large(a, t, nbatch, strata, levels, smaller, large | (stores_through(bytes, kThroughSample, whole) ? 1u << 31 : 0u), lds, s);
     auto* const kernel = strata == 16   ? k_per_sample_lds<16>
                          : strata == 32 ? k_per_sample_lds<32>
                          : strata == 64 ? k_per_sample_lds<64>

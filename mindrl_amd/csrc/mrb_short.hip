@@ -71,9 +71,13 @@ hipError_t launch_short_gather(const RowTable* table, const ShortIo& io, const I
                                uint64_t calls, int64_t n, uint32_t blocks, bool with_indices, hipStream_t s) {
     if (blocks > (indices ? kGatherFew : kGatherFewDrawn)) {
         dim3 grid(0);
-        for (int f = 0; f < t.nfields; ++f) grid.x += put_blocks(t.prefix[f + 1] - t.prefix[f], kWG);
+        bool whole = true;
+        for (int f = 0; f < t.nfields; ++f) {
+            grid.x += put_blocks(t.prefix[f + 1] - t.prefix[f], kWG);
+            if (t.vec_log2[f] == 4) whole = whole && whole_pieces(t, f);
+        }
         launch_kernel(k_short_gather_many, grid, dim3(kWG), 0, s, table, indices, seed, calls, (uint32_t)count, (uint32_t)n,
-                      (with_indices ? 1 : 0) | (stores_through(batch_bytes(t), kThroughGather) ? 2 : 0), io);
+                      (with_indices ? 1 : 0) | (stores_through(batch_bytes(t), kThroughGather, whole) ? 2 : 0), io);
         return hipGetLastError();
     }
     launch_kernel(k_short_gather, dim3(blocks, (uint32_t)t.nfields), dim3(kWG), 0, s, table, indices, seed, calls, (uint32_t)count, (uint32_t)n,

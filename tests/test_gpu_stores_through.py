@@ -1,4 +1,4 @@
-"""Batches on both sides of the sizes from which their rows are stored through the caches (store_granule, mrb_rows.h), by each of the
+"""Batches on both sides of the sizes from which, and up to which, their rows are stored through the caches (store_granule, mrb_rows.h), by each of the
 kernels that do so: a workgroup to a row with one and with several large fields, the same with the next observation, a wave to a
 row, and granules numbered over all rows. Rows against the buffer's own at the returned slots, byte for byte, also of calls replayed
 from a graph into tensors that have been cleared."""
@@ -10,7 +10,7 @@ from gpu_util import random_rows, to_dev, torch_types
 
 pytestmark = pytest.mark.gpu
 
-LINE, GATHERS_LINE = 20 << 20, 40 << 20
+LINE, GATHERS_LINE, BROKEN_LINE = 20 << 20, 40 << 20, 160 << 20  # samples and gathers from the first and the second on; stores that end within 64 bytes up to the last
 ROWS = {  # (the second field: a slot number)
     "frames": ([(84, 84, 4), (1,), (1,)], [np.uint8, np.int64, np.float32]),
     "odd": ([(48, 51, 3), (1,), (307,), (1,), (9,)], [np.uint8, np.int64, np.float32, np.bool_, np.float16]),
@@ -124,3 +124,20 @@ def test_returns(shape):
         assert np.array_equal(out.detach().cpu().numpy(), want)
         assert np.array_equal(gx.cpu().numpy(), grad)
         assert np.array_equal(gv.cpu().numpy(), c[-1] * grad[-1])
+
+
+@pytest.mark.parametrize("rows", ["frames", "odd", "wave", "flat"])
+def test_more_than_the_memorys_cache_takes(rows):
+    from mindrl_amd.core import PriorityReplayBuffer, UniformReplayBuffer
+    cap, size = 700, row_bytes(*ROWS[rows])
+    for n in (BROKEN_LINE // size, BROKEN_LINE // size + 9):
+        b, new = filled(lambda s, t: UniformReplayBuffer(n, cap, s, t, seed=3), rows, cap, lambda b, new: b.insert(new))
+        given = torch.randint(0, cap, (n,), device="cuda")
+        same_rows(b.sample(indices=given), new, given)
+        b.check()
+        b.destroy()
+        b, new = filled(lambda s, t: PriorityReplayBuffer(0.6, cap, n, s, t, seed0=3), rows, cap, lambda b, new: b.insert(*new))
+        out = b.sample(0.4)
+        same_rows(out[2:], new, out[0])
+        b.check()
+        b.destroy()
