@@ -21,22 +21,50 @@ namespace mrb {
 // sum .. calls repeat members of `a` as plain leading parameters: those are preloaded into scalar
 // registers, so the staging loads go out when the wave starts instead of a round trip to the
 // kernel-argument segment later.
-// kLarge: fields that bring every thread eight granules and more are copied by themselves, four granules of a thread in flight: what a
-// granule's field is need not be looked up for each, and where it lies is a multiplication instead of a division - these kernels, not the
-// memory, were what bounded large rows. Batches of more than 20 MB are stored through the L2 (store_granule). us, all by the lookup / so:
-//   row       1 x 12,288 rows   1 x 16,384     2 x 12,288     5 x 8192       5 x 16,384     1 x 65,536
-//   1 KB                                                                     36.6 / 30.9    31.7 / 25.8
+// kLarge: large fields are copied by themselves, four granules of a thread in flight: what a granule's field is need not be looked up for
+// each, and where it lies is a multiplication instead of a division - these kernels, not the memory, were what bounded large rows. Batches
+// of more than 20 MB are stored through the L2 (store_granule). us, all by the lookup / so, from 2 * 10^5 rows:
+//   row       1 x 12,288 rows   1 x 16,384     2 x 12,288     5 x 8192       5 x 16,384     1 x 65,536     1 x 131,072 (256 strata to a workgroup)
+//   128 B                                                                                                  16.2 / 12.8
+//   512 B                                                                                                  45.6 / 28.7
+//   1 KB                                                                     36.6 / 30.9    31.7 / 25.8    78.4 / 47.0
 //   2.4 KB                                     32.8 / 25.4    47.0 / 42.2    87.3 / 84.9    73.5 / 69.2
-//   3 KB      23.8 / 20.3       28.0 / 24.9    42.2 / 31.8   (61.6 / 66.0   114.4 / 132     96.4 / 106.5)
 //   4 KB      26.4 / 21.3       34.1 / 26.5    49.8 / 42.5    74.5 / 70.7                   115.1 / 106.4
 //   6 KB      38.8 / 27.6       46.2 / 38.4    70.2 / 62.5   102.0 / 100.5
-// (3 KB: rows of no whole granules, which lose in brackets: kLargeOdd. With ordinary loads 2.4 KB 28.6, 45.1, 3 KB 41.6, 65.5, 4 KB 45.4, 71.2.)
+// (With ordinary loads 2.4 KB 28.6, 45.1, 4 KB 45.4, 71.2.)
+// A field is large with 2048 granules and more for a workgroup's strata. (Batches of fewer strata than a workgroup has bring a thread
+// less, and are not slower so: 4096 batches of 3 rows of 4.8 KB 39.6 / 35.3, of 8 rows of 2 KB 39.6 / 36.1, of 8 rows of twice 1 KB 38.7 / 39.3,
+// 2048 of 40 rows of twice 512 bytes 37.8 / 38.3.)
+// But rows of a small buffer come from the caches, many of them several times, and the streaming loads of this copy do not find
+// them there for long; least of all the rows of no whole granules, whose lines two granules share. What the rows held take is compared with
+// a line for odd rows, and for others with one for batches of up to 64 MB and one for larger ones. us, all by the lookup / so, by the MB of the rows held, each behind calls of the other:
+//                                                    10            20            30            45            64            90            128           180           256
+//   1 KB, 1 x 42,000 (43 MB)                    19.8 / 13.7   19.8 / 15.5   19.5 / 17.7   20.1 / 17.7   20.9 / 17.8   21.6 / 18.2
+//   3 KB, 1 x 21,000 (65 MB)                    23.3 / 16.9   23.7 / 19.9   24.5 / 23.9   25.7 / 23.5   27.1 / 23.4   28.3 / 23.7
+//   1 KB, 1 x 80,000 (83 MB)                                  23.2 / 26.6   24.1 / 27.7   25.6 / 26.5   27.4 / 26.1   28.9 / 27.8
+//   4 KB, 1 x 21,000 (86 MB)                                  28.4 / 25.3   29.2 / 30.7   30.6 / 30.4   31.8 / 28.9   33.5 / 29.2
+//   4 KB, 2 x 6200 (51 MB)                      18.7 / 18.1   19.6 / 20.9   20.2 / 19.8   21.2 / 20.8   21.7 / 21.4   22.8 / 22.0
+//   1 KB, 2 x 31,000 (64 MB)                    20.1 / 20.9   21.3 / 23.4   22.5 / 21.8   23.8 / 22.3   24.7 / 23.3   25.3 / 24.0
+//   2.4 KB, 5 x 5000 (60 MB)                    21.9 / 24.6   23.3 / 24.4   24.0 / 24.8   25.0 / 25.5   25.7 / 25.6   26.5 / 25.7
+//   3 KB, 5 x 5000 (77 MB)                      25.3 / 27.9   27.1 / 28.0   28.0 / 29.3   28.7 / 30.0   29.9 / 30.5   30.6 / 30.6   31.6 / 30.7
+//   1.1 KB (odd), 1 x 42,000 (47 MB)            22.5 / 18.3   22.1 / 22.0   21.9 / 24.8   22.8 / 24.5                 24.5 / 23.8   25.3 / 23.9   26.3 / 24.3
+//   1.1 KB (odd), 5 x 5000 (28 MB)              14.9 / 18.2   15.9 / 17.9   16.3 / 17.9   16.8 / 17.9   17.2 / 18.1   17.4 / 18.1   17.9 / 18.1   18.4 / 18.4   18.7 / 18.6
+//   3 KB (odd), 1 x 12,400 (43 MB)              20.3 / 17.8   20.0 / 22.1   19.9 / 23.3   20.4 / 22.5   21.4 / 22.0   22.2 / 22.1   22.7 / 22.5   23.3 / 22.6   24.4 / 23.0
+//   1.1 KB (odd), 5 x 12,500 (69 MB)            23.1 / 30.0   24.2 / 33.4   25.2 / 30.8   26.4 / 30.1   27.7 / 30.1   28.7 / 30.4   29.7 / 30.4   30.8 / 31.0   32.6 / 31.2
+//   3 KB (odd), 5 x 5000 (87 MB)                              32.3 / 38.0   33.4 / 38.9   34.4 / 39.2   35.5 / 40.0   36.4 / 39.8   37.2 / 40.4   40.2 / 40.1   43.5 / 40.5
+//   512 B, 1 x 98,400 (51 MB, 256 strata)       30.1 / 14.8   30.4 / 20.2   30.6 / 20.2   31.2 / 20.7
+//   512 B, 1 x 180,000 (94 MB, 256 strata)                    33.1 / 29.0   33.9 / 28.9   34.4 / 28.3   35.8 / 29.0   37.6 / 31.6
+// (Where nothing else comes between calls, the lookup finds more of 30 to 100 MB in the memory's cache: 60 MB, 1 KB 1 x 42,000 18.6 / 17.6,
+// 2 x 10,500 12.3 / 12.2, 5 x 5000 13.2 / 14.0, 2.4 KB 5 x 5000 23.7 / 25.7, 4 KB 2 x 10,500 33.3 / 30.3; of odd ones 100 MB, 1.1 KB 5 x 5000 15.8 / 18.2.
+// Odd rows in batches of more than 96 MB keep the lookup, whatever the buffer.)
 // ---------------------------------------------------------------------------
 constexpr int kLargeTrip = 4;
-constexpr uint64_t kLargeOdd = 96ull << 20;  // bytes of a batch up to which rows of no whole granules are copied so
-inline bool large_field(const IoTable& t, int f, int strata, uint64_t bytes) {
-    return t.vec_log2[f] == 4 && t.units[f] * (uint64_t)strata >= (uint64_t)(2 * kLargeTrip * kWG) && t.units[f] <= 1u << 14 &&
-           (t.row_bytes[f] % 16 == 0 || bytes <= kLargeOdd);
+constexpr uint64_t kLargeOdd = 96ull << 20;
+inline bool large_field(const IoTable& t, int f, int strata, int64_t nbatch, uint64_t bytes, uint64_t held) {
+    if (t.vec_log2[f] != 4 || t.units[f] * (uint64_t)strata < (uint64_t)(2 * kLargeTrip * kWG) || t.units[f] > 1u << 14) return false;
+    const uint64_t mb = 1 << 20;
+    if (t.row_bytes[f] % 16 != 0) return bytes <= kLargeOdd && held > 144 * mb;
+    return strata == 256 || held > (bytes > 64 * mb ? 56 * mb : nbatch > 1 ? 24 * mb : 0);
 }
 __device__ __forceinline__ uint8_t* uniform_pointer(uint8_t* p) {
     const uint64_t v = (uint64_t)p;

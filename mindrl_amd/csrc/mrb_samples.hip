@@ -21,10 +21,13 @@ hipError_t launch_per_sample_lds(const SampleArgs& a, const IoTable& t, int64_t 
                                  hipStream_t s) {
     const uint32_t ntop = (2u << levels) < 4 ? 4 : (2u << levels);
     const uint64_t bytes = batch_bytes(t);
+    uint64_t held = 0;
+    for (int f = 0; f < t.nfields; ++f) held += t.row_bytes[f];
+    held *= (uint64_t)(a.size >= 0 ? a.size : a.capacity);
     uint32_t large = 0, smaller = rest;
     bool whole = true;
     for (int f = 0; f < t.nfields; ++f) {
-        if (!large_field(t, f, strata, bytes)) continue;
+        if (!large_field(t, f, strata, nbatch, bytes, held)) continue;
         large |= 1u << f;
         smaller -= t.units[f];
         whole = whole && whole_pieces(t, f);
