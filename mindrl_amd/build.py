@@ -25,7 +25,7 @@ HIPCC_FLAGS = [
 ]
 
 
-SOURCES = ["mrb.hip", "mrb_push_many.hip", "mrb_range.hip", "mrb_range_one.hip", "mrb_returns.hip", "mrb_sample_lanes.hip", "mrb_samples.hip", "mrb_samples_large.hip", "mrb_short.hip", "mrb_silent.hip"]
+SOURCES = ["mrb.hip", "mrb_push_many.hip", "mrb_range.hip", "mrb_range_one.hip", "mrb_returns.hip", "mrb_returns_streamed.hip", "mrb_sample_lanes.hip", "mrb_samples.hip", "mrb_samples_large.hip", "mrb_short.hip", "mrb_silent.hip"]
 
 
 def _native_commands(tmp, obj):

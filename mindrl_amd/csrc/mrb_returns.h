@@ -51,7 +51,9 @@ namespace mrb {
 // A single group shares no line, and who reads its results next finds them in the L2 they went through only where they may stay: as
 // non-temporal ones. us, non-temporal / through, alone and with the maximum over the steps behind it: [20, 1] 3.14 / 3.33, 5.9 / 6.3,
 // [64, 8] 3.01 / 3.04, 10.7 / 13.3, [128, 8] 3.51 / 3.56, 15.5 / 22.0, [1000, 16] 11.2 / 11.1, 17.6 / 18.8; of several groups [20, 17] 3.14 / 2.92, 7.3 / 6.8,
-// [128, 17] 3.94 / 3.55, 20.3 / 15.4, [128, 128] 3.63 / 3.66, 12.5 / 11.1, [1000, 100] 11.9 / 11.5, 36.1 / 29.5.
+// [128, 17] 3.94 / 3.55, 20.3 / 15.4, [128, 128] 3.63 / 3.66, 12.5 / 11.1, [1000, 100] 11.9 / 11.5, 36.1 / 29.5. (2048 columns are where such a
+// reader loses, [300, 2048] 20.0 / 26.4 where [300, 1000] gains, 33.8 / 26.0; and of some 4095 columns the gradient does near the line,
+// [1950, 4095] 21.3 / 22.3.)
 // kCols is small so that a few thousand columns spread over all
 // compute units, several workgroups to each when there are more. The pad of four floats puts the sixteen columns'
 // 16-byte reads into different banks, and the movers' scalar writes likewise.
@@ -68,13 +70,15 @@ constexpr int kDrChunk = 64;  // steps
 constexpr int kDrAhead = 3;   // chunks on their way from memory at any time
 constexpr int kDrBuffers = 3;
 constexpr int kDrPitch = kDrChunk + 4;
-constexpr int64_t kDrThrough = 8 << 20;  // results of several groups up to which they are stored through the L2 (sixteen and thirty-two columns)
+constexpr int64_t kDrThrough = 8 << 20;
+inline bool returns_through(int64_t timesteps, int64_t cols, int group) { return group < 64 && cols > group && timesteps * cols <= kDrThrough; }
 
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));      // four floats at any float's address
 typedef uint32_t u32_u __attribute__((aligned(1)));                         // four flags at any address
 #define MRB_GLOBAL __attribute__((address_space(1)))
 
-template <bool kBack, bool kQuad, int kCols, int kMovers>
+// kThrough: the results are stored through the L2 (a kernel of its own: with both in one, a call of few columns took 1 to 3 % longer).
+template <bool kBack, bool kQuad, int kCols, int kMovers, bool kThrough>
 __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
     const float* __restrict__ x, const uint8_t* __restrict__ done, float* __restrict__ end_value, float* __restrict__ out,
     int64_t timesteps, int64_t batch, int64_t inner, float gamma) {
@@ -88,7 +92,6 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
     __shared__ float s_x[kDrBuffers][kCols][kDrPitch];  // a step's value in, its result out
     __shared__ float s_f[kDrBuffers][kCols][kDrPitch];  // its factor (1 - done) * gamma
     const int64_t cols = batch * inner;
-    const bool through = kCols < 64 && timesteps * cols <= (cols > kCols ? kDrThrough : 0);
     // Workgroups are dealt to the chip's eight dies in turn, and each die has its own L2. Neighbouring column groups
     // share cache lines (a group's flags of a step are kCols bytes), so they go to the SAME die.
     const uint32_t groups = (uint32_t)((cols + kCols - 1) / kCols), per = groups >> 3, more = groups & 7u, die = blockIdx.x & 7u;
@@ -276,8 +279,7 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
         }
         wave_lds_fence();  // (the next chunk goes over what other lanes have read)
     };
-    auto store_as = [&](auto how, int64_t c, const f32x4 (&v)[kPer], auto whole, int last) {
-        constexpr bool kThrough = decltype(how)::value;
+    auto store = [&](int64_t c, const f32x4 (&v)[kPer], auto whole, int last) {
         char* const bo = reinterpret_cast<char*>(out + base_of(c) * cols);
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
@@ -298,10 +300,6 @@ __global__ __launch_bounds__(64 + kMovers) void k_discounted_return_tiled(
                     }
             }
         }
-    };
-    auto store = [&](int64_t c, const f32x4 (&v)[kPer], auto whole, int last) {
-        if (through) store_as(std::true_type{}, c, v, whole, last);  // uniform
-        else store_as(std::false_type{}, c, v, whole, last);
     };
     const int end = last_of(nchunks - 1);  // the last chunk's last step
 #pragma unroll

@@ -1,24 +1,7 @@
-// The instantiations of k_discounted_return_tiled and the rule that chooses among them.
-#include "mrb_returns.h"
-#include "mrb_launch.h"
+// Most instantiations of k_discounted_return_tiled and the rule that chooses among them.
+#include "mrb_returns_launch.h"
 
 namespace mrb {
-
-namespace {
-
-template <bool kQuad, int kCols, int kMovers>
-void launch(bool back, const float* x, const uint8_t* done, float* end_value, float* out, int64_t timesteps, int64_t batch,
-            int64_t inner, float gamma, hipStream_t s) {
-    const dim3 grid((uint32_t)((batch * inner + kCols - 1) / kCols)), threads(64 + kMovers);
-    if (back)
-        launch_kernel((k_discounted_return_tiled<true, kQuad, kCols, kMovers>), grid, threads, 0, s, x, done, end_value, out,
-                      timesteps, batch, inner, gamma);
-    else
-        launch_kernel((k_discounted_return_tiled<false, kQuad, kCols, kMovers>), grid, threads, 0, s, x, done, end_value, out,
-                      timesteps, batch, inner, gamma);
-}
-
-}  // namespace
 
 // Columns per workgroup. Narrow groups spread the recurrence's waves and the memory traffic over more compute units; wide ones read
 // longer pieces of a row, which the memory serves better, and which counts when the call is more than the caches hold. Measured, us for
@@ -31,12 +14,15 @@ hipError_t launch_discounted_return_tiled(bool back, const float* x, const uint8
                                           int64_t timesteps, int64_t batch, int64_t inner, float gamma, hipStream_t s) {
     const int64_t cols = batch * inner;
     const bool quad = inner == 1 && cols >= 4;
-    if (cols <= 4096 || timesteps < 128)
-        (quad ? launch<true, 16, 256> : launch<false, 16, 256>)(back, x, done, end_value, out, timesteps, batch, inner, gamma, s);
-    else if (cols <= 8192)
-        (quad ? launch<true, 32, 256> : launch<false, 32, 512>)(back, x, done, end_value, out, timesteps, batch, inner, gamma, s);
+    const int group = cols <= 4096 || timesteps < 128 ? 16 : cols <= 8192 ? 32 : 64;
+    if (group < 64 && !returns_through(timesteps, cols, group))
+        launch_returns_streamed(group, quad, back, x, done, end_value, out, timesteps, batch, inner, gamma, s);
+    else if (group == 16)
+        (quad ? launch_returns<true, 16, 256, true> : launch_returns<false, 16, 256, true>)(back, x, done, end_value, out, timesteps, batch, inner, gamma, s);
+    else if (group == 32)
+        (quad ? launch_returns<true, 32, 256, true> : launch_returns<false, 32, 512, true>)(back, x, done, end_value, out, timesteps, batch, inner, gamma, s);
     else
-        launch<false, 64, 512>(back, x, done, end_value, out, timesteps, batch, inner, gamma, s);
+        launch_returns<false, 64, 512, false>(back, x, done, end_value, out, timesteps, batch, inner, gamma, s);
     return hipGetLastError();
 }
 

@@ -6,7 +6,7 @@ using namespace mrb;
 
 int wrong = 0;
 
-template <bool kBack, bool kQuad, int kCols, int kMovers>
+template <bool kBack, bool kQuad, int kCols, int kMovers, bool kThrough>
 void check(int64_t timesteps, int64_t batch, int64_t inner) {
     const int64_t cols = batch * inner;
     const float gamma = 0.97f;
@@ -28,7 +28,7 @@ void check(int64_t timesteps, int64_t batch, int64_t inner) {
     g_through = 0;
     for (uint32_t g = 0; g < (uint32_t)((cols + kCols - 1) / kCols); ++g) {
         const bool ended = sim::run(g, 64 + kMovers, [&] {
-            k_discounted_return_tiled<kBack, kQuad, kCols, kMovers>(x.data(), done.data(), end.data(), out.data(), timesteps, batch, inner, gamma);
+            k_discounted_return_tiled<kBack, kQuad, kCols, kMovers, kThrough>(x.data(), done.data(), end.data(), out.data(), timesteps, batch, inner, gamma);
         });
         if (!ended) ++wrong, printf("lanes wait at different places\n");
     }
@@ -36,20 +36,33 @@ void check(int64_t timesteps, int64_t batch, int64_t inner) {
     for (int64_t i = 0; i < timesteps * cols; ++i) differ += memcmp(&out[i], &want[i], 4) != 0;
     for (int64_t c = 0; kBack && c < cols; ++c) differ += memcmp(&end[c], &want_end[c], 4) != 0;
     // (the last group's columns are moved back, so some results are stored twice)
-    const bool through = kCols < 64 && cols > kCols;
-    if (through ? g_through < timesteps * cols : g_through != 0) ++wrong, printf("%lld columns by %d: %lld stored through\n", (long long)cols, kCols, (long long)g_through);
+    if (kThrough ? g_through < timesteps * cols : g_through != 0) ++wrong, printf("%lld columns by %d: %lld stored through\n", (long long)cols, kCols, (long long)g_through);
     if (differ) ++wrong, printf("back %d quad %d columns %d: %lld x %lld x %lld: %lld differ\n", kBack, kQuad, kCols, (long long)timesteps, (long long)batch, (long long)inner, (long long)differ);
 }
 
 template <bool kQuad, int kCols, int kMovers>
 void both(int64_t batch, int64_t inner) {
     for (const int64_t timesteps : {1, 16, 33, 64, 65, 128, 150, 193, 256, 321}) {
-        check<false, kQuad, kCols, kMovers>(timesteps, batch, inner);
-        check<true, kQuad, kCols, kMovers>(timesteps, batch, inner);
+        check<false, kQuad, kCols, kMovers, false>(timesteps, batch, inner);
+        check<true, kQuad, kCols, kMovers, false>(timesteps, batch, inner);
+        if (kCols == 64) continue;
+        check<false, kQuad, kCols, kMovers, kCols != 64>(timesteps, batch, inner);
+        check<true, kQuad, kCols, kMovers, kCols != 64>(timesteps, batch, inner);
     }
 }
 
+// Which calls store their results through the L2.
+void rule(bool want, int64_t timesteps, int64_t cols, int group) {
+    if (returns_through(timesteps, cols, group) != want) ++wrong, printf("%lld x %lld by %d: %d\n", (long long)timesteps, (long long)cols, group, !want);
+}
+
 int main(int argc, char** argv) {
+    for (const int group : {16, 32}) {
+        for (const int64_t timesteps : {1, 20, 2000, 1000000}) rule(false, timesteps, 1, group), rule(false, timesteps, group, group);
+        rule(true, 1, group + 1, group), rule(true, 2000, group + 1, group);
+        rule(true, kDrThrough / 1024, 1024, group), rule(false, kDrThrough / 1024, 1025, group);
+    }
+    rule(false, 1, 65, 64), rule(false, 100, 16384, 64);
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "quads") both<true, 16, 256>(23, 1), both<true, 16, 256>(5, 1);
     else if (what == "columns") both<false, 16, 256>(7, 3), both<false, 16, 256>(3, 1);

@@ -203,7 +203,7 @@ def test_only_the_staging_calls_wait_or_allocate_beyond_the_abi():
     assert "Py_BEGIN_ALLOW_THREADS ready = src.stage(r, stream);" in more_sources()["native.cpp"]
 
 
-@pytest.mark.parametrize("source,count", [("mrb_range.hip", 7), ("mrb_samples.hip", 4), ("mrb_returns.hip", 10)])
+@pytest.mark.parametrize("source,count", [("mrb_range.hip", 7), ("mrb_samples.hip", 4), ("mrb_returns.hip", 10), ("mrb_returns_streamed.hip", 8)])
 def test_kernels_of_the_other_files_use_no_scratch_memory(source, count, tmp_path):
     """As test_kernels_use_no_scratch_memory, for the kernels outside mrb.hip."""
     import subprocess
