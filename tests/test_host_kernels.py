@@ -7,7 +7,7 @@ import subprocess
 import pytest
 
 
-@pytest.mark.parametrize("source,count", [("mrb_range_one.hip", 10), ("mrb_short.hip", 5), ("mrb_push_many.hip", 3)])
+@pytest.mark.parametrize("source,count", [("mrb_range_one.hip", 10), ("mrb_short.hip", 5), ("mrb_push_many.hip", 3), ("mrb_samples_large.hip", 4), ("mrb_silent.hip", 1)])
 def test_kernels_use_no_scratch_memory(source, count, tmp_path):
     from mindrl_amd import build
     out = tmp_path / "kernels.s"
@@ -32,7 +32,7 @@ def test_kernels_use_no_scratch_memory(source, count, tmp_path):
         assert 0 <= lds - (8 * leaves + 12 * (leaves // 256)) <= 1088, (name, lds)
 
 
-@pytest.mark.parametrize("source", ["mrb.hip", "mrb_short.hip", "mrb_returns.hip"])
+@pytest.mark.parametrize("source", ["mrb.hip", "mrb_short.hip", "mrb_returns.hip", "mrb_samples_large.hip"])
 def test_stores_written_in_assembly_keep_their_registers(source, tmp_path):
     """A 16-byte store's registers may be written two wait states behind it, which the compiler does not look after in inline assembly."""
     from mindrl_amd import build
