@@ -873,29 +873,34 @@ constexpr int64_t kElectMax = 1024;
 // Whether an update of few entries goes by runs of leaves in k_range_one, whose workgroups read the priorities with the indices and
 // leave where they have no entry, rather than in k_tree_range. us, k_range_one / k_tree_range:
 //   levels   entries   random         one by one
-//   20       1024       6.9 /  7.3
-//   20       1500       8.0 /  7.7     7.4 /  7.5
-//   20       3000                      9.4 /  9.7
-//   20       4096       9.3 /  8.9    10.8 / 11.3    (the line of 4096 is where these two take turns)
-//   21        512       6.4 /  7.1
-//   21       1024       7.5 /  7.5
-//   22       1024       7.8 /  8.0
+//   20       1024       6.7 /  7.3     6.1 /  7.3
+//   20       1500       7.8 /  7.5     7.5 /  7.7
+//   20       3000       8.5 /  8.2     8.6 /  9.0
+//   20       4096       8.8 /  8.5    10.6 / 11.1    (the line of 4096 is where these two take turns)
+//   21        512       6.4 /  7.2     5.6 /  6.7
+//   21       1024       7.4 /  7.6     6.3 /  7.4
+//   22       1024       7.4 /  7.9     6.7 /  7.9
 // Trees of fewer than 8 levels have no whole tile, those of more than 22 more than 256 runs.
 bool takes_range_one(const Per& b, int64_t n) {
     return b.fused && n <= (b.depth <= 20 ? kOneMostEntries : kElectMax) && b.depth >= 8 && b.depth <= 22;
 }
 
-// Whether an update of more entries goes by runs of leaves (launch_tree_range). us, by stamps and tiles / by runs:
-//   levels   entries
-//   12         8192    10.0 /  9.6
-//   12       16,384    11.4 / 13.8
-//   14       16,384    11.7 / 11.2
-//   14       32,768    12.5 / 16.7
-//   20       16,384    14.4 / 14.1
-//   20       32,768    15.4 / 18.7
-//   23         2048    14.9 / 14.9     (more than a tile above the runs, and many runs without an entry)
-//   24         2048    15.9 / 23.3
-// On 21 levels and more what its entries drive is the other way: see takes_sparse.
+// Whether an update of more entries goes by runs of leaves (launch_tree_range). us, by stamps and tiles / by runs, slots at random; in the
+// order that a sample returns them; one after the other:
+//   levels   entries    random          sample's        one by one
+//   12         8192      9.2 /  9.4                      7.9 /  7.2
+//   12       16,384     10.5 / 13.7                      8.1 /  9.6
+//   14         8192     10.1 /  8.7      9.2 /  6.6      9.2 /  6.7
+//   14       12,000     10.2 / 10.6      9.3 /  7.5      9.2 /  7.7
+//   14       16,384     10.3 / 11.5      9.2 /  8.1      9.3 /  7.8
+//   14       32,768     10.9 / 16.7                      9.2 / 10.6
+//   18       12,000     10.1 / 10.2      9.5 /  8.5      9.1 /  8.6
+//   18       16,384     10.3 / 10.9      9.7 /  9.0      9.3 /  9.3
+//   20         8192     11.4 /  9.6     11.1 /  8.6      9.9 / 11.6
+//   20       16,384     11.9 / 12.2     11.4 / 10.1      9.9 / 13.1
+//   20       32,768     12.9 / 16.9                      9.9 / 15.6
+// (The line of 16,384 is the sample's order's.) Trees of more than 22 levels have more than one tile above the runs. On 21 levels and more
+// what its entries drive is the other way: see takes_sparse.
 bool takes_range(const Per& b, int64_t n) {
     if (!b.fused || b.depth < 12 || b.depth > 22) return false;
     return !takes_range_one(b, n) && n <= (b.depth >= 21 ? 3072 : b.depth == 12 ? 8192 : 16384);
@@ -906,23 +911,27 @@ bool takes_range(const Per& b, int64_t n) {
 // of the tree. us per call, the other way / by entries, slots at random; in the order that a sample returns them; one after the
 // other; half of them and all of them the same:
 //   levels  entries    random         sample's       one by one     half           all
-//   21        3,073     9.2 /  9.6     8.5 /  9.3    10.8 /  8.8    10.0 /  9.2     9.6 /  8.1    by runs
-//   21        4,096     9.9 /  9.7     9.2 /  9.4    12.1 /  9.0    11.5 /  9.6    10.8 /  8.4    by runs
-//   21        8,192    11.8 / 10.4    11.6 /  9.9    12.2 /  9.1    16.2 / 10.9    15.0 /  9.1    by runs
-//   21       16,384    14.9 / 11.5    13.4 / 10.7    18.8 /  9.2    24.5 / 13.4    24.1 / 10.6    by runs
-//   22        3,073    10.1 /  9.8     9.5 /  9.6    11.2 /  8.9    11.1 /  9.3    10.4 /  8.2    by runs
-//   22        8,192    13.1 / 10.4    12.6 / 10.2    12.4 /  9.1    16.3 / 11.6    15.4 /  9.2    by runs
+//   21        2,048     8.1 /  9.3     7.8 /  9.1     9.1 /  8.8     9.1 /  9.3     8.8 /  8.1    by runs
+//   21        3,073     8.7 /  9.5     8.2 /  9.2    10.8 /  8.8    10.4 /  9.4    10.1 /  8.3    by runs
+//   21        4,096     9.3 /  9.6     8.8 /  9.3    11.7 /  9.0    11.8 /  9.6    11.3 /  8.5    by runs
+//   21        8,192    10.3 / 10.0     9.4 /  9.6    15.7 /  8.9    15.1 / 10.8    14.8 /  9.1    by runs
+//   21       16,384    13.6 / 11.0    11.5 / 10.1    18.4 /  9.0    24.1 / 13.0    24.0 / 10.5    by runs
+//   22        2,048     8.6 /  9.3     8.3 /  9.1     9.6 /  8.7     9.2 /  9.0     9.1 /  8.0    by runs
+//   22        3,073     9.3 /  9.5     8.9 /  9.3    11.5 /  9.0    10.4 /  9.4    10.2 /  8.2    by runs
+//   22        8,192    11.8 / 10.0    11.0 /  9.8    16.4 /  9.0    15.8 / 10.9    15.3 /  9.1    by runs
 // and by tiles / by entries, at random, one after the other:
-//   21       32,768    20.7 / 13.5                   10.9 /  9.5
-//   21       65,536    23.4 / 19.7                   11.0 / 11.6    (the line lies in front of what loses in one order)
-//   21      131,072    27.9 / 29.0
-//   22       32,768    29.6 / 13.9
-//   22      131,072    38.7 / 32.0                   14.6 / 13.2
-//   22      200,000    43.3 / 43.0                   15.2 / 16.2
-//   23      131,072      56 / 34;   262,144   66 / 56 and 19.7 / 18.2;   524,288   83 / 95
-//   24      131,072      93 / 36;   262,144  116 / 63 and 27 / 18;       524,288  138 / 156
-//   25      262,144     189 / 110;  524,288  235 / 173
-//   26      524,288     368 / 338 and 75 / 50;   1,048,576   458 / 599;   deeper trees were not measured
+//   21       32,768    17.5 / 13.2                   11.6 /  9.5
+//   21       65,536    20.3 / 16.9                   11.6 / 10.3
+//   21      131,072    24.9 / 23.6                   12.3 / 11.6
+//   22       32,768    26.6 / 13.6                   14.5 /  9.5
+//   22      131,072    35.4 / 25.1                   15.5 / 11.7
+//   22      200,000    39.8 / 34.3                   16.1 / 14.6
+//   23      131,072      49 / 27 and 19.2 / 11.7;   262,144   58 / 44 and 20.6 / 16.3;   524,288   73 / 76 and 23.3 / 24.7
+//   24      131,072      72 / 31 and 26.9 / 12.0;   262,144   90 / 53 and 27.4 / 16.6;   524,288  109 / 94 and 30.3 / 25.1
+//   25      262,144     151 / 73 and 43.8 / 19.7;   524,288  192 / 127 and 46.7 / 30.9;  1,048,576  237 / 220 and 52.3 / 50.1
+//   26      524,288     290 / 240 and 77.6 / 47.8;  1,048,576   372 / 438;   deeper trees were not measured
+// (The lines of 21, 22 and 24 levels lie at half of what the entries could take: they were drawn when an entry's block was ten pieces of
+// lines instead of four.)
 bool takes_sparse(const Per& b, int64_t n) {
     const int share = b.depth == 22 || b.depth == 23 ? 5 : b.depth <= 25 ? 6 : b.depth == 26 ? 7 : 8;
     return b.s_g0 > 0 && n > kElectMax && n <= b.leaves >> share;
@@ -1725,14 +1734,21 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
 //   8-byte rows, 2^24 slots   2048 rows 6.8 / 6.1, 4096 8.6 / 6.1, 16,384 23 / 6.1
 //   153 bytes, 10^6           2048 rows 6.6 / 7.3, 3000 7.4 / 7.4, 4096 8.9 / 7.3, 16,384 22 / 7.9, 65,536 71 / 13.3
 //   521 bytes, 2^20           4096 rows 8.3 / 8.9, 6000 11.8 / 9.5, 16,384 22 / 11.1
-//   3 KB, 2 * 10^5            8192 rows 17.9 / 21.0, 16,384 29.1 / 26.1; 6 KB: 8192 31.6 / 32.0, 16,384 58 / 39.5
+//   (sixteen lanes, or a wave, / LDS-top)   8192 rows       10,240          12,288          14,336          16,384          20,480
+//   2.4 KB, 2 * 10^5                       12.3 / 13.2     15.4 / 14.8     16.3 / 15.6     21.2 / 18.0     22.2 / 18.8     24.3 / 21.9
+//   3 KB                                   13.9 / 13.2     16.7 / 15.8     17.8 / 16.9     22.6 / 19.4     23.7 / 20.7     26.5 / 24.5
+//   3.5 KB in an odd field and others      17.6 / 16.6     21.5 / 20.4     22.4 / 21.1     31.5 / 25.5     32.5 / 26.3     35.6 / 31.3
+//   4 KB                                   16.7 / 15.9     19.7 / 19.1     21.2 / 20.5     28.7 / 24.1     29.8 / 25.5     33.1 / 31.3
+//   6 KB                                   21.8 / 20.4     26.7 / 26.0     30.0 / 27.7     34.4 / 33.0     37.4 / 34.7     45.0 / 41.9
+// (The line of 12,288 was drawn before large fields had a loop of their own; 3 to 6 % from 8192 rows on are left there.)
 // and 16 / 32 / 64 / 256 strata to a workgroup: 153 bytes, 16,384 rows 8.5 / 7.9 / 8.7 / 16.1, 65,536 25 / 17 / 13.3 /
-// 16.7, 262,144 84 / 51 / 38 / 31; 521 bytes, 8192 rows 9.6 / 10.7 / 14.0 / 34.5, 32,768 21 / 13.8 / 16.8 / 36; 3 KB,
-// 65,536 rows 99 / 96 / 91 / 201.
+// 16.7, 262,144 84 / 51 / 38 / 31; 521 bytes, 8192 rows 9.6 / 10.7 / 14.0 / 34.5, 32,768 21 / 13.8 / 16.8 / 36; 1 KB, 20,480 rows 13.0 / 12.5 / 13.0 /
+// 21.9, 131,072 70 / 50 / 46 / 43; 3 KB, 12,288 rows 16.9 / 17.6 / 20.4 / 51, 32,768 38.0 / 34.8 / 34.5 / 58, 65,536 67.5 / 64.8 / 62.6 / 69.6.
 // A workgroup has the strata of one batch only, so batches of a few rows leave most of it idle while it stages the top all
 // the same (batches x rows of one): 8-byte rows, 10^6 slots 4096 x 1 6.6 / 20, 4096 x 2 11.0 / 20.6, 2048 x 4 10.9 / 12.1,
-// 2048 x 6 14.6 / 9.9, 1024 x 8 10.8 / 6.4; 521 bytes 2048 x 4 11.0 / 13.8, 4096 x 5 26 / 22; 3 KB 4096 x 3 21 / 30, 4096 x 6
-// 36 / 43, 2048 x 8 26 / 26. (A row above 4 KB takes a whole workgroup there: 6 KB 4096 x 3 46 / 43.)
+// 2048 x 6 14.6 / 9.9, 1024 x 8 10.8 / 6.4. (By sixteen lanes rows of 521 bytes and more lose nothing to small batches: 521 bytes
+// 2048 x 4 6.3 / 12.7, 4096 x 5 13.0 / 22.6, 3 KB 4096 x 3 18.1 / 30.1, 4096 x 6 31.2 / 39.3, 2048 x 8 24.0 / 25.7, 6 KB 4096 x 3 30.4 / 40.8, 2048 x 8
+// 38.1 / 39.0. The fewest rows of a batch were drawn before there were these, and let 4096 x 5 and the rows of 6 KB through.)
 // `lanes`: whether sixteen lanes to a stratum could take it (takes_lanes), which are the better ones longer than a wave is. us,
 // LDS-top / lanes:
 //   row        slots       8192 rows      10,240        12,288        14,336        16,384        18,000        20,480
@@ -1746,7 +1762,6 @@ int mrb_per_update_push(int64_t h, const int64_t* indices, const float* prioriti
 //   521        4 * 10^6     9.2 / 6.0     9.8 / 7.3    10.2 / 7.7    10.7 / 9.0    10.9 / 9.2    11.6 / 11.3   11.8 / 11.8
 //   899        2 * 10^5                                 9.8 / 9.5                  10.8 / 14.2
 //   1 KB       2 * 10^5                                18.9 / 10.9 (a wave's)      12.4 / 14.2
-//   2.4 KB     2 * 10^5                                                            21.5 / 22.9
 // (Of rows with nothing but scalars the line, 14,336, is right for some trees and 5 % off for others.)
 static bool takes_lds(int64_t nbatch, int64_t batch, uint64_t rest, bool lanes) {
     const int64_t rows = nbatch * batch, fewest = rest <= 64 ? 5 : rest <= 256 ? 8 : 1;

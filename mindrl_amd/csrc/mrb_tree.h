@@ -16,7 +16,7 @@ constexpr int kBlockNodes = 256;  // nodes of a tile (a float4 per lane of a wav
 // takes a tile's leaves and goes on from its root, and who walks up from a leaf takes the leaves around it in the trip that brings the siblings
 // (push_one_levels, tree_paths_body: a push of one row with its priority on 2^20 leaves 2.6 -> 2.35 us, 64 entries on 2^23 10.2 -> 8.0). An export
 // writes them first (k_tree_silent). They are
-// 448 of the 511 nodes above a tile of 256 leaves, and 14 of the 16 above a block of 16 - six of the ten pieces of lines that an entry's
+// 224 of the 255 nodes above a tile of 256 leaves, and 14 of the 15 above a block of 16 - six of the ten pieces of lines that an entry's
 // block costs k_tree_sparse. us per update, all levels / without these:
 //   entries   levels   random         ascending            entries   levels   random, ascending in turn
 //    65,536   24       24.6 / 19.5    22.8 / 18.4           2048     21        8.4 / 7.8
