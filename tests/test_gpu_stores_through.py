@@ -22,7 +22,7 @@ ROWS = {  # (the second field: a slot number)
 
 def same_rows(out, stored, slots):
     for o, s in zip(out, stored):
-        want = s.reshape(s.shape[0], -1)[slots.reshape(-1)].reshape(o.shape)
+        want = s.reshape(s.shape[0], -1)[slots.reshape(-1).clamp(max=s.shape[0] - 1)].reshape(o.shape)  # (as the rows are: a number past them is no index)
         assert torch.equal(o.contiguous().view(torch.uint8), want.contiguous().view(torch.uint8))
 
 
