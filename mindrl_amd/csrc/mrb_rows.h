@@ -435,8 +435,8 @@ using g16 = MRB_GLOBAL granule16_u;
 //   gather, 2432 (k_rows_gather_rows)                                                               137 / 128       176 / 165       346 / 323
 //   gather, 2400                                                                                    153 / 145       183 / 194       358 / 395
 // So such batches are stored so up to 160 MB, others without an end (measured up to 1.8 GB: sample, 28,224 bytes 690 / 659).
-// Not stored so are single rows, rows of few granules, and those of k_per_sample_rows, of k_per_sample_lds and of k_per_sample_lanes
-// (whose lanes store pieces of many rows at once and are slower so at every size: 7.5 KB 32.2 / 35.8 with 64 MB).
+// Not stored so is what k_rows_gather, k_short_gather, k_per_sample_rows, k_per_sample_lds and k_per_sample_lanes copy (the last one's lanes store
+// pieces of many rows at once and are slower so at every size: 7.5 KB 32.2 / 35.8 with 64 MB).
 template <bool kThrough>
 __device__ __forceinline__ void store_granule(g16* to, granule_t v) {
     if (kThrough) store_through((void*)to, v);
